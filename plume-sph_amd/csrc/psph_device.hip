@@ -5,15 +5,15 @@
 // grid whose edge covers the largest kernel support).  Every step:
 //   1. cell keys -> radix sort (key, index) -> gather every field (neighbours
 //      are then contiguous: cell rows along x are contiguous index ranges);
-//   2. targets (bc 100/99) are compacted and cut into "chunks" of <= 64
-//      consecutive targets inside one (y,z) cell row;
-//   3. pair passes: one 64-lane wavefront per chunk.  The chunk's candidate
-//      range for each neighbouring (y,z) row is one contiguous slice; it is
-//      staged 64 candidates at a time into LDS with coalesced loads (derived
-//      per-candidate terms such as 1/rho and p/rho^2 are computed once, by the
-//      staging lane), then every lane walks the tile with broadcast LDS reads.
-//      No list is materialised; the reference's list membership rule is
-//      evaluated per pair (same bucket, or |dx| <= 4.25 h_i per axis).
+//   2. targets (bc 100/99) are compacted and cut into "chunks" of <= 32
+//      consecutive targets of a cell and "groups" of 8;
+//   3. pair passes: one 64-lane wavefront per group, 8 targets x 8 streams of
+//      candidates.  Per step and group, every tile (64 consecutive particles)
+//      that can hold a pair gets a 64-bit mask of the particles that can be
+//      one; a pass stages each such tile in LDS and evaluates the masked
+//      particles, re-testing its own exact kernel box.  The reference's list
+//      membership rule is evaluated per pair (same bucket, or |dx| <= 4.25 h_i
+//      per axis) where the kernel box can reach past it.
 // No MFMA: there is no dense contraction.  Reductions are deterministic
 // (min/max via integer atomics on positive doubles; sums via fixed-order
 // block partials).
@@ -220,7 +220,8 @@ __global__ void k_tile_counts(uint32_t ncells, const uint32_t *cs, uint32_t *tcn
   tcnt[c] = c == ncells ? 0u : (cs[c + 1] - cs[c] + kWave - 1) / kWave;
 }
 
-// Bounding box of every tile, rounded outwards to float: [lo, hi] per tile.
+// Bounding box of every tile, rounded outwards to float: [lo, hi] per tile, and
+// in the w components the bits of its first particle and its particle count.
 // One wavefront per tile; the tile's cell is found by bisection of toff.
 __global__ __launch_bounds__(kWave) void k_tile_boxes(uint32_t ncells, const uint32_t *cs, const uint32_t *toff,
                                                       const double *x, const double *y, const double *z,
@@ -239,8 +240,9 @@ __global__ __launch_bounds__(kWave) void k_tile_boxes(uint32_t ncells, const uin
   const double ax = wave_min(px), ay = wave_min(py), az = wave_min(pz);
   const double bx = wave_max(px), by = wave_max(py), bz = wave_max(pz);
   if (threadIdx.x == 0) {
-    tbox[2 * t] = make_float4(__double2float_rd(ax), __double2float_rd(ay), __double2float_rd(az), 0.f);
-    tbox[2 * t + 1] = make_float4(__double2float_ru(bx), __double2float_ru(by), __double2float_ru(bz), 0.f);
+    tbox[2 * t] = make_float4(__double2float_rd(ax), __double2float_rd(ay), __double2float_rd(az), __uint_as_float(base));
+    tbox[2 * t + 1] = make_float4(__double2float_ru(bx), __double2float_ru(by), __double2float_ru(bz),
+                                  __uint_as_float(end - base));
   }
 }
 
@@ -530,24 +532,50 @@ __global__ __launch_bounds__(kWave) void k_pairs(PairCommon pc, typename P::Args
 }
 
 // ---------------------------------------------------------------------------
-// Visit lists.  The RHS, density and filter passes of a step see the same
-// positions, smoothing lengths and list-time data, so the exact candidate
-// scan is done once per step: for every chunk, the tiles that meet its grown
-// box and hold a pair of any of the three passes, each with one 32-bit hit
-// mask per lane (bit b <-> candidate sub + b kSub of the lane's target).  The
-// mask is a superset: list membership and in_support are exact, the kernel
-// box is widened to cut * max(h_ij, h_i) (the union of the three passes'
-// boxes) with a relative margin of 1e-12; each pass re-tests its own exact box
-// and masks on the set bits only.
+// Group passes.  The RHS, density and filter passes take their targets in
+// groups of kGroup consecutive targets of a cell, one wavefront per group.  For
+// every group and tile that can hold a pair of it, a 64-bit mask made once per
+// step says which of the tile's particles can be a pair of one of the group's
+// targets in any of the passes.  A pass stages the tile in LDS, queues the
+// masked particles, and evaluates kStreams of them at a time against all
+// kGroup targets: lane = target + kGroup * stream, so a lane keeps its target
+// and its partial sums in registers and reads a particle's record from LDS, and
+// each pair re-tests the pass's exact kernel box.
+//
+// Why 8 x 8: the larger the group, the fewer staged tiles a target costs, but
+// the fewer of the queued particles are pairs of a given target.  On the
+// lattice after an adaptation (3 h = 4.5 spacings) 55-62 % of the evaluated
+// lanes are pairs with 8 targets, 65-69 % with 4, 46-54 % with 16; walking bit
+// masks of 32 targets x 2 lanes, where a wave ran as long as its fullest lane,
+// had 41 %.
+// Measured and not kept: a record per lane held against 4 targets in turn, the
+// records gathered from the caches (65-76 cycles of the return path per 16-byte
+// load, which kept it busy 90 % of the density and filter passes) or from
+// windows of tiles that 4 or 8 waves stage together (60 % of the wave time went
+// into the windows' barriers); the next tile through registers while one is
+// worked on (density and filter 7.5 -> 25 ms at 4M).
+// Against the masks of 32 targets x 2 lanes, us per launch (RHS, density, filter,
+// masks): 1M FP64 6755, 3231, 2733, 560 (before: 8257, 3894, 3049, 992); 4M
+// FP32-exp 15446, 7663, 7451, 1933 (18057, 8047, 6634, 3843); 1.7k FP64 in 65k
+// particles, where 54 waves of 32 targets left the chip idle, 117, 80, 76, 22
+// (508, 299, 273, 151).
 // ---------------------------------------------------------------------------
-static_assert(kWave / kSub <= 32, "visit masks hold one bit per candidate of a lane's share");
+constexpr int kGroup = 8;                      // targets of a group
+constexpr int kStreams = kWave / kGroup;       // particles evaluated at a time
+constexpr int kGroupsPerChunk = kChunk / kGroup;
 
-struct VisitList {
-  const uint32_t *off;      // first visit of each chunk
-  const uint32_t *num;      // visits written for each chunk
-  const uint2 *ent;         // (first particle, particle count) of the visited tile
-  const uint32_t *mask;     // per visit, kWave lane masks
+// Positions (x, y) and (z, h / 2) of every particle.
+struct Geom {
+  const double2 *xy, *zh;
 };
+
+__global__ void k_geom(uint32_t n, const double *x, const double *y, const double *z, const double *h, double2 *xy,
+                       double2 *zh) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  xy[i] = make_double2(x[i], y[i]);
+  zh[i] = make_double2(z[i], 0.5 * h[i]);
+}
 
 // tiles that meet each chunk's grown box (an upper bound on its visits);
 // one wavefront per chunk, chunk = blockIdx.x, zero past the last chunk; the
@@ -567,57 +595,6 @@ __device__ inline uint32_t count_meeting_tiles(const Traversal &tr, const ChunkB
   return cnt;
 }
 
-// The chunk's grown box for the visit lists: per target the widest kernel
-// box of the three passes, cutx max((h_i + h_max) / 2, h_i), with a relative
-// margin of 1e-9 (the traversal's reach bounds it with h_i = h_max).
-__device__ inline ChunkBox chunk_pass_box(const Traversal &tr, const double *p, double h, double cutx,
-                                          double h_max) {
-  ChunkBox b;
-  const int nn[3] = {tr.g.nx, tr.g.ny, tr.g.nz};
-  const double r = cutx * fmax(0.5 * h + 0.5 * h_max, h) * (1 + 1e-9);
-  for (int d = 0; d < 3; d++) {
-    const double lo = wave_min(p[d] - r), hi = wave_max(p[d] + r);
-    b.lo[d] = __double2float_rd(lo);
-    b.hi[d] = __double2float_ru(hi);
-    if (tr.g.inv_e > 0) {
-      b.c0[d] = cell_of(lo, tr.g.lo[d], tr.g.inv_e, nn[d]);
-      b.c1[d] = cell_of(hi, tr.g.lo[d], tr.g.inv_e, nn[d]);
-    } else {
-      b.c0[d] = b.c1[d] = 0;
-    }
-  }
-  return b;
-}
-
-__global__ __launch_bounds__(kWave) void k_visit_count(PairCommon pc, const double *h, double cutx, double h_max,
-                                                       uint32_t *vcount) {
-  const uint32_t chunk = blockIdx.x;
-  const uint32_t nch = *pc.nchunks;
-  if (chunk >= nch) {
-    if (threadIdx.x == 0) vcount[chunk] = 0;
-    return;
-  }
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const uint32_t slot = (uint32_t)threadIdx.x / kSub;
-  const uint32_t i = pc.targets[cf + (slot < cc ? slot : 0)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const ChunkBox box = chunk_pass_box(pc.tr, xi, h[i], cutx, h_max);
-  const uint32_t cnt = count_meeting_tiles(pc.tr, box);
-  if (threadIdx.x == 0) vcount[chunk] = cnt;
-}
-
-// The scan is transposed: lane l holds candidate c(l) = 2 (l mod 32) + l / 32
-// of the tile (so the ballot of a test over the 64 lanes is, in its low and
-// high halves, exactly the masks of a target's sub-lanes 0 and 1), and the
-// wave loops over the chunk's targets.  A target is skipped for a tile when
-// its widened box misses the tile's box (one vector test for all 32 targets,
-// then a scalar loop over the survivors), which drops about half of the
-// (target, tile) combinations of a chunk's grown box.
-struct VisitTgt {
-  double x, y, z, chh;       // position, cutx h / 2
-  double ch, lf, supp, wide; // cutx h, list box, in_support box, widest union box
-};
-
 // m &= ~(1 << b) for a wave-uniform 64-bit mask in scalar registers: one
 // s_bitset0_b64 (the and-not of a shifted one takes two scalar instructions)
 __device__ inline void clear_bit_u(uint64_t &m, uint32_t b) {
@@ -633,189 +610,410 @@ __device__ inline void set_lane(uint32_t &v, uint32_t value, uint32_t lane) {
   asm volatile("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(v) : "s"(value), "s"(lane) : "m0");
 }
 
-// FAST: for every target of the chunk the widened box lies inside both its
-// list box (4.25 h at list time) and its in_support box (CUTOFF2 h), and is
-// narrower than a bucket (so it reaches the adjacent buckets only): those
-// tests cannot fail for a candidate inside the widened box.
-template <int D>
-__global__ __launch_bounds__(kWave) void k_visit_masks(PairCommon pc, const double *h, double cutoff2, double cutx,
-                                                       double h_max, const uint32_t *voff, uint32_t *vnum,
-                                                       uint2 *vent, uint32_t *vmask) {
-  static_assert(kSub == 2, "the transposed scan maps the ballot halves onto two sub-lanes");
-  __shared__ VisitTgt tg[kChunk];
-  __shared__ uint32_t trb[kChunk];
-  const uint32_t nch = *pc.nchunks;
-  const uint32_t per = (nch + kXcds - 1) / kXcds;
-  const uint32_t local = blockIdx.x / kXcds;
-  if (local >= per) return;
-  const uint32_t chunk = (blockIdx.x % kXcds) * per + local;
-  if (chunk >= nch) return;
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const int lane = threadIdx.x;
-  // lanes 0..cc-1 own one target each: its record in LDS, its float box in registers
-  const bool owner = (uint32_t)lane < cc;
-  const uint32_t i = pc.targets[cf + (owner ? (uint32_t)lane : 0u)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const double hi = h[i], hh_i = 0.5 * hi;
-  const double lf_i = pc.list_factor * pc.h_list[i], supp_i = cutoff2 * hi;
-  const double widest = cutx * fmax(hh_i + 0.5 * h_max, hi);
-  if (owner) {
-    tg[lane] = VisitTgt{xi[0], xi[1], xi[2], cutx * hh_i, cutx * hi, lf_i, supp_i, widest};
-    trb[lane] = pc.refb[i];
-  }
-  float blo[3], bhi[3];
-  for (int d = 0; d < 3; d++) {
-    blo[d] = D == 3 || d == 0 ? __double2float_rd(xi[d] - widest) : -INFINITY;
-    bhi[d] = D == 3 || d == 0 ? __double2float_ru(xi[d] + widest) : INFINITY;
-  }
-  const bool fast = __all(!owner || (widest <= supp_i &&
-                                     (pc.list_all != 0 || (widest <= lf_i && widest * (1 + 1e-12) < pc.del))));
-  // the chunk's grown box (same as the passes': every lane's target counts)
-  const uint32_t slot = (uint32_t)lane / kSub;
-  const uint32_t ib = pc.targets[cf + (slot < cc ? slot : 0u)];
-  const double xb[3] = {pc.x[ib], pc.y[ib], pc.z[ib]};
-  const ChunkBox box = chunk_pass_box(pc.tr, xb, h[ib], cutx, h_max);
-  __syncthreads();
-  const GridDesc &g = pc.tr.g;
-  const uint32_t cq = 2u * ((uint32_t)lane & 31u) + ((uint32_t)lane >> 5);   // this lane's candidate
-  const uint32_t w0 = voff[chunk];
-  uint32_t w = w0;
-  for (int cz = box.c0[2]; cz <= box.c1[2]; cz++)
-    for (int cy = box.c0[1]; cy <= box.c1[1]; cy++)
-      for (int cx = box.c0[0]; cx <= box.c1[0]; cx++) {
-        const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx + cx;
-        const uint32_t lo = pc.tr.cs[cell], hi_ = pc.tr.cs[cell + 1];
-        uint32_t tl = pc.tr.toff[cell];
-        for (uint32_t base = lo; base < hi_; base += kWave, tl++) {
-          if (!tile_meets(box, pc.tr.tbox, tl)) continue;
-          const uint32_t cnt = min((uint32_t)kWave, hi_ - base);
-          // targets whose widened box meets the tile's box
-          const float4 tlo = pc.tr.tbox[2 * tl], thi = pc.tr.tbox[2 * tl + 1];
-          bool meets = owner && !(tlo.x > bhi[0] || thi.x < blo[0]);
-          if (D == 3) meets = meets && !(tlo.y > bhi[1] || thi.y < blo[1] || tlo.z > bhi[2] || thi.z < blo[2]);
-          uint64_t tm = __ballot(meets);
-          if (!tm) continue;
-          const bool valid = cq < cnt;
-          const uint32_t j = base + (valid ? cq : 0u);
-          const double cxp = valid ? pc.x[j] : kFar;
-          const double cyp = valid ? pc.y[j] : kFar;
-          const double czp = valid ? pc.z[j] : kFar;
-          const double chh = valid ? cutx * (0.5 * h[j]) : 0.0;
-          const uint32_t crb = valid ? pc.refb[j] : ~0u;
-          uint32_t mask = 0;
-          // the same loop with and without the list and support tests (the
-          // wave-uniform choice taken outside it)
-          auto scan = [&](auto fast_c) {
-            while (tm) {
-              const uint32_t t = (uint32_t)__builtin_ctzll(tm);
-              clear_bit_u(tm, t);
-              const VisitTgt T = tg[t];
-              double amax = fabs(T.x - cxp);
-              if (D == 3) amax = fmax(amax, fmax(fabs(T.y - cyp), fabs(T.z - czp)));
-              // amax <= cutx max(h_ij, h_t), with cutx h_ij ~ cutx hh_t + cutx hh_j
-              // (the 1e-12 margin of cutx covers the rounding of the split sum,
-              // taken as amax - cutx hh_j <= cutx hh_t)
-              uint64_t bal;
-              if constexpr (decltype(fast_c)::value) {
-                // one ballot per compare: each compare writes its lane mask directly
-                bal = __ballot(amax - chh <= T.chh) | __ballot(amax <= T.ch);
-              } else {
-                bool in = (amax - chh <= T.chh) | (amax <= T.ch);
-                in &= (pc.list_all != 0) | (crb == trb[t]) |
-                      ((amax <= T.lf) & ((pc.list_adj == 0) || refb_adjacent(crb, trb[t])));
-                in &= amax <= T.supp;
-                bal = __ballot(in);
-              }
-              // lanes 2t and 2t+1 (target t's sub-lanes) take the two halves:
-              // t and the ballot are wave-uniform (scalar registers), so each
-              // half is written into its one lane
-              set_lane(mask, (uint32_t)bal, 2u * t);
-              set_lane(mask, (uint32_t)(bal >> 32), 2u * t + 1u);
-            }
-          };
-          if (fast) scan(std::true_type{}); else scan(std::false_type{});
-          if (__ballot(mask != 0)) {
-            if (lane == 0) vent[w] = make_uint2(base, cnt);
-            __builtin_nontemporal_store(mask, vmask + (size_t)w * kWave + lane);
-            w++;
-          }
-        }
-      }
-  if (lane == 0) vnum[chunk] = w - w0;
+__device__ inline uint32_t lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
 
-// A pair pass over the visit lists: stage each visited tile, test the pass's
-// exact kernel box and masks on the set bits, and run the pair arithmetic.
-struct NoArith {};
-struct ArithPos { double x[kWave], y[kWave], z[kWave]; };
+// v of lane ^ (the lanes of a row of 16), by DPP moves
+template <int CTRL>
+__device__ inline double row_move(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+// v_permlane32_swap exchanges a's upper half with b's lower, v_permlane16_swap
+// a's odd rows with b's even ones: the sum of the two results then holds a's
+// partial sums on one half (the even rows) and b's on the other.
+template <int ROWS>
+__device__ inline double swap_add(double a, double b) {
+  const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+  auto lo = ROWS == 2 ? __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false)
+                      : __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+  auto hi = ROWS == 2 ? __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false)
+                      : __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+  return __longlong_as_double((long long)((uint64_t)hi[0] << 32 | lo[0])) +
+         __longlong_as_double((long long)((uint64_t)hi[1] << 32 | lo[1]));
+}
+// The tiles a group visits, with a 64-bit mask of the particles that can be a
+// pair of one of its targets in any of the passes.
+struct GroupLists {
+  uint4 *visit;             // x, y: first particle and count of the tile; z, w: the mask
+  uint32_t *off, *num;      // per group: first visit, visits
+  uint32_t *fast;           // per group: list membership and in_support cannot fail for a masked
+                            // particle inside a pass's kernel box
+  uint32_t *cursor;         // visits handed out
+  uint32_t cap;             // visits that visit holds
+};
 
-// FROZEN (a frozen replay): the predicates read pc.x (the recorded run's
-// positions) and the pair arithmetic pc.ax; otherwise both are pc.x.
-template <int D, class P, bool FROZEN = false>
-__global__ __launch_bounds__(kWave) void k_pairs_v(PairCommon pc, VisitList vl, typename P::Args a) {
-  __shared__ double sx[kWave], sy[kWave], sz[kWave];
-  __shared__ uint8_t sgh[kWave];   // boundary ghost (bc 1, 2), one byte each
-  __shared__ typename P::Tile tile;
-  __shared__ typename std::conditional<FROZEN, ArithPos, NoArith>::type sa;
-  const uint32_t nch = *pc.nchunks;
-  const uint32_t per = (nch + kXcds - 1) / kXcds;
+struct GroupCommon {
+  Geom g;
+  GroupLists gl;
+  double cutx;               // cut with a relative margin of 1e-12
+  double h_max;
+};
+
+// The group of this workgroup, its target for this lane (lane % kGroup; past
+// the last target the lanes repeat it) and the number of its targets; 0 for none.
+__device__ inline uint32_t my_group(const PairCommon &pc, uint32_t &gid, uint32_t &i) {
+  const uint32_t ngr = *pc.nchunks * kGroupsPerChunk;
+  const uint32_t per = (ngr + kXcds - 1) / kXcds;
+  const uint32_t local = blockIdx.x / kXcds;
+  if (local >= per) return 0;
+  gid = (blockIdx.x % kXcds) * per + local;
+  if (gid >= ngr) return 0;
+  const uint32_t chunk = gid / kGroupsPerChunk, t0 = gid % kGroupsPerChunk * kGroup;
+  const uint32_t cc = pc.ccount[chunk];
+  if (t0 >= cc) return 0;
+  const uint32_t nt = min((uint32_t)kGroup, cc - t0);
+  i = pc.targets[pc.cfirst[chunk] + t0 + min(threadIdx.x % kGroup, nt - 1u)];
+  return nt;
+}
+
+__device__ inline double group_min(double v) {
+  for (int o = 1; o < kGroup; o <<= 1) v = fmin(v, __shfl_xor(v, o));
+  return v;
+}
+__device__ inline double group_max(double v) {
+  for (int o = 1; o < kGroup; o <<= 1) v = fmax(v, __shfl_xor(v, o));
+  return v;
+}
+
+// |x_k - c_k| - b_k <= max(chh + cutx h_j / 2, ch) holds on every axis for each
+// particle j that is a pair of one of the group's targets in any of the passes
+// (b with room for the rounding of c and of the differences).
+struct GroupBox {
+  double c[3], b[3];
+  double chh, ch;            // cutx h / 2 and cutx h of the group's largest h
+  float lo[3], up[3];        // the grown box
+};
+
+// One wavefront per share of a chunk: kGroupsPerChunk / nsplit groups.  The
+// tiles whose box meets a group's grown box are counted to find room for the
+// visits, then their particles are read, once for all the wave's groups, and
+// tested.  A wave that finds no room only counts: the host grows the array and
+// calls again.  A whole chunk per wave reads a tile once for four groups (at 4M
+// the reads of one group per wave ran at 8 TB/s of L2: 6.1 ms against 3.8); a
+// small set of particles has too few chunks to fill the chip and takes a group
+// per wave.
+template <int D>
+__global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommon gc, const double *h, double cutoff2,
+                                                       uint32_t nsplit) {
+  __shared__ GroupBox gb[kGroupsPerChunk];
+  __shared__ uint32_t rowpre[kWave], rowtile[kWave];
+  const uint32_t units = *pc.nchunks * nsplit;
+  const uint32_t per = (units + kXcds - 1) / kXcds;
   const uint32_t local = blockIdx.x / kXcds;
   if (local >= per) return;
-  const uint32_t chunk = (blockIdx.x % kXcds) * per + local;
-  if (chunk >= nch) return;
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
+  const uint32_t unit = (blockIdx.x % kXcds) * per + local;
+  if (unit >= units) return;
+  const uint32_t chunk = unit / nsplit, share = kGroupsPerChunk / nsplit, g0 = unit % nsplit * share;
+  const uint32_t cc = pc.ccount[chunk];
+  if (g0 * kGroup >= cc) return;
+  const uint32_t ng = min(share, (cc - g0 * kGroup + kGroup - 1) / kGroup);
   const int lane = threadIdx.x;
-  const uint32_t slot = (uint32_t)lane / P::kSub, sub = (uint32_t)lane % P::kSub;
-  const bool active = slot < cc;
-  const uint32_t i = pc.targets[cf + (active ? slot : 0)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  double xa[3] = {xi[0], xi[1], xi[2]};
-  if constexpr (FROZEN) { xa[0] = pc.ax[i]; xa[1] = pc.ay[i]; xa[2] = pc.az[i]; }
-  typename P::Tgt t;
-  P::load_target(a, i, t);
-  P::init(tile, lane);
-  __syncthreads();
-  P::begin_pass(a, t, 0);
-  const uint32_t v0 = vl.off[chunk], nv = vl.num[chunk];
-  for (uint32_t v = 0; v < nv; v++) {
-    const uint2 e = vl.ent[v0 + v];
-    const uint32_t base = e.x, cnt = e.y;
-    if ((uint32_t)lane < cnt) {
-      const uint32_t j = base + lane;
-      sx[lane] = pc.x[j]; sy[lane] = pc.y[j]; sz[lane] = pc.z[j];
-      if constexpr (FROZEN) { sa.x[lane] = pc.ax[j]; sa.y[lane] = pc.ay[j]; sa.z[lane] = pc.az[j]; }
-      if (pc.gflag) { const int b = pc.bc[j]; sgh[lane] = b == 1 || b == 2; }
-      P::stage(a, j, tile, lane);
-    }
-    // streamed once per pass: keep it out of the caches that hold the tiles
-    uint32_t mask = __builtin_nontemporal_load(vl.mask + (size_t)(v0 + v) * kWave + lane);
-    __syncthreads();
-    if (active) {
-      while (mask) {
-        const uint32_t b = (uint32_t)__builtin_ctz(mask);
-        mask &= mask - 1;
-        const uint32_t q = sub + b * P::kSub;
-        double dx[3];
-        dx[0] = xi[0] - sx[q];
-        double amax = fabs(dx[0]);
-        if (D == 3) {
-          dx[1] = xi[1] - sy[q]; dx[2] = xi[2] - sz[q];
-          amax = fmax(amax, fmax(fabs(dx[1]), fabs(dx[2])));
-        }
-        if (pc.cut.outside(amax, P::hker(a, t, tile, q)) || !P::extra(a, t, tile, q, base + q, i)) continue;
-        if constexpr (FROZEN) {
-          dx[0] = xa[0] - sa.x[q];
-          if (D == 3) { dx[1] = xa[1] - sa.y[q]; dx[2] = xa[2] - sa.z[q]; }
-        }
-        P::pair(a, t, tile, q, base + q, i, dx, amax);
-        if (pc.gflag && sgh[q]) pc.gflag[base + q] = 1u;
+  // kGroup lanes own a group's targets; past the last target they repeat it
+  const uint32_t i = pc.targets[pc.cfirst[chunk] + min(g0 * kGroup + min((uint32_t)lane, ng * kGroup - 1u), cc - 1u)];
+  const GridDesc &g = pc.tr.g;
+  const int nn[3] = {g.nx, g.ny, g.nz};
+  int c0[3] = {0, 0, 0}, c1[3] = {0, 0, 0};
+  bool fast;
+  {
+    const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
+    const double hi = h[i];
+    const double lf = pc.list_factor * pc.h_list[i], supp = cutoff2 * hi;
+    // fast: the widest kernel box of the passes lies inside the list box and the
+    // in_support box of every target and is narrower than a bucket, so that list
+    // membership and in_support cannot fail for a particle inside it
+    double widest = gc.cutx * fmax(0.5 * hi + 0.5 * gc.h_max, hi);
+    fast = widest <= supp && (pc.list_all != 0 || (widest <= lf && widest * (1 + 1e-12) < pc.del));
+    GroupBox B;
+    const double hg = group_max(hi);
+    widest = gc.cutx * fmax(0.5 * hg + 0.5 * gc.h_max, hg) * (1 + 1e-9);
+    B.chh = gc.cutx * (0.5 * hg);
+    B.ch = gc.cutx * hg;
+    for (int d = 0; d < 3; d++) {
+      const double lo = group_min(xi[d]), up = group_max(xi[d]);
+      B.c[d] = 0.5 * lo + 0.5 * up;
+      B.b[d] = fmax(up - B.c[d], B.c[d] - lo);
+      B.b[d] += 2e-15 * (fabs(B.c[d]) + B.b[d]);
+      B.lo[d] = D == 3 || d == 0 ? __double2float_rd(lo - widest) : -INFINITY;
+      B.up[d] = D == 3 || d == 0 ? __double2float_ru(up + widest) : INFINITY;
+      if (g.inv_e > 0) {
+        // the cells any of the groups reaches
+        c0[d] = __builtin_amdgcn_readfirstlane(cell_of(wave_min((double)B.lo[d]), g.lo[d], g.inv_e, nn[d]));
+        c1[d] = __builtin_amdgcn_readfirstlane(cell_of(wave_max((double)B.up[d]), g.lo[d], g.inv_e, nn[d]));
       }
     }
-    __syncthreads();
+    if (lane % kGroup == 0 && (uint32_t)lane / kGroup < ng) gb[lane / kGroup] = B;
   }
-  if constexpr (P::kSub > 1) P::combine(t);
-  P::end_pass(a, t, 0, i, active);
-  if (active && sub == 0) P::finish(a, t, i, pc.err);
+  const uint64_t fb = __ballot(fast);
+  const int rows_y = c1[1] - c0[1] + 1, nrow = rows_y * (c1[2] - c0[2] + 1);
+  uint32_t off[kGroupsPerChunk] = {}, num[kGroupsPerChunk] = {};
+  for (int write = 0; write < 2; write++) {
+    for (int rb = 0; rb < nrow; rb += kWave) {
+      // the tiles of a row of cells are consecutive: first tile of each row, and
+      // how many tiles the rows before it hold
+      uint32_t first = 0, len = 0;
+      if (rb + lane < nrow) {
+        const int cy = c0[1] + (rb + lane) % rows_y, cz = c0[2] + (rb + lane) / rows_y;
+        const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx;
+        first = pc.tr.toff[cell + c0[0]];
+        len = pc.tr.toff[cell + c1[0] + 1] - first;
+      }
+      uint32_t upto = len;
+      for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t v = __shfl_up(upto, o);
+        if (lane >= o) upto += v;
+      }
+      __syncthreads();
+      rowpre[lane] = upto - len;
+      rowtile[lane] = first;
+      __syncthreads();
+      const uint32_t total = __builtin_amdgcn_readlane(upto, kWave - 1);
+      for (uint32_t kb = 0; kb < total; kb += kWave) {
+        // the lanes test a tile each
+        const uint32_t k = kb + lane;
+        uint32_t meets = 0;
+        float4 tlo = make_float4(0.f, 0.f, 0.f, 0.f), thi = tlo;
+        if (k < total) {
+          uint32_t ra = 0;                          // the last row that starts at or before k
+          for (uint32_t o = kWave / 2; o > 0; o >>= 1)
+            if (rowpre[ra + o] <= k) ra += o;
+          const uint32_t t = rowtile[ra] + (k - rowpre[ra]);
+          tlo = pc.tr.tbox[2 * t];
+          thi = pc.tr.tbox[2 * t + 1];
+          for (uint32_t q = 0; q < ng; q++) {
+            const GroupBox &B = gb[q];
+            const bool out = tlo.x > B.up[0] || thi.x < B.lo[0] || tlo.y > B.up[1] || thi.y < B.lo[1] ||
+                             tlo.z > B.up[2] || thi.z < B.lo[2];
+            meets |= out ? 0u : 1u << q;
+          }
+        }
+        if (!write) {
+#pragma unroll
+          for (uint32_t q = 0; q < kGroupsPerChunk; q++) num[q] += (uint32_t)__popcll(__ballot((meets >> q) & 1u));
+          continue;
+        }
+        uint64_t tm = __ballot(meets != 0);
+        uint32_t mlo[kGroupsPerChunk] = {}, mhi[kGroupsPerChunk] = {};   // this lane's tile's masks
+        while (tm) {
+          const uint32_t l = (uint32_t)__builtin_ctzll(tm);
+          clear_bit_u(tm, l);
+          const uint32_t base = __builtin_amdgcn_readlane(__float_as_uint(tlo.w), l);
+          const uint32_t cnt = __builtin_amdgcn_readlane(__float_as_uint(thi.w), l);
+          const uint32_t gm = __builtin_amdgcn_readlane(meets, l);
+          const uint32_t j = base + min((uint32_t)lane, cnt - 1u);
+          const double2 xy = gc.g.xy[j], zh = gc.g.zh[j];
+          const double chh = gc.cutx * zh.y;
+          const uint64_t valid = cnt < kWave ? (1ull << cnt) - 1 : ~0ull;
+#pragma unroll
+          for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
+            if (!((gm >> q) & 1u)) continue;
+            const GroupBox &B = gb[q];
+            double d = fabs(xy.x - B.c[0]) - B.b[0];
+            if (D == 3) d = fmax(d, fmax(fabs(xy.y - B.c[1]) - B.b[1], fabs(zh.x - B.c[2]) - B.b[2]));
+            const uint64_t in = (__ballot(d - chh <= B.chh) | __ballot(d <= B.ch)) & valid;
+            set_lane(mlo[q], (uint32_t)in, l);
+            set_lane(mhi[q], (uint32_t)(in >> 32), l);
+          }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
+          const uint64_t has = __ballot((mlo[q] | mhi[q]) != 0);
+          if (mlo[q] | mhi[q])
+            gc.gl.visit[(size_t)off[q] + num[q] + lanes_below(has)] =
+                make_uint4(__float_as_uint(tlo.w), __float_as_uint(thi.w), mlo[q], mhi[q]);
+          num[q] += (uint32_t)__popcll(has);
+        }
+      }
+    }
+    if (!write) {
+      uint32_t room = 0, at = 0;
+      for (uint32_t q = 0; q < kGroupsPerChunk; q++) room += num[q];
+      if (lane == 0) at = atomicAdd(gc.gl.cursor, room);
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (at + room > gc.gl.cap || at + room < at) return;
+      for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
+        off[q] = at;
+        at += num[q];
+        num[q] = 0;
+      }
+    }
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
+    const uint32_t gid = chunk * kGroupsPerChunk + g0 + q;
+    if (lane == 0 && q < ng) {
+      gc.gl.off[gid] = off[q];
+      gc.gl.num[gid] = num[q];
+      gc.gl.fast[gid] = ((fb >> (q * kGroup)) & 0xffu) == 0xffu ? 1u : 0u;
+    }
+  }
+}
+
+// 64 lanes' 16 (4) bytes from memory to consecutive LDS places
+template <int BYTES>
+__device__ inline void load_to_lds(const void *from, void *to) {
+  auto *g = (const __attribute__((address_space(1))) uint32_t *)from;
+  auto *l = (__attribute__((address_space(3))) uint32_t *)to;
+  if constexpr (BYTES == 16) __builtin_amdgcn_global_load_lds(g, l, 16, 0, 0);
+  else __builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
+}
+
+// A tile's particles: positions, then the pass's record arrays (NA16 of 16
+// bytes a particle, NA4 of 4).  Place kWave is out of every kernel's reach.
+template <class P>
+struct TileLds {
+  double2 xy[kWave + 1], zh[kWave + 1];
+  float4 a16[P::NA16][kWave + 1];
+  float a4[P::NA4 ? P::NA4 : 1][P::NA4 ? kWave + 1 : 1];
+  __device__ const double2 *d2(int k) const { return (const double2 *)a16[k]; }
+  __device__ const float4 *f4(int k) const { return a16[k]; }
+  __device__ const float *f1(int k) const { return a4[k]; }
+};
+
+template <class T>
+using const_ptr = const __attribute__((address_space(4))) T *;   // read by scalar loads where uniform
+
+// v plus its value kGroup, 2 kGroup, ... lanes on: the sum over the streams, on
+// every lane (order fixed)
+__device__ inline double stream_sum(double v) {
+  static_assert(kGroup == 8, "lane = target + 8 stream");
+  v += row_move<0x128>(v);                        // row_ror 8
+  v = swap_add<1>(v, v);
+  return swap_add<2>(v, v);
+}
+
+// A pair pass over groups.  Each pass supplies: Tgt (the lane's target), Rec
+// (one particle) and load() of it from a staged tile, pack(), which writes the
+// arrays the tiles are loaded from, hker() (h of the kernel-box test),
+// pair_d(), which adds to the target's NACC partial sums, and finish() for the
+// lane that holds a target's totals.
+//
+// Bound by VALU issue.  Whatever is left in the queue after a tile stays in the
+// registers of its streams (nl of them) while the next tile is staged.
+//
+// FROZEN (a frozen replay): the predicates read g's and pc.x (the recorded
+// run's positions) and the pair arithmetic pc.ax; otherwise both are pc.x.
+template <int D, class P, bool FROZEN>
+__global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, GroupCommon gc, typename P::Args a) {
+  __shared__ TileLds<P> st;
+  __shared__ uint8_t queue[2 * kWave];             // places in the tile
+  uint32_t gid, i;
+  const uint32_t nt = my_group(pc, gid, i);
+  if (!nt) return;
+  const int lane = threadIdx.x;
+  const uint32_t stream = (uint32_t)lane / kGroup, slot = (uint32_t)lane % kGroup;
+  typename P::Own own;
+  typename P::Tgt T;
+  P::load_target(a, i, T, own);
+  // a lane without a target of its own meets nothing
+  const double xi[3] = {slot < nt ? pc.x[i] : -kFar, pc.y[i], pc.z[i]};
+  double xa[3] = {0, 0, 0};
+  if constexpr (FROZEN) { xa[0] = pc.ax[i]; xa[1] = pc.ay[i]; xa[2] = pc.az[i]; }
+  if (lane == 0) {
+    st.xy[kWave] = make_double2(kFar, kFar);
+    st.zh[kWave] = make_double2(kFar, 0.0);
+  }
+  double acc[P::NACC];
+#pragma unroll
+  for (int k = 0; k < P::NACC; k++) acc[k] = 0;
+  uint32_t npairs = 0;                             // of all targets (wave-uniform)
+  uint64_t bad = 0;                                // lanes that met an invalid neighbour (wave-uniform)
+  const bool slow = FROZEN || gc.gl.fast[gid] == 0 || pc.gflag != nullptr;
+  const uint32_t nv = __builtin_amdgcn_readfirstlane(gc.gl.num[gid]);
+  const_ptr<uint32_t> vis = (const_ptr<uint32_t>)(uintptr_t)(gc.gl.visit + __builtin_amdgcn_readfirstlane(gc.gl.off[gid]));
+  uint32_t ahead[4] = {0, 0, 0, 0};                // the next visit
+  if (nv)
+    for (int k = 0; k < 4; k++) ahead[k] = vis[k];
+  double2 xy, zh;
+  uint32_t j = 0;
+  typename P::Rec r;
+  uint32_t nq = 0, nl = 0;                         // queued places, streams that hold theirs in registers
+  for (uint32_t v = 0; v <= nv; v++) {
+    uint32_t base = 0;
+    uint64_t m = 0;
+    const uint32_t held = nl;
+    if (v < nv) {
+      base = ahead[0];
+      const uint32_t cnt = ahead[1];
+      m = (uint64_t)ahead[3] << 32 | ahead[2];
+      const_ptr<uint32_t> e = vis + (size_t)min(v + 1, nv - 1) * 4;
+      for (int k = 0; k < 4; k++) ahead[k] = e[k];
+      const uint32_t from = base + min((uint32_t)lane, cnt - 1u);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last tile has been read
+      load_to_lds<16>(gc.g.xy + from, st.xy);
+      load_to_lds<16>(gc.g.zh + from, st.zh);
+#pragma unroll
+      for (int k = 0; k < P::NA16; k++) load_to_lds<16>(a.pk.f4(k) + from, st.a16[k]);
+#pragma unroll
+      for (int k = 0; k < P::NA4; k++) load_to_lds<4>(a.pk.f1(P::NA16 + k) + from, st.a4[k]);
+      if ((m >> lane) & 1) queue[held + lanes_below(m)] = (uint8_t)lane;
+    } else {
+      if (!held) break;
+      // the last block's other streams take the place out of reach
+      m = 0xffu >> held;
+      if ((uint32_t)lane < kStreams - held) queue[held + lane] = (uint8_t)kWave;
+    }
+    nq = held + (uint32_t)__popcll(m);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // tile and queue are there
+    for (uint32_t q = 0; q < nq; q += kStreams) {
+      const uint32_t take = min(nq - q, (uint32_t)kStreams);
+      if (stream >= nl && stream < take) {
+        const uint32_t p = queue[q + stream];
+        xy = st.xy[p];
+        zh = st.zh[p];
+        P::load(st, p, r);
+        j = base + p;
+      }
+      nl = take;
+      if (take < kStreams) break;
+      nl = 0;
+      double dx[3];
+      dx[0] = xi[0] - xy.x;
+      double amax = fabs(dx[0]);
+      if (D == 3) {
+        dx[1] = xi[1] - xy.y; dx[2] = xi[2] - zh.x;
+        amax = fmax(amax, fmax(fabs(dx[1]), fabs(dx[2])));
+      }
+      const double hk = P::hker(T, zh.y);
+      uint64_t in = __ballot(!pc.cut.outside(amax, hk));
+      if (slow) {
+        const bool mine = (in >> lane) & 1;
+        // list membership (neighs.cc:37-211: same bucket or 4.25 h_i box) and in_support
+        const uint32_t rj = mine ? pc.refb[j] : 0u, ri = pc.refb[i];
+        bool ok = mine & ((pc.list_all != 0) | (rj == ri) |
+                          ((amax <= pc.list_factor * pc.h_list[i]) & ((pc.list_adj == 0) || refb_adjacent(rj, ri))));
+        ok &= amax <= a.cutoff2 * a.h[i];
+        if (pc.gflag) {
+          // recorded step: the boundary ghosts (bc 1, 2) met as neighbours
+          const int bj = ok ? pc.bc[j] : 0;
+          ok &= P::counts_ghost(bj);
+          if (ok && (bj == 1 || bj == 2)) pc.gflag[j] = 1u;
+        }
+        if constexpr (FROZEN) {
+          const uint32_t ja = ok ? j : i;
+          dx[0] = xa[0] - pc.ax[ja];
+          if (D == 3) { dx[1] = xa[1] - pc.ay[ja]; dx[2] = xa[2] - pc.az[ja]; }
+        }
+        in = __ballot(ok);
+      }
+      if constexpr (P::kCountPairs) {
+        npairs += (uint32_t)__popcll(in);
+        bad |= in & __ballot(!P::valid(r));
+      }
+      if (__builtin_amdgcn_inverse_ballot_w64(in)) P::template pair_d<D>(a, T, r, hk, dx, amax, acc);
+    }
+  }
+  double sum[P::NACC];
+#pragma unroll
+  for (int k = 0; k < P::NACC; k++) sum[k] = stream_sum(acc[k]);
+  for (int o = 32; o >= kGroup; o >>= 1) bad |= bad >> o;
+  if ((uint32_t)lane < nt) P::finish(a, own, sum, ((bad >> lane) & 1u) != 0, i, pc.err);
+  // pairs of the group's targets, without the targets themselves
+  if constexpr (P::kCountPairs)
+    if (lane == 0 && npairs > nt) atomicAdd(a.pairs, (unsigned long long)(npairs - nt));
 }
 
 // sum of v over the kSub lanes of a target (lanes slot*kSub .. +kSub-1)
@@ -854,12 +1052,21 @@ constexpr double kCutMargin = 1.0 + 1e-12;
 // the pair predicate (phase 1) is FP64 in both, so both forms visit exactly
 // the same pairs; accumulators, integration and the EOS stay FP64.
 // ---------------------------------------------------------------------------
-template <class R> __device__ inline R rexp(R x);
-template <> __device__ inline double rexp<double>(double x) { return exp(x); }
-template <> __device__ inline float rexp<float>(float x) { return __expf(x); }
+// 1 / x in FP64 for normal x and 1 / x: the hardware estimate and two Newton
+// steps whose last rounds once (within a rounding of the quotient).  5
+// instructions; the IEEE division takes 10 and the scaling that the quotients
+// here, far from the ends of the range, do not need.
+__device__ inline double rcp_newton(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
 template <class R> __device__ inline R rrcp(R x);
-template <> __device__ inline double rrcp<double>(double x) { return 1.0 / x; }
+template <> __device__ inline double rrcp<double>(double x) { return rcp_newton(x); }
 template <> __device__ inline float rrcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
+template <class R> __device__ inline R rfma(R a, R b, R c);
+template <> __device__ inline double rfma<double>(double a, double b, double c) { return fma(a, b, c); }
+template <> __device__ inline float rfma<float>(float a, float b, float c) { return fmaf(a, b, c); }
 // |x| as the source modifier of the consuming instruction (x < 0 ? -x : x
 // would cost a compare and a select)
 template <class R> __device__ inline R rabs(R x);
@@ -884,8 +1091,34 @@ __device__ inline double exp_neg_tab(double e, const double *tab) {
   return tab[(int)k] * p;
 }
 
+// exp(-e) in FP64 for e >= 0 without a table (Cody and Waite's reduction: e = -k
+// ln 2 - r with k an integer, |r| <= ln 2 / 2, ln 2 in two parts; then 1 + r +
+// r^2 q(r) with q the degree-9 polynomial through the Chebyshev nodes of the
+// interval, computed for this file in 60-digit arithmetic: truncation 1.7e-17).
+// Measured over 0 <= e <= 27.5: 1.0 ulp at most, 0.30 ulp rms (the table form
+// below: 1.9 and 0.47; the C library's: 0.51 and 0.29).  16 VALU instructions
+// and no LDS.
+__device__ inline double exp_neg(double e) {
+  const double magic = 6755399441055744.0;               // 1.5 * 2^52: kd's low word is k
+  const double kd = fma(e, -1.4426950408889634, magic), k = kd - magic;
+  double r = fma(k, -0.6931471805598903, -e);
+  r = fma(k, -5.497923018708371e-14, r);
+  double p = 2.510038549551032e-08;
+  p = fma(p, r, 2.7620088445409746e-07); p = fma(p, r, 2.7557268459997064e-06);
+  p = fma(p, r, 2.4801521295954376e-05); p = fma(p, r, 0.00019841269863053618);
+  p = fma(p, r, 0.0013888888917213717); p = fma(p, r, 0.008333333333330062);
+  p = fma(p, r, 0.04166666666662413); p = fma(p, r, 0.16666666666666669);
+  p = fma(p, r, 0.5); p = fma(p, r, 1.0); p = fma(p, r, 1.0);
+  return __builtin_amdgcn_ldexp(p, (int)(uint32_t)__double_as_longlong(kd));
+}
+
+// exp(-e), e >= 0, in the pair arithmetic's type
+template <class R> __device__ inline R rexp_neg(R e);
+template <> __device__ inline double rexp_neg<double>(double e) { return exp_neg(e); }
+template <> __device__ inline float rexp_neg<float>(float e) { return __expf(-e); }
+
 // The exponential of the FP32-pair forms' FP64 weights.  FX false
-// (PSPH_FP32_PAIR): exp_neg_tab, FP64 throughout.  FX true (PSPH_FP32_EXP):
+// (PSPH_FP32_PAIR): exp_neg, FP64 throughout.  FX true (PSPH_FP32_EXP):
 // the FP32 hardware exponential 2^-tf of the argument t = e log2(e), formed
 // in FP64 and rounded once to tf: a relative error of the instruction's own
 // (about one FP32 ulp) plus t 2^-24 ln 2 from the rounding of t (largest at
@@ -893,17 +1126,22 @@ __device__ inline double exp_neg_tab(double e, const double *tab) {
 // h, 1/h and the norm stay FP64.  Taking the rounding of t back out (times
 // 1 - (t - tf) ln 2) halves the form's difference to FP64 over the bench's
 // steps and costs 4 % of the step: not kept.
-template <bool FX> constexpr int wtab_size() { return FX ? 1 : kETab; }
-template <bool FX> __device__ inline void wtab_fill(double *tab, int lane) {
-  if constexpr (!FX) etab_fill(tab, lane);
-}
 constexpr double kLog2e = 1.4426950408889634;
 // 2^-t of the FX form (t >= 0 in FP64)
 __device__ inline double exp2_neg_fx(double t) { return (double)__builtin_amdgcn_exp2f(-(float)t); }
-template <bool FX> __device__ inline double exp_neg_w(double e, const double *tab) {
-  if constexpr (!FX) return exp_neg_tab(e, tab);
+template <bool FX> __device__ inline double exp_neg_w(double e) {
+  if constexpr (!FX) return exp_neg(e);
   else return exp2_neg_fx(e * kLog2e);
 }
+
+// The particle records that a pass reads, in arrays of 16-byte pieces (the last
+// may be narrower): neighbouring lanes take neighbouring pieces.
+struct Packs {
+  void *p[5];
+  __device__ double2 *d2(int k) const { return (double2 *)p[k]; }
+  __device__ float4 *f4(int k) const { return (float4 *)p[k]; }
+  __device__ float *f1(int k) const { return (float *)p[k]; }
+};
 
 template <class R> __device__ inline R pow16(R x) {
   x *= x; x *= x; x *= x;
@@ -924,6 +1162,7 @@ struct RhsArgs {
   int lans, dim;
   EosConst eos;
   unsigned long long *pairs;
+  Packs pk;
 };
 
 // Pair terms, written with the halves folded: c2 = c_i + c_j = 2 c_ab,
@@ -937,9 +1176,6 @@ struct RhsArgs {
 // about 1 % of their size, and FP32 rounding there is what the velocities
 // feel.  The kernel value comes from the exp table (FP64 at FP32-like cost);
 // viscosity, heat conduction and the energy work terms stay FP32.
-template <bool FX> struct RhsMixTile { double m64[kWave], mpv64[kWave], etab[wtab_size<FX>()]; float mV[kWave]; };
-template <class R> struct RhsTileR { R PV2[kWave]; };
-
 // -2 pi^(-D/2): grad W = G dx with G = -2 W / h^2 = kGradNorm h^-(D+2) exp(-r^2/h^2)
 template <int D> constexpr double kGradNorm = -2.0 * kInvSqrtPi * kInvSqrtPi * kInvSqrtPi;
 template <> constexpr double kGradNorm<1> = -2.0 * kInvSqrtPi;
@@ -948,76 +1184,94 @@ template <class R, bool MIXED = std::is_same<R, float>::value, bool FX = false>
 struct RhsPass {
   using Args = RhsArgs;
   static constexpr bool kMixed = MIXED;
-  struct Tile : std::conditional<kMixed, RhsMixTile<FX>, RhsTileR<R>>::type {
-    double hh[kWave];       // h / 2
-    R m[kWave], V[kWave], rho[kWave], c[kWave], T[kWave], cp[kWave];
-    R vx[kWave], vy[kWave], vz[kWave];
-  };
+  static constexpr bool kCountPairs = true;
+  static constexpr int NACC = 4;               // 0-2: the velocity sums, 3: the energy sum (2 de/dt)
+  struct Own { bool bad; };
   struct Tgt {
-    double hi, hh, supp, rv[3], re, pv64;
+    double hh, pv64;
     R rhoi, Vi, pvsqi, ci, Ti, cpi, vel[3];
-    unsigned npairs;
-    int bad;
   };
-  __device__ static void init(Tile &s, int lane) {
-    if constexpr (kMixed) wtab_fill<FX>(s.etab, lane);
-  }
-  static constexpr int kSub = ::kSub;
-  __device__ static void combine(Tgt &t) {
-    for (int k = 0; k < 3; k++) t.rv[k] = sub_sum<kSub>(t.rv[k]);
-    t.re = sub_sum<kSub>(t.re);
-    t.npairs = sub_sum_u<kSub>(t.npairs);
-    t.bad = sub_sum_u<kSub>((uint32_t)t.bad) ? 1 : 0;
-  }
-  __device__ static int npasses(const Args &) { return 1; }
-  __device__ static void begin_pass(const Args &, Tgt &, int) {}
-  __device__ static void end_pass(const Args &, Tgt &, int, uint32_t, bool) {}
-  __device__ static bool want(const Tgt &) { return true; }
-  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t) {
-    t.hi = a.h[i];
-    t.hh = 0.5 * t.hi;
-    t.supp = a.cutoff2 * t.hi;
+  // a neighbour; m64, mpv64 (m p / rho^2) and mV (m / rho) only in the mixed
+  // form, PV2 (p / rho^2) only in the others
+  struct Rec {
+    double m64, mpv64;
+    R m, V, rho, c, T, cp, vx, vy, vz, PV2, mV;
+  };
+  static constexpr int kWaves = 4;             // per SIMD: at most 128 VGPRs
+  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t, Own &o) {
+    t.hh = 0.5 * a.h[i];
     const double rho = a.rho[i];
-    t.bad = !(rho > 0) ? 1 : 0;
+    o.bad = !(rho > 0);
     const double Vi = 1.0 / rho;
     t.pv64 = a.p[i] * Vi * Vi;
     t.rhoi = (R)rho; t.Vi = (R)Vi; t.pvsqi = (R)t.pv64;
     t.ci = (R)a.c[i]; t.Ti = (R)a.T[i]; t.cpi = (R)a.cp[i];
     if (a.lans) { t.vel[0] = (R)a.svx[i]; t.vel[1] = (R)a.svy[i]; t.vel[2] = (R)a.svz[i]; }
     else { t.vel[0] = (R)a.vx[i]; t.vel[1] = (R)a.vy[i]; t.vel[2] = (R)a.vz[i]; }
-    t.rv[0] = t.rv[1] = t.rv[2] = 0; t.re = 0; t.npairs = 0;
   }
-  __device__ static void stage(const Args &a, uint32_t j, Tile &s, int l) {
+  __device__ static void pack(const Args &a, uint32_t j) {
     const double rj = a.rho[j];
     const double V = 1.0 / rj;
     const double pv = a.p[j] * V * V;
     const double mj = a.m[j];
-    s.hh[l] = 0.5 * a.h[j]; s.m[l] = (R)mj; s.V[l] = (R)V; s.rho[l] = (R)rj;
-    if constexpr (kMixed) { s.m64[l] = mj; s.mpv64[l] = mj * pv; s.mV[l] = (float)(mj * V); }
-    else s.PV2[l] = (R)pv;
-    s.c[l] = (R)a.c[j]; s.T[l] = (R)a.T[j]; s.cp[l] = (R)a.cp[j];
-    if (a.lans) { s.vx[l] = (R)a.svx[j]; s.vy[l] = (R)a.svy[j]; s.vz[l] = (R)a.svz[j]; }
-    else { s.vx[l] = (R)a.vx[j]; s.vy[l] = (R)a.vy[j]; s.vz[l] = (R)a.vz[j]; }
+    const double *ux = a.lans ? a.svx : a.vx, *uy = a.lans ? a.svy : a.vy, *uz = a.lans ? a.svz : a.vz;
+    const R c = (R)a.c[j], T = (R)a.T[j], cp = (R)a.cp[j], vx = (R)ux[j], vy = (R)uy[j], vz = (R)uz[j];
+    if constexpr (kMixed) {
+      a.pk.d2(0)[j] = make_double2(mj, mj * pv);
+      a.pk.f4(1)[j] = make_float4((R)V, (R)rj, c, T);
+      a.pk.f4(2)[j] = make_float4(cp, vx, vy, vz);
+      a.pk.f1(3)[j] = (float)(mj * V);
+    } else if constexpr (std::is_same<R, float>::value) {
+      a.pk.f4(0)[j] = make_float4((R)mj, (R)V, (R)rj, c);
+      a.pk.f4(1)[j] = make_float4(T, cp, (R)pv, vx);
+      a.pk.f1(2)[j] = vy;
+      a.pk.f1(3)[j] = vz;
+    } else {
+      a.pk.d2(0)[j] = make_double2(mj, V);
+      a.pk.d2(1)[j] = make_double2(rj, c);
+      a.pk.d2(2)[j] = make_double2(T, cp);
+      a.pk.d2(3)[j] = make_double2(pv, vx);
+      a.pk.d2(4)[j] = make_double2(vy, vz);
+    }
+  }
+  static constexpr int NA16 = kMixed ? 3 : std::is_same<R, float>::value ? 2 : 5;
+  static constexpr int NA4 = kMixed ? 1 : std::is_same<R, float>::value ? 2 : 0;
+  template <class L>
+  __device__ static void load(const L &a, uint32_t j, Rec &r) {
+    if constexpr (kMixed) {
+      const double2 u = a.d2(0)[j];
+      const float4 v = a.f4(1)[j], w = a.f4(2)[j];
+      r.m64 = u.x; r.mpv64 = u.y; r.m = (R)u.x;
+      r.V = v.x; r.rho = v.y; r.c = v.z; r.T = v.w;
+      r.cp = w.x; r.vx = w.y; r.vy = w.z; r.vz = w.w;
+      r.mV = a.f1(0)[j];
+    } else if constexpr (std::is_same<R, float>::value) {
+      const float4 u = a.f4(0)[j], v = a.f4(1)[j];
+      r.m = u.x; r.V = u.y; r.rho = u.z; r.c = u.w;
+      r.T = v.x; r.cp = v.y; r.PV2 = v.z; r.vx = v.w; r.vy = a.f1(0)[j]; r.vz = a.f1(1)[j];
+    } else {
+      const double2 p0 = a.d2(0)[j], p1 = a.d2(1)[j], p2 = a.d2(2)[j], p3 = a.d2(3)[j], p4 = a.d2(4)[j];
+      r.m = p0.x; r.V = p0.y; r.rho = p1.x; r.c = p1.y; r.T = p2.x; r.cp = p2.y;
+      r.PV2 = p3.x; r.vx = p3.y; r.vy = p4.x; r.vz = p4.y;
+    }
   }
   // h_ij = (h_i + h_j)/2 (ME_UPDATE_SML 2).  The reference skips j == i; here
   // the target meets itself once, with dx = 0 and v_ij = 0, and every term it
   // adds is an exact zero (f dx, f v.r, no viscosity for v.r = 0, no heat for
-  // |v_ij . dx| = 0), so no test is spent on it; finish leaves it out of the
-  // pair count.
-  __device__ static double hker(const Args &, const Tgt &t, const Tile &s, uint32_t q) { return t.hh + s.hh[q]; }
-  __device__ static bool extra(const Args &, const Tgt &, const Tile &, uint32_t, uint32_t, uint32_t) { return true; }
+  // |v_ij . dx| = 0), so no test is spent on it; the pair count leaves it out.
+  __device__ static double hker(const Tgt &t, double hhj) { return t.hh + hhj; }
+  __device__ static bool counts_ghost(int) { return true; }
+  __device__ static bool valid(const Rec &r) { return r.rho > R(0); }        // assert(uvecj[0] > 0)
   template <int D>
-  __device__ static void pair_d(const Args &a, Tgt &t, const Tile &s, uint32_t q, uint32_t, uint32_t,
-                                const double *dxd, double) {
-    t.npairs++;
-    if (!(s.rho[q] > R(0))) { t.bad = 1; return; }      // assert(uvecj[0] > 0)
-    if constexpr (kMixed) pair_mixed<D>(a, t, s, q, dxd);
-    else pair_plain<D>(a, t, s, q, dxd);
+  __device__ static void pair_d(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *dxd, double,
+                                double *acc) {
+    if constexpr (kMixed) pair_mixed<D>(a, t, s, hijd, dxd, acc);
+    else pair_plain<D>(a, t, s, hijd, dxd, acc);
   }
   template <int D>
-  __device__ static void pair_plain(const Args &a, Tgt &t, const Tile &s, uint32_t q, const double *dxd) {
-    const R rhoj = s.rho[q];
-    const R h = (R)(t.hh + s.hh[q]);
+  __device__ static void pair_plain(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *dxd, double *acc) {
+    const R rhoj = s.rho;
+    const R h = (R)hijd;
     const R ih = rrcp<R>(h);
     R dx[3], dist_sq = 0, expt = 0;
 #pragma unroll
@@ -1030,27 +1284,31 @@ struct RhsPass {
     const R ih2 = ih * ih;
     const R ihD = (D == 3) ? ih2 * ih : ih;
     // G = -2 W / h^2: grad W = G dx
-    const R G = (R(kGradNorm<D>) * ih2) * (ihD * rexp<R>(-expt));
-    const R Vj = s.V[q];
+    const R G = (R(kGradNorm<D>) * ih2) * (ihD * rexp_neg<R>(expt));
+    const R Vj = s.V;
     R vij[3];
-    vij[0] = t.vel[0] - s.vx[q];
-    if (D == 3) { vij[1] = t.vel[1] - s.vy[q]; vij[2] = t.vel[2] - s.vz[q]; }
-    const R c2 = t.ci + s.c[q];
-    R vrab = 0, dotvv = 0;
+    vij[0] = t.vel[0] - s.vx;
+    if (D == 3) { vij[1] = t.vel[1] - s.vy; vij[2] = t.vel[2] - s.vz; }
+    const R c2 = t.ci + s.c;
+    // (fused explicitly: the heat term needs the products v_k dx_k rounded, and
+    // the compiler would sum those)
+    R vrab = 0;
 #pragma unroll
-    for (int k = 0; k < D; k++) { vrab += dx[k] * vij[k]; dotvv += vij[k] * vij[k]; }
+    for (int k = 0; k < D; k++) vrab = rfma<R>(dx[k], vij[k], vrab);
+    const R dotvv = D == 3 ? rfma<R>(vij[2], vij[2], rfma<R>(vij[0], vij[0], vij[1] * vij[1])) : vij[0] * vij[0];
     // art_vis (sph_lib.cc:402-424): Pi = (beta mu - alpha c) mu / rho_ab for
     // approaching pairs, mu = h v.r / (r^2 + ata h^2)
-    R vis = 0;
-    if (vrab < R(0)) {
+    R vis;
+    {
       const R rs = t.rhoi + rhoj;
       const R den = dist_sq + R(a.ata) * h * h;
       const R r = rrcp<R>(den * rs);
       const R miu = h * vrab * (rs * r);
       vis = (R(a.beta2) * miu - R(a.alpha) * c2) * miu * (den * r);
+      vis = vrab < R(0) ? vis : R(0);
     }
     if (a.lans) vis -= R(a.eps_half) * dotvv * Vj;        // SPH_epsilon_mom
-    const R mpv = s.m[q] * (s.PV2[q] + t.pvsqi + vis);
+    const R mpv = s.m * (s.PV2 + t.pvsqi + vis);
     R heat = 0;
     if (a.lans && D == 3) {
       // k_ij F_ij of SPH_epsilon_heat_conductivity (6-arg, sph_lib.cc:1399-1439)
@@ -1060,25 +1318,24 @@ struct RhsPass {
 #pragma unroll
       for (int k = 0; k < D; k++) dotvr += rabs<R>(vij[k] * dx[k]);
       const R wr = G * dist_sq;
-      if (dotvr != R(0) && wr != R(0)) {
-        const R cp2 = s.cp[q] + t.cpi;
-        const R kF = R(a.kheat) * cp2 * dotvv * wr * rrcp<R>(dotvr * h * c2);
-        heat = s.m[q] * Vj * t.Vi * (t.Ti - s.T[q]) * kF;
-      }
+      const R cp2 = s.cp + t.cpi;
+      const R kF = R(a.kheat) * cp2 * dotvv * wr * rrcp<R>(dotvr * h * c2);
+      heat = s.m * Vj * t.Vi * (t.Ti - s.T) * kF;
+      heat = ((dotvr != R(0)) & (wr != R(0))) ? heat : R(0);
     }
     R de = 0;
     const R Gm = mpv * G;
 #pragma unroll
     for (int k = 0; k < D; k++) {
       const R f = Gm * dx[k];
-      t.rv[k] -= (double)f;
-      de += f * vij[k];
+      acc[k] -= (double)f;
+      de = rfma<R>(f, vij[k], de);
     }
-    t.re += (double)(de + heat);
+    acc[3] += (double)(de + heat);
   }
   template <int D>
-  __device__ static void pair_mixed(const Args &a, Tgt &t, const Tile &s, uint32_t q, const double *dxd) {
-    const double hd = t.hh + s.hh[q];
+  __device__ static void pair_mixed(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *dxd, double *acc) {
+    const double hd = hijd;
     const float h = (float)hd;
     const float ih = rrcp<float>(h);
     const double ih64 = (double)ih * fma(-hd, (double)ih, 2.0);     // one Newton step: ~1e-14
@@ -1089,61 +1346,62 @@ struct RhsPass {
 #pragma unroll
     for (int k = 0; k < D; k++) { r2 = fma(dxd[k], dxd[k], r2); dx[k] = (float)dxd[k]; }
     // G = -2 W / h^2: grad W = G dx
-    const double G64 = (kGradNorm<D> * ih2) * (ihD * exp_neg_w<FX>(r2 * ih2, s.etab));
+    const double G64 = (kGradNorm<D> * ih2) * (ihD * exp_neg_w<FX>(r2 * ih2));
     const float G = (float)G64, dist_sq = (float)r2;
-    const float Vj = s.V[q], rhoj = s.rho[q];
+    const float Vj = s.V, rhoj = s.rho;
     float vij[3];
-    vij[0] = t.vel[0] - s.vx[q];
-    if (D == 3) { vij[1] = t.vel[1] - s.vy[q]; vij[2] = t.vel[2] - s.vz[q]; }
-    const float c2 = t.ci + s.c[q];
-    float vrab = 0, dotvv = 0;
+    vij[0] = t.vel[0] - s.vx;
+    if (D == 3) { vij[1] = t.vel[1] - s.vy; vij[2] = t.vel[2] - s.vz; }
+    const float c2 = t.ci + s.c;
+    float vrab = 0;
 #pragma unroll
-    for (int k = 0; k < D; k++) { vrab += dx[k] * vij[k]; dotvv += vij[k] * vij[k]; }
-    float vis = 0;
-    if (vrab < 0.f) {
+    for (int k = 0; k < D; k++) vrab = fmaf(dx[k], vij[k], vrab);
+    const float dotvv = D == 3 ? fmaf(vij[2], vij[2], fmaf(vij[0], vij[0], vij[1] * vij[1])) : vij[0] * vij[0];
+    float vis;
+    {
       const float rs = t.rhoi + rhoj;
       const float den = dist_sq + (float)a.ata * h * h;
       const float r = rrcp<float>(den * rs);
       const float miu = h * vrab * (rs * r);
       vis = ((float)a.beta2 * miu - (float)a.alpha * c2) * miu * (den * r);
+      vis = vrab < 0.f ? vis : 0.f;
     }
     if (a.lans) vis -= (float)a.eps_half * dotvv * Vj;
     // pressure part in FP64, viscous part in FP32; f = (M_p + M_v) G dx
-    const double f = fma(s.m64[q], t.pv64, s.mpv64[q]) * G64 + (double)(s.m[q] * vis * G);
+    const double f = fma(s.m64, t.pv64, s.mpv64) * G64 + (double)(s.m * vis * G);
 #pragma unroll
-    for (int k = 0; k < D; k++) t.rv[k] = fma(-f, dxd[k], t.rv[k]);
+    for (int k = 0; k < D; k++) acc[k] = fma(-f, dxd[k], acc[k]);
     float heat = 0;
     if (a.lans && D == 3) {
       float dotvr = 0;
 #pragma unroll
       for (int k = 0; k < D; k++) dotvr += rabs<float>(vij[k] * dx[k]);
       const float wr = G * dist_sq;
-      if (dotvr != 0.f && wr != 0.f) {
-        const float cp2 = s.cp[q] + t.cpi;
-        const float kF = (float)a.kheat * cp2 * dotvv * wr * rrcp<float>(dotvr * h * c2);
-        heat = s.mV[q] * t.Vi * (t.Ti - s.T[q]) * kF;
-      }
+      const float cp2 = s.cp + t.cpi;
+      const float kF = (float)a.kheat * cp2 * dotvv * wr * rrcp<float>(dotvr * h * c2);
+      heat = s.mV * t.Vi * (t.Ti - s.T) * kF;
+      heat = ((dotvr != 0.f) & (wr != 0.f)) ? heat : 0.f;
     }
-    t.re += fma(f, (double)vrab, (double)heat);
+    acc[3] += fma(f, (double)vrab, (double)heat);
   }
-  __device__ static void finish(const Args &a, Tgt &t, uint32_t i, int *err) {
-    if (t.bad) { raise_err(err, PSPH_EINVARIANT, i); return; }
+  __device__ static bool finish(const Args &a, const Own &o, const double *sum, bool bad, uint32_t i, int *err) {
+    if (o.bad || bad) { raise_err(err, PSPH_EINVARIANT, i); return false; }
     const double gz = -a.g, dt = a.dt;
     // v += dt rhs_v; gravity on the last axis; e += dt (rhs_e + v_last g)
     // (mom_engr_update.cc:372-388); the velocity in the energy term is the
-    // FP64 one of the target; t.re holds 2 rhs_e
+    // FP64 one of the target; sum[3] holds 2 rhs_e
     const double vl = a.dim == 3 ? (a.lans ? a.svz[i] : a.vz[i]) : (a.lans ? a.svx[i] : a.vx[i]);
-    double nv0 = a.vx[i] + dt * (t.rv[0]);
-    double nv1 = a.vy[i] + dt * (t.rv[1]);
-    double nv2 = a.vz[i] + dt * (t.rv[2]);
+    double nv0 = a.vx[i] + dt * (sum[0]);
+    double nv1 = a.vy[i] + dt * (sum[1]);
+    double nv2 = a.vz[i] + dt * (sum[2]);
     if (a.dim == 3) nv2 += dt * gz; else nv0 += dt * gz;
-    const double ne = a.e[i] + dt * (0.5 * t.re + vl * gz);
+    const double ne = a.e[i] + dt * (0.5 * sum[3] + vl * gz);
     a.o_vx[i] = nv0; a.o_vy[i] = nv1; a.o_vz[i] = nv2;
     a.o_e[i] = ne;
     double p, c, T, gam, cp = a.cp[i];
     eos_dev(a.eos, a.rho[i], ne, a.xi[i], p, c, T, gam, &cp);
     a.o_p[i] = p; a.o_c[i] = c; a.o_T[i] = T; a.o_gam[i] = gam; a.o_cp[i] = cp;
-    if (t.npairs > 1) atomicAdd(a.pairs, (unsigned long long)(t.npairs - 1));   // without the target itself
+    return true;
   }
 };
 
@@ -1162,6 +1420,7 @@ struct DensArgs {
   double *o_wn;            // optional: energy-smoothing normalisation (adjoint recompute)
   int e_sq16;              // e_ratio^2 == 16: exp(-16 x) = exp(-x)^16 by four squarings
   double e_norm;           // the energy-smoothing kernel's norm times h^D: (e_ratio / sqrt(pi))^D
+  Packs pk;
 };
 
 // pi^(-D/2): W = kNorm h^-D exp(-s^2)
@@ -1173,9 +1432,6 @@ template <> constexpr double kNorm<1> = kInvSqrtPi;
 // pair adds to both sums without selecting between them; a candidate that
 // does not contribute (contr_dens false or another phase) stages zero masses
 // and mr = 0, so its terms are exact zeros and no pair tests for it.
-template <bool FX> struct DensMixTile { double m1[kWave], m2[kWave], mr64[kWave], e64[kWave], etab[wtab_size<FX>()]; };
-template <class R> struct DensTileR { R m1[kWave], m2[kWave], mr[kWave], e[kWave]; };
-
 // The FP32-pair form evaluates the density and energy-smoothing weights in
 // FP64 with the exp table: the pressure gradient of the next step amplifies
 // relative errors of rho and e by its cancellation.
@@ -1183,49 +1439,47 @@ template <class R, bool MIXED = std::is_same<R, float>::value, bool FX = false>
 struct DensPass {
   using Args = DensArgs;
   static constexpr bool kMixed = MIXED;
-  // the mixed form stages only the FP64 copies it reads
-  struct Tile : std::conditional<kMixed, DensMixTile<FX>, DensTileR<R>>::type {
-    double hh[kWave];       // h / 2
-  };
-  __device__ static void init(Tile &s, int lane) {
-    if constexpr (kMixed) wtab_fill<FX>(s.etab, lane);
-  }
-  struct Tgt { double hi, hh, supp, r1, r2, wn, en; };
-  static constexpr int kSub = ::kSub;
-  __device__ static void combine(Tgt &t) {
-    t.r1 = sub_sum<kSub>(t.r1); t.r2 = sub_sum<kSub>(t.r2);
-    t.wn = sub_sum<kSub>(t.wn); t.en = sub_sum<kSub>(t.en);
-  }
-  __device__ static int npasses(const Args &) { return 1; }
-  __device__ static void begin_pass(const Args &, Tgt &, int) {}
-  __device__ static void end_pass(const Args &, Tgt &, int, uint32_t, bool) {}
-  __device__ static bool want(const Tgt &) { return true; }
-  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t) {
-    t.hi = a.h[i]; t.hh = 0.5 * t.hi; t.supp = a.cutoff2 * t.hi;
-    t.r1 = t.r2 = t.wn = t.en = 0;
-  }
-  __device__ static void stage(const Args &a, uint32_t j, Tile &s, int l) {
-    s.hh[l] = 0.5 * a.h[j];
+  static constexpr bool kCountPairs = false;
+  static constexpr int NACC = 4;               // r1, r2, wn, en
+  struct Own {};
+  struct Tgt { double hh; };
+  using W = typename std::conditional<kMixed, double, R>::type;   // the mixed form reads FP64 copies only
+  struct Rec { W m1, m2, mr, e; };
+  static constexpr int kWaves = 4;             // per SIMD: at most 128 VGPRs
+  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t, Own &) { t.hh = 0.5 * a.h[i]; }
+  __device__ static void pack(const Args &a, uint32_t j) {
     const int ph = a.phase[j];
     const int ok = (contr_dens(a.pghost, a.bc[j]) && (ph == 1 || ph == 2)) ? ph : 0;
     const double mj = a.m[j];
     const double m1 = ok == 1 ? mj : 0.0, m2 = ok == 2 ? mj : 0.0;
     const double mr = ok ? mj / a.rho[j] : 0.0, e = ok ? a.e[j] : 0.0;
-    if constexpr (kMixed) {
-      s.m1[l] = m1; s.m2[l] = m2; s.mr64[l] = mr; s.e64[l] = e;
+    if constexpr (std::is_same<W, float>::value) {
+      a.pk.f4(0)[j] = make_float4((W)m1, (W)m2, (W)mr, (W)e);
     } else {
-      s.m1[l] = (R)m1; s.m2[l] = (R)m2; s.mr[l] = (R)mr; s.e[l] = (R)e;
+      a.pk.d2(0)[j] = make_double2(m1, m2);
+      a.pk.d2(1)[j] = make_double2(mr, e);
+    }
+  }
+  static constexpr int NA16 = std::is_same<W, float>::value ? 1 : 2, NA4 = 0;
+  template <class L>
+  __device__ static void load(const L &a, uint32_t j, Rec &r) {
+    if constexpr (std::is_same<W, float>::value) {
+      const float4 u = a.f4(0)[j];
+      r = Rec{u.x, u.y, u.z, u.w};
+    } else {
+      const double2 u = a.d2(0)[j], v = a.d2(1)[j];
+      r = Rec{u.x, u.y, v.x, v.y};
     }
   }
   // kernel at h_ij (DENSITY_UPDATE_SML 11); contr_dens and the phase are in
-  // the staged masses.  The energy-smoothing kernel (support 0.75 h_ij) lies
+  // the packed masses.  The energy-smoothing kernel (support 0.75 h_ij) lies
   // inside that box.
-  __device__ static double hker(const Args &, const Tgt &t, const Tile &s, uint32_t q) { return t.hh + s.hh[q]; }
-  __device__ static bool extra(const Args &, const Tgt &, const Tile &, uint32_t, uint32_t, uint32_t) { return true; }
+  __device__ static double hker(const Tgt &t, double hhj) { return t.hh + hhj; }
+  __device__ static bool counts_ghost(int) { return true; }
+  __device__ static bool valid(const Rec &) { return true; }
   template <int D>
-  __device__ static void pair_d(const Args &a, Tgt &t, const Tile &s, uint32_t q, uint32_t, uint32_t,
-                                const double *ds, double amax) {
-    const double hijd = t.hh + s.hh[q];
+  __device__ static void pair_d(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *ds, double amax,
+                                double *acc) {
     if constexpr (kMixed && FX) {
       // The FP32-exp form: the weights in FP32 (reciprocal of h_ij, s^2, the
       // exponential, the norm), the sums in FP64.  Over the 4M bench window
@@ -1240,13 +1494,13 @@ struct DensPass {
       const float ex = __builtin_amdgcn_exp2f(-(r2 * (ih2 * (float)kLog2e)));
       const float ihD = (D == 3) ? ih2 * ih : ih;
       const double wk = (double)(((float)kNorm<D> * ihD) * ex);
-      t.r1 = fma(wk, s.m1[q], t.r1);
-      t.r2 = fma(wk, s.m2[q], t.r2);
+      acc[0] = fma(wk, s.m1, acc[0]);
+      acc[1] = fma(wk, s.m2, acc[1]);
       if (a.energy_smooth && !a.cut.outside(a.e_ratio * amax, hijd)) {
         const float ee = a.e_sq16 ? pow16(ex) : __builtin_amdgcn_exp2f(-(float)(a.e_ratio * a.e_ratio) * (r2 * (ih2 * (float)kLog2e)));
-        const double vr = (double)(((float)a.e_norm * ihD) * ee) * s.mr64[q];
-        t.wn += vr;
-        t.en += vr * s.e64[q];
+        const double vr = (double)(((float)a.e_norm * ihD) * ee) * s.mr;
+        acc[2] += vr;
+        acc[3] += vr * s.e;
       }
     } else if constexpr (kMixed) {
       const float ih32 = rrcp<float>((float)hijd);
@@ -1257,16 +1511,16 @@ struct DensPass {
       const double ih2 = ih * ih;
       const double expt = r2 * ih2;
       const double ihD = (D == 3) ? ih2 * ih : ih;
-      const double ex = exp_neg_w<FX>(expt, s.etab);
+      const double ex = exp_neg_w<FX>(expt);
       // one of m1, m2 is 0: that sum gains an exact zero
       const double wk = (kNorm<D> * ihD) * ex;
-      t.r1 = fma(wk, s.m1[q], t.r1);
-      t.r2 = fma(wk, s.m2[q], t.r2);
+      acc[0] = fma(wk, s.m1, acc[0]);
+      acc[1] = fma(wk, s.m2, acc[1]);
       if (a.energy_smooth && !a.cut.outside(a.e_ratio * amax, hijd)) {
-        const double ee = a.e_sq16 ? pow16(ex) : exp_neg_w<FX>(a.e_ratio * a.e_ratio * expt, s.etab);
-        const double vr = (a.e_norm * ihD) * (ee * s.mr64[q]);
-        t.wn += vr;
-        t.en += vr * s.e64[q];
+        const double ee = a.e_sq16 ? pow16(ex) : exp_neg_w<FX>(a.e_ratio * a.e_ratio * expt);
+        const double vr = (a.e_norm * ihD) * (ee * s.mr);
+        acc[2] += vr;
+        acc[3] += vr * s.e;
       }
     } else {
     const R hij = (R)hijd;
@@ -1278,33 +1532,33 @@ struct DensPass {
       expt += sk * sk;
     }
     const R ihD = (D == 3) ? ih * ih * ih : ih;
-    const R ex = rexp<R>(-expt);
+    const R ex = rexp_neg<R>(expt);
     const R wk = (R(kNorm<D>) * ihD) * ex;
-    t.r1 += (double)(wk * s.m1[q]);
-    t.r2 += (double)(wk * s.m2[q]);
+    acc[0] += (double)(wk * s.m1);
+    acc[1] += (double)(wk * s.m2);
     if (a.energy_smooth) {
       // weight(4 ds / h_ij, h_ij / 4) m_j / rho_j (HAVE_ENERGY_SMOOTH 1); exact FP64 box test
       if (!a.cut.outside(a.e_ratio * amax, hijd)) {
         const R e2 = R(a.e_ratio * a.e_ratio);
-        const R vr = (R(a.e_norm) * ihD) * ((a.e_sq16 ? pow16(ex) : rexp<R>(-(e2 * expt))) * s.mr[q]);
-        t.wn += (double)vr;
-        t.en += (double)(vr * s.e[q]);
+        const R vr = (R(a.e_norm) * ihD) * ((a.e_sq16 ? pow16(ex) : rexp_neg<R>(e2 * expt)) * s.mr);
+        acc[2] += (double)vr;
+        acc[3] += (double)(vr * s.e);
       }
     }
     }
   }
-  __device__ static void finish(const Args &a, Tgt &t, uint32_t i, int *err) {
+  __device__ static bool finish(const Args &a, const Own &, const double *sum, bool, uint32_t i, int *err) {
     double density = 0.0;
-    density += t.r1;
-    density += t.r2;
-    const double xi = t.r2 / density;
+    density += sum[0];
+    density += sum[1];
+    const double xi = sum[1] / density;
     double e = a.e[i];
     if (a.energy_smooth) {
-      if (!(t.wn > 0)) { raise_err(err, PSPH_EINVARIANT, i); return; }
-      e = t.en / t.wn;
-      if (a.o_wn) a.o_wn[i] = t.wn;
+      if (!(sum[2] > 0)) { raise_err(err, PSPH_EINVARIANT, i); return false; }
+      e = sum[3] / sum[2];
+      if (a.o_wn) a.o_wn[i] = sum[2];
     }
-    if (!(density > 0) || !(xi <= 1)) { raise_err(err, PSPH_EINVARIANT, i); return; }
+    if (!(density > 0) || !(xi <= 1)) { raise_err(err, PSPH_EINVARIANT, i); return false; }
     a.o_rho[i] = density;
     a.o_e[i] = e;
     a.xi[i] = xi;
@@ -1312,6 +1566,7 @@ struct DensPass {
     double p, c, T, gam, cp = a.cp[i];
     eos_dev(a.eos, density, e, xi, p, c, T, gam, &cp);
     a.p[i] = p; a.c[i] = c; a.T[i] = T; a.gam[i] = gam; a.cp[i] = cp;
+    return true;
   }
 };
 
@@ -1324,10 +1579,7 @@ struct VsmArgs {
   double *svx, *svy, *svz;
   double cutoff, cutoff2;
   double *o_wn;            // optional: the filter's normalisation sum (adjoint recompute)
-  // the per-pair contr_vel test is skipped (a non-contributing candidate
-  // stages m / rho = 0, so its terms are exact zeros) unless the step is
-  // recorded, where the boundary-ghost marks follow the tested pairs
-  int ok_test;
+  Packs pk;
 };
 
 // The FP32-pair form evaluates the filter weights in FP64 from the exp table
@@ -1335,59 +1587,41 @@ struct VsmArgs {
 // FP32 weights (relative error ~3e-7, dominated by the rounding of s^2 and of
 // h) made the velocity filter the largest source of FP32-vs-FP64 difference,
 // ~15x the RHS's FP32 terms.
-template <bool FX> struct VsmMixTile { double mr64[kWave], v64[3][kWave], etab[wtab_size<FX>()]; };
-template <class R> struct VsmTileR { R mr[kWave], vx[kWave], vy[kWave], vz[kWave]; };
-
+//
+// A neighbour that is not contr_vel packs m / rho = 0, so its terms are exact
+// zeros and no pair tests for it (in a recorded step the boundary-ghost marks
+// do).
 template <class R, bool FX = false>
 struct VsmPass {
   using Args = VsmArgs;
   static constexpr bool kMixed = std::is_same<R, float>::value;
-  struct Tile : std::conditional<kMixed, VsmMixTile<FX>, VsmTileR<R>>::type {
-    int ok[kWave];
-  };
-  __device__ static void init(Tile &s, int lane) {
-    if constexpr (kMixed) wtab_fill<FX>(s.etab, lane);
-  }
-  struct Tgt { double hi, supp, ih2, nrm, v64[3], dv[3], wn; R ih, v[3]; };
-  static constexpr int kSub = ::kSub;
-  __device__ static void combine(Tgt &t) {
-    for (int k = 0; k < 3; k++) t.dv[k] = sub_sum<kSub>(t.dv[k]);
-    t.wn = sub_sum<kSub>(t.wn);
-  }
-  __device__ static int npasses(const Args &) { return 1; }
-  __device__ static void begin_pass(const Args &, Tgt &, int) {}
-  __device__ static void end_pass(const Args &, Tgt &, int, uint32_t, bool) {}
-  __device__ static bool want(const Tgt &) { return true; }
-  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t) {
-    t.hi = a.h[i]; t.supp = a.cutoff2 * t.hi;
-    const double ih = 1.0 / t.hi;
-    const double nk = kInvSqrtPi * ih;
-    t.ih = (R)ih;
-    t.ih2 = FX ? ih * ih * kLog2e : ih * ih;    // the FX form's exponential takes s^2 log2(e)
-    t.nrm = a.vy ? nk * nk * nk : nk;
+  static constexpr bool kCountPairs = false;
+  static constexpr int NACC = 4;               // 0-2: the velocity differences, 3: the weights
+  struct Own {};
+  struct Tgt { double hi, ih2, v64[3]; double ih; };
+  struct Rec { double mr, v[3]; };
+  static constexpr int kWaves = 4;             // per SIMD: at most 128 VGPRs
+  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t, Own &) {
+    t.hi = a.h[i];
+    t.ih = 1.0 / t.hi;
+    t.ih2 = FX ? t.ih * t.ih * kLog2e : t.ih * t.ih;    // the FX form's exponential takes s^2 log2(e)
     t.v64[0] = a.vx[i]; t.v64[1] = a.vy ? a.vy[i] : 0; t.v64[2] = a.vz ? a.vz[i] : 0;
-    for (int k = 0; k < 3; k++) t.v[k] = (R)t.v64[k];
-    t.dv[0] = t.dv[1] = t.dv[2] = 0; t.wn = 0;
   }
-  __device__ static void stage(const Args &a, uint32_t j, Tile &s, int l) {
-    const double v[3] = {a.vx[j], a.vy ? a.vy[j] : 0.0, a.vz ? a.vz[j] : 0.0};
-    const int ok = contr_vel(a.bc[j]);
-    if constexpr (kMixed) {
-      s.mr64[l] = ok ? a.m[j] / a.rho[j] : 0.0;
-      for (int k = 0; k < 3; k++) s.v64[k][l] = v[k];
-    } else {
-      s.mr[l] = ok ? (R)(a.m[j] / a.rho[j]) : R(0);
-      s.vx[l] = (R)v[0]; s.vy[l] = (R)v[1]; s.vz[l] = (R)v[2];
-    }
-    s.ok[l] = ok;
+  __device__ static void pack(const Args &a, uint32_t j) {
+    a.pk.d2(0)[j] = make_double2(contr_vel(a.bc[j]) ? a.m[j] / a.rho[j] : 0.0, a.vx[j]);
+    a.pk.d2(1)[j] = make_double2(a.vy ? a.vy[j] : 0.0, a.vz ? a.vz[j] : 0.0);
   }
-  __device__ static double hker(const Args &, const Tgt &t, const Tile &, uint32_t) { return t.hi; }
-  __device__ static bool extra(const Args &a, const Tgt &, const Tile &s, uint32_t q, uint32_t, uint32_t) {
-    return !a.ok_test || s.ok[q] != 0;
+  static constexpr int NA16 = 2, NA4 = 0;
+  template <class L>
+  __device__ static void load(const L &a, uint32_t j, Rec &r) {
+    const double2 u = a.d2(0)[j], v = a.d2(1)[j];
+    r = Rec{u.x, {u.y, v.x, v.y}};
   }
+  __device__ static double hker(const Tgt &t, double) { return t.hi; }
+  __device__ static bool counts_ghost(int b) { return contr_vel(b); }
+  __device__ static bool valid(const Rec &) { return true; }
   template <int D>
-  __device__ static void pair_d(const Args &a, Tgt &t, const Tile &s, uint32_t q, uint32_t, uint32_t,
-                                const double *ds, double) {
+  __device__ static void pair_d(const Args &, const Tgt &t, const Rec &s, double, const double *ds, double, double *acc) {
     if constexpr (kMixed) {
       double r2 = 0;
 #pragma unroll
@@ -1395,34 +1629,34 @@ struct VsmPass {
       // the weight without the kernel's norm, which cancels in dv / wn
       double ew;
       if constexpr (FX) ew = exp2_neg_fx(r2 * t.ih2);
-      else ew = exp_neg_tab(r2 * t.ih2, s.etab);
-      const double w = ew * s.mr64[q];
+      else ew = exp_neg(r2 * t.ih2);
+      const double w = ew * s.mr;
 #pragma unroll
-      for (int k = 0; k < D; k++) t.dv[k] = fma(w, s.v64[k][q] - t.v64[k], t.dv[k]);
-      t.wn += w;
-    }
-    else {
+      for (int k = 0; k < D; k++) acc[k] = fma(w, s.v[k] - t.v64[k], acc[k]);
+      acc[3] += w;
+    } else {
       R expt = 0;
 #pragma unroll
       for (int k = 0; k < D; k++) {
         R sk = (R)ds[k] * t.ih;
         expt += sk * sk;
       }
-      const R mvw = rexp<R>(-expt) * s.mr[q];        // the norm cancels in dv / wn
-      t.dv[0] += (double)(mvw * (s.vx[q] - t.v[0]));
-      if (D == 3) {
-        t.dv[1] += (double)(mvw * (s.vy[q] - t.v[1]));
-        t.dv[2] += (double)(mvw * (s.vz[q] - t.v[2]));
-      }
-      t.wn += (double)mvw;
+      const R mvw = rexp_neg<R>(expt) * s.mr;           // the norm cancels in dv / wn
+#pragma unroll
+      for (int k = 0; k < D; k++) acc[k] += mvw * (s.v[k] - t.v64[k]);
+      acc[3] += mvw;
     }
   }
-  __device__ static void finish(const Args &a, Tgt &t, uint32_t i, int *err) {
-    if (!(t.wn > 0)) { raise_err(err, PSPH_EINVARIANT, i); return; }
-    const double iw = 1.0 / t.wn;
-    if (a.o_wn) a.o_wn[i] = t.wn * t.nrm;          // the normalisation sum with the kernel's norm
-    a.svx[i] = t.v64[0] + t.dv[0] * iw;
-    if (a.svy) { a.svy[i] = t.v64[1] + t.dv[1] * iw; a.svz[i] = t.v64[2] + t.dv[2] * iw; }
+  __device__ static bool finish(const Args &a, const Own &, const double *sum, bool, uint32_t i, int *err) {
+    if (!(sum[3] > 0)) { raise_err(err, PSPH_EINVARIANT, i); return false; }
+    const double iw = 1.0 / sum[3];
+    if (a.o_wn) {                                    // the normalisation sum with the kernel's norm
+      const double nk = kInvSqrtPi * (1.0 / a.h[i]);
+      a.o_wn[i] = sum[3] * (a.vy ? nk * nk * nk : nk);
+    }
+    a.svx[i] = a.vx[i] + sum[0] * iw;
+    if (a.svy) { a.svy[i] = a.vy[i] + sum[1] * iw; a.svz[i] = a.vz[i] + sum[2] * iw; }
+    return true;
   }
 };
 
@@ -1450,9 +1684,8 @@ struct AdaptPass {
   struct Tile {
     R m[kWave];
     int ok[kWave];
-    double etab[wtab_size<FX>()];
   };
-  __device__ static void init(Tile &s, int lane) { wtab_fill<FX>(s.etab, lane); }
+  __device__ static void init(Tile &, int) {}
   struct Tgt { double mi, hcur, Hs, supp, rho_star; R iHs, norm; bool done; };
   static constexpr int kSub = ::kSub;
   __device__ static void combine(Tgt &t) { t.rho_star = sub_sum<kSub>(t.rho_star); }
@@ -1485,7 +1718,7 @@ struct AdaptPass {
       R sk = (R)dx[k] * t.iHs;
       expt += sk * sk;
     }
-    t.rho_star += (double)(t.norm * (R)exp_neg_w<FX>((double)expt, s.etab) * s.m[q]);
+    t.rho_star += (double)(t.norm * (R)exp_neg_w<FX>((double)expt) * s.m[q]);
   }
   __device__ static void end_pass(const Args &a, Tgt &t, int, uint32_t, bool active) {
     if (!active || t.done) return;
@@ -2034,11 +2267,14 @@ struct psph_ctx {
   bool grid_valid = false;
   GridDesc grid{};
   double reach_main = 0;       // per-axis reach of the RHS / density / filter predicates
-  // visit lists of the RHS / density / filter passes (built once per step)
-  bool vis_valid = false;
-  uint32_t *vcount = nullptr, *voff = nullptr, *vnum = nullptr, *vmask = nullptr;
-  uint2 *vent = nullptr;
-  size_t vchunk_cap = 0, vis_cap = 0;
+  // the group passes' lists and positions (made once per step) and particle records
+  bool lists_valid = false;
+  uint4 *gvisit = nullptr;
+  uint32_t *goff = nullptr, *gnum = nullptr, *gfast = nullptr, *gcursor = nullptr;
+  size_t gchunk_cap = 0;
+  uint32_t gvisit_cap = 0;
+  double2 *gxy = nullptr, *gzh = nullptr;
+  void *pk[5] = {};
   double h_max = 0;
   // clock (TimeProps)
   double time = 0, next_output = 0;
@@ -2196,9 +2432,10 @@ extern "C" int psph_destroy(psph_ctx *c) {
   void *ptrs[] = {c->usp, c->isp, c->h_list, c->pid, c->pid_sp, c->refb, c->key_a, c->key_b, c->idx_a, c->idx_b,
                   c->flags, c->tpos, c->targets, c->cfirst, c->ccount, c->cs, c->tcnt, c->toff,
                   c->cchunks, c->coff, c->tbox, c->nchunks, c->cub, c->d_u64, c->d_err, c->d_part,
-                  c->vcount, c->voff, c->vnum, c->vmask, c->vent, c->px, c->py, c->pz,
+                  c->gvisit, c->goff, c->gnum, c->gfast, c->gcursor, c->gxy, c->gzh, c->px, c->py, c->pz,
                   c->d_occ, c->d_conv, c->d_sides};
   for (auto p : ptrs) if (p) hipFree(p);
+  for (auto p : c->pk) if (p) hipFree(p);
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -2511,7 +2748,7 @@ extern "C" int psph_neighbors(psph_ctx *c) {
   HIP_TRY(hipGetLastError());
   tm.stop();
   c->grid_valid = true;
-  c->vis_valid = false;
+  c->lists_valid = false;
   return 0;
 }
 
@@ -2571,75 +2808,106 @@ static void launch_pairs(psph_ctx *c, const PairCommon &pc, const typename P::Ar
     hipLaunchKernelGGL((k_pairs<1, Bound<1, P>>), nb, kWave, 0, c->stream, pc, a);
 }
 
-// Visit lists of the current step (positions, h and targets fixed since the
-// last psph_neighbors / adaptation): count the tiles each chunk meets, scan,
-// then write the tiles with hits and their lane masks.
-static int ensure_visits(psph_ctx *c) {
-  if (c->vis_valid) return 0;
+static GroupCommon group_common(psph_ctx *c) {
+  GroupCommon gc{};
+  gc.g = Geom{c->gxy, c->gzh};
+  gc.gl = GroupLists{c->gvisit, c->goff, c->gnum, c->gfast, c->gcursor, c->gvisit_cap};
+  gc.cutx = c->cfg.cutoff * (1.0 + 1e-12);     // a superset of the three passes' kernel boxes
+  gc.h_max = c->h_max;
+  return gc;
+}
+
+// Lists and positions of the group passes (positions, h and targets fixed since
+// the last psph_neighbors / adaptation).
+static int ensure_lists(psph_ctx *c) {
+  if (c->lists_valid) return 0;
   StageTimer tm(c, 1);
-  const PairCommon pc = make_common(c, c->reach_main);
-  const unsigned G = chunk_grid(c->n, c->grid.ncells, kChunk);
-  if ((size_t)G + 1 > c->vchunk_cap) {
-    uint32_t **arrs[] = {&c->vcount, &c->voff, &c->vnum};
+  if (!c->gxy) PSPH_TRY(dmalloc((void **)&c->gxy, c->cap * sizeof(double2)));
+  if (!c->gzh) PSPH_TRY(dmalloc((void **)&c->gzh, c->cap * sizeof(double2)));
+  for (auto &p : c->pk)
+    if (!p) PSPH_TRY(dmalloc(&p, c->cap * 16));
+  if (!c->gcursor) PSPH_TRY(dmalloc((void **)&c->gcursor, 4));
+  if (c->chunk_cap > c->gchunk_cap) {
+    uint32_t **arrs[] = {&c->goff, &c->gnum, &c->gfast};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)G + 1) * 4));
-    c->vchunk_cap = (size_t)G + 1;
+    c->gchunk_cap = 0;
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, c->chunk_cap * kGroupsPerChunk * 4));
+    c->gchunk_cap = c->chunk_cap;
   }
-  // a superset of the three passes' kernel boxes with a relative margin
-  const double cutx = c->cfg.cutoff * (1.0 + 1e-12);
-  hipLaunchKernelGGL(k_visit_count, G, kWave, 0, c->stream, pc, c->f.h, cutx, c->h_max, c->vcount);
-  hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, (int *)c->vcount + G, 0, 1);
-  HIP_TRY(hipGetLastError());
-  PSPH_TRY(excl_scan(c, c->vcount, c->voff, (size_t)G + 1));
-  uint32_t total = 0;
-  HIP_TRY(hipMemcpyAsync(&total, c->voff + G, 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  if ((size_t)total > c->vis_cap) {
-    if (c->vmask) hipFree(c->vmask);
-    if (c->vent) hipFree(c->vent);
-    c->vmask = nullptr; c->vent = nullptr;
-    const size_t cap = (size_t)total + total / 8 + 1024;
-    PSPH_TRY(dmalloc((void **)&c->vmask, cap * kWave * 4));
-    PSPH_TRY(dmalloc((void **)&c->vent, cap * sizeof(uint2)));
-    c->vis_cap = cap;
+  const PairCommon pc = make_common(c, c->reach_main);
+  hipLaunchKernelGGL(k_geom, blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, pc.x, pc.y, pc.z, c->f.h, c->gxy, c->gzh);
+  // a group per wave up to a quarter of a million particles: at 77k 0.15 ms against
+  // 0.20 with half a chunk; a chunk per wave beyond
+  const uint32_t nsplit = c->n < (1u << 18) ? kGroupsPerChunk : 1;
+  const unsigned G = chunk_grid(c->n, c->grid.ncells, kChunk) * nsplit;
+  for (;;) {
+    const GroupCommon gc = group_common(c);
+    hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, (int *)c->gcursor, 0, 1);
+    if (c->cfg.dim == 3)
+      hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
+    else
+      hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
+    HIP_TRY(hipGetLastError());
+    uint32_t total = 0;
+    HIP_TRY(hipMemcpyAsync(&total, c->gcursor, 4, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (total <= c->gvisit_cap) break;
+    // the visits outgrew their memory: this call only counted
+    if (c->gvisit) hipFree(c->gvisit);
+    c->gvisit = nullptr;
+    c->gvisit_cap = 0;
+    const size_t want = std::min<size_t>((size_t)total + total / 8 + 1024, 0xffffffffu);
+    PSPH_TRY(dmalloc((void **)&c->gvisit, want * sizeof(uint4)));
+    c->gvisit_cap = (uint32_t)want;
   }
-  if (c->cfg.dim == 3)
-    hipLaunchKernelGGL(k_visit_masks<3>, G, kWave, 0, c->stream, pc, c->f.h, c->cfg.cutoff2, cutx, c->h_max,
-                       c->voff, c->vnum, c->vent, c->vmask);
-  else
-    hipLaunchKernelGGL(k_visit_masks<1>, G, kWave, 0, c->stream, pc, c->f.h, c->cfg.cutoff2, cutx, c->h_max,
-                       c->voff, c->vnum, c->vent, c->vmask);
-  HIP_TRY(hipGetLastError());
-  c->vis_valid = true;
+  c->lists_valid = true;
   return 0;
 }
 
-// the RHS, density and filter passes run over the visit lists; PM, PP, PD:
-// the pass in the FP32-pair, FP32-pure and FP64 forms
-template <int D, class P>
-static void launch_visit_pass(psph_ctx *c, const PairCommon &pc, const VisitList &vl, const typename P::Args &a) {
-  const unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk);
-  if (c->tape.mode == 2 && c->tape.frozen)
-    hipLaunchKernelGGL((k_pairs_v<D, Bound<D, P>, true>), nb, kWave, 0, c->stream, pc, vl, a);
-  else
-    hipLaunchKernelGGL((k_pairs_v<D, Bound<D, P>>), nb, kWave, 0, c->stream, pc, vl, a);
+// A pass's outputs for its targets go to spare arrays; the other particles keep
+// their values: the kernel that packs the pass's records copies those.
+struct FieldCopy {
+  const double *src[9];
+  double *dst[9];
+  int nf;
+};
+template <class P>
+__global__ void k_pack(uint32_t n, typename P::Args a, const int32_t *bc, FieldCopy fc) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  P::pack(a, i);
+  if (fc.nf && !need_neigh(bc[i]))
+    for (int q = 0; q < fc.nf; q++) fc.dst[q][i] = fc.src[q][i];
 }
+
+template <int D, class P>
+static void launch_group_pass(psph_ctx *c, const PairCommon &pc, const GroupCommon &gc, const typename P::Args &a,
+                              const FieldCopy &fc) {
+  hipLaunchKernelGGL((k_pack<P>), blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, a, c->f.bc, fc);
+  const unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk) * kGroupsPerChunk;
+  if (c->tape.mode == 2 && c->tape.frozen)
+    hipLaunchKernelGGL((k_group_pass<D, P, true>), nb, kWave, 0, c->stream, pc, gc, a);
+  else
+    hipLaunchKernelGGL((k_group_pass<D, P, false>), nb, kWave, 0, c->stream, pc, gc, a);
+}
+// the RHS, density and filter passes; PM, PX, PP, PD: the pass in the FP32-pair,
+// FP32-exp, FP32-pure and FP64 forms
 template <class PM, class PX, class PP, class PD>
-static int launch_visits(psph_ctx *c, const typename PD::Args &a) {
-  PSPH_TRY(ensure_visits(c));
+static int launch_groups(psph_ctx *c, typename PD::Args a, const FieldCopy &fc) {
   const PairCommon pc = make_common(c, c->reach_main);
-  const VisitList vl{c->voff, c->vnum, c->vent, c->vmask};
+  const GroupCommon gc = group_common(c);
+  for (int k = 0; k < 5; k++) a.pk.p[k] = c->pk[k];
   const int form = c->cfg.precision;
   if (c->cfg.dim == 3) {
-    if (form == PSPH_FP32_PAIR) launch_visit_pass<3, PM>(c, pc, vl, a);
-    else if (form == PSPH_FP32_EXP) launch_visit_pass<3, PX>(c, pc, vl, a);
-    else if (form == PSPH_FP32_PURE) launch_visit_pass<3, PP>(c, pc, vl, a);
-    else launch_visit_pass<3, PD>(c, pc, vl, a);
+    if (form == PSPH_FP32_PAIR) launch_group_pass<3, PM>(c, pc, gc, a, fc);
+    else if (form == PSPH_FP32_EXP) launch_group_pass<3, PX>(c, pc, gc, a, fc);
+    else if (form == PSPH_FP32_PURE) launch_group_pass<3, PP>(c, pc, gc, a, fc);
+    else launch_group_pass<3, PD>(c, pc, gc, a, fc);
   } else {
-    if (form == PSPH_FP32_PAIR) launch_visit_pass<1, PM>(c, pc, vl, a);
-    else if (form == PSPH_FP32_EXP) launch_visit_pass<1, PX>(c, pc, vl, a);
-    else if (form == PSPH_FP32_PURE) launch_visit_pass<1, PP>(c, pc, vl, a);
-    else launch_visit_pass<1, PD>(c, pc, vl, a);
+    if (form == PSPH_FP32_PAIR) launch_group_pass<1, PM>(c, pc, gc, a, fc);
+    else if (form == PSPH_FP32_EXP) launch_group_pass<1, PX>(c, pc, gc, a, fc);
+    else if (form == PSPH_FP32_PURE) launch_group_pass<1, PP>(c, pc, gc, a, fc);
+    else launch_group_pass<1, PD>(c, pc, gc, a, fc);
   }
   return 0;
 }
@@ -2660,7 +2928,7 @@ static int reduce_hmax(psph_ctx *c, double *out) {
 
 // the later passes of a step use the new h: widen the reach
 static void set_reach(psph_ctx *c, double hmax) {
-  c->vis_valid = false;                // h changed
+  c->lists_valid = false;                // h changed
   c->h_max = hmax;
   c->reach_main = c->cfg.cutoff * hmax * (1 + 1e-9);
 }
@@ -2709,19 +2977,6 @@ static int h_by_id(psph_ctx *c, double *tab, int replay) {
   return 0;
 }
 
-// A pass writes its outputs for its targets (need_neigh) into spare arrays;
-// the other particles keep their values: one launch copies those.
-struct FieldCopy {
-  const double *src[9];
-  double *dst[9];
-  int nf;
-};
-__global__ void k_copy_nontargets(uint32_t n, const int32_t *bc, FieldCopy fc) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || need_neigh(bc[i])) return;
-  for (int q = 0; q < fc.nf; q++) fc.dst[q][i] = fc.src[q][i];
-}
-
 extern "C" int psph_rhs(psph_ctx *c, double dt) {
   if (!c) return fail(PSPH_EINVAL, "null ctx");
   if (!c->grid_valid) return fail(PSPH_EINVAL, "rhs: call psph_neighbors first");
@@ -2730,12 +2985,9 @@ extern "C" int psph_rhs(psph_ctx *c, double dt) {
   // outputs go to spare arrays; non-targets keep their values
   double *ov[9] = {c->dsp[1], c->dsp[2], c->dsp[3], c->dsp[4], c->dsp[5], c->dsp[6], c->dsp[7], c->dsp[8], c->dsp[9]};
   double *src[9] = {c->f.vx, c->f.vy, c->f.vz, c->f.e, c->f.p, c->f.c, c->f.T, c->f.gam, c->f.cp};
-  if (n) {
-    FieldCopy fc{};
-    for (int q = 0; q < 9; q++) { fc.src[q] = src[q]; fc.dst[q] = ov[q]; }
-    fc.nf = 9;
-    hipLaunchKernelGGL(k_copy_nontargets, blocks(n), 256, 0, c->stream, n, c->f.bc, fc);
-  }
+  FieldCopy fc{};
+  for (int q = 0; q < 9; q++) { fc.src[q] = src[q]; fc.dst[q] = ov[q]; }
+  fc.nf = 9;
   RhsArgs a{};
   a.h = c->f.h; a.m = c->f.m; a.rho = c->f.rho; a.p = c->f.p; a.c = c->f.c; a.T = c->f.T; a.cp = c->f.cp;
   a.vx = c->f.vx; a.vy = c->f.vy; a.vz = c->f.vz; a.svx = c->f.svx; a.svy = c->f.svy; a.svz = c->f.svz;
@@ -2747,10 +2999,10 @@ extern "C" int psph_rhs(psph_ctx *c, double dt) {
   a.beta2 = 2.0 * k.beta; a.kheat = 20.0 * k.eps_half / k.prandtl;
   a.lans = k.lans; a.dim = k.dim; a.eos = eos_const(k); a.pairs = c->d_u64 + 2;
   hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 2, 0ull, 1);
-  if (n) PSPH_TRY(ensure_visits(c));
+  if (n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 3);
-    if (n) PSPH_TRY((launch_visits<RhsPass<float>, RhsPass<float, true, true>, RhsPass<float, false>, RhsPass<double>>(c, a)));
+    if (n) PSPH_TRY((launch_groups<RhsPass<float>, RhsPass<float, true, true>, RhsPass<float, false>, RhsPass<double>>(c, a, fc)));
   }
   HIP_TRY(hipGetLastError());
   std::swap(c->f.vx, c->dsp[1]); std::swap(c->f.vy, c->dsp[2]); std::swap(c->f.vz, c->dsp[3]);
@@ -2765,13 +3017,10 @@ extern "C" int psph_density(psph_ctx *c) {
   if (!c->grid_valid) return fail(PSPH_EINVAL, "density: call psph_neighbors first");
   const psph_config &k = c->cfg;
   uint32_t n = (uint32_t)c->n;
-  if (n) {
-    FieldCopy fc{};
-    fc.src[0] = c->f.rho; fc.dst[0] = c->dsp[1];
-    fc.src[1] = c->f.e; fc.dst[1] = c->dsp[2];
-    fc.nf = 2;
-    hipLaunchKernelGGL(k_copy_nontargets, blocks(n), 256, 0, c->stream, n, c->f.bc, fc);
-  }
+  FieldCopy fc{};
+  fc.src[0] = c->f.rho; fc.dst[0] = c->dsp[1];
+  fc.src[1] = c->f.e; fc.dst[1] = c->dsp[2];
+  fc.nf = 2;
   DensArgs a{};
   a.h = c->f.h; a.m = c->f.m; a.rho = c->f.rho; a.e = c->f.e; a.bc = c->f.bc; a.phase = c->f.phase;
   a.o_rho = c->dsp[1]; a.o_e = c->dsp[2]; a.xi = c->f.xi; a.p = c->f.p; a.c = c->f.c; a.T = c->f.T;
@@ -2785,10 +3034,10 @@ extern "C" int psph_density(psph_ctx *c) {
     const double en = kInvSqrtPi * k.e_smooth_ratio;
     a.e_norm = k.dim == 3 ? en * en * en : en;
   }
-  if (n) PSPH_TRY(ensure_visits(c));
+  if (n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 4);
-    if (n) PSPH_TRY((launch_visits<DensPass<float>, DensPass<float, true, true>, DensPass<float, false>, DensPass<double>>(c, a)));
+    if (n) PSPH_TRY((launch_groups<DensPass<float>, DensPass<float, true, true>, DensPass<float, false>, DensPass<double>>(c, a, fc)));
   }
   HIP_TRY(hipGetLastError());
   std::swap(c->f.rho, c->dsp[1]);
@@ -2806,11 +3055,10 @@ extern "C" int psph_vsmooth(psph_ctx *c) {
   a.bc = c->f.bc; a.svx = c->f.svx; a.svy = k.dim == 3 ? c->f.svy : nullptr; a.svz = k.dim == 3 ? c->f.svz : nullptr;
   a.cutoff = k.cutoff; a.cutoff2 = k.cutoff2;
   a.o_wn = c->rec ? c->rec->d[RF_WNV] : nullptr;
-  a.ok_test = c->rec ? 1 : 0;
-  if (c->n) PSPH_TRY(ensure_visits(c));
+  if (c->n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 5);
-    if (c->n) PSPH_TRY((launch_visits<VsmPass<float>, VsmPass<float, true>, VsmPass<float>, VsmPass<double>>(c, a)));
+    if (c->n) PSPH_TRY((launch_groups<VsmPass<float>, VsmPass<float, true>, VsmPass<float>, VsmPass<double>>(c, a, FieldCopy{})));
   }
   HIP_TRY(hipGetLastError());
   return check_err(c, "vsmooth");
