@@ -555,9 +555,9 @@ __global__ __launch_bounds__(kWave) void k_pairs(PairCommon pc, typename P::Args
 // into the windows' barriers); the next tile through registers while one is
 // worked on (density and filter 7.5 -> 25 ms at 4M).
 // Against the masks of 32 targets x 2 lanes, us per launch (RHS, density, filter,
-// masks): 1M FP64 6755, 3231, 2733, 560 (before: 8257, 3894, 3049, 992); 4M
-// FP32-exp 15446, 7663, 7451, 1933 (18057, 8047, 6634, 3843); 1.7k FP64 in 65k
-// particles, where 54 waves of 32 targets left the chip idle, 117, 80, 76, 22
+// masks): 1M FP64 6808, 3168, 2589, 563 (before: 8257, 3894, 3049, 992); 4M
+// FP32-exp 14990, 7235, 6838, 1939 (18057, 8047, 6634, 3843); 1.7k FP64 in 65k
+// particles, where 54 waves of 32 targets left the chip idle, 112, 75, 68, 22
 // (508, 299, 273, 151).
 // ---------------------------------------------------------------------------
 constexpr int kGroup = 8;                      // targets of a group
@@ -921,7 +921,7 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
   for (int k = 0; k < P::NACC; k++) acc[k] = 0;
   uint32_t npairs = 0;                             // of all targets (wave-uniform)
   uint64_t bad = 0;                                // lanes that met an invalid neighbour (wave-uniform)
-  const bool slow = FROZEN || gc.gl.fast[gid] == 0 || pc.gflag != nullptr;
+  const bool slow = FROZEN || __builtin_amdgcn_readfirstlane(gc.gl.fast[gid]) == 0 || pc.gflag != nullptr;
   const uint32_t nv = __builtin_amdgcn_readfirstlane(gc.gl.num[gid]);
   const_ptr<uint32_t> vis = (const_ptr<uint32_t>)(uintptr_t)(gc.gl.visit + __builtin_amdgcn_readfirstlane(gc.gl.off[gid]));
   uint32_t ahead[4] = {0, 0, 0, 0};                // the next visit
@@ -930,7 +930,7 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
   double2 xy, zh;
   uint32_t j = 0;
   typename P::Rec r;
-  uint32_t nq = 0, nl = 0;                         // queued places, streams that hold theirs in registers
+  uint32_t nl = 0;                                 // streams that hold their particle in registers
   for (uint32_t v = 0; v <= nv; v++) {
     uint32_t base = 0;
     uint64_t m = 0;
@@ -956,19 +956,19 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
       m = 0xffu >> held;
       if ((uint32_t)lane < kStreams - held) queue[held + lane] = (uint8_t)kWave;
     }
-    nq = held + (uint32_t)__popcll(m);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // tile and queue are there
-    for (uint32_t q = 0; q < nq; q += kStreams) {
-      const uint32_t take = min(nq - q, (uint32_t)kStreams);
-      if (stream >= nl && stream < take) {
-        const uint32_t p = queue[q + stream];
-        xy = st.xy[p];
-        zh = st.zh[p];
-        P::load(st, p, r);
-        j = base + p;
-      }
-      nl = take;
-      if (take < kStreams) break;
+    // the streams below nl hold theirs
+    auto load = [&](const uint8_t *at) {
+      const uint32_t p = at[stream];
+      xy = st.xy[p];
+      zh = st.zh[p];
+      P::load(st, p, r);
+      if (slow) j = base + p;
+    };
+    const uint8_t *qp = queue;
+    uint32_t left = held + (uint32_t)__popcll(m);
+    for (; left >= kStreams; left -= kStreams, qp += kStreams) {
+      if (stream >= nl) load(qp);
       nl = 0;
       double dx[3];
       dx[0] = xi[0] - xy.x;
@@ -1005,6 +1005,8 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
       }
       if (__builtin_amdgcn_inverse_ballot_w64(in)) P::template pair_d<D>(a, T, r, hk, dx, amax, acc);
     }
+    if (stream >= nl && stream < left) load(qp);
+    nl = left;
   }
   double sum[P::NACC];
 #pragma unroll
@@ -1197,7 +1199,8 @@ struct RhsPass {
     double m64, mpv64;
     R m, V, rho, c, T, cp, vx, vy, vz, PV2, mV;
   };
-  static constexpr int kWaves = 4;             // per SIMD: at most 128 VGPRs
+  // waves per SIMD: 96 VGPRs hold the FP32-exp and FP32-pure forms, 128 the others
+  static constexpr int kWaves = std::is_same<R, double>::value || (MIXED && !FX) ? 4 : 5;
   __device__ static void load_target(const Args &a, uint32_t i, Tgt &t, Own &o) {
     t.hh = 0.5 * a.h[i];
     const double rho = a.rho[i];
