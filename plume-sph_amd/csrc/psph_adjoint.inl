@@ -1198,73 +1198,136 @@ struct BcondAdjIn {
   const double *gx, *gy, *gz;       // positions at the search (wall ghosts do not move)
   const double *h, *m, *rho, *vx, *vy, *vz, *e, *xi;   // the values the refresh read
   const double *wrec;
-  const uint32_t *cs;
+  const uint32_t *toff;
+  const float4 *tbox;
   GridDesc grid;
   double h_new;                      // h of an erupt ghost that turned real in update_pos
   double rfac;                       // per-axis reach over h (both support tests, with margin)
 };
 
-__global__ void k_adj_bcond_contr(uint32_t n, BcondArgs g, BcondAdjIn in, BcondAdj cf, LamPtrs l) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const int b = in.bcn[j];
-  if (b != 100 && b != 99 && b != 1) return;        // contr_image (particle.h:562-565)
-  const double pj[3] = {in.xn[j], in.yn[j], in.zn[j]};
-  int bj[3];
-  if (!bucket_of(g, pj, bj)) return;
-  // images lie in the ground bucket layer or the one above it
-  if (bj[2] > g.bzg + 2) return;
-  const double hj = in.bc0[j] == 0 ? in.h_new : in.h[j];
-  const double mj[3] = {pj[0], pj[1], 2 * g.zg - pj[2]};
-  const double reach = in.rfac * hj;
-  const int nn[3] = {in.grid.nx, in.grid.ny, in.grid.nz};
-  int c0[3], c1[3];
+// One wavefront per kAdjGroup consecutive particles; those that contribute
+// gather the wall ghosts that hold their image.  The tiles within reach of the
+// mirror points are tested a lane each, and those with a refreshed ghost taken
+// in turn, a ghost a lane, against every contributor; a lane adds its ghosts'
+// shares to each contributor's sums, which are summed over the lanes at the end
+// in a fixed order.  A thread per contributor that walked the cells alone was a
+// chain of loads, one ghost after the other: 3108 -> 285 us per reversed step at
+// 30k real particles (228k in all).  The chain row, tile, ghost bounds it still.
+constexpr int kAdjGroup = 4;
+__global__ __launch_bounds__(kWave, 2) void k_adj_bcond_contr(uint32_t n, BcondArgs g, BcondAdjIn in, BcondAdj cf,
+                                                              LamPtrs l) {
+  constexpr int NS = 10;                    // vx, vy, vz, e, xi, rho, m, x, y, z
+  __shared__ TileScratch scratch;
+  const int lane = threadIdx.x;
+  const uint32_t j = blockIdx.x * kAdjGroup + (uint32_t)lane;
+  // the contributors, on the first lanes
+  double p[3] = {0, 0, 0}, mir[3] = {0, 0, 0}, h = 1, reach = 0, ir = 0, m = 0, v[3] = {0, 0, 0}, e = 0, xi = 0;
+  int b[3] = {0, 0, 0};
+  bool act = lane < kAdjGroup && j < n && contr_image(in.bcn[j]);
+  if (act) {
+    p[0] = in.xn[j]; p[1] = in.yn[j]; p[2] = in.zn[j];
+    // images lie in the ground bucket layer or the one above it
+    act = bucket_of(g, p, b) && b[2] <= g.bzg + 2;
+  }
+  const uint32_t acts = (uint32_t)__ballot(act);
+  if (!acts) return;
+  double lo[3], hi[3];
+  if (act) {
+    h = in.bc0[j] == 0 ? in.h_new : in.h[j];
+    reach = in.rfac * h;
+    ir = 1.0 / in.rho[j]; m = in.m[j];
+    v[0] = in.vx[j]; v[1] = in.vy[j]; v[2] = in.vz[j];
+    e = in.e[j]; xi = in.xi[j];
+    mir[0] = p[0]; mir[1] = p[1]; mir[2] = 2 * g.zg - p[2];
+  }
   for (int k = 0; k < 3; k++) {
-    if (in.grid.inv_e > 0) {
-      c0[k] = cell_of(mj[k] - reach, in.grid.lo[k], in.grid.inv_e, nn[k]);
-      c1[k] = cell_of(mj[k] + reach, in.grid.lo[k], in.grid.inv_e, nn[k]);
-    } else {
-      c0[k] = c1[k] = 0;
+    lo[k] = act ? mir[k] - reach : HUGE_VAL;
+    hi[k] = act ? mir[k] + reach : -HUGE_VAL;
+    for (int o = 1; o < kAdjGroup; o <<= 1) {
+      lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
+      hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
     }
   }
-  const double ir = 1.0 / in.rho[j], mj_ = in.m[j];
-  const double vj[3] = {in.vx[j], in.vy[j], in.vz[j]}, ej = in.e[j], xij = in.xi[j];
-  const double ih = 1.0 / hj, nk = kInvSqrtPi * ih, nk3 = nk * nk * nk;
-  double lvx = 0, lvy = 0, lvz = 0, le = 0, lxi = 0, lrho = 0, lm = 0, lx[3] = {0, 0, 0};
-  for (int cz = c0[2]; cz <= c1[2]; cz++)
-    for (int cy = c0[1]; cy <= c1[1]; cy++)
-      for (int cx = c0[0]; cx <= c1[0]; cx++) {
-        const uint32_t cell = ((uint32_t)cz * in.grid.ny + cy) * in.grid.nx + cx;
-        for (uint32_t q = in.cs[cell], qe = in.cs[cell + 1]; q < qe; q++) {
-          if (in.bc0[q] != 2 || !(in.wrec[q] > 0)) continue;
-          const double refc[3] = {in.gx[q], in.gy[q], 2 * g.zg - in.gz[q]};
-          int bi[3];
-          if (!bucket_of(g, refc, bi)) continue;
-          if (abs(bj[0] - bi[0]) > 1 || abs(bj[1] - bi[1]) > 1 || abs(bj[2] - bi[2]) > 1) continue;
-          const double amax = fmax(fabs(refc[0] - pj[0]), fmax(fabs(refc[1] - pj[1]), fabs(refc[2] - pj[2])));
-          if (!(amax <= g.cutoff2 * hj) || g.cut.outside(amax, hj)) continue;
-          const double dx[3] = {refc[0] - pj[0], refc[1] - pj[1], refc[2] - pj[2]};
-          double expt = 0;
-          for (int k = 0; k < 3; k++) { const double sk = dx[k] * ih; expt += sk * sk; }
-          const double w = nk3 * exp(-expt);
-          const double mw = mj_ * w, mwr = mw * ir;
-          const bool nbr = bj[0] != bi[0] || bj[1] != bi[1] || bj[2] != bi[2];
-          const double av[3] = {cf.f[BA_AVX][q], cf.f[BA_AVY][q], cf.f[BA_AVZ][q]};
-          const double ae = cf.f[BA_AE][q], axi = nbr ? cf.f[BA_AXI][q] : 0.0;
-          const double s = av[0] * vj[0] + av[1] * vj[1] + av[2] * vj[2] + ae * ej + axi * xij + cf.f[BA_B][q];
-          const double lw = cf.f[BA_ARHO][q] + s * ir;
-          lvx += av[0] * mwr; lvy += av[1] * mwr; lvz += av[2] * mwr;
-          le += ae * mwr;
-          lxi += axi * mwr;
-          lrho -= s * mwr * ir;
-          lm += lw * w;
-          const double gw = lw * mw * 2 * ih * ih;          // dW/dx_j = W 2 (r_i - x_j) / h^2
-          for (int k = 0; k < 3; k++) lx[k] += gw * dx[k];
+  int c0[3] = {0, 0, 0}, c1[3] = {0, 0, 0};
+  const int nn[3] = {in.grid.nx, in.grid.ny, in.grid.nz};
+  if (in.grid.inv_e > 0)
+    for (int k = 0; k < 3; k++) {
+      c0[k] = __builtin_amdgcn_readfirstlane(cell_of(lo[k], in.grid.lo[k], in.grid.inv_e, nn[k]));
+      c1[k] = __builtin_amdgcn_readfirstlane(cell_of(hi[k], in.grid.lo[k], in.grid.inv_e, nn[k]));
+    }
+  // what a contributor brings to its pairs, read back where used
+  struct Contr { double p[3], mir[3], reach, h, ih2, nk3, ir, m, v[3], e, xi; int b[3]; };
+  __shared__ Contr con[kAdjGroup];
+  if (lane < kAdjGroup) {
+    const double ih = 1.0 / h, nk = kInvSqrtPi * ih;
+    Contr c;
+    for (int k = 0; k < 3; k++) { c.p[k] = p[k]; c.mir[k] = mir[k]; c.v[k] = v[k]; c.b[k] = b[k]; }
+    c.reach = reach; c.h = h; c.ih2 = ih * ih; c.nk3 = nk * nk * nk;
+    c.ir = ir; c.m = m; c.e = e; c.xi = xi;
+    con[lane] = c;
+  }
+  double s[NS][kAdjGroup];
+#pragma unroll
+  for (int q = 0; q < NS; q++)
+    for (int u = 0; u < kAdjGroup; u++) s[q][u] = 0;
+  tiles_in_reach(in.toff, in.tbox, in.grid, c0, c1, scratch, 0, 1, [&](const float4 &tlo, const float4 &thi) {
+    // wall ghosts do not move: the tile's box holds them still
+    uint32_t near = 0;
+#pragma unroll
+    for (int u = 0; u < kAdjGroup; u++) near |= box_distance(tlo, thi, con[u].mir) <= con[u].reach ? 1u << u : 0u;
+    return near & acts;
+  }, [&](uint32_t (*todo)[3], uint32_t nt) {
+    const uint32_t kept = tiles_holding(todo, nt, [&](uint32_t q) { return in.bc0[q] == 2 && in.wrec[q] > 0; });
+    for (uint32_t t = 0; t < kept; t++) {
+      const uint32_t base = __builtin_amdgcn_readfirstlane(todo[t][0]);
+      const uint32_t cnt = __builtin_amdgcn_readfirstlane(todo[t][1]);
+      const uint32_t gm = __builtin_amdgcn_readfirstlane(todo[t][2]);
+      const uint32_t q = base + min((uint32_t)lane, cnt - 1u);
+      const double r0 = in.gx[q], r1 = in.gy[q], r2 = 2 * g.zg - in.gz[q];
+      const double refc[3] = {r0, r1, r2};
+      int bi[3];
+      const bool ok = (uint32_t)lane < cnt && in.bc0[q] == 2 && in.wrec[q] > 0 && bucket_of(g, refc, bi);
+      if (!__any(ok)) continue;
+      double a0 = 0, a1 = 0, a2 = 0, ae = 0, ax = 0, ar = 0, ab = 0;
+      if (ok) {
+        a0 = cf.f[BA_AVX][q]; a1 = cf.f[BA_AVY][q]; a2 = cf.f[BA_AVZ][q];
+        ae = cf.f[BA_AE][q]; ax = cf.f[BA_AXI][q]; ar = cf.f[BA_ARHO][q]; ab = cf.f[BA_B][q];
+      }
+#pragma unroll
+      for (int u = 0; u < kAdjGroup; u++) {
+        if (!((gm >> u) & 1)) continue;
+        asm volatile("" ::: "memory");
+        const Contr &c = con[u];
+        const int d0 = c.b[0] - bi[0], d1 = c.b[1] - bi[1], d2 = c.b[2] - bi[2];
+        const double dx[3] = {r0 - c.p[0], r1 - c.p[1], r2 - c.p[2]};
+        const double amax = fmax(fabs(dx[0]), fmax(fabs(dx[1]), fabs(dx[2])));
+        const bool near = max(abs(d0), max(abs(d1), abs(d2))) <= 1;
+        if (ok & near & (amax <= g.cutoff2 * c.h) & !g.cut.outside(amax, c.h)) {
+          const double w = c.nk3 * exp_neg((dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]) * c.ih2);
+          const double mw = c.m * w, mwr = mw * c.ir;
+          const double axi = (d0 | d1 | d2) != 0 ? ax : 0.0;
+          const double sj = a0 * c.v[0] + a1 * c.v[1] + a2 * c.v[2] + ae * c.e + axi * c.xi + ab;
+          const double lw = ar + sj * c.ir;
+          s[0][u] = fma(a0, mwr, s[0][u]);
+          s[1][u] = fma(a1, mwr, s[1][u]);
+          s[2][u] = fma(a2, mwr, s[2][u]);
+          s[3][u] = fma(ae, mwr, s[3][u]);
+          s[4][u] = fma(axi, mwr, s[4][u]);
+          s[5][u] -= sj * mwr * c.ir;
+          s[6][u] = fma(lw, w, s[6][u]);
+          const double gw = lw * mw * 2 * c.ih2;            // dW/dx_j = W 2 (r_i - x_j) / h^2
+          for (int k = 0; k < 3; k++) s[7 + k][u] = fma(gw, dx[k], s[7 + k][u]);
         }
       }
-  l.f[L_VX][j] += lvx; l.f[L_VY][j] += lvy; l.f[L_VZ][j] += lvz;
-  l.f[L_E][j] += le; l.f[L_XI][j] += lxi; l.f[L_RHO][j] += lrho; l.f[L_M][j] += lm;
-  l.f[L_X][j] += lx[0]; l.f[L_Y][j] += lx[1]; l.f[L_Z][j] += lx[2];
+    }
+  });
+  constexpr int to[NS] = {L_VX, L_VY, L_VZ, L_E, L_XI, L_RHO, L_M, L_X, L_Y, L_Z};
+  const uint32_t u = (uint32_t)lane / 16;
+#pragma unroll
+  for (int q = 0; q < NS; q++) {
+    const double t = wave_sum4(s[q][0], s[q][1], s[q][2], s[q][3]);
+    if (lane % 16 == 0 && ((acts >> u) & 1)) l.f[to[q]][blockIdx.x * kAdjGroup + u] += t;
+  }
 }
 
 static int adj_bcond(psph_ctx *c, Adjoint &A, const StepRec &R, ThetaGrad &th) {
@@ -1288,11 +1351,12 @@ static int adj_bcond(psph_ctx *c, Adjoint &A, const StepRec &R, ThetaGrad &th) {
   in.vx = R.d[RF_V1X]; in.vy = R.d[RF_V1Y]; in.vz = R.d[RF_V1Z];
   in.e = R.d[RF_E2]; in.xi = R.d[RF_XI2];
   in.wrec = R.d[RF_BW];
-  in.cs = R.cs;
+  in.toff = R.toff;
+  in.tbox = R.tbox;
   in.grid = R.grid;
   in.h_new = k.ratio_sml_dx * k.h_air;
   in.rfac = std::min(k.cutoff, k.cutoff2) * (1 + 1e-9) + 1e-12;
-  hipLaunchKernelGGL(k_adj_bcond_contr, blocks(n), 256, 0, st, n, g, in, cf, l);
+  hipLaunchKernelGGL(k_adj_bcond_contr, blocks(n, kAdjGroup), kWave, 0, st, n, g, in, cf, l);
   HIP_TRY(hipGetLastError());
   return 0;
 }

@@ -1840,167 +1840,318 @@ __device__ inline bool bucket_of(const BcondArgs &a, const double *p, int *b) {
   return ok;
 }
 
-// One wavefront per kBcondSpan consecutive particles (in cell order, so a
-// wave's ghosts and their images are compact): the wave stages the candidate cells'
-// particles 64 at a time into LDS, with their bucket indices and 1/rho; each
-// lane holding an imaged ghost marks the staged candidates that reach its
-// image, then walks only those, in index order.
-// consecutive particles per wavefront: 32 (lanes 32-63 only stage and test
-// candidates) gives twice the waves to hide the staging latency behind;
-// 1.74 ms per refresh at 4M against 1.83 ms with 64 and 2.19 ms with 16
-constexpr uint32_t kBcondSpan = 32;
-__global__ __launch_bounds__(kWave) void k_bcond(uint32_t n, BcondArgs a) {
-  __shared__ double sx[kWave], sy[kWave], sz[kWave], sh[kWave], smw[kWave], sir[kWave];
-  __shared__ double svx[kWave], svy[kWave], svz[kWave], se[kWave], sxi[kWave];
-  __shared__ double sqx[kWave], sqy[kWave], sqz[kWave];
-  __shared__ int sbk[3][kWave];
-  const int lane = threadIdx.x;
-  const uint32_t i = blockIdx.x * kBcondSpan + lane;
-  double coord[3] = {0, 0, 0}, refc[3] = {0, 0, 0};
-  int bi[3] = {0, 0, 0};
-  bool act = false;
-  if ((uint32_t)lane < kBcondSpan && i < n && a.bc[i] == 2) {
-    coord[0] = a.x[i]; coord[1] = a.y[i]; coord[2] = a.z[i];
-    int bg[3];
-    if (bucket_of(a, coord, bg) && bg[2] == a.bzg) {
-      refc[0] = coord[0]; refc[1] = coord[1]; refc[2] = 2 * a.zg - coord[2];
-      act = bucket_of(a, refc, bi);
+// Particle::contr_image (particle.h:562-565)
+__device__ inline bool contr_image(int bc) { return bc == 100 || bc == 99 || bc == 1; }
+
+// the image of wall ghost i and its bucket, if it has one
+__device__ inline bool ghost_image(const BcondArgs &a, uint32_t i, double *coord, double *refc, int *bi) {
+  if (a.bc[i] != 2) return false;
+  coord[0] = a.x[i]; coord[1] = a.y[i]; coord[2] = a.z[i];
+  int bg[3];
+  if (!bucket_of(a, coord, bg) || bg[2] != a.bzg) return false;
+  refc[0] = coord[0]; refc[1] = coord[1]; refc[2] = 2 * a.zg - coord[2];
+  return bucket_of(a, refc, bi);
+}
+
+// Every tile of the cell box c0..c1 for which near() (a lane per tile; a mask of
+// the wave's items that the tile may concern) is not 0, by one wave, `part` of
+// `parts` that share them in turn.  take(todo, count) gets up to 2 kWave of them:
+// first particle, particle count, mask.
+struct TileScratch {
+  uint32_t rowpre[kWave], rowtile[kWave];
+  uint32_t todo[2 * kWave][3];
+};
+template <class Near, class Take>
+__device__ __forceinline__ void tiles_in_reach(const uint32_t *toff, const float4 *tbox, const GridDesc &g,
+                                               const int *c0, const int *c1, TileScratch &sc, uint32_t part,
+                                               uint32_t parts, Near near, Take take) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  const uint32_t ry = (uint32_t)(c1[1] - c0[1] + 1), rows = ry * (uint32_t)(c1[2] - c0[2] + 1);
+  uint32_t nt = 0, seen = 0;
+  for (uint32_t rb = 0; rb < rows; rb += kWave) {
+    // the lanes take a row of cells each: its first tile, tiles up to it
+    const uint32_t r = rb + lane;
+    uint32_t first = 0, len = 0;
+    if (r < rows) {
+      const uint32_t row = ((uint32_t)(c0[2] + (int)(r / ry)) * g.ny + (uint32_t)(c0[1] + (int)(r % ry))) * g.nx;
+      first = toff[row + c0[0]];
+      len = toff[row + c1[0] + 1] - first;
     }
-  }
-  if (!__any(act)) return;
-  // Each active lane's cells within reach of its image form a box, walked
-  // in increasing cell index with a cursor; the wave visits the union of the
-  // boxes in that order (the smallest pending cell of any lane next).  A
-  // lane's hits therefore come cell by cell in increasing index, as in the
-  // bounding-box walk, without the cells between far-apart images (a wave's
-  // ghosts can straddle two rows of cells).
-  const int nn[3] = {a.g.nx, a.g.ny, a.g.nz};
-  int c0[3], c1[3], cur[3];
-  for (int k = 0; k < 3; k++) {
-    if (a.g.inv_e > 0) {
-      c0[k] = cell_of(refc[k] - a.reach, a.g.lo[k], a.g.inv_e, nn[k]);
-      c1[k] = cell_of(refc[k] + a.reach, a.g.lo[k], a.g.inv_e, nn[k]);
-    } else {
-      c0[k] = c1[k] = 0;
+    uint32_t upto = len;
+    for (uint32_t o = 1; o < kWave; o <<= 1) {
+      const uint32_t v = (uint32_t)__shfl_up((int)upto, o);
+      if (lane >= o) upto += v;
     }
-    cur[k] = c0[k];
-  }
-  constexpr uint32_t kDone = 0xffffffffu;
-  uint32_t mine = act ? ((uint32_t)cur[2] * a.g.ny + cur[1]) * a.g.nx + cur[0] : kDone;
-  double u0 = 0, u1 = 0, u2 = 0, u3 = 0, u4 = 0, wnorm = 0, ks = 0;
-  for (;;) {
-    uint32_t cell = mine;
-    for (int o = 32; o > 0; o >>= 1) cell = min(cell, (uint32_t)__shfl_xor((int)cell, o));
-    if (cell == kDone) break;
-    const bool here = mine == cell;
-    if (here) {
-      if (++cur[0] > c1[0]) {
-        cur[0] = c0[0];
-        if (++cur[1] > c1[1]) {
-          cur[1] = c0[1];
-          ++cur[2];
-        }
+    sc.rowpre[lane] = upto - len;
+    sc.rowtile[lane] = first;
+    const uint32_t ntiles = __builtin_amdgcn_readlane(upto, kWave - 1);
+    const bool last = rb + kWave >= rows;         // its first turn takes what is left, also without tiles
+    for (uint32_t kb = 0; kb < ntiles || (last && kb == 0); kb += kWave) {
+      const uint32_t k = kb + lane;
+      uint32_t m = 0, base = 0, cnt = 0;
+      if (k < ntiles) {
+        uint32_t ra = 0;                          // the last row that starts at or before k
+        for (uint32_t o = kWave / 2; o > 0; o >>= 1)
+          if (sc.rowpre[ra + o] <= k) ra += o;
+        const uint32_t t = sc.rowtile[ra] + (k - sc.rowpre[ra]);
+        const float4 tlo = tbox[2 * t], thi = tbox[2 * t + 1];
+        base = __float_as_uint(tlo.w);
+        cnt = __float_as_uint(thi.w);
+        m = near(tlo, thi);
       }
-      mine = cur[2] > c1[2] ? kDone : ((uint32_t)cur[2] * a.g.ny + cur[1]) * a.g.nx + cur[0];
+      const uint64_t all = __ballot(m != 0);
+      const bool mine = m != 0 && (seen + lanes_below(all)) % parts == part;
+      seen += (uint32_t)__popcll(all);
+      const uint64_t mt = __ballot(mine);
+      if (mine) {
+        uint32_t *e = sc.todo[nt + lanes_below(mt)];
+        e[0] = base; e[1] = cnt; e[2] = m;
+      }
+      nt += (uint32_t)__popcll(mt);
+      if (nt > kWave || (last && kb + kWave >= ntiles)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        take(sc.todo, nt);
+        nt = 0;
+      }
     }
-    const uint32_t lo = a.cs[cell], hi = a.cs[cell + 1];
-    uint32_t tl = a.toff[cell];
-    for (uint32_t base = lo; base < hi; base += kWave, tl++) {
-      // A tile is staged only if some lane of this cell's box can reach it:
-      // its particles have moved by at most the displacement that the reach
-      // includes, so the tile box at grid time within reach of the image is
+  }
+}
+
+// of the tiles in todo (count of them), those that hold a particle for which
+// of(j) is true, moved to the front; four tiles' loads at a time
+template <class Of>
+__device__ __forceinline__ uint32_t tiles_holding(uint32_t (*todo)[3], uint32_t count, Of of) {
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  uint32_t kept = 0;
+  for (uint32_t t = 0; t < count; t += 4) {
+    uint32_t e[4][3];
+    bool has[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const uint32_t *p = todo[min(t + u, count - 1)];
+      for (int d = 0; d < 3; d++) e[u][d] = __builtin_amdgcn_readfirstlane(p[d]);
+      has[u] = of(e[u][0] + min(lane, e[u][1] - 1u));
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (t + u >= count || !__any(has[u])) continue;
+      if (lane < 3) todo[kept][lane] = lane == 0 ? e[u][0] : lane == 1 ? e[u][1] : e[u][2];
+      kept++;
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  return kept;
+}
+
+// the largest per-axis distance of r from a tile's box
+__device__ inline double box_distance(const float4 &lo, const float4 &hi, const double *r) {
+  return fmax(fmax(fmax((double)lo.x - r[0], r[0] - (double)hi.x), fmax((double)lo.y - r[1], r[1] - (double)hi.y)),
+              fmax((double)lo.z - r[2], r[2] - (double)hi.z));
+}
+
+// Wall-ghost refresh.  A workgroup takes kBcondGroup consecutive particles that
+// hold an imaged ghost (in cell order, so their images are compact); its waves
+// share the tiles within reach.  A wave tests the tiles, a lane each, drops
+// those without a contributor, then takes the others in turn: a particle a
+// lane, whose weight and fields stay in registers while the images pass by, and
+// whose successor's loads are under way meanwhile.  Each lane adds its
+// particle's share to every ghost's sums; they are summed over lanes and waves
+// at the end, in a fixed order.
+//
+// Bound by VALU issue (57 % of the time at 228k particles), then by the chain of
+// loads row, tile, particle.  A lane per ghost that walked its own hits ran as
+// long as the fullest lane and left the chip to one wave per 32 particles, most
+// of them without a ghost: us per refresh 600 -> 118 at 228k particles (30k
+// real), 962 -> 396 at 1M, 1440 -> 888 at 4M.  8 ghosts by 2 waves of 2 per
+// SIMD; 4 ghosts by 2 waves of 3 per SIMD take 127, 435, 984, by 4 waves 132,
+// 498, 1149: a group's own work (images, rows, tile tests) is done by each wave.
+constexpr int kBcondGroup = 8;                 // consecutive particles: 7 sums each in registers
+constexpr int kBcondWaves = 2;
+constexpr unsigned kBcondGrid = 1024;          // workgroups: 4 per CU, all resident
+
+// the groups with an imaged ghost, in any order (a group's result does not
+// depend on its place)
+__global__ void k_bcond_list(uint32_t n, BcondArgs a, uint32_t *list, unsigned long long *count) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = threadIdx.x & (kWave - 1);
+  double coord[3], refc[3];
+  int bi[3];
+  const uint64_t act = __ballot(i < n && ghost_image(a, i, coord, refc, bi));
+  const bool first = lane % kBcondGroup == 0 && ((act >> lane) & ((1u << kBcondGroup) - 1));
+  const uint64_t has = __ballot(first);
+  if (!has) return;
+  uint32_t at = 0;
+  if (lane == 0) at = (uint32_t)atomicAdd(count, (unsigned long long)__popcll(has));
+  at = __builtin_amdgcn_readfirstlane(at);
+  if (first) list[at + lanes_below(has)] = i / kBcondGroup;
+}
+
+// the four values' sums over the wave: row r of 16 lanes gets value r's, in
+// every lane
+__device__ inline double wave_sum4(double v0, double v1, double v2, double v3) {
+  double v = swap_add<1>(swap_add<2>(v0, v2), swap_add<2>(v1, v3));
+  v += row_move<0x128>(v);                        // row_ror 8, 4, 2, 1
+  v += row_move<0x124>(v);
+  v += row_move<0x122>(v);
+  v += row_move<0x121>(v);
+  return v;
+}
+
+// a candidate as it lies in memory
+template <bool FROZEN>
+struct BcondRaw {
+  double x, y, z, h, m, rho, vx, vy, vz, e, xi, px, py, pz;
+  int bc;
+  __device__ void read(const BcondArgs &a, const uint32_t *tile, int lane) {
+    const uint32_t j = __builtin_amdgcn_readfirstlane(tile[0]) +
+                       min((uint32_t)lane, __builtin_amdgcn_readfirstlane(tile[1]) - 1u);
+    bc = a.bc[j];
+    x = a.x[j]; y = a.y[j]; z = a.z[j];
+    if constexpr (FROZEN) { px = a.px[j]; py = a.py[j]; pz = a.pz[j]; }
+    h = a.h[j]; m = a.m[j]; rho = a.rho[j];
+    vx = a.vx[j]; vy = a.vy[j]; vz = a.vz[j];
+    e = a.e[j]; xi = a.xi[j];
+  }
+};
+
+// FROZEN: a frozen replay, where the support tests read px, py, pz
+template <bool FROZEN>
+__global__ __launch_bounds__(kBcondWaves * kWave, 2) void k_bcond(uint32_t n, BcondArgs a, const uint32_t *list,
+                                                                const unsigned long long *count) {
+  constexpr int NS = 7;                           // rho, v, e, normaliser, xi
+  __shared__ double part[2][kBcondWaves][NS][kBcondGroup];
+  struct Image { double r[3]; int b[3]; };
+  // a wave's own: the images are read back where used, not kept in registers
+  __shared__ Image image[kBcondWaves][kBcondGroup];
+  __shared__ TileScratch scratch[kBcondWaves];
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t total = __builtin_amdgcn_readfirstlane((uint32_t)*count);
+  // an XCD's workgroups share a stretch of the list
+  const uint32_t per = (total + kXcds - 1) / kXcds, xcd = blockIdx.x % kXcds;
+  const uint32_t end = min(total, (xcd + 1) * per);
+  uint32_t turn = 0;
+  for (uint32_t k = xcd * per + blockIdx.x / kXcds; k < end; k += gridDim.x / kXcds, turn++) {
+    const uint32_t i = __builtin_amdgcn_readfirstlane(list[k]) * kBcondGroup + (uint32_t)lane;
+    double at[3], refc[3] = {0, 0, 0};
+    int bi[3] = {0, 0, 0};
+    const bool act = lane < kBcondGroup && i < n && ghost_image(a, i, at, refc, bi);
+    Image *img = image[wave];
+    const uint32_t acts = (uint32_t)__ballot(act);
+    if (lane < kBcondGroup)
+      for (int d = 0; d < 3; d++) { img[lane].r[d] = refc[d]; img[lane].b[d] = bi[d]; }
+    double lo[3], hi[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      lo[d] = act ? refc[d] : HUGE_VAL;
+      hi[d] = act ? refc[d] : -HUGE_VAL;
+      for (int o = 1; o < kBcondGroup; o <<= 1) {
+        lo[d] = fmin(lo[d], __shfl_xor(lo[d], o));
+        hi[d] = fmax(hi[d], __shfl_xor(hi[d], o));
+      }
+    }
+    int c0[3], c1[3];
+    const int nn[3] = {a.g.nx, a.g.ny, a.g.nz};
+    for (int d = 0; d < 3; d++) {
+      c0[d] = c1[d] = 0;
+      if (a.g.inv_e > 0) {
+        c0[d] = __builtin_amdgcn_readfirstlane(cell_of(lo[d] - a.reach, a.g.lo[d], a.g.inv_e, nn[d]));
+        c1[d] = __builtin_amdgcn_readfirstlane(cell_of(hi[d] + a.reach, a.g.lo[d], a.g.inv_e, nn[d]));
+      }
+    }
+    double s[NS][kBcondGroup];
+#pragma unroll
+    for (int q = 0; q < NS; q++)
+      for (int g = 0; g < kBcondGroup; g++) s[q][g] = 0;
+    tiles_in_reach(a.toff, a.tbox, a.g, c0, c1, scratch[wave], wave, kBcondWaves, [&](const float4 &tlo, const float4 &thi) {
+      // A tile's particles have moved by at most the displacement that the
+      // reach includes: its box at grid time within reach of an image is
       // necessary for any of them to be within the kernel box now.
-      const float4 tlo = a.tbox[2 * tl], thi = a.tbox[2 * tl + 1];
-      const bool near_t = here && fmax((double)tlo.x - refc[0], refc[0] - (double)thi.x) <= a.reach &&
-                          fmax((double)tlo.y - refc[1], refc[1] - (double)thi.y) <= a.reach &&
-                          fmax((double)tlo.z - refc[2], refc[2] - (double)thi.z) <= a.reach;
-      if (!__any(near_t)) continue;
-      const uint32_t j = base + lane;
-      bool ok = false;
-      if (j < hi) {
-        const int b = a.bc[j];
-        const double qj[3] = {a.px[j], a.py[j], a.pz[j]};
+      uint32_t near = 0;
+#pragma unroll
+      for (int g = 0; g < kBcondGroup; g++) near |= box_distance(tlo, thi, img[g].r) <= a.reach ? 1u << g : 0u;
+      return near & acts;
+    }, [&](uint32_t (*todo)[3], uint32_t nt) {
+      // without the tiles that hold no contributor (wall ghosts only)
+      const uint32_t kept = tiles_holding(todo, nt, [&](uint32_t j) { return contr_image(a.bc[j]); });
+      BcondRaw<FROZEN> nx;
+      if (kept) nx.read(a, todo[0], lane);
+      for (uint32_t t = 0; t < kept; t++) {
+        const BcondRaw<FROZEN> c = nx;
+        const uint32_t gm = __builtin_amdgcn_readfirstlane(todo[t][2]);
+        const uint32_t n_in = __builtin_amdgcn_readfirstlane(todo[t][1]);
+        if (t + 1 < kept) nx.read(a, todo[t + 1], lane);
+        double q[3] = {c.x, c.y, c.z};
+        if constexpr (FROZEN) { q[0] = c.px; q[1] = c.py; q[2] = c.pz; }
         int bj[3];
-        ok = (b == 100 || b == 99 || b == 1) && bucket_of(a, qj, bj);   // contr_image (particle.h:562-565)
-        if (ok) {
-          sx[lane] = a.x[j]; sy[lane] = a.y[j]; sz[lane] = a.z[j];
-          sqx[lane] = qj[0]; sqy[lane] = qj[1]; sqz[lane] = qj[2];
-          sh[lane] = a.h[j]; smw[lane] = a.m[j]; sir[lane] = 1.0 / a.rho[j];
-          svx[lane] = a.vx[j]; svy[lane] = a.vy[j]; svz[lane] = a.vz[j];
-          se[lane] = a.e[j]; sxi[lane] = a.xi[j];
-          for (int k = 0; k < 3; k++) sbk[k][lane] = bj[k];
-        }
-      }
-      if (!ok) sbk[0][lane] = -1000;            // never within one bucket of an image
-      const bool any_contr = __any(ok);          // e.g. tiles of wall ghosts only
-      __syncthreads();
-      const uint32_t cnt = min((uint32_t)kWave, hi - base);
-      if (any_contr) {
-        // phase 1, transposed: lane l tests staged candidate l against the
-        // image of each lane within reach of the tile, one lane g at a time;
-        // lane g keeps the ballot (bit q: candidate q reaches g's image)
-        uint64_t mask = 0;
-        uint64_t need = __ballot(near_t);
-        const bool cand = (uint32_t)lane < cnt;
-        const double ox = sqx[lane], oy = sqy[lane], oz = sqz[lane], oh = sh[lane];
-        const int o0 = sbk[0][lane], o1 = sbk[1][lane], o2 = sbk[2][lane];
-        while (need) {
-          const int g = __builtin_ctzll(need);
-          need &= need - 1;
-          const double r0 = __shfl(refc[0], g), r1 = __shfl(refc[1], g), r2 = __shfl(refc[2], g);
-          const int b0 = __shfl(bi[0], g), b1 = __shfl(bi[1], g), b2 = __shfl(bi[2], g);
-          const bool near = abs(o0 - b0) <= 1 && abs(o1 - b1) <= 1 && abs(o2 - b2) <= 1;
-          const double amax = fmax(fabs(r0 - ox), fmax(fabs(r1 - oy), fabs(r2 - oz)));
+        const bool ok = (uint32_t)lane < n_in && contr_image(c.bc) && bucket_of(a, q, bj);
+        const double ih = rcp_newton(c.h), ih2 = ih * ih, nk = kInvSqrtPi * ih;
+        const double mk = c.m * (nk * nk * nk), mr = mk * rcp_newton(c.rho);
+#pragma unroll
+        for (int g = 0; g < kBcondGroup; g++) {
+          if (!((gm >> g) & 1)) continue;
+          asm volatile("" ::: "memory");
+          const double r0 = img[g].r[0], r1 = img[g].r[1], r2 = img[g].r[2];
+          const int d0 = bj[0] - img[g].b[0], d1 = bj[1] - img[g].b[1], d2 = bj[2] - img[g].b[2];
+          const double amax = fmax(fabs(r0 - q[0]), fmax(fabs(r1 - q[1]), fabs(r2 - q[2])));
+          const bool nb = max(abs(d0), max(abs(d1), abs(d2))) <= 1;
           // in_support; W = 0 outside the kernel box
-          const bool in = cand & near & (amax <= a.cutoff2 * oh) & !a.cut.outside(amax, oh);
-          const uint64_t bal = __ballot(in);
-          mask = lane == g ? bal : mask;
-        }
-        // phase 2: the lane's own hits, in index order
-        while (mask) {
-          const uint32_t q = (uint32_t)__builtin_ctzll(mask);
-          mask &= mask - 1;
-          const double hj = sh[q];
-          const double dx[3] = {refc[0] - sx[q], refc[1] - sy[q], refc[2] - sz[q]};
-          const double ih = 1.0 / hj;
-          double expt = 0;
-          for (int k = 0; k < 3; k++) { const double sk = dx[k] * ih; expt += sk * sk; }
-          const double nk = kInvSqrtPi * ih;
-          const double w = nk * nk * nk * exp(-expt);
-          const double ir = sir[q];
-          const double mw = smw[q] * w;
-          u0 += mw;
-          u1 += mw * svx[q] * ir;
-          u2 += mw * svy[q] * ir;
-          u3 += mw * svz[q] * ir;
-          u4 += mw * se[q] * ir;
-          wnorm += mw * ir;
-          if (sbk[0][q] != bi[0] || sbk[1][q] != bi[1] || sbk[2][q] != bi[2]) ks += mw * sxi[q] * ir;
+          if (ok & nb & (amax <= a.cutoff2 * c.h) & !a.cut.outside(amax, c.h)) {
+            const double dx = r0 - c.x, dy = r1 - c.y, dz = r2 - c.z;
+            const double ex = exp_neg((dx * dx + dy * dy + dz * dz) * ih2);
+            const double w = mr * ex;
+            s[0][g] = fma(mk, ex, s[0][g]);
+            s[1][g] = fma(w, c.vx, s[1][g]);
+            s[2][g] = fma(w, c.vy, s[2][g]);
+            s[3][g] = fma(w, c.vz, s[3][g]);
+            s[4][g] = fma(w, c.e, s[4][g]);
+            s[5][g] += w;
+            s[6][g] = fma(w, (d0 | d1 | d2) != 0 ? c.xi : 0.0, s[6][g]);   // not from the image's own bucket
+          }
         }
       }
-      __syncthreads();
+    });
+    double (*pt)[NS][kBcondGroup] = part[turn & 1];
+#pragma unroll
+    for (int q = 0; q < NS; q++)
+#pragma unroll
+      for (int g = 0; g < kBcondGroup; g += 4) {
+        const double v = wave_sum4(s[q][g], s[q][g + 1], s[q][g + 2], s[q][g + 3]);
+        if (lane % 16 == 0) pt[wave][q][g + lane / 16] = v;
+      }
+    __syncthreads();
+    // a wave in turn finishes; the others go on with the next group, and its
+    // sums' places are written again only past the next barrier
+    if (wave != turn % kBcondWaves || lane >= kBcondGroup || !((acts >> lane) & 1)) continue;
+    asm volatile("" ::: "memory");
+    const double coord[3] = {a.x[i], a.y[i], a.z[i]}, *mirror = img[lane].r;
+    double u[NS];
+#pragma unroll
+    for (int q = 0; q < NS; q++) {
+      u[q] = 0;
+      for (int w = 0; w < kBcondWaves; w++) u[q] += pt[w][q][lane];
     }
+    const double wnorm = u[5];
+    if (a.wrec && i < a.wrec_n) a.wrec[i] = wnorm;
+    double nrm[3];
+    mirror_normal(coord, mirror, nrm);
+    if (wnorm > 0) {
+      u[0] /= wnorm; u[1] /= wnorm; u[2] /= wnorm; u[3] /= wnorm; u[4] /= wnorm;
+      u[6] /= wnorm;
+    } else {
+      u[0] = 1; u[1] = u[2] = u[3] = u[4] = 0; u[6] = 0;
+    }
+    const double vdotn = u[1] * nrm[0] + u[2] * nrm[1] + u[3] * nrm[2];
+    a.rho[i] = u[0];
+    a.vx[i] = u[1] - 2 * vdotn * nrm[0];
+    a.vy[i] = u[2] - 2 * vdotn * nrm[1];
+    a.vz[i] = u[3] - 2 * vdotn * nrm[2];
+    a.e[i] = u[4];
+    a.xi[i] = u[6];
+    double p, c, T, gam, cp = a.cp[i];
+    eos_dev(a.eos, u[0], u[4], u[6], p, c, T, gam, &cp);
+    a.p[i] = p; a.c[i] = c; a.T[i] = T; a.gam[i] = gam; a.cp[i] = cp;
   }
-  if (!act) return;
-  if (a.wrec && i < a.wrec_n) a.wrec[i] = wnorm;
-  double nrm[3];
-  mirror_normal(coord, refc, nrm);
-  if (wnorm > 0) {
-    u0 /= wnorm; u1 /= wnorm; u2 /= wnorm; u3 /= wnorm; u4 /= wnorm;
-    ks = ks / wnorm;
-  } else {
-    u0 = 1; u1 = u2 = u3 = u4 = 0; ks = 0;
-  }
-  const double vdotn = u1 * nrm[0] + u2 * nrm[1] + u3 * nrm[2];
-  a.rho[i] = u0;
-  a.vx[i] = u1 - 2 * vdotn * nrm[0];
-  a.vy[i] = u2 - 2 * vdotn * nrm[1];
-  a.vz[i] = u3 - 2 * vdotn * nrm[2];
-  a.e[i] = u4;
-  a.xi[i] = ks;
-  double p, c, T, gam, cp = a.cp[i];
-  eos_dev(a.eos, u0, u4, ks, p, c, T, gam, &cp);
-  a.p[i] = p; a.c[i] = c; a.T[i] = T; a.gam[i] = gam; a.cp[i] = cp;
 }
 
 // largest per-axis speed of the particles update_pos moves (reals with the
@@ -3217,7 +3368,13 @@ static int apply_bcond_grid(psph_ctx *c, double disp, double *wrec = nullptr, si
   a.px = qx ? qx : c->f.x; a.py = qx ? qy : c->f.y; a.pz = qx ? qz : c->f.z;
   const double hm = std::max(c->h_max, k.ratio_sml_dx * k.h_air);
   a.reach = k.cutoff * hm * (1 + 1e-9) + disp * (1 + 1e-9);
-  hipLaunchKernelGGL(k_bcond, blocks(c->n, kBcondSpan), kWave, 0, c->stream, (uint32_t)c->n, a);
+  const uint32_t n = (uint32_t)c->n;
+  unsigned long long *count = c->d_u64 + 5;
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, count, 0ull, 1);
+  hipLaunchKernelGGL(k_bcond_list, blocks(n), 256, 0, c->stream, n, a, c->usp, count);
+  const unsigned grid = std::min(kBcondGrid, (n / kBcondGroup / kXcds + 1) * kXcds);
+  if (qx) hipLaunchKernelGGL(k_bcond<true>, grid, kBcondWaves * kWave, 0, c->stream, n, a, c->usp, count);
+  else hipLaunchKernelGGL(k_bcond<false>, grid, kBcondWaves * kWave, 0, c->stream, n, a, c->usp, count);
   HIP_TRY(hipGetLastError());
   return 0;
 }
