@@ -256,9 +256,8 @@ __device__ inline uint32_t refb_pack(uint32_t x, uint32_t y, uint32_t z) { retur
 // buckets at most one apart on every axis: per field 1024 + a - b + 1 (the
 // guard bits 10 and 21 stop borrows between fields), (a - b + 1) mod 1024 for z
 __device__ inline bool refb_adjacent(uint32_t a, uint32_t b) {
-  if (a == kDead || b == kDead) return false;
   const uint32_t d = ((a | 0x00200400u) - b) + 0x00400801u;
-  return ((d & 0x7ffu) - 1024u <= 2u) & (((d >> 11) & 0x7ffu) - 1024u <= 2u) & ((d >> 22) <= 2u);
+  return (a != kDead) & (b != kDead) & ((d & 0x7ffu) - 1024u <= 2u) & (((d >> 11) & 0x7ffu) - 1024u <= 2u) & ((d >> 22) <= 2u);
 }
 
 // the smoothing length at list time, and the reference bucket
@@ -407,132 +406,66 @@ __device__ inline ChunkBox chunk_list_box(const PairCommon &pc, const double *p,
   return b;
 }
 
-// Work split of a wavefront: kChunk targets (consecutive in the cell's fine
-// Morton order, so they sit within ~2 particle spacings of each other), each
-// served by kSub lanes that take every kSub-th candidate of a staged tile.
-// The wave streams the union of its targets' neighbourhoods; with so compact
-// a chunk that union is little more than one neighbourhood, and a lane's hit
-// count per tile is bounded by 64 / kSub, so lanes rarely idle in phase 2.
-// The kSub partial sums of a target are combined by a fixed shuffle tree.
-#ifndef PSPH_SUB_LANES
-#define PSPH_SUB_LANES 2
-#endif
-constexpr int kSub = PSPH_SUB_LANES;
+// A chunk: up to kChunk targets, consecutive in the cell's fine Morton order, so
+// they sit within ~2 particle spacings of each other and the union of their
+// neighbourhoods is little more than one of them.  The reverse pair passes serve
+// each of a chunk's rows with kSub lanes that take every kSub-th candidate of a
+// staged tile; the partial sums are combined by a fixed shuffle tree.
+constexpr int kSub = 2;
 constexpr double kFar = 1.0e300;
 constexpr int kChunk = kWave / kSub;
 
-// Each pass supplies: Tile (LDS SoA), Tgt (registers), stage(), pair(),
-// combine() (sums a target's sub-lane partials), finish().
-template <int D, class P>
-__global__ __launch_bounds__(kWave) void k_pairs(PairCommon pc, typename P::Args a) {
+// List materialisation (parity checks only): one wavefront per chunk, a target a
+// lane.  The candidates accepted are exactly the reference's list
+// (neighs.cc:37-211).  out null counts, else device indices are written from
+// offset[i] on.
+template <int D>
+__global__ __launch_bounds__(kWave) void k_list(PairCommon pc, uint32_t *count, const uint32_t *offset, uint32_t *out) {
   __shared__ double sx[kWave], sy[kWave], sz[kWave];
   __shared__ uint32_t srefb[kWave];
-  __shared__ uint8_t sgh[kWave];   // boundary ghost (bc 1, 2), one byte each
-  __shared__ typename P::Tile tile;
-  // XCD-aware order: workgroups are dealt round-robin to the 8 XCDs, so
-  // XCD x runs workgroups x, x+8, ...; give it the contiguous chunk range
-  // [x*per, (x+1)*per) so neighbouring chunks share that XCD's L2.
-  const uint32_t nch = *pc.nchunks;
-  const uint32_t per = (nch + kXcds - 1) / kXcds;
-  const uint32_t local = blockIdx.x / kXcds;
-  if (local >= per) return;
-  const uint32_t chunk = (blockIdx.x % kXcds) * per + local;
-  if (chunk >= nch) return;
+  const uint32_t chunk = blockIdx.x;
+  if (chunk >= *pc.nchunks) return;
   const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const int lane = threadIdx.x;
-  const uint32_t slot = (uint32_t)lane / P::kSub, sub = (uint32_t)lane % P::kSub;
-  const bool active = slot < cc;
-  using Mask = typename std::conditional<(kWave / P::kSub > 32), uint64_t, uint32_t>::type;
-  const uint32_t i = pc.targets[cf + (active ? slot : 0)];
-
-  double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const uint32_t rb_i = pc.refb[i];
-  const double lf_i = pc.list_factor * pc.h_list[i];
-  typename P::Tgt t;
-  P::load_target(a, i, t);
-  // a chunk none of whose targets wants the pass (converged in an earlier
-  // iteration of the adaptive h) skips the traversal
-  if (!__any(active && P::want(t))) {
-    if (active && sub == 0) P::finish(a, t, i, pc.err);
-    return;
-  }
-  // the passes run here (adaptive h, list materialisation) accept list
-  // members only: the chunk visits the region its lists can reach
-  const ChunkBox box = chunk_list_box(pc, xi, lf_i, rb_i);
+  const uint32_t lane = threadIdx.x;
+  const bool active = lane < cc;
+  const uint32_t i = pc.targets[cf + (active ? lane : 0)];
+  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
+  const uint32_t rb = pc.refb[i];
+  const double lf = pc.list_factor * pc.h_list[i];
+  const ChunkBox box = chunk_list_box(pc, xi, lf, rb);
   const GridDesc &g = pc.tr.g;
-  P::init(tile, lane);
-  __syncthreads();
-
-  for (int pass = 0; pass < P::npasses(a); pass++) {
-    P::begin_pass(a, t, pass);
-    for (int cz = box.c0[2]; cz <= box.c1[2]; cz++)
-      for (int cy = box.c0[1]; cy <= box.c1[1]; cy++)
-        for (int cx = box.c0[0]; cx <= box.c1[0]; cx++) {
-          const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx + cx;
-          const uint32_t lo = pc.tr.cs[cell], hi = pc.tr.cs[cell + 1];
-          uint32_t tl = pc.tr.toff[cell];
-          for (uint32_t base = lo; base < hi; base += kWave, tl++) {
-            if (!tile_meets(box, pc.tr.tbox, tl)) continue;
-            const uint32_t j = base + lane;
-            if (j < hi) {
-              sx[lane] = pc.x[j]; sy[lane] = pc.y[j]; sz[lane] = pc.z[j];
-              srefb[lane] = pc.refb[j];
-              if (pc.gflag) { const int b = pc.bc[j]; sgh[lane] = b == 1 || b == 2; }
-              P::stage(a, j, tile, lane);
-            } else {
-              // empty slot: a position no predicate accepts (|dx| > every support)
-              sx[lane] = sy[lane] = sz[lane] = kFar;
-              srefb[lane] = ~0u;
-              sgh[lane] = 0;
-            }
-            __syncthreads();
-            const uint32_t cnt = min((uint32_t)kWave, hi - base);
-            if (active && P::want(t)) {
-              // phase 1: exact FP64 predicate on this lane's share of the tile,
-              // without branches (the same trip count on every lane, q < 64)
-              Mask mask = 0;
-              const uint32_t nb = (cnt + P::kSub - 1) / P::kSub;
-#pragma unroll 4
-              for (uint32_t b = 0; b < nb; b++) {
-                const uint32_t q = sub + b * P::kSub;
-                double amax = fabs(xi[0] - sx[q]);
-                if (D == 3) amax = fmax(amax, fmax(fabs(xi[1] - sy[q]), fabs(xi[2] - sz[q])));
-                // inside the kernel box (exact, see CutTest), list membership
-                // (neighs.cc:37-211: same bucket or 4.25 h_i box), in_support
-                // and the pass's own mask
-                bool in = !pc.cut.outside(amax, P::hker(a, t, tile, q));
-                in &= (pc.list_all != 0) | (srefb[q] == rb_i) |
-                      ((amax <= lf_i) & ((pc.list_adj == 0) || refb_adjacent(srefb[q], rb_i)));
-                in &= (q < cnt) & (amax <= t.supp) & P::extra(a, t, tile, q, base + q, i);
-                mask |= (Mask)in << b;
-              }
-              // phase 2: each lane walks its own hits
-              while (mask) {
-                const uint32_t b = (uint32_t)__builtin_ctzll((uint64_t)mask);
-                mask &= mask - 1;
-                const uint32_t q = sub + b * P::kSub;
-                double dx[3];
-                dx[0] = xi[0] - sx[q];
-                double amax = fabs(dx[0]);
-                if (D == 3) {
-                  dx[1] = xi[1] - sy[q]; dx[2] = xi[2] - sz[q];
-                  amax = fmax(amax, fmax(fabs(dx[1]), fabs(dx[2])));
-                }
-                P::pair(a, t, tile, q, base + q, i, dx, amax);
-                if (pc.gflag && sgh[q]) pc.gflag[base + q] = 1u;
-              }
-            }
-            __syncthreads();
+  uint32_t n = 0, o = active && out ? offset[i] : 0;
+  for (int cz = box.c0[2]; cz <= box.c1[2]; cz++)
+    for (int cy = box.c0[1]; cy <= box.c1[1]; cy++)
+      for (int cx = box.c0[0]; cx <= box.c1[0]; cx++) {
+        const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx + cx;
+        const uint32_t je = pc.tr.cs[cell + 1];
+        uint32_t tl = pc.tr.toff[cell];
+        for (uint32_t base = pc.tr.cs[cell]; base < je; base += kWave, tl++) {
+          if (!tile_meets(box, pc.tr.tbox, tl)) continue;
+          const uint32_t js = min(base + lane, je - 1);
+          sx[lane] = pc.x[js]; sy[lane] = pc.y[js]; sz[lane] = pc.z[js];
+          srefb[lane] = pc.refb[js];
+          __syncthreads();
+          const uint32_t cnt = active ? min((uint32_t)kWave, je - base) : 0;
+          for (uint32_t q = 0; q < cnt; q++) {
+            double amax = fabs(xi[0] - sx[q]);
+            if (D == 3) amax = fmax(amax, fmax(fabs(xi[1] - sy[q]), fabs(xi[2] - sz[q])));
+            // same bucket or the 4.25 h_i box (neighs.cc:37-211)
+            bool in = (amax <= lf) & ((pc.list_adj == 0) | refb_adjacent(srefb[q], rb));
+            in |= (srefb[q] == rb) | (pc.list_all != 0);
+            if (!in) continue;
+            if (out) out[o + n] = base + q;
+            n++;
           }
+          __syncthreads();
         }
-    if constexpr (P::kSub > 1) P::combine(t);
-    P::end_pass(a, t, pass, i, active);
-  }
-  if (active && sub == 0) P::finish(a, t, i, pc.err);
+      }
+  if (active && !out) count[i] = n;
 }
 
 // ---------------------------------------------------------------------------
-// Group passes.  The RHS, density and filter passes take their targets in
+// Group passes.  The RHS, density, filter and adaptive-h passes take their targets in
 // groups of kGroup consecutive targets of a cell, one wavefront per group.  For
 // every group and tile that can hold a pair of it, a 64-bit mask made once per
 // step says which of the tile's particles can be a pair of one of the group's
@@ -558,11 +491,12 @@ __global__ __launch_bounds__(kWave) void k_pairs(PairCommon pc, typename P::Args
 // masks): 1M FP64 6808, 3168, 2589, 563 (before: 8257, 3894, 3049, 992); 4M
 // FP32-exp 14990, 7235, 6838, 1939 (18057, 8047, 6634, 3843); 1.7k FP64 in 65k
 // particles, where 54 waves of 32 targets left the chip idle, 112, 75, 68, 22
-// (508, 299, 273, 151).
+// (508, 299, 273, 151), and 32, 19, 17 with 8 waves a group.
 // ---------------------------------------------------------------------------
 constexpr int kGroup = 8;                      // targets of a group
 constexpr int kStreams = kWave / kGroup;       // particles evaluated at a time
 constexpr int kGroupsPerChunk = kChunk / kGroup;
+constexpr int kMaxSplit = 8;                   // waves that share a group
 
 // Positions (x, y) and (z, h / 2) of every particle.
 struct Geom {
@@ -642,7 +576,7 @@ struct GroupLists {
   uint32_t *off, *num;      // per group: first visit, visits
   uint32_t *fast;           // per group: list membership and in_support cannot fail for a masked
                             // particle inside a pass's kernel box
-  uint32_t *cursor;         // visits handed out
+  unsigned long long *cursor;   // visits handed out
   uint32_t cap;             // visits that visit holds
 };
 
@@ -651,6 +585,10 @@ struct GroupCommon {
   GroupLists gl;
   double cutx;               // cut with a relative margin of 1e-12
   double h_max;
+  // lists for an iteration of the adaptive h: the kernel's h over h (0: lists
+  // for the three passes) and the targets that have converged
+  double c_smooth;
+  const uint32_t *done;
 };
 
 // The group of this workgroup, its target for this lane (lane % kGroup; past
@@ -725,15 +663,30 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
     // fast: the widest kernel box of the passes lies inside the list box and the
     // in_support box of every target and is narrower than a bucket, so that list
     // membership and in_support cannot fail for a particle inside it
-    double widest = gc.cutx * fmax(0.5 * hi + 0.5 * gc.h_max, hi);
-    fast = widest <= supp && (pc.list_all != 0 || (widest <= lf && widest * (1 + 1e-12) < pc.del));
     GroupBox B;
-    const double hg = group_max(hi);
-    widest = gc.cutx * fmax(0.5 * hg + 0.5 * gc.h_max, hg) * (1 + 1e-9);
-    B.chh = gc.cutx * (0.5 * hg);
-    B.ch = gc.cutx * hg;
+    double widest;
+    bool in = true;                  // the target takes part
+    if (gc.c_smooth > 0) {
+      // the kernel box of c_smooth h_i, and of the list no particle beyond its
+      // box and the target's bucket
+      const double hs = hi * gc.c_smooth;
+      const double box = gc.cutx * hs;
+      fast = box <= cutoff2 * hs && (pc.list_all != 0 || (box <= lf && box * (1 + 1e-12) < pc.del));
+      in = gc.done[i] == 0;
+      const double w = pc.list_all ? box : fmin(box, fmax(lf, pc.del * (1 + 1e-9)));
+      B.chh = -HUGE_VAL;
+      B.ch = group_max(in ? w : 0.0);
+      widest = B.ch * (1 + 1e-9);
+    } else {
+      widest = gc.cutx * fmax(0.5 * hi + 0.5 * gc.h_max, hi);
+      fast = widest <= supp && (pc.list_all != 0 || (widest <= lf && widest * (1 + 1e-12) < pc.del));
+      const double hg = group_max(hi);
+      widest = gc.cutx * fmax(0.5 * hg + 0.5 * gc.h_max, hg) * (1 + 1e-9);
+      B.chh = gc.cutx * (0.5 * hg);
+      B.ch = gc.cutx * hg;
+    }
     for (int d = 0; d < 3; d++) {
-      const double lo = group_min(xi[d]), up = group_max(xi[d]);
+      const double lo = group_min(in ? xi[d] : kFar), up = group_max(in ? xi[d] : -kFar);
       B.c[d] = 0.5 * lo + 0.5 * up;
       B.b[d] = fmax(up - B.c[d], B.c[d] - lo);
       B.b[d] += 2e-15 * (fabs(B.c[d]) + B.b[d]);
@@ -746,6 +699,7 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
       }
     }
     if (lane % kGroup == 0 && (uint32_t)lane / kGroup < ng) gb[lane / kGroup] = B;
+    if (!__any(in)) c1[0] = c0[0] - 1, c1[1] = c0[1] - 1;
   }
   const uint64_t fb = __ballot(fast);
   const int rows_y = c1[1] - c0[1] + 1, nrow = rows_y * (c1[2] - c0[2] + 1);
@@ -829,11 +783,12 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
       }
     }
     if (!write) {
-      uint32_t room = 0, at = 0;
+      uint32_t room = 0;
+      unsigned long long first = 0;
       for (uint32_t q = 0; q < kGroupsPerChunk; q++) room += num[q];
-      if (lane == 0) at = atomicAdd(gc.gl.cursor, room);
-      at = __builtin_amdgcn_readfirstlane(at);
-      if (at + room > gc.gl.cap || at + room < at) return;
+      if (lane == 0) first = atomicAdd(gc.gl.cursor, (unsigned long long)room);
+      uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)first);
+      if (__builtin_amdgcn_readfirstlane((uint32_t)(first >> 32)) || (unsigned long long)at + room > gc.gl.cap) return;
       for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
         off[q] = at;
         at += num[q];
@@ -867,10 +822,20 @@ template <class P>
 struct TileLds {
   double2 xy[kWave + 1], zh[kWave + 1];
   float4 a16[P::NA16][kWave + 1];
-  float a4[P::NA4 ? P::NA4 : 1][P::NA4 ? kWave + 1 : 1];
+  float a4[P::NA4 ? P::NA4 : 1][P::NA4 ? kWave + 4 : 4];   // (whole 16 bytes)
   __device__ const double2 *d2(int k) const { return (const double2 *)a16[k]; }
   __device__ const float4 *f4(int k) const { return a16[k]; }
   __device__ const float *f1(int k) const { return a4[k]; }
+};
+
+// one wave's LDS; the tile's place takes the wave's sums at the end
+template <class P>
+struct GroupLds {
+  union {
+    TileLds<P> st;
+    struct { double sum[P::NACC][kGroup]; uint64_t bad; uint32_t npairs; } tot;
+  };
+  uint8_t queue[2 * kWave];                        // places in the tile
 };
 
 template <class T>
@@ -894,27 +859,42 @@ __device__ inline double stream_sum(double v) {
 // Bound by VALU issue.  Whatever is left in the queue after a tile stays in the
 // registers of its streams (nl of them) while the next tile is staged.
 //
+// The waves of a workgroup (blockDim.x / 64) share a group: each takes its visits
+// in turn, in LDS of its own, and the first adds up their sums.
+//
 // FROZEN (a frozen replay): the predicates read g's and pc.x (the recorded
 // run's positions) and the pair arithmetic pc.ax; otherwise both are pc.x.
 template <int D, class P, bool FROZEN>
-__global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, GroupCommon gc, typename P::Args a) {
-  __shared__ TileLds<P> st;
-  __shared__ uint8_t queue[2 * kWave];             // places in the tile
+__global__ __launch_bounds__(kMaxSplit * kWave, P::kWaves) void k_group_pass(PairCommon pc, GroupCommon gc,
+                                                                             typename P::Args a) {
+  extern __shared__ char lds[];                    // a GroupLds<P> per wave
   uint32_t gid, i;
   const uint32_t nt = my_group(pc, gid, i);
   if (!nt) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), split = blockDim.x / kWave;
+  GroupLds<P> &own_lds = ((GroupLds<P> *)lds)[wave];
+  TileLds<P> &st = own_lds.st;
+  uint8_t *const queue = own_lds.queue;
   const uint32_t stream = (uint32_t)lane / kGroup, slot = (uint32_t)lane % kGroup;
   typename P::Own own;
   typename P::Tgt T;
   P::load_target(a, i, T, own);
   // a lane without a target of its own meets nothing
-  const double xi[3] = {slot < nt ? pc.x[i] : -kFar, pc.y[i], pc.z[i]};
+  const double xi[3] = {slot < nt && P::wants(T) ? pc.x[i] : -kFar, pc.y[i], pc.z[i]};
   double xa[3] = {0, 0, 0};
   if constexpr (FROZEN) { xa[0] = pc.ax[i]; xa[1] = pc.ay[i]; xa[2] = pc.az[i]; }
   if (lane == 0) {
     st.xy[kWave] = make_double2(kFar, kFar);
     st.zh[kWave] = make_double2(kFar, 0.0);
+  }
+  // what membership takes of the target: kept where every pair is tested
+  uint32_t ri = 0;
+  double lf = 0, supp = 0;
+  if constexpr (P::kRefb) {
+    ri = pc.refb[i];
+    lf = pc.list_factor * pc.h_list[i];
+    supp = P::support(a, i);
   }
   double acc[P::NACC];
 #pragma unroll
@@ -925,13 +905,13 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
   const uint32_t nv = __builtin_amdgcn_readfirstlane(gc.gl.num[gid]);
   const_ptr<uint32_t> vis = (const_ptr<uint32_t>)(uintptr_t)(gc.gl.visit + __builtin_amdgcn_readfirstlane(gc.gl.off[gid]));
   uint32_t ahead[4] = {0, 0, 0, 0};                // the next visit
-  if (nv)
-    for (int k = 0; k < 4; k++) ahead[k] = vis[k];
+  if (wave < nv)
+    for (int k = 0; k < 4; k++) ahead[k] = vis[(size_t)wave * 4 + k];
   double2 xy, zh;
   uint32_t j = 0;
   typename P::Rec r;
   uint32_t nl = 0;                                 // streams that hold their particle in registers
-  for (uint32_t v = 0; v <= nv; v++) {
+  for (uint32_t v = wave;; v += split) {
     uint32_t base = 0;
     uint64_t m = 0;
     const uint32_t held = nl;
@@ -939,7 +919,7 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
       base = ahead[0];
       const uint32_t cnt = ahead[1];
       m = (uint64_t)ahead[3] << 32 | ahead[2];
-      const_ptr<uint32_t> e = vis + (size_t)min(v + 1, nv - 1) * 4;
+      const_ptr<uint32_t> e = vis + (size_t)min(v + split, nv - 1) * 4;
       for (int k = 0; k < 4; k++) ahead[k] = e[k];
       const uint32_t from = base + min((uint32_t)lane, cnt - 1u);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the last tile has been read
@@ -982,14 +962,23 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
       if (slow) {
         const bool mine = (in >> lane) & 1;
         // list membership (neighs.cc:37-211: same bucket or 4.25 h_i box) and in_support
-        const uint32_t rj = mine ? pc.refb[j] : 0u, ri = pc.refb[i];
-        bool ok = mine & ((pc.list_all != 0) | (rj == ri) |
-                          ((amax <= pc.list_factor * pc.h_list[i]) & ((pc.list_adj == 0) || refb_adjacent(rj, ri))));
-        ok &= amax <= a.cutoff2 * a.h[i];
+        uint32_t rj;
+        if constexpr (P::kRefb) {
+          rj = r.refb;
+        } else {
+          rj = mine ? pc.refb[j] : 0u;
+          ri = pc.refb[i];
+          lf = pc.list_factor * pc.h_list[i];
+          supp = P::support(a, i);
+        }
+        bool member = amax <= lf;
+        if (pc.list_adj != 0) member &= refb_adjacent(rj, ri);
+        member |= (rj == ri) | (pc.list_all != 0);
+        bool ok = mine & member & (amax <= supp);
         if (pc.gflag) {
           // recorded step: the boundary ghosts (bc 1, 2) met as neighbours
           const int bj = ok ? pc.bc[j] : 0;
-          ok &= P::counts_ghost(bj);
+          ok &= P::counts_ghost(a, bj);
           if (ok && (bj == 1 || bj == 2)) pc.gflag[j] = 1u;
         }
         if constexpr (FROZEN) {
@@ -1005,6 +994,7 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
       }
       if (__builtin_amdgcn_inverse_ballot_w64(in)) P::template pair_d<D>(a, T, r, hk, dx, amax, acc);
     }
+    if (v >= nv) break;
     if (stream >= nl && stream < left) load(qp);
     nl = left;
   }
@@ -1012,6 +1002,20 @@ __global__ __launch_bounds__(kWave, P::kWaves) void k_group_pass(PairCommon pc, 
 #pragma unroll
   for (int k = 0; k < P::NACC; k++) sum[k] = stream_sum(acc[k]);
   for (int o = 32; o >= kGroup; o >>= 1) bad |= bad >> o;
+  if (split > 1) {
+    // the waves' sums, added in their order
+    if (lane < kGroup)
+      for (int k = 0; k < P::NACC; k++) own_lds.tot.sum[k][lane] = sum[k];
+    if (lane == 0) { own_lds.tot.bad = bad; own_lds.tot.npairs = npairs; }
+    __syncthreads();
+    if (wave != 0) return;
+    for (uint32_t w = 1; w < split; w++) {
+      const GroupLds<P> &o = ((GroupLds<P> *)lds)[w];
+      for (int k = 0; k < P::NACC; k++) sum[k] += o.tot.sum[k][lane % kGroup];
+      bad |= o.tot.bad;
+      npairs += o.tot.npairs;
+    }
+  }
   if ((uint32_t)lane < nt) P::finish(a, own, sum, ((bad >> lane) & 1u) != 0, i, pc.err);
   // pairs of the group's targets, without the targets themselves
   if constexpr (P::kCountPairs)
@@ -1024,35 +1028,11 @@ __device__ inline double sub_sum(double v) {
   for (int o = 1; o < S; o <<= 1) v += __shfl_xor(v, o);
   return v;
 }
-template <int S>
-__device__ inline uint32_t sub_sum_u(uint32_t v) {
-  for (int o = 1; o < S; o <<= 1) v += (uint32_t)__shfl_xor((int)v, o);
-  return v;
-}
-
-__device__ inline bool in_support(const double *dx, double h, int D) {
-  for (int k = 0; k < D; k++)
-    if (fabs(dx[k]) > h) return false;
-  return true;
-}
-
 constexpr double kInvSqrtPi = 0.564189583547756;   // sph_lib.cc:207
 
-// |dx_k| > 3 h (1 + 1e-12) on any axis implies fl(dx_k / h) > 3: the pair is
-// outside the kernel box and contributes exactly zero.
-template <int D>
-__device__ inline bool beyond(const double *dx, double bound) {
-  bool out = fabs(dx[0]) > bound;
-  if (D == 3) out = out || fabs(dx[1]) > bound || fabs(dx[2]) > bound;
-  return out;
-}
-constexpr double kCutMargin = 1.0 + 1e-12;
-
-// Each pass supplies, besides load_target/stage/pair/finish:
-//   hker(q):  smoothing length of the kernel-box test, extra(q): masks.
 // The pair arithmetic type R is double (FP64 form) or float (FP32-pair form):
-// the pair predicate (phase 1) is FP64 in both, so both forms visit exactly
-// the same pairs; accumulators, integration and the EOS stay FP64.
+// the pair predicate is FP64 in both, so both forms visit exactly the same
+// pairs; accumulators, integration and the EOS stay FP64.
 // ---------------------------------------------------------------------------
 // 1 / x in FP64 for normal x and 1 / x: the hardware estimate and two Newton
 // steps whose last rounds once (within a rounding of the quotient).  5
@@ -1263,7 +1243,10 @@ struct RhsPass {
   // adds is an exact zero (f dx, f v.r, no viscosity for v.r = 0, no heat for
   // |v_ij . dx| = 0), so no test is spent on it; the pair count leaves it out.
   __device__ static double hker(const Tgt &t, double hhj) { return t.hh + hhj; }
-  __device__ static bool counts_ghost(int) { return true; }
+  __device__ static bool counts_ghost(const Args &, int) { return true; }
+  __device__ static double support(const Args &a, uint32_t i) { return a.cutoff2 * a.h[i]; }
+  __device__ static bool wants(const Tgt &) { return true; }
+  static constexpr bool kRefb = false;
   __device__ static bool valid(const Rec &r) { return r.rho > R(0); }        // assert(uvecj[0] > 0)
   template <int D>
   __device__ static void pair_d(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *dxd, double,
@@ -1478,7 +1461,10 @@ struct DensPass {
   // the packed masses.  The energy-smoothing kernel (support 0.75 h_ij) lies
   // inside that box.
   __device__ static double hker(const Tgt &t, double hhj) { return t.hh + hhj; }
-  __device__ static bool counts_ghost(int) { return true; }
+  __device__ static bool counts_ghost(const Args &, int) { return true; }
+  __device__ static double support(const Args &a, uint32_t i) { return a.cutoff2 * a.h[i]; }
+  __device__ static bool wants(const Tgt &) { return true; }
+  static constexpr bool kRefb = false;
   __device__ static bool valid(const Rec &) { return true; }
   template <int D>
   __device__ static void pair_d(const Args &a, const Tgt &t, const Rec &s, double hijd, const double *ds, double amax,
@@ -1621,7 +1607,10 @@ struct VsmPass {
     r = Rec{u.x, {u.y, v.x, v.y}};
   }
   __device__ static double hker(const Tgt &t, double) { return t.hi; }
-  __device__ static bool counts_ghost(int b) { return contr_vel(b); }
+  __device__ static bool counts_ghost(const Args &, int b) { return contr_vel(b); }
+  __device__ static double support(const Args &a, uint32_t i) { return a.cutoff2 * a.h[i]; }
+  __device__ static bool wants(const Tgt &) { return true; }
+  static constexpr bool kRefb = false;
   __device__ static bool valid(const Rec &) { return true; }
   template <int D>
   __device__ static void pair_d(const Args &, const Tgt &t, const Rec &s, double, const double *ds, double, double *acc) {
@@ -1671,121 +1660,74 @@ struct VsmPass {
 struct AdaptArgs {
   const double *m;
   const int32_t *bc;
+  const uint32_t *refb;
   double *h;
   uint32_t *done;
   double cutoff, cutoff2, c_smooth, eta, ratio, thresh;
   int pghost, dim;
+  Packs pk;
 };
 
-// The kernel value comes from the FP64 exp table (exp_neg_tab, about an ulp),
-// or in the FX form (PSPH_FP32_EXP) from the FP32 exponential of the FP64
-// argument: its rounding is independent from pair to pair, so rho* and h
-// move by ~1e-9 relative over a particle's ~2000 list pairs.
+// The exponential is FP64 (exp_neg), or in the FX form (PSPH_FP32_EXP) the FP32
+// exponential of the FP64 argument: its rounding is independent from pair to
+// pair, so rho* and h move by ~1e-9 relative over a particle's ~2000 list pairs.
+// A candidate that does not contribute (contr_dens false) has a zero mass.  The
+// kernel box (4.5 h) reaches past the list box (4.25 h of list time), so list
+// membership is tested for every pair: the record carries the bucket.  Each
+// iteration has visits of its own, for the boxes of the h it starts from and the
+// targets that have not converged.  Bound by VALU issue.  60k targets, an
+// iteration (visits in brackets): 2264 us with a bit mask of 32 targets x 2
+// lanes, 577 (170) with groups.
 template <class R, bool FX = false>
 struct AdaptPass {
   using Args = AdaptArgs;
-  struct Tile {
-    R m[kWave];
-    int ok[kWave];
-  };
-  __device__ static void init(Tile &, int) {}
-  struct Tgt { double mi, hcur, Hs, supp, rho_star; R iHs, norm; bool done; };
-  static constexpr int kSub = ::kSub;
-  __device__ static void combine(Tgt &t) { t.rho_star = sub_sum<kSub>(t.rho_star); }
-  __device__ static int npasses(const Args &) { return 1; }
-  __device__ static void begin_pass(const Args &a, Tgt &t, int) {
-    t.Hs = t.hcur * a.c_smooth;
-    const double iHs = 1.0 / t.Hs;
-    t.iHs = (R)iHs;
-    t.supp = a.cutoff2 * t.Hs;
-    const double nk = kInvSqrtPi * iHs;
-    t.norm = (R)(a.dim == 3 ? nk * nk * nk : nk);
-    t.rho_star = 0;
+  static constexpr bool kCountPairs = false;
+  static constexpr int NACC = 1;
+  struct Own { double hcur; };
+  struct Tgt { double Hs, iHs; bool done; };
+  struct Rec { R m; uint32_t refb; };
+  static constexpr int kWaves = 6;             // per SIMD: at most 80 VGPRs
+  static constexpr bool kRefb = true;
+  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t, Own &o) {
+    o.hcur = a.h[i];
+    t.Hs = o.hcur * a.c_smooth;
+    t.iHs = 1.0 / t.Hs;
+    t.done = a.done[i] != 0;
   }
-  __device__ static bool want(const Tgt &t) { return !t.done; }
-  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t) {
-    t.mi = a.m[i]; t.hcur = a.h[i]; t.done = a.done[i] != 0;
+  __device__ static void pack(const Args &a, uint32_t j) {
+    a.pk.d2(0)[j] = make_double2(contr_dens(a.pghost, a.bc[j]) ? a.m[j] : 0.0,
+                                 __longlong_as_double((long long)a.refb[j]));
   }
-  __device__ static void stage(const Args &a, uint32_t j, Tile &s, int l) {
-    s.m[l] = (R)a.m[j];
-    s.ok[l] = contr_dens(a.pghost, a.bc[j]);
+  static constexpr int NA16 = 1, NA4 = 0;
+  template <class L>
+  __device__ static void load(const L &a, uint32_t j, Rec &r) {
+    const double2 u = a.d2(0)[j];
+    r = Rec{u.x, (uint32_t)__double_as_longlong(u.y)};
   }
-  __device__ static double hker(const Args &, const Tgt &t, const Tile &, uint32_t) { return t.Hs; }
-  __device__ static bool extra(const Args &, const Tgt &, const Tile &s, uint32_t q, uint32_t, uint32_t) { return s.ok[q] != 0; }
+  __device__ static double hker(const Tgt &t, double) { return t.Hs; }
+  __device__ static double support(const Args &a, uint32_t i) { return a.cutoff2 * (a.h[i] * a.c_smooth); }
+  __device__ static bool wants(const Tgt &t) { return !t.done; }
+  __device__ static bool counts_ghost(const Args &a, int b) { return contr_dens(a.pghost, b); }
+  __device__ static bool valid(const Rec &) { return true; }
   template <int D>
-  __device__ static void pair_d(const Args &a, Tgt &t, const Tile &s, uint32_t q, uint32_t, uint32_t,
-                                const double *dx, double) {
+  __device__ static void pair_d(const Args &, const Tgt &t, const Rec &s, double, const double *dx, double, double *acc) {
     R expt = 0;
 #pragma unroll
     for (int k = 0; k < D; k++) {
-      R sk = (R)dx[k] * t.iHs;
+      const R sk = (R)dx[k] * t.iHs;
       expt += sk * sk;
     }
-    t.rho_star += (double)(t.norm * (R)exp_neg_w<FX>((double)expt) * s.m[q]);
+    acc[0] += exp_neg_w<FX>(expt) * s.m;
   }
-  __device__ static void end_pass(const Args &a, Tgt &t, int, uint32_t, bool active) {
-    if (!active || t.done) return;
-    double Hold = t.hcur;
-    double Hnew = (a.dim == 3) ? a.eta * cbrt(t.mi / t.rho_star) : a.eta * (t.mi / t.rho_star);
-    t.hcur = a.ratio * Hnew;
-    if (fabs((Hnew - Hold) / Hold) < a.thresh) t.done = true;
-  }
-  __device__ static void finish(const Args &a, Tgt &t, uint32_t i, int *) {
-    a.h[i] = t.hcur;
-    a.done[i] = t.done ? 1u : 0u;
-  }
-};
-
-// ---------------------------------------------------------------------------
-// List materialisation (parity checks only): the candidates the skeleton's
-// membership rule accepts are exactly the reference's list (neighs.cc:37-211).
-// mode 0 counts, mode 1 writes device indices at offsets[i].
-// ---------------------------------------------------------------------------
-struct ListPass {
-  template <class T> __device__ static void init(T &, int) {}
-  struct Args {
-    int mode;
-    uint32_t *count;
-    const uint32_t *offset;
-    uint32_t *out;
-    double cutoff;
-  };
-  struct Tile { int dummy; };
-  struct Tgt { uint32_t n, o; double supp; };
-  static constexpr int kSub = 1;
-  __device__ static void combine(Tgt &) {}
-  __device__ static int npasses(const Args &) { return 1; }
-  __device__ static void begin_pass(const Args &, Tgt &, int) {}
-  __device__ static void end_pass(const Args &, Tgt &, int, uint32_t, bool) {}
-  __device__ static bool want(const Tgt &) { return true; }
-  __device__ static void load_target(const Args &a, uint32_t i, Tgt &t) {
-    t.n = 0;
-    t.o = a.mode ? a.offset[i] : 0;
-    t.supp = HUGE_VAL;
-  }
-  __device__ static void stage(const Args &, uint32_t, Tile &, int) {}
-  __device__ static double bound(const Args &, const Tgt &, const Tile &, uint32_t) { return HUGE_VAL; }
-  __device__ static double hker(const Args &, const Tgt &, const Tile &, uint32_t) { return HUGE_VAL; }
-  __device__ static bool extra(const Args &, const Tgt &, const Tile &, uint32_t, uint32_t, uint32_t) { return true; }
-  template <int D>
-  __device__ static void pair_d(const Args &a, Tgt &t, const Tile &, uint32_t, uint32_t j, uint32_t,
-                                const double *, double) {
-    if (a.mode) a.out[t.o + t.n] = j;
-    t.n++;
-  }
-  __device__ static void finish(const Args &a, Tgt &t, uint32_t i, int *) {
-    if (!a.mode) a.count[i] = t.n;
-  }
-};
-
-// Binds the dimension into the pass's pair routine for the skeleton.
-template <int D, class P>
-struct Bound : P {
-  // dx: the pair's position difference; amax: max_k |dx_k| of the positions
-  // the predicates read (the same dx except in a frozen replay)
-  __device__ static void pair(const typename P::Args &a, typename P::Tgt &t, const typename P::Tile &s,
-                             uint32_t q, uint32_t j, uint32_t i, const double *dx, double amax) {
-    P::template pair_d<D>(a, t, s, q, j, i, dx, amax);
+  __device__ static bool finish(const Args &a, const Own &o, const double *sum, bool, uint32_t i, int *) {
+    if (a.done[i] != 0) return true;
+    const double nk = kInvSqrtPi * (1.0 / (o.hcur * a.c_smooth));
+    const double rho_star = sum[0] * (a.dim == 3 ? nk * nk * nk : nk);
+    const double m = a.m[i];
+    const double Hnew = a.dim == 3 ? a.eta * cbrt(m / rho_star) : a.eta * (m / rho_star);
+    a.h[i] = a.ratio * Hnew;
+    if (fabs((Hnew - o.hcur) / o.hcur) < a.thresh) a.done[i] = 1u;
+    return true;
   }
 };
 
@@ -2424,7 +2366,9 @@ struct psph_ctx {
   // the group passes' lists and positions (made once per step) and particle records
   bool lists_valid = false;
   uint4 *gvisit = nullptr;
-  uint32_t *goff = nullptr, *gnum = nullptr, *gfast = nullptr, *gcursor = nullptr;
+  uint32_t *goff = nullptr, *gnum = nullptr, *gfast = nullptr;
+  uint32_t ngroups = 0;              // of the lists last built
+  unsigned long long *gcursor = nullptr;
   size_t gchunk_cap = 0;
   uint32_t gvisit_cap = 0;
   double2 *gxy = nullptr, *gzh = nullptr;
@@ -2557,8 +2501,8 @@ extern "C" int psph_create(const psph_config *cfg, size_t capacity, psph_ctx **o
     if (!rc) rc = dmalloc((void **)pp, capacity * 4);
   if (!rc) rc = dmalloc((void **)&c->flags, (capacity + 1) * 4);
   if (!rc) rc = dmalloc((void **)&c->tpos, (capacity + 1) * 4);
-  if (!rc) rc = dmalloc((void **)&c->nchunks, 4);
   if (!rc) rc = dmalloc((void **)&c->d_u64, 8 * 8);
+  if (!rc) { c->gcursor = c->d_u64 + 6; c->nchunks = (uint32_t *)(c->d_u64 + 7); }   // read in one copy
   if (!rc) rc = dmalloc((void **)&c->d_err, 2 * sizeof(int));
   if (!rc) rc = dmalloc((void **)&c->d_part, kRedBlocks * 8 * 8);
   if (rc) { psph_destroy(c); return rc; }
@@ -2585,8 +2529,8 @@ extern "C" int psph_destroy(psph_ctx *c) {
   for (auto p : c->dsp) if (p) hipFree(p);
   void *ptrs[] = {c->usp, c->isp, c->h_list, c->pid, c->pid_sp, c->refb, c->key_a, c->key_b, c->idx_a, c->idx_b,
                   c->flags, c->tpos, c->targets, c->cfirst, c->ccount, c->cs, c->tcnt, c->toff,
-                  c->cchunks, c->coff, c->tbox, c->nchunks, c->cub, c->d_u64, c->d_err, c->d_part,
-                  c->gvisit, c->goff, c->gnum, c->gfast, c->gcursor, c->gxy, c->gzh, c->px, c->py, c->pz,
+                  c->cchunks, c->coff, c->tbox, c->cub, c->d_u64, c->d_err, c->d_part,
+                  c->gvisit, c->goff, c->gnum, c->gfast, c->gxy, c->gzh, c->px, c->py, c->pz,
                   c->d_occ, c->d_conv, c->d_sides};
   for (auto p : ptrs) if (p) hipFree(p);
   for (auto p : c->pk) if (p) hipFree(p);
@@ -2953,13 +2897,11 @@ static unsigned chunk_grid(size_t n, size_t ncells, size_t csz) {
   return (unsigned)((ub + kXcds - 1) / kXcds * kXcds);
 }
 
-template <class P>
-static void launch_pairs(psph_ctx *c, const PairCommon &pc, const typename P::Args &a) {
-  unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk);
-  if (c->cfg.dim == 3)
-    hipLaunchKernelGGL((k_pairs<3, Bound<3, P>>), nb, kWave, 0, c->stream, pc, a);
-  else
-    hipLaunchKernelGGL((k_pairs<1, Bound<1, P>>), nb, kWave, 0, c->stream, pc, a);
+static void launch_list(psph_ctx *c, double reach, uint32_t *count, const uint32_t *offset, uint32_t *out) {
+  const PairCommon pc = make_common(c, reach);
+  const unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk);
+  if (c->cfg.dim == 3) hipLaunchKernelGGL(k_list<3>, nb, kWave, 0, c->stream, pc, count, offset, out);
+  else hipLaunchKernelGGL(k_list<1>, nb, kWave, 0, c->stream, pc, count, offset, out);
 }
 
 static GroupCommon group_common(psph_ctx *c) {
@@ -2971,16 +2913,12 @@ static GroupCommon group_common(psph_ctx *c) {
   return gc;
 }
 
-// Lists and positions of the group passes (positions, h and targets fixed since
-// the last psph_neighbors / adaptation).
-static int ensure_lists(psph_ctx *c) {
-  if (c->lists_valid) return 0;
-  StageTimer tm(c, 1);
+// memory of the group passes: positions, record arrays, per-group offsets
+static int group_memory(psph_ctx *c) {
   if (!c->gxy) PSPH_TRY(dmalloc((void **)&c->gxy, c->cap * sizeof(double2)));
   if (!c->gzh) PSPH_TRY(dmalloc((void **)&c->gzh, c->cap * sizeof(double2)));
   for (auto &p : c->pk)
     if (!p) PSPH_TRY(dmalloc(&p, c->cap * 16));
-  if (!c->gcursor) PSPH_TRY(dmalloc((void **)&c->gcursor, 4));
   if (c->chunk_cap > c->gchunk_cap) {
     uint32_t **arrs[] = {&c->goff, &c->gnum, &c->gfast};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
@@ -2988,32 +2926,56 @@ static int ensure_lists(psph_ctx *c) {
     for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, c->chunk_cap * kGroupsPerChunk * 4));
     c->gchunk_cap = c->chunk_cap;
   }
-  const PairCommon pc = make_common(c, c->reach_main);
+  return 0;
+}
+
+static void launch_geom(psph_ctx *c, const PairCommon &pc) {
   hipLaunchKernelGGL(k_geom, blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, pc.x, pc.y, pc.z, c->f.h, c->gxy, c->gzh);
+}
+
+// the groups' visits for the boxes that c_smooth and done say (GroupCommon)
+static int build_lists(psph_ctx *c, const PairCommon &pc, double c_smooth, const uint32_t *done) {
   // a group per wave up to a quarter of a million particles: at 77k 0.15 ms against
   // 0.20 with half a chunk; a chunk per wave beyond
   const uint32_t nsplit = c->n < (1u << 18) ? kGroupsPerChunk : 1;
   const unsigned G = chunk_grid(c->n, c->grid.ncells, kChunk) * nsplit;
   for (;;) {
-    const GroupCommon gc = group_common(c);
-    hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, (int *)c->gcursor, 0, 1);
+    GroupCommon gc = group_common(c);
+    gc.c_smooth = c_smooth;
+    gc.done = done;
+    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->gcursor, 0ull, 1);
     if (c->cfg.dim == 3)
       hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
     else
       hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
     HIP_TRY(hipGetLastError());
-    uint32_t total = 0;
-    HIP_TRY(hipMemcpyAsync(&total, c->gcursor, 4, hipMemcpyDeviceToHost, c->stream));
+    unsigned long long got[2] = {0, 0};         // visits; chunks (nchunks)
+    HIP_TRY(hipMemcpyAsync(got, c->gcursor, 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (total <= c->gvisit_cap) break;
+    const unsigned long long total = got[0];
+    c->ngroups = (uint32_t)got[1] * kGroupsPerChunk;
+    if (total <= c->gvisit_cap) return 0;
     // the visits outgrew their memory: this call only counted
+    constexpr unsigned long long kMost = 0xffffffffull;      // GroupLists::off
+    if (total > kMost) return fail(PSPH_ENOMEM, "%llu tile visits exceed the maximum of %llu", total, kMost);
     if (c->gvisit) hipFree(c->gvisit);
     c->gvisit = nullptr;
     c->gvisit_cap = 0;
-    const size_t want = std::min<size_t>((size_t)total + total / 8 + 1024, 0xffffffffu);
-    PSPH_TRY(dmalloc((void **)&c->gvisit, want * sizeof(uint4)));
+    const unsigned long long want = std::min(total + total / 8 + 1024, kMost);
+    PSPH_TRY(dmalloc((void **)&c->gvisit, (size_t)want * sizeof(uint4)));
     c->gvisit_cap = (uint32_t)want;
   }
+}
+
+// Lists and positions of the group passes (positions, h and targets fixed since
+// the last psph_neighbors / adaptation).
+static int ensure_lists(psph_ctx *c) {
+  if (c->lists_valid) return 0;
+  StageTimer tm(c, 1);
+  PSPH_TRY(group_memory(c));
+  const PairCommon pc = make_common(c, c->reach_main);
+  launch_geom(c, pc);
+  PSPH_TRY(build_lists(c, pc, 0.0, nullptr));
   c->lists_valid = true;
   return 0;
 }
@@ -3034,23 +2996,46 @@ __global__ void k_pack(uint32_t n, typename P::Args a, const int32_t *bc, FieldC
     for (int q = 0; q < fc.nf; q++) fc.dst[q][i] = fc.src[q][i];
 }
 
-template <int D, class P>
-static void launch_group_pass(psph_ctx *c, const PairCommon &pc, const GroupCommon &gc, const typename P::Args &a,
-                              const FieldCopy &fc) {
+// Waves per group.  A group alone is a chain of tile loads and pair blocks;
+// where groups are fewer than the chip has room for (about 5000 waves), several
+// waves share one.  RHS, density, filter, us, with 1 / 2 / 4 / 8 waves: 256
+// groups (FP64) 119, 74, 68 / 74, 45, 40 / 43, 27, 24 / 32, 19, 17; 4308 groups
+// (FP32-exp) 192, 105, 93 / 161, 95, 85 / 142, 87, 78 / 169, 108, 96; 10784
+// groups 364, 210, 188 / 341, 194, 175 / 332, 196, 177 / 406, 259, 232; 20416
+// groups (FP32-pair) 763, 500, 424 / 760, 490, 414 / 760, 485, 417 / 865, 594,
+// 513; 400k targets (FP32-pure) 1522, 832, 1083 / 1522, 828, 1081 / 1568, 874,
+// 1118.
+static unsigned group_split(uint32_t ngroups) {
+  return ngroups <= 1024 ? kMaxSplit : ngroups <= 16384 ? 4 : 1;
+}
+
+template <class P>
+static void launch_pack(psph_ctx *c, typename P::Args &a, const FieldCopy &fc) {
+  for (int k = 0; k < 5; k++) a.pk.p[k] = c->pk[k];
   hipLaunchKernelGGL((k_pack<P>), blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, a, c->f.bc, fc);
-  const unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk) * kGroupsPerChunk;
-  if (c->tape.mode == 2 && c->tape.frozen)
-    hipLaunchKernelGGL((k_group_pass<D, P, true>), nb, kWave, 0, c->stream, pc, gc, a);
-  else
-    hipLaunchKernelGGL((k_group_pass<D, P, false>), nb, kWave, 0, c->stream, pc, gc, a);
+}
+template <int D, class P>
+static void launch_group_kernel(psph_ctx *c, const PairCommon &pc, const GroupCommon &gc, const typename P::Args &a,
+                                bool frozen) {
+  const unsigned nb = (c->ngroups + kXcds - 1) / kXcds * kXcds;
+  if (!nb) return;
+  const unsigned split = group_split(c->ngroups);
+  const size_t lds = split * sizeof(GroupLds<P>);
+  if (frozen) hipLaunchKernelGGL((k_group_pass<D, P, true>), nb, split * kWave, lds, c->stream, pc, gc, a);
+  else hipLaunchKernelGGL((k_group_pass<D, P, false>), nb, split * kWave, lds, c->stream, pc, gc, a);
+}
+template <int D, class P>
+static void launch_group_pass(psph_ctx *c, const PairCommon &pc, const GroupCommon &gc, typename P::Args a,
+                              const FieldCopy &fc) {
+  launch_pack<P>(c, a, fc);
+  launch_group_kernel<D, P>(c, pc, gc, a, c->tape.mode == 2 && c->tape.frozen);
 }
 // the RHS, density and filter passes; PM, PX, PP, PD: the pass in the FP32-pair,
 // FP32-exp, FP32-pure and FP64 forms
 template <class PM, class PX, class PP, class PD>
-static int launch_groups(psph_ctx *c, typename PD::Args a, const FieldCopy &fc) {
+static int launch_groups(psph_ctx *c, const typename PD::Args &a, const FieldCopy &fc) {
   const PairCommon pc = make_common(c, c->reach_main);
   const GroupCommon gc = group_common(c);
-  for (int k = 0; k < 5; k++) a.pk.p[k] = c->pk[k];
   const int form = c->cfg.precision;
   if (c->cfg.dim == 3) {
     if (form == PSPH_FP32_PAIR) launch_group_pass<3, PM>(c, pc, gc, a, fc);
@@ -3091,25 +3076,32 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
   if (!c) return fail(PSPH_EINVAL, "null ctx");
   if (!c->grid_valid) return fail(PSPH_EINVAL, "adapt_h: call psph_neighbors first");
   const psph_config &k = c->cfg;
-  const bool all = k.list_all || k.dim == 1;
-  // the list never reaches past the own bucket or the 4.25 h_i box of list time
-  const double list_reach = all ? HUGE_VAL : std::max(k.list_factor * c->h_max, k.bucket_edge);
   AdaptArgs a{};
-  a.m = c->f.m; a.bc = c->f.bc; a.h = c->f.h; a.done = c->usp;
+  a.m = c->f.m; a.bc = c->f.bc; a.refb = c->refb; a.h = c->f.h; a.done = c->usp;
   a.cutoff = k.cutoff; a.cutoff2 = k.cutoff2; a.c_smooth = k.c_smooth; a.eta = k.eta;
   a.ratio = k.ratio_sml_dx; a.thresh = k.thresh; a.pghost = k.pghost_contrib; a.dim = k.dim;
-  if (c->n) HIP_TRY(hipMemsetAsync(c->usp, 0, c->n * 4, c->stream));
   double hmax = c->h_max;
-  for (int it = 0; it < k.num_loop; it++) {
-    const double reach = std::min(k.cutoff * k.c_smooth * hmax, list_reach) * (1 + 1e-9);
-    {
+  if (c->n && k.num_loop > 0) {
+    HIP_TRY(hipMemsetAsync(c->usp, 0, c->n * 4, c->stream));
+    PSPH_TRY(group_memory(c));
+    const PairCommon pc = make_common(c, c->reach_main);
+    launch_geom(c, pc);
+    // FP64 arithmetic in every form (h enters every later pass, and a
+    // relative error of h moves every kernel value by ~|s|^2 times as
+    // much); the FX form takes its exponentials from the FP32 instruction
+    const bool fx = k.precision == PSPH_FP32_EXP;
+    if (fx) launch_pack<AdaptPass<double, true>>(c, a, FieldCopy{});
+    else launch_pack<AdaptPass<double>>(c, a, FieldCopy{});
+    for (int it = 0; it < k.num_loop; it++) {
       StageTimer tm(c, 2);
-      // FP64 arithmetic in every form (h enters every later pass, and a
-      // relative error of h moves every kernel value by ~|s|^2 times as
-      // much); the FX form takes its exponentials from the FP32 instruction
-      if (c->n) {
-        if (k.precision == PSPH_FP32_EXP) launch_pairs<AdaptPass<double, true>>(c, make_common(c, reach), a);
-        else launch_pairs<AdaptPass<double>>(c, make_common(c, reach), a);
+      PSPH_TRY(build_lists(c, pc, k.c_smooth, c->usp));
+      const GroupCommon gc = group_common(c);
+      if (k.dim == 3) {
+        if (fx) launch_group_kernel<3, AdaptPass<double, true>>(c, pc, gc, a, false);
+        else launch_group_kernel<3, AdaptPass<double>>(c, pc, gc, a, false);
+      } else {
+        if (fx) launch_group_kernel<1, AdaptPass<double, true>>(c, pc, gc, a, false);
+        else launch_group_kernel<1, AdaptPass<double>>(c, pc, gc, a, false);
       }
     }
     HIP_TRY(hipGetLastError());
@@ -3549,9 +3541,8 @@ extern "C" int psph_diag_height(psph_ctx *c, double *H) {
   return 0;
 }
 
-// Neighbour lists for parity checks, produced on the GPU by the same
-// skeleton and membership rule as the physics passes, then mapped to read
-// order and sorted (the reference's list order is bucket-insertion history;
+// Neighbour lists for parity checks, produced on the GPU by the membership rule
+// of the physics passes, then mapped to read order and sorted (the reference's list order is bucket-insertion history;
 // the set is what every pass consumes).
 extern "C" int psph_get_neighbors(psph_ctx *c, int64_t *offsets, size_t n_cap, uint32_t *idx, size_t idx_cap) {
   if (!c || !offsets) return fail(PSPH_EINVAL, "null argument");
@@ -3565,8 +3556,7 @@ extern "C" int psph_get_neighbors(psph_ctx *c, int64_t *offsets, size_t n_cap, u
   PSPH_TRY(dmalloc((void **)&cnt, ((size_t)n + 1) * 4));
   PSPH_TRY(dmalloc((void **)&off, ((size_t)n + 1) * 4));
   HIP_TRY(hipMemsetAsync(cnt, 0, ((size_t)n + 1) * 4, c->stream));
-  ListPass::Args a{0, cnt, nullptr, nullptr, k.cutoff};
-  if (n) launch_pairs<ListPass>(c, make_common(c, r), a);
+  if (n) launch_list(c, r, cnt, nullptr, nullptr);
   size_t bytes = 0;
   HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, cnt, off, (int)n + 1, c->stream));
   PSPH_TRY(ensure_cub(c, bytes));
@@ -3575,8 +3565,7 @@ extern "C" int psph_get_neighbors(psph_ctx *c, int64_t *offsets, size_t n_cap, u
   HIP_TRY(hipMemcpyAsync(&total, off + n, 4, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   PSPH_TRY(dmalloc((void **)&out, ((size_t)total + 1) * 4));
-  a = ListPass::Args{1, cnt, off, out, k.cutoff};
-  if (n) launch_pairs<ListPass>(c, make_common(c, r), a);
+  if (n) launch_list(c, r, cnt, off, out);
   std::vector<uint32_t> hoff(n + 1), hout(total);
   HIP_TRY(hipMemcpyAsync(hoff.data(), off, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost, c->stream));
   if (total) HIP_TRY(hipMemcpyAsync(hout.data(), out, (size_t)total * 4, hipMemcpyDeviceToHost, c->stream));

@@ -102,3 +102,27 @@ def test_1d_step_equals_oracle(n_left):
         compare(G.read(), S.particles(), FLOAT_FIELDS_1D, REL_TOL_FP64)
     say(f"Sod {n_left}: equal")
 
+
+
+@pytest.mark.parametrize("form", ["fp64", "exp"])
+@pytest.mark.parametrize("name", ["1 target", "9 targets", "33 targets", "h spread", "list inside kernel box",
+                                  "support inside kernel box"])
+def test_adaptive_h_equals_oracle(name, form):
+    """An adaptation of three iterations, of which the converged targets leave
+    the later ones; the FP32-exp form's exponential moves h by ~1e-9."""
+    cfg, P = plume(**CASES[name])
+    cfg.num_loop = 3
+    if form == "exp":
+        cfg.precision = psph.PSPH_FP32_EXP
+    S = oracle.State(cfg, P)
+    S.neighbors()
+    S.adaptive_sml()
+    with psph.Solver(cfg, len(P)) as G:
+        G.load(P)
+        G.search_neighs_consth()
+        G.adaptive_sml()
+        h = G.read()["h"]
+    hs = S.particles()["h"]
+    err = float(np.max(np.abs(h - hs) / hs))
+    say(f"{name}, {form}: {int((hs != P['h']).sum())} adapted, max rel err of h {err:.2e}")
+    assert err < (REL_TOL_FP64 if form == "fp64" else 1e-7)
