@@ -161,231 +161,157 @@ __global__ void k_adj_rhs_pre(uint32_t n, const int32_t *bc, double dt, double g
 
 // ---------------------------------------------------------------------------
 // Adjoint pair passes.  Rows: the particles whose state can depend on the
-// inputs (real particles, erupt ghosts, boundary ghosts next to targets),
-// in chunks of kChunk consecutive rows of one cell.
+// inputs (real particles, erupt ghosts, boundary ghosts next to targets), in
+// groups as the targets of the forward passes (k_group_lists, k_order_targets).
 // ---------------------------------------------------------------------------
 struct AdjCommon {
-  const double *x, *y, *z, *h, *h_list;
-  const uint32_t *refb, *rows, *cfirst, *ccount, *nchunks;
-  const int32_t *bc;
-  Traversal tr;
-  int list_all;
-  int list_adj;              // some list box may reach past the adjacent buckets
-  double list_factor, cutoff2;
-  CutTest cut;
+  PairCommon p;              // targets: the rows
+  const double *h;
+  double cutoff2;
 };
 
-// Visit lists of a reversed step, shared by its three adjoint passes: for
-// every chunk of rows, the tiles that meet its grown box and hold a candidate
-// of either role of any pass, with two 32-bit masks per lane (own role,
-// neighbour role; bit b <-> candidate sub + b kSub).  List membership,
-// in_support and the row/candidate target tests are exact; the kernel box is
-// widened to the union of the passes' boxes (cut * max(h_s, h_ij), h_s the
-// summing particle's h) with a relative margin of 1e-12.  Each pass re-tests
-// its own box and masks on the set bits.
-static_assert(kWave / kSub <= 32, "the adjoint's role masks hold one bit per candidate of a lane's share");
+constexpr int kAdjSplit = 4;  // waves that share a group where groups are few (as in the forward passes)
 
-struct AdjVisits {
-  const uint32_t *off, *num;
-  const uint2 *ent;          // (first particle, particle count) of the visited tile
-  const uint64_t *mask;      // per visit and lane: own-role mask | neighbour-role mask << 32
-};
-
-__global__ __launch_bounds__(kWave) void k_adj_visit_count(AdjCommon pc, uint32_t *vcount) {
-  const uint32_t chunk = blockIdx.x;
-  const uint32_t nch = *pc.nchunks;
-  if (chunk >= nch) {
-    if (threadIdx.x == 0) vcount[chunk] = 0;
-    return;
-  }
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const uint32_t slot = (uint32_t)threadIdx.x / kSub;
-  const uint32_t i = pc.rows[cf + (slot < cc ? slot : 0)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const ChunkBox box = chunk_box(pc.tr, xi);
-  const uint32_t cnt = count_meeting_tiles(pc.tr, box);
-  if (threadIdx.x == 0) vcount[chunk] = cnt;
-}
-
-// The scan is transposed as the forward one (k_visit_masks): lane l holds
-// candidate 2 (l mod 32) + l / 32 of the tile, the wave loops over the
-// chunk's rows, and the two ballots of a row's role tests are, in their low
-// and high halves, the masks of the row's two sub-lanes.  A row is skipped
-// for a tile when its distance to the tile's box exceeds cut * max(h_i,
-// h_max of the tile): both roles' kernel boxes, cut * max(h_s, h_ij) with h_s
-// the summing particle's h, lie within that reach for every candidate of the
-// tile, and the rounded pair quantities stay on the same side of it (a
-// rounded mean lies between its operands; rounding is monotonic), so the
-// masks are exactly those of testing every row.
-struct AdjVisitRow {
-  double x, y, z, h, lf, supp;   // position, h, list box, in_support box
-  uint32_t refb;
-  int tgt;                       // need_neigh: the row sums (own role)
-};
-
-__global__ __launch_bounds__(kWave) void k_adj_visit_masks(AdjCommon pc, double cutx, const uint32_t *voff,
-                                                           uint32_t *vnum, uint2 *vent, uint64_t *vmask) {
-  static_assert(kSub == 2, "the transposed scan maps the ballot halves onto two sub-lanes");
-  __shared__ AdjVisitRow rw[kChunk];
-  const uint32_t nch = *pc.nchunks;
-  const uint32_t per = (nch + kXcds - 1) / kXcds;
-  const uint32_t local = blockIdx.x / kXcds;
-  if (local >= per) return;
-  const uint32_t chunk = (blockIdx.x % kXcds) * per + local;
-  if (chunk >= nch) return;
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const int lane = threadIdx.x;
-  // lanes 0..cc-1 own one row each: its record in LDS, its position in registers
-  const bool owner = (uint32_t)lane < cc;
-  const uint32_t i = pc.rows[cf + (owner ? (uint32_t)lane : 0u)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const double hi = pc.h[i];
-  if (owner)
-    rw[lane] = AdjVisitRow{xi[0], xi[1], xi[2], hi, pc.list_factor * pc.h_list[i], pc.cutoff2 * hi,
-                           pc.refb[i], (int)need_neigh(pc.bc[i])};
-  // the chunk's grown box (every lane's row counts, as in the passes)
-  const uint32_t slot = (uint32_t)lane / kSub;
-  const uint32_t ib = pc.rows[cf + (slot < cc ? slot : 0u)];
-  const double xb[3] = {pc.x[ib], pc.y[ib], pc.z[ib]};
-  const ChunkBox box = chunk_box(pc.tr, xb);
-  __syncthreads();
-  const GridDesc &g = pc.tr.g;
-  const uint32_t cq = 2u * ((uint32_t)lane & 31u) + ((uint32_t)lane >> 5);   // this lane's candidate
-  const uint32_t w0 = voff[chunk];
-  uint32_t w = w0;
-  for (int cz = box.c0[2]; cz <= box.c1[2]; cz++)
-    for (int cy = box.c0[1]; cy <= box.c1[1]; cy++)
-      for (int cx = box.c0[0]; cx <= box.c1[0]; cx++) {
-        const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx + cx;
-        const uint32_t lo = pc.tr.cs[cell], hi_ = pc.tr.cs[cell + 1];
-        uint32_t tl = pc.tr.toff[cell];
-        for (uint32_t base = lo; base < hi_; base += kWave, tl++) {
-          if (!tile_meets(box, pc.tr.tbox, tl)) continue;
-          const uint32_t cnt = min((uint32_t)kWave, hi_ - base);
-          const bool valid = cq < cnt;
-          const uint32_t j = base + (valid ? cq : 0u);
-          const double cxp = valid ? pc.x[j] : kFar;
-          const double cyp = valid ? pc.y[j] : kFar;
-          const double czp = valid ? pc.z[j] : kFar;
-          const double hj = valid ? pc.h[j] : 0.0;
-          const double lfj = valid ? pc.list_factor * pc.h_list[j] : 0.0;
-          const uint32_t crb = valid ? pc.refb[j] : ~0u;
-          const bool nn_j = valid && need_neigh(pc.bc[j]);
-          const double c2hj = pc.cutoff2 * hj;
-          // rows within reach of the tile in either role
-          const double hmax_t = wave_max(hj);
-          const float4 tlo = pc.tr.tbox[2 * tl], thi = pc.tr.tbox[2 * tl + 1];
-          const double r_i = cutx * fmax(hi, hmax_t);
-          const double dxl = fmax((double)tlo.x - xi[0], xi[0] - (double)thi.x);
-          const double dyl = fmax((double)tlo.y - xi[1], xi[1] - (double)thi.y);
-          const double dzl = fmax((double)tlo.z - xi[2], xi[2] - (double)thi.z);
-          const bool meets = owner && dxl <= r_i && dyl <= r_i && dzl <= r_i;
-          uint64_t tm = __ballot(meets);
-          if (!tm) continue;
-          uint32_t mown = 0, mnbr = 0;   // this lane's halves of the two role ballots
-          while (tm) {
-            const uint32_t t = (uint32_t)__builtin_ctzll(tm);
-            clear_bit_u(tm, t);
-            const AdjVisitRow R = rw[t];
-            const double amax = fmax(fabs(R.x - cxp), fmax(fabs(R.y - cyp), fabs(R.z - czp)));
-            const bool same = (pc.list_all != 0) | (crb == R.refb);
-            const bool adj = (pc.list_adj == 0) || refb_adjacent(crb, R.refb);
-            const double hij = 0.5 * (R.h + hj);
-            // row t sums, this lane's candidate is its neighbour
-            const bool own = (R.tgt != 0) & (same | ((amax <= R.lf) & adj)) & (amax <= R.supp) &
-                             (amax <= cutx * fmax(R.h, hij));
-            // this lane's candidate sums, row t is its neighbour
-            const bool nbr = nn_j & (same | ((amax <= lfj) & adj)) & (amax <= c2hj) & (amax <= cutx * fmax(hj, hij));
-            const uint64_t bo = __ballot(own), bn = __ballot(nbr);
-            // lanes 2t and 2t+1 (row t's sub-lanes) take the two halves of
-            // each ballot (one v_writelane each)
-            set_lane(mown, (uint32_t)bo, 2u * t);
-            set_lane(mown, (uint32_t)(bo >> 32), 2u * t + 1u);
-            set_lane(mnbr, (uint32_t)bn, 2u * t);
-            set_lane(mnbr, (uint32_t)(bn >> 32), 2u * t + 1u);
-          }
-          const uint64_t mask = (uint64_t)mnbr << 32 | mown;
-          if (__ballot(mask != 0)) {
-            if (lane == 0) vent[w] = make_uint2(base, cnt);
-            __builtin_nontemporal_store(mask, vmask + (size_t)w * kWave + lane);
-            w++;
-          }
-        }
-      }
-  if (lane == 0) vnum[chunk] = w - w0;
-}
-
-// An adjoint pair pass over the visit lists.  For row i and candidate j it
-// evaluates the forward pass's exact pair predicate with i as the summing
-// particle (own role, i a target) and with j as the summing particle
-// (neighbour role, j a target), and calls pair() once with both flags and
-// dx = x_i - x_j.  Within a pass, dx given to an own()/nbr() role routine is
-// always summing minus neighbour.
+// one wave's LDS: a tile's particles (place kWave is out of every reach), the
+// pass's records and the queue; the wave's sums take the tile's place
 template <class P>
-__global__ __launch_bounds__(kWave) void k_adj_pairs(AdjCommon pc, AdjVisits vl, typename P::Args a) {
-  __shared__ double sx[kWave], sy[kWave], sz[kWave], sh[kWave];
-  __shared__ typename P::Tile tile;
-  const uint32_t nch = *pc.nchunks;
-  const uint32_t per = (nch + kXcds - 1) / kXcds;
-  const uint32_t local = blockIdx.x / kXcds;
-  if (local >= per) return;
-  const uint32_t chunk = (blockIdx.x % kXcds) * per + local;
-  if (chunk >= nch) return;
-  const uint32_t cf = pc.cfirst[chunk], cc = pc.ccount[chunk];
-  const int lane = threadIdx.x;
-  // kSub lanes per row, taking alternate candidates of each tile
-  const uint32_t slot = (uint32_t)lane / kSub, sub = (uint32_t)lane % kSub;
-  const bool active = slot < cc;
-  const uint32_t i = pc.rows[cf + (active ? slot : 0)];
-  const double xi[3] = {pc.x[i], pc.y[i], pc.z[i]};
-  const double hi = pc.h[i];
+struct AdjLds {
+  union {
+    struct {
+      double x[kWave + 1], y[kWave + 1], z[kWave + 1], h[kWave + 1], lf[kWave + 1];
+      uint32_t refb[kWave + 1];
+      int32_t tgt[kWave + 1];
+      typename P::Tile tile;
+    };
+    double sum[P::NACC][kGroup];
+  };
+  uint8_t queue[2 * kWave];
+};
+
+// For row i and candidate j a pass evaluates the forward pass's exact pair
+// predicate (kernel box, list membership, in_support) with i as the summing
+// particle (own role, i a target) and with j as the summing particle (neighbour
+// role, j a target), and calls pair() once with both flags and dx = x_i - x_j.
+// Within a pass, dx given to an own()/nbr() role routine is always summing minus
+// neighbour.
+//
+// Bound by VALU issue (about 400 FP64 instructions a pair in the RHS).  8 rows x 8
+// streams of a queue of the candidates that any row of the group can meet, as in
+// k_group_pass, because the rows' own hit lists differ in length: a wave of 32 rows
+// x 2 lanes that walked a bit mask per lane ran as long as its fullest lane, and at
+// 30k rows there was one such wave per SIMD.  us per step at 30k rows (RHS, density,
+// filter, lists): 1406, 495, 504, 343 before, 1019, 358, 363, 125 so.
+template <class P>
+__global__ __launch_bounds__(kAdjSplit * kWave, P::kWaves) void k_adj_pass(AdjCommon pc, GroupLists gl, typename P::Args a) {
+  extern __shared__ char lds[];                    // an AdjLds<P> per wave
+  uint32_t gid, i;
+  const uint32_t nt = my_group(pc.p, gid, i);
+  if (!nt) return;
+  const int lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), split = blockDim.x / kWave;
+  AdjLds<P> &st = ((AdjLds<P> *)lds)[wave];
+  const uint32_t stream = (uint32_t)lane / kGroup, slot = (uint32_t)lane % kGroup;
+  // a lane without a row of its own meets nothing
+  const double xi[3] = {slot < nt ? pc.p.x[i] : -kFar, pc.p.y[i], pc.p.z[i]};
+  const double hi = pc.h[i], lfi = pc.p.list_factor * pc.p.h_list[i], supi = pc.cutoff2 * hi;
+  const uint32_t rbi = pc.p.refb[i];
+  const bool tgt = need_neigh(pc.p.bc[i]);
   typename P::Row t;
   P::load_row(a, i, t);
-  P::init(tile, lane);
-  __syncthreads();
-  const uint32_t v0 = vl.off[chunk], nv = vl.num[chunk];
-  for (uint32_t v = 0; v < nv; v++) {
-    const uint2 e = vl.ent[v0 + v];
-    const uint32_t base = e.x, cnt = e.y;
-    if ((uint32_t)lane < cnt) {
-      const uint32_t j = base + lane;
-      sx[lane] = pc.x[j]; sy[lane] = pc.y[j]; sz[lane] = pc.z[j];
-      sh[lane] = pc.h[j];
-      P::stage(a, j, tile, lane);
-    }
-    const uint64_t m64 = __builtin_nontemporal_load(vl.mask + (size_t)(v0 + v) * kWave + lane);
-    const uint2 m = make_uint2((uint32_t)m64, (uint32_t)(m64 >> 32));
-    __syncthreads();
-    if (active) {
-      uint32_t mb = m.x | m.y;
-      while (mb) {
-        const uint32_t b = (uint32_t)__builtin_ctz(mb);
-        mb &= mb - 1;
-        const uint32_t q = sub + b * kSub, jq = base + q;
-        const double dx[3] = {xi[0] - sx[q], xi[1] - sy[q], xi[2] - sz[q]};
-        const double amax = fmax(fabs(dx[0]), fmax(fabs(dx[1]), fabs(dx[2])));
-        // all operands evaluated (no short-circuit branches), combined as ints
-        const bool fo = ((int)((m.x >> b) & 1u) & (int)P::own_ok(t, tile, q, jq, i) &
-                         (int)!pc.cut.outside(amax, P::hker_own(hi, sh[q]))) != 0;
-        const bool fn = ((int)((m.y >> b) & 1u) & (int)P::nbr_ok(t, tile, q, jq, i) &
-                         (int)!pc.cut.outside(amax, P::hker_nbr(hi, sh[q]))) != 0;
-        if (fo | fn) P::pair(a, t, tile, q, dx, amax, hi, sh[q], fo, fn);
-      }
-    }
-    __syncthreads();
+  double acc[P::NACC];
+#pragma unroll
+  for (int k = 0; k < P::NACC; k++) acc[k] = 0;
+  if (lane == 0) {
+    st.x[kWave] = st.y[kWave] = st.z[kWave] = kFar;
+    st.h[kWave] = st.lf[kWave] = 0;
+    st.refb[kWave] = kDead;
+    st.tgt[kWave] = 0;
   }
-  P::combine(t);
-  if (active && sub == 0) P::finish(a, t, i);
+  const uint32_t nv = __builtin_amdgcn_readfirstlane(gl.num[gid]);
+  const_ptr<uint32_t> vis = (const_ptr<uint32_t>)(uintptr_t)(gl.visit + __builtin_amdgcn_readfirstlane(gl.off[gid]));
+  uint32_t ahead[4] = {0, 0, 0, 0};                // the next visit
+  if (wave < nv)
+    for (int k = 0; k < 4; k++) ahead[k] = vis[(size_t)wave * 4 + k];
+  // the particle of this lane's stream; streams below nl hold theirs from the
+  // tile before
+  double xj[3], hj, lfj;
+  uint32_t rbj, j = 0;
+  int32_t tgj;
+  typename P::Rec r;
+  uint32_t nl = 0;
+  for (uint32_t v = wave;; v += split) {
+    uint32_t base = 0;
+    uint64_t m = 0;
+    const uint32_t held = nl;
+    if (v < nv) {
+      base = ahead[0];
+      m = (uint64_t)ahead[3] << 32 | ahead[2];
+      const_ptr<uint32_t> e = vis + (size_t)min(v + split, nv - 1) * 4;
+      for (int k = 0; k < 4; k++) ahead[k] = e[k];
+      if ((m >> lane) & 1) {
+        // (masked places lie below the tile's count)
+        const uint32_t q = base + lane;
+        st.x[lane] = pc.p.x[q]; st.y[lane] = pc.p.y[q]; st.z[lane] = pc.p.z[q];
+        st.h[lane] = pc.h[q];
+        st.lf[lane] = pc.p.list_factor * pc.p.h_list[q];
+        st.refb[lane] = pc.p.refb[q];
+        st.tgt[lane] = need_neigh(pc.p.bc[q]) ? 1 : 0;
+        P::stage(a, q, st.tile, lane);
+        st.queue[held + lanes_below(m)] = (uint8_t)lane;
+      }
+    } else {
+      if (!held) break;
+      // the last block's other streams take the place out of reach
+      m = 0xffu >> held;
+      if ((uint32_t)lane < kStreams - held) st.queue[held + lane] = (uint8_t)kWave;
+    }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own LDS writes are there
+    auto load = [&](const uint8_t *at) {
+      const uint32_t p = at[stream];
+      xj[0] = st.x[p]; xj[1] = st.y[p]; xj[2] = st.z[p];
+      hj = st.h[p]; lfj = st.lf[p]; rbj = st.refb[p]; tgj = st.tgt[p];
+      P::load(st.tile, min(p, (uint32_t)kWave - 1u), r);
+      j = base + p;
+    };
+    const uint8_t *qp = st.queue;
+    uint32_t left = held + (uint32_t)__popcll(m);
+    for (; left >= kStreams; left -= kStreams, qp += kStreams) {
+      if (stream >= nl) load(qp);
+      nl = 0;
+      const double dx[3] = {xi[0] - xj[0], xi[1] - xj[1], xi[2] - xj[2]};
+      const double amax = fmax(fabs(dx[0]), fmax(fabs(dx[1]), fabs(dx[2])));
+      const bool same = (pc.p.list_all != 0) | (rbj == rbi);
+      const bool adj = (pc.p.list_adj == 0) || refb_adjacent(rbj, rbi);
+      // all operands evaluated (no short-circuit branches), combined as ints
+      const bool fo = ((int)tgt & (int)(same | ((amax <= lfi) & adj)) & (int)(amax <= supi) &
+                       (int)P::own_ok(t, r, j != i) & (int)!pc.p.cut.outside(amax, P::hker_own(hi, hj))) != 0;
+      const bool fn = ((int)(tgj != 0) & (int)(same | ((amax <= lfj) & adj)) & (int)(amax <= pc.cutoff2 * hj) &
+                       (int)P::nbr_ok(t, r, j != i) & (int)!pc.p.cut.outside(amax, P::hker_nbr(hi, hj))) != 0;
+      if (fo | fn) P::pair(a, t, r, dx, amax, hi, hj, fo, fn, acc);
+    }
+    if (v >= nv) break;
+    if (stream >= nl && stream < left) load(qp);
+    nl = left;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the tile has been read
+    __builtin_amdgcn_wave_barrier();
+  }
+  double sum[P::NACC];
+#pragma unroll
+  for (int k = 0; k < P::NACC; k++) sum[k] = stream_sum(acc[k]);
+  if (split > 1) {
+    // the waves' sums, added in their order
+    if (lane < kGroup)
+      for (int k = 0; k < P::NACC; k++) st.sum[k][lane] = sum[k];
+    __syncthreads();
+    if (wave != 0) return;
+    for (uint32_t w = 1; w < split; w++)
+      for (int k = 0; k < P::NACC; k++) sum[k] += ((AdjLds<P> *)lds)[w].sum[k][lane % kGroup];
+  }
+  if ((uint32_t)lane < nt) P::finish(a, sum, i);
 }
 
 __device__ inline double dot3(const double *a, const double *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
-
-// 1 / x in FP64: hardware reciprocal refined by two Newton steps
-__device__ inline double rcp64(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  r = r * fma(-x, r, 2.0);
-  return r * fma(-x, r, 2.0);
-}
 
 // --- velocity filter (smooth_velocity.cc:25-165) ----------------------------
 struct VsmAdj {
@@ -396,19 +322,19 @@ struct VsmAdj {
     LamPtrs l;
   };
   struct Tile {
-    double mr[kWave], ih2[kWave], nrm[kWave], v[3][kWave], a[3][kWave], c[kWave], etab[kETab];
+    double mr[kWave], ih2[kWave], nrm[kWave], v[3][kWave], a[3][kWave], c[kWave];
     int ok[kWave];
   };
-  struct Row { double imi, irho, mr, ih2, nrm, v[3], a[3], c, g[3], gv[3], gm, grho; bool ok; };
-  __device__ static void init(Tile &s, int lane) { etab_fill(s.etab, lane); }
+  struct Rec { double mr, ih2, nrm, v[3], a[3], c; int ok; };
+  struct Row { double imi, irho, mr, ih2, nrm, v[3], a[3], c; bool ok; };
+  static constexpr int kWaves = 3;             // per SIMD: at most 168 VGPRs
+  static constexpr int NACC = 8;               // 0-2: x, 3-5: v, 6: m, 7: rho
   __device__ static void load_row(const Args &A, uint32_t i, Row &t) {
     const double mi = A.m[i], rhoi = A.rho[i], ih = 1.0 / A.h[i], nk = kInvSqrtPi * ih;
     t.imi = 1.0 / mi; t.irho = 1.0 / rhoi; t.mr = mi * t.irho;
     t.ih2 = ih * ih; t.nrm = nk * nk * nk;
     t.v[0] = A.v0[i]; t.v[1] = A.v1[i]; t.v[2] = A.v2[i];
     t.a[0] = A.ax[i]; t.a[1] = A.ay[i]; t.a[2] = A.az[i]; t.c = A.ac[i];
-    for (int k = 0; k < 3; k++) t.g[k] = t.gv[k] = 0;
-    t.gm = t.grho = 0;
     t.ok = contr_vel(A.bc[i]);
   }
   __device__ static void stage(const Args &A, uint32_t j, Tile &s, int l) {
@@ -419,46 +345,38 @@ struct VsmAdj {
     s.a[0][l] = A.ax[j]; s.a[1][l] = A.ay[j]; s.a[2][l] = A.az[j]; s.c[l] = A.ac[j];
     s.ok[l] = contr_vel(A.bc[j]);
   }
+  __device__ static void load(const Tile &s, uint32_t q, Rec &r) {
+    r = Rec{s.mr[q], s.ih2[q], s.nrm[q], {s.v[0][q], s.v[1][q], s.v[2][q]}, {s.a[0][q], s.a[1][q], s.a[2][q]},
+            s.c[q], s.ok[q]};
+  }
   __device__ static double hker_own(double hi, double) { return hi; }
   __device__ static double hker_nbr(double, double hj) { return hj; }
-  __device__ static bool own_ok(const Row &, const Tile &s, uint32_t q, uint32_t, uint32_t) { return s.ok[q] != 0; }
-  __device__ static bool nbr_ok(const Row &t, const Tile &, uint32_t, uint32_t, uint32_t) { return t.ok; }
-  __device__ static void own(const Args &, Row &t, const Tile &s, uint32_t q, const double *dx, double,
-                             double, double) {
-    const double w = t.nrm * exp_neg_tab(dot3(dx, dx) * t.ih2, s.etab) * s.mr[q];
-    const double gw = t.a[0] * s.v[0][q] + t.a[1] * s.v[1][q] + t.a[2] * s.v[2][q] - t.c;
-    const double f = -2.0 * gw * w * t.ih2;
-    for (int k = 0; k < 3; k++) t.g[k] += f * dx[k];
-  }
-  __device__ static void nbr(const Args &, Row &t, const Tile &s, uint32_t q, const double *dx, double,
-                             double, double) {
-    const double ih2 = s.ih2[q];
-    const double w = s.nrm[q] * exp_neg_tab(dot3(dx, dx) * ih2, s.etab) * t.mr;
-    const double a[3] = {s.a[0][q], s.a[1][q], s.a[2][q]};
-    const double gw = dot3(a, t.v) - s.c[q];
-    for (int k = 0; k < 3; k++) t.gv[k] += a[k] * w;
-    t.gm += gw * w * t.imi;
-    t.grho -= gw * w * t.irho;
-    const double f = -2.0 * gw * w * ih2;
-    for (int k = 0; k < 3; k++) t.g[k] -= f * dx[k];
-  }
+  __device__ static bool own_ok(const Row &, const Rec &r, bool) { return r.ok != 0; }
+  __device__ static bool nbr_ok(const Row &t, const Rec &, bool) { return t.ok; }
   // the two roles use different kernels (h_i and h_j): nothing to share
-  __device__ static void pair(const Args &A, Row &t, const Tile &s, uint32_t q, const double *dx, double amax,
-                              double hi, double hj, bool fo, bool fn) {
-    if (fo) own(A, t, s, q, dx, amax, hi, hj);
+  __device__ static void pair(const Args &, const Row &t, const Rec &s, const double *dx, double, double, double,
+                              bool fo, bool fn, double *acc) {
+    const double r2 = dot3(dx, dx);
+    if (fo) {
+      const double w = t.nrm * exp_neg(r2 * t.ih2) * s.mr;
+      const double gw = dot3(t.a, s.v) - t.c;
+      const double f = -2.0 * gw * w * t.ih2;
+      for (int k = 0; k < 3; k++) acc[k] += f * dx[k];
+    }
     if (fn) {
-      const double dn[3] = {-dx[0], -dx[1], -dx[2]};
-      nbr(A, t, s, q, dn, amax, hi, hj);
+      const double w = s.nrm * exp_neg(r2 * s.ih2) * t.mr;
+      const double gw = dot3(s.a, t.v) - s.c;
+      for (int k = 0; k < 3; k++) acc[3 + k] += s.a[k] * w;
+      acc[6] += gw * w * t.imi;
+      acc[7] -= gw * w * t.irho;
+      const double f = -2.0 * gw * w * s.ih2;
+      for (int k = 0; k < 3; k++) acc[k] += f * dx[k];
     }
   }
-  __device__ static void combine(Row &t) {
-    for (int k = 0; k < 3; k++) { t.g[k] = sub_sum<kSub>(t.g[k]); t.gv[k] = sub_sum<kSub>(t.gv[k]); }
-    t.gm = sub_sum<kSub>(t.gm); t.grho = sub_sum<kSub>(t.grho);
-  }
-  __device__ static void finish(const Args &A, Row &t, uint32_t i) {
-    for (int k = 0; k < 3; k++) { A.l.f[L_X + k][i] += t.g[k]; A.l.f[L_VX + k][i] += t.gv[k]; }
-    A.l.f[L_M][i] += t.gm;
-    A.l.f[L_RHO][i] += t.grho;
+  __device__ static void finish(const Args &A, const double *sum, uint32_t i) {
+    for (int k = 0; k < 3; k++) { A.l.f[L_X + k][i] += sum[k]; A.l.f[L_VX + k][i] += sum[3 + k]; }
+    A.l.f[L_M][i] += sum[6];
+    A.l.f[L_RHO][i] += sum[7];
   }
 };
 
@@ -474,18 +392,18 @@ struct DensAdj {
     LamPtrs l;
   };
   struct Tile {
-    double m[kWave], irho[kWave], e1[kWave], s1[kWave], s2[kWave], sen[kWave], swn[kWave], etab[kETab];
+    double m[kWave], irho[kWave], e1[kWave], s1[kWave], s2[kWave], sen[kWave], swn[kWave];
     int ok[kWave];
   };
-  struct Row { double mi, imi, irho, e1i, s1, s2, sen, swn, g[3], gm, grho, ge; int ok; };
-  __device__ static void init(Tile &s, int lane) { etab_fill(s.etab, lane); }
+  struct Rec { double m, irho, e1, s1, s2, sen, swn; int ok; };
+  struct Row { double mi, irho, e1i, s1, s2, sen, swn; int ok; };
+  static constexpr int kWaves = 4;             // per SIMD: at most 128 VGPRs
+  static constexpr int NACC = 6;               // 0-2: x, 3: m, 4: rho, 5: e
   __device__ static void load_row(const Args &A, uint32_t i, Row &t) {
-    t.mi = A.m[i]; t.imi = 1.0 / t.mi; t.irho = 1.0 / A.rho[i]; t.e1i = A.e1[i];
+    t.mi = A.m[i]; t.irho = 1.0 / A.rho[i]; t.e1i = A.e1[i];
     t.s1 = A.s1[i]; t.s2 = A.s2[i]; t.sen = A.sen[i]; t.swn = A.swn[i];
     const int ph = A.phase[i];
     t.ok = (contr_dens(A.pghost, A.bc[i]) && (ph == 1 || ph == 2)) ? ph : 0;
-    t.g[0] = t.g[1] = t.g[2] = 0;
-    t.gm = t.grho = t.ge = 0;
   }
   __device__ static void stage(const Args &A, uint32_t j, Tile &s, int l) {
     s.m[l] = A.m[j]; s.irho[l] = 1.0 / A.rho[j]; s.e1[l] = A.e1[j];
@@ -493,68 +411,67 @@ struct DensAdj {
     const int ph = A.phase[j];
     s.ok[l] = (contr_dens(A.pghost, A.bc[j]) && (ph == 1 || ph == 2)) ? ph : 0;
   }
+  __device__ static void load(const Tile &s, uint32_t q, Rec &r) {
+    r = Rec{s.m[q], s.irho[q], s.e1[q], s.s1[q], s.s2[q], s.sen[q], s.swn[q], s.ok[q]};
+  }
   __device__ static double hker_own(double hi, double hj) { return 0.5 * (hi + hj); }
   __device__ static double hker_nbr(double hi, double hj) { return 0.5 * (hj + hi); }
-  __device__ static bool own_ok(const Row &, const Tile &s, uint32_t q, uint32_t, uint32_t) { return s.ok[q] != 0; }
-  __device__ static bool nbr_ok(const Row &t, const Tile &, uint32_t, uint32_t, uint32_t) { return t.ok != 0; }
+  __device__ static bool own_ok(const Row &, const Rec &r, bool) { return r.ok != 0; }
+  __device__ static bool nbr_ok(const Row &t, const Rec &, bool) { return t.ok != 0; }
   // kernel values of the pair: wm / m_j (density) and the energy weight / (m_j / rho_j)
-  __device__ static void weights(const Args &A, const Tile &s, double r2, double amax, double h, double &w,
-                                 double &we, double &ih2, bool &ebox) {
-    const double ih = rcp64(h);
+  __device__ static void weights(const Args &A, double r2, double amax, double h, double &w, double &we, double &ih2,
+                                 bool &ebox) {
+    const double ih = rcp_newton(h);
     ih2 = ih * ih;
     const double nk = kInvSqrtPi * ih;
-    const double ex = exp_neg_tab(r2 * ih2, s.etab);
+    const double ex = exp_neg(r2 * ih2);
     w = nk * nk * nk * ex;
     ebox = A.energy_smooth && !A.cut.outside(A.e_ratio * amax, h);
     we = 0;
     if (ebox) {
       const double nke = nk * A.e_ratio;
-      we = nke * nke * nke * (A.e_sq16 ? pow16(ex) : exp_neg_tab(A.e_ratio * A.e_ratio * r2 * ih2, s.etab));
+      we = nke * nke * nke * (A.e_sq16 ? pow16(ex) : exp_neg(A.e_ratio * A.e_ratio * r2 * ih2));
     }
   }
   // h_ij is symmetric: both roles share the pair's two kernel weights.
   // dx = x_i - x_j; the neighbour role's position term, 2 f (x_j - x_i) added,
   // is the same subtraction as the own role's.
-  __device__ static void pair(const Args &A, Row &t, const Tile &s, uint32_t q, const double *dx, double amax,
-                              double hi, double hj, bool fo, bool fn) {
+  __device__ static void pair(const Args &A, const Row &t, const Rec &s, const double *dx, double amax, double hi,
+                              double hj, bool fo, bool fn, double *acc) {
     double w, we, ih2;
     bool ebox;
-    weights(A, s, dot3(dx, dx), amax, 0.5 * (hi + hj), w, we, ih2, ebox);
+    weights(A, dot3(dx, dx), amax, 0.5 * (hi + hj), w, we, ih2, ebox);
     double f = 0;
     if (fo) {
-      const double lr = s.ok[q] == 1 ? t.s1 : t.s2;
-      f = lr * (w * s.m[q]) * ih2;
+      const double lr = s.ok == 1 ? t.s1 : t.s2;
+      f = lr * (w * s.m) * ih2;
       if (ebox) {
-        const double vr = we * s.m[q] * s.irho[q];
-        const double gvr = t.swn + t.sen * s.e1[q];
+        const double vr = we * s.m * s.irho;
+        const double gvr = t.swn + t.sen * s.e1;
         f += gvr * vr * (A.e_ratio * A.e_ratio) * ih2;
       }
-      for (int k = 0; k < 3; k++) t.g[k] -= 2.0 * f * dx[k];
+      for (int k = 0; k < 3; k++) acc[k] -= 2.0 * f * dx[k];
     }
     if (fn) {
-      const double lr = t.ok == 1 ? s.s1[q] : s.s2[q];
+      const double lr = t.ok == 1 ? s.s1 : s.s2;
       f = lr * (w * t.mi) * ih2;
-      t.gm += lr * w;
+      acc[3] += lr * w;
       if (ebox) {
         const double vr = we * t.mi * t.irho;
-        const double gvr = s.swn[q] + s.sen[q] * t.e1i;
-        t.ge += s.sen[q] * vr;
-        t.gm += gvr * we * t.irho;
-        t.grho -= gvr * vr * t.irho;
+        const double gvr = s.swn + s.sen * t.e1i;
+        acc[5] += s.sen * vr;
+        acc[3] += gvr * we * t.irho;
+        acc[4] -= gvr * vr * t.irho;
         f += gvr * vr * (A.e_ratio * A.e_ratio) * ih2;
       }
-      for (int k = 0; k < 3; k++) t.g[k] -= 2.0 * f * dx[k];
+      for (int k = 0; k < 3; k++) acc[k] -= 2.0 * f * dx[k];
     }
   }
-  __device__ static void combine(Row &t) {
-    for (int k = 0; k < 3; k++) t.g[k] = sub_sum<kSub>(t.g[k]);
-    t.gm = sub_sum<kSub>(t.gm); t.grho = sub_sum<kSub>(t.grho); t.ge = sub_sum<kSub>(t.ge);
-  }
-  __device__ static void finish(const Args &A, Row &t, uint32_t i) {
-    for (int k = 0; k < 3; k++) A.l.f[L_X + k][i] += t.g[k];
-    A.l.f[L_M][i] += t.gm;
-    A.l.f[L_RHO][i] += t.grho;
-    A.l.f[L_E][i] += t.ge;
+  __device__ static void finish(const Args &A, const double *sum, uint32_t i) {
+    for (int k = 0; k < 3; k++) A.l.f[L_X + k][i] += sum[k];
+    A.l.f[L_M][i] += sum[3];
+    A.l.f[L_RHO][i] += sum[4];
+    A.l.f[L_E][i] += sum[5];
   }
 };
 
@@ -576,15 +493,15 @@ struct RhsGeo {
   bool avis, heat;
 };
 
-__device__ inline RhsGeo rhs_geo(const RhsAdjConst &k, const double *etab, const double *dx, const double *vij,
+__device__ inline RhsGeo rhs_geo(const RhsAdjConst &k, const double *dx, const double *vij,
                                  double h, const RhsSide &S, const RhsSide &N) {
   RhsGeo q;
   q.h = h;
-  const double ih = rcp64(h);
+  const double ih = rcp_newton(h);
   q.ih2 = ih * ih;
   q.r2 = dot3(dx, dx);
   const double nk = kInvSqrtPi * ih;
-  const double W = nk * nk * nk * exp_neg_tab(q.r2 * q.ih2, etab);
+  const double W = nk * nk * nk * exp_neg(q.r2 * q.ih2);
   q.G = -2.0 * q.ih2 * W;
   q.vrab = dot3(dx, vij);
   q.dotvv = dot3(vij, vij);
@@ -594,7 +511,7 @@ __device__ inline RhsGeo rhs_geo(const RhsAdjConst &k, const double *etab, const
   if (q.avis) {
     const double rhoab = 0.5 * (S.rho + N.rho);
     const double den = q.r2 + k.ata * h * h;
-    const double inv = rcp64(den * rhoab);
+    const double inv = rcp_newton(den * rhoab);
     q.irhoab = den * inv;
     q.iden = rhoab * inv;
     q.mu = h * q.vrab * q.iden;
@@ -607,7 +524,7 @@ __device__ inline RhsGeo rhs_geo(const RhsAdjConst &k, const double *etab, const
   q.cpab = q.hinv = 0;
   if (q.heat) {
     q.cpab = 0.5 * (S.cp + N.cp);
-    q.hinv = rcp64(q.dotvr * h * q.cab);
+    q.hinv = rcp_newton(q.dotvr * h * q.cab);
   }
   return q;
 }
@@ -691,16 +608,16 @@ struct RhsAdj {
   };
   struct Tile {
     double m[kWave], im[kWave], rho[kWave], V[kWave], p[kWave], c[kWave], T[kWave], cp[kWave], u[3][kWave];
-    double a[3][kWave], ae[kWave], etab[kETab];
+    double a[3][kWave], ae[kWave];
   };
-  struct Row { RhsSide me; double a[3], ae, g[3], gu[3], gm, grho, gp, gc, gT, gcp; };
-  __device__ static void init(Tile &s, int lane) { etab_fill(s.etab, lane); }
+  struct Rec { RhsSide it; double a[3], ae; };
+  struct Row { RhsSide me; double a[3], ae; };
+  static constexpr int kWaves = 2;             // per SIMD: 3 would spill (1019 us to 3720)
+  static constexpr int NACC = 12;              // 0-2: x, 3-5: u, 6: m, 7: rho, 8: p, 9: c, 10: T, 11: cp
   __device__ static void load_row(const Args &A, uint32_t i, Row &t) {
     const double m = A.m[i], rho = A.rho[i];
     t.me = RhsSide{m, 1.0 / m, rho, 1.0 / rho, A.p[i], A.c[i], A.T[i], A.cp[i], {A.u0[i], A.u1[i], A.u2[i]}};
     t.a[0] = A.a0[i]; t.a[1] = A.a1[i]; t.a[2] = A.a2[i]; t.ae = A.ae[i];
-    for (int k = 0; k < 3; k++) t.g[k] = t.gu[k] = 0;
-    t.gm = t.grho = t.gp = t.gc = t.gT = t.gcp = 0;
   }
   __device__ static void stage(const Args &A, uint32_t j, Tile &s, int l) {
     const double m = A.m[j], rho = A.rho[j];
@@ -709,43 +626,40 @@ struct RhsAdj {
     s.u[0][l] = A.u0[j]; s.u[1][l] = A.u1[j]; s.u[2][l] = A.u2[j];
     s.a[0][l] = A.a0[j]; s.a[1][l] = A.a1[j]; s.a[2][l] = A.a2[j]; s.ae[l] = A.ae[j];
   }
-  __device__ static RhsSide side(const Tile &s, uint32_t q) {
-    return RhsSide{s.m[q], s.im[q], s.rho[q], s.V[q], s.p[q], s.c[q], s.T[q], s.cp[q], {s.u[0][q], s.u[1][q], s.u[2][q]}};
+  __device__ static void load(const Tile &s, uint32_t q, Rec &r) {
+    r.it = RhsSide{s.m[q], s.im[q], s.rho[q], s.V[q], s.p[q], s.c[q], s.T[q], s.cp[q],
+                   {s.u[0][q], s.u[1][q], s.u[2][q]}};
+    for (int k = 0; k < 3; k++) r.a[k] = s.a[k][q];
+    r.ae = s.ae[q];
   }
   __device__ static double hker_own(double hi, double hj) { return 0.5 * (hi + hj); }
   __device__ static double hker_nbr(double hi, double hj) { return 0.5 * (hj + hi); }
-  __device__ static bool own_ok(const Row &, const Tile &, uint32_t, uint32_t j, uint32_t i) { return j != i; }
-  __device__ static bool nbr_ok(const Row &, const Tile &, uint32_t, uint32_t j, uint32_t i) { return j != i; }
+  __device__ static bool own_ok(const Row &, const Rec &, bool other) { return other; }
+  __device__ static bool nbr_ok(const Row &, const Rec &, bool other) { return other; }
   // dx = x_i - x_j (row minus candidate); the neighbour role sees -dx, -v_ij
-  __device__ static void pair(const Args &A, Row &t, const Tile &s, uint32_t q, const double *dx, double,
-                              double hi, double hj, bool fo, bool fn) {
-    const RhsSide J = side(s, q);
+  __device__ static void pair(const Args &A, const Row &t, const Rec &s, const double *dx, double, double hi,
+                              double hj, bool fo, bool fn, double *acc) {
+    const RhsSide &J = s.it;
     const double vij[3] = {t.me.vel[0] - J.vel[0], t.me.vel[1] - J.vel[1], t.me.vel[2] - J.vel[2]};
-    const RhsGeo G = rhs_geo(A.k, s.etab, dx, vij, 0.5 * (hi + hj), t.me, J);
+    const RhsGeo G = rhs_geo(A.k, dx, vij, 0.5 * (hi + hj), t.me, J);
     RhsGrad g;
     if (fo) {
       rhs_role(A.k, G, dx, vij, t.me, J, t.a, t.ae, g);
-      for (int k = 0; k < 3; k++) { t.g[k] += g.dx[k]; t.gu[k] += g.vij[k]; }
-      t.grho += g.rho_s; t.gp += g.p_s; t.gc += g.c_s; t.gT += g.T_s; t.gcp += g.cp_s;
+      for (int k = 0; k < 3; k++) { acc[k] += g.dx[k]; acc[3 + k] += g.vij[k]; }
+      acc[7] += g.rho_s; acc[8] += g.p_s; acc[9] += g.c_s; acc[10] += g.T_s; acc[11] += g.cp_s;
     }
     if (fn) {
       const double dn[3] = {-dx[0], -dx[1], -dx[2]}, vn[3] = {-vij[0], -vij[1], -vij[2]};
-      const double a[3] = {s.a[0][q], s.a[1][q], s.a[2][q]};
-      rhs_role(A.k, G, dn, vn, J, t.me, a, s.ae[q], g);
-      for (int k = 0; k < 3; k++) { t.g[k] -= g.dx[k]; t.gu[k] -= g.vij[k]; }
-      t.gm += g.m_n; t.grho += g.rho_n; t.gp += g.p_n; t.gc += g.c_n; t.gT += g.T_n; t.gcp += g.cp_n;
+      rhs_role(A.k, G, dn, vn, J, t.me, s.a, s.ae, g);
+      for (int k = 0; k < 3; k++) { acc[k] -= g.dx[k]; acc[3 + k] -= g.vij[k]; }
+      acc[6] += g.m_n; acc[7] += g.rho_n; acc[8] += g.p_n; acc[9] += g.c_n; acc[10] += g.T_n; acc[11] += g.cp_n;
     }
   }
-  __device__ static void combine(Row &t) {
-    for (int k = 0; k < 3; k++) { t.g[k] = sub_sum<kSub>(t.g[k]); t.gu[k] = sub_sum<kSub>(t.gu[k]); }
-    t.gm = sub_sum<kSub>(t.gm); t.grho = sub_sum<kSub>(t.grho); t.gp = sub_sum<kSub>(t.gp);
-    t.gc = sub_sum<kSub>(t.gc); t.gT = sub_sum<kSub>(t.gT); t.gcp = sub_sum<kSub>(t.gcp);
-  }
-  __device__ static void finish(const Args &A, Row &t, uint32_t i) {
+  __device__ static void finish(const Args &A, const double *sum, uint32_t i) {
     const int u0 = A.k.lans ? L_SVX : L_VX;
-    for (int k = 0; k < 3; k++) { A.l.f[L_X + k][i] += t.g[k]; A.l.f[u0 + k][i] += t.gu[k]; }
-    A.l.f[L_M][i] += t.gm; A.l.f[L_RHO][i] += t.grho; A.l.f[L_P][i] += t.gp;
-    A.l.f[L_C][i] += t.gc; A.l.f[L_T][i] += t.gT; A.l.f[L_CP][i] += t.gcp;
+    for (int k = 0; k < 3; k++) { A.l.f[L_X + k][i] += sum[k]; A.l.f[u0 + k][i] += sum[3 + k]; }
+    A.l.f[L_M][i] += sum[6]; A.l.f[L_RHO][i] += sum[7]; A.l.f[L_P][i] += sum[8];
+    A.l.f[L_C][i] += sum[9]; A.l.f[L_T][i] += sum[10]; A.l.f[L_CP][i] += sum[11];
   }
 };
 
@@ -806,14 +720,9 @@ struct Adjoint {
   double *part = nullptr;     // reduction partials
   // chunks of adjoint rows
   uint32_t *flags = nullptr, *tpos = nullptr, *rows = nullptr, *cchunks = nullptr, *coff = nullptr;
-  uint32_t *cfirst = nullptr, *ccount = nullptr, *nchunks = nullptr;
-  uint32_t *tcell = nullptr;
-  size_t n_cap = 0, rows_cap = 0, chunk_cap = 0, tcell_cap = 0;
-  // visit lists of the step being reversed
-  uint32_t *vcount = nullptr, *voff = nullptr, *vnum = nullptr;
-  uint2 *vent = nullptr;
-  uint64_t *vmask = nullptr;
-  size_t vchunk_cap = 0, vis_cap = 0;
+  uint32_t *cfirst = nullptr, *ccount = nullptr;
+  unsigned long long *made = nullptr;   // visits handed out, chunks
+  size_t n_cap = 0, chunk_cap = 0, cell_cap = 0;
 };
 
 static void dev_fields(psph_ctx *c, double **d, uint32_t **u, int32_t **i) {
@@ -861,7 +770,7 @@ static void adjoint_free(psph_ctx *c) {
   for (auto p : A->l) if (p) hipFree(p);
   for (auto p : A->aux) if (p) hipFree(p);
   void *ptrs[] = {A->part, A->flags, A->tpos, A->rows, A->cchunks, A->coff, A->cfirst, A->ccount,
-                  A->nchunks, A->tcell, A->vcount, A->voff, A->vnum, A->vent, A->vmask};
+                  A->made};
   for (auto p : ptrs) if (p) hipFree(p);
   delete A;
   c->adj = nullptr;
@@ -1049,86 +958,69 @@ static int dev_sum(psph_ctx *c, Adjoint &A, const double *v, size_t n, double *o
   return 0;
 }
 
-// chunks of adjoint rows of one step (<= 64 consecutive rows of one cell)
+// groups of adjoint rows of one step (chunks of kChunk consecutive rows of a cell)
 static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
   const uint32_t n = (uint32_t)R.n;
   const GridDesc &g = R.grid;
   const uint32_t ncells = g.ncells;
   hipStream_t s = c->stream;
   if (n + 1 > A.n_cap) {
-    void *ptrs[] = {A.flags, A.tpos, A.rows};
-    for (auto p : ptrs) if (p) hipFree(p);
+    uint32_t **arrs[] = {&A.flags, &A.tpos, &A.rows};
+    for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
+    A.n_cap = 0;
     const size_t cap = std::max<size_t>(c->cap, n) + 1;
-    PSPH_TRY(dmalloc((void **)&A.flags, cap * 4));
-    PSPH_TRY(dmalloc((void **)&A.tpos, cap * 4));
-    PSPH_TRY(dmalloc((void **)&A.rows, cap * 4));
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, cap * 4));
     A.n_cap = cap;
   }
-  if (ncells + 1 > A.tcell_cap) {
-    void *ptrs[] = {A.cchunks, A.coff, A.tcell};
-    for (auto p : ptrs) if (p) hipFree(p);
-    PSPH_TRY(dmalloc((void **)&A.cchunks, ((size_t)ncells + 1) * 4));
-    PSPH_TRY(dmalloc((void **)&A.coff, ((size_t)ncells + 1) * 4));
-    PSPH_TRY(dmalloc((void **)&A.tcell, ((size_t)ncells + 1) * 4));
-    A.tcell_cap = (size_t)ncells + 1;
+  if (ncells + 1 > A.cell_cap) {
+    uint32_t **arrs[] = {&A.cchunks, &A.coff};
+    for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
+    A.cell_cap = 0;
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)ncells + 1) * 4));
+    A.cell_cap = (size_t)ncells + 1;
   }
   const size_t chunks_ub = n / kChunk + (size_t)ncells + 1;
   if (chunks_ub > A.chunk_cap) {
-    void *ptrs[] = {A.cfirst, A.ccount};
-    for (auto p : ptrs) if (p) hipFree(p);
-    PSPH_TRY(dmalloc((void **)&A.cfirst, chunks_ub * 4));
-    PSPH_TRY(dmalloc((void **)&A.ccount, chunks_ub * 4));
+    uint32_t **arrs[] = {&A.cfirst, &A.ccount};
+    for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
+    A.chunk_cap = 0;
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, chunks_ub * 4));
     A.chunk_cap = chunks_ub;
   }
-  if (!A.nchunks) PSPH_TRY(dmalloc((void **)&A.nchunks, 4));
+  if (!A.made) {
+    PSPH_TRY(dmalloc((void **)&A.made, 2 * 8));
+    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, A.made, 0ull, 2);
+  }
   hipLaunchKernelGGL(k_adj_row_flags, blocks(n + 1), 256, 0, s, n, R.bc, R.gflag, A.flags);
   PSPH_TRY(excl_scan(c, A.flags, A.tpos, (size_t)n + 1));
   if (n) hipLaunchKernelGGL(k_targets, blocks(n), 256, 0, s, n, A.flags, A.tpos, A.rows);
   hipLaunchKernelGGL(k_cell_chunks, blocks(ncells + 1), 256, 0, s, ncells, R.cs, A.tpos, (uint32_t)kChunk, A.cchunks);
   PSPH_TRY(excl_scan(c, A.cchunks, A.coff, (size_t)ncells + 1));
   hipLaunchKernelGGL(k_chunks, blocks(ncells + 1), 256, 0, s, ncells, R.cs, A.tpos, A.coff,
-                     (uint32_t)kChunk, A.cfirst, A.ccount, A.nchunks);
+                     (uint32_t)kChunk, A.cfirst, A.ccount, (uint32_t *)(A.made + 1));
+  if (n) launch_order(c, n, ncells, R.cs, A.tpos, R.d[RF_X], R.d[RF_Y], R.d[RF_Z], A.rows);
   HIP_TRY(hipGetLastError());
   return 0;
 }
 
-// visit lists of the step's row chunks (count, scan, masks)
-static int adj_visits(psph_ctx *c, Adjoint &A, const StepRec &R, const AdjCommon &pc, AdjVisits &vl) {
-  const unsigned G = chunk_grid(R.n, R.grid.ncells, kChunk);
-  if ((size_t)G + 1 > A.vchunk_cap) {
-    uint32_t **arrs[] = {&A.vcount, &A.voff, &A.vnum};
-    for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)G + 1) * 4));
-    A.vchunk_cap = (size_t)G + 1;
-  }
-  hipLaunchKernelGGL(k_adj_visit_count, G, kWave, 0, c->stream, pc, A.vcount);
-  hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, (int *)A.vcount + G, 0, 1);
-  HIP_TRY(hipGetLastError());
-  PSPH_TRY(excl_scan(c, A.vcount, A.voff, (size_t)G + 1));
-  uint32_t total = 0;
-  HIP_TRY(hipMemcpyAsync(&total, A.voff + G, 4, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  if ((size_t)total > A.vis_cap) {
-    if (A.vmask) hipFree(A.vmask);
-    if (A.vent) hipFree(A.vent);
-    A.vmask = nullptr;
-    A.vent = nullptr;
-    const size_t cap = (size_t)total + total / 8 + 1024;
-    PSPH_TRY(dmalloc((void **)&A.vmask, cap * kWave * sizeof(uint64_t)));
-    PSPH_TRY(dmalloc((void **)&A.vent, cap * sizeof(uint2)));
-    A.vis_cap = cap;
-  }
-  hipLaunchKernelGGL(k_adj_visit_masks, G, kWave, 0, c->stream, pc, c->cfg.cutoff * (1.0 + 1e-12), A.voff, A.vnum,
-                     A.vent, A.vmask);
-  HIP_TRY(hipGetLastError());
-  vl = AdjVisits{A.voff, A.vnum, A.vent, A.vmask};
+// the visits of the row groups (they take the place of the context's own, which
+// the next search makes again)
+static int adj_lists(psph_ctx *c, Adjoint &A, const StepRec &R, const AdjCommon &pc, GroupLists &gl, uint32_t &ngroups) {
+  c->lists_valid = false;
+  PSPH_TRY(group_memory(c, R.n / kChunk + (size_t)R.grid.ncells + 1));
+  hipLaunchKernelGGL(k_geom, blocks(R.n), 256, 0, c->stream, (uint32_t)R.n, pc.p.x, pc.p.y, pc.p.z, pc.h, c->gxy, c->gzh);
+  const ListOf of{R.n, R.grid.ncells, pc.h, R.hmax, A.made, true};
+  PSPH_TRY(build_lists(c, pc.p, of, 0.0, nullptr, ngroups));
+  gl = group_common(c).gl;
   return 0;
 }
 
 template <class P>
-static void launch_adj(psph_ctx *c, const AdjCommon &pc, const AdjVisits &vl, const StepRec &R,
-                       const typename P::Args &a) {
-  hipLaunchKernelGGL((k_adj_pairs<P>), chunk_grid(R.n, R.grid.ncells, kChunk), kWave, 0, c->stream, pc, vl, a);
+static void launch_adj(psph_ctx *c, const AdjCommon &pc, const GroupLists &gl, uint32_t ngroups, const typename P::Args &a) {
+  const unsigned nb = (ngroups + kXcds - 1) / kXcds * kXcds;
+  if (!nb) return;
+  const unsigned split = ngroups <= 16384 ? kAdjSplit : 1;
+  hipLaunchKernelGGL((k_adj_pass<P>), nb, split * kWave, split * sizeof(AdjLds<P>), c->stream, pc, gl, a);
 }
 
 struct ThetaGrad { double v = 0, T = 0, ng0 = 0; };
@@ -1414,25 +1306,31 @@ static int reverse_step(psph_ctx *c, Adjoint &A, StepRec &R, ThetaGrad &th) {
   // 3. position update
   hipLaunchKernelGGL(k_adj_pos, blocks(n), 256, 0, st, n, R.bc, R.erupting, k.lans, R.dt, l);
   PSPH_TRY(adj_rows(c, A, R));
-  AdjCommon pc;
-  pc.x = R.d[RF_X]; pc.y = R.d[RF_Y]; pc.z = R.d[RF_Z]; pc.h = R.d[RF_H]; pc.h_list = R.d[RF_HLIST];
-  pc.refb = R.refb; pc.rows = A.rows;
-  pc.cfirst = A.cfirst; pc.ccount = A.ccount; pc.nchunks = A.nchunks;
-  pc.bc = R.bc;
-  pc.tr = Traversal{R.cs, R.toff, R.tbox, R.grid, R.reach};
-  pc.list_all = k.list_all ? 1 : 0;
-  pc.list_adj = list_adj(k, R.hmax);
-  pc.list_factor = k.list_factor; pc.cutoff2 = k.cutoff2;
-  pc.cut = cut_test(k.cutoff);
-  AdjVisits vl;
-  PSPH_TRY(adj_visits(c, A, R, pc, vl));
+  AdjCommon pc{};
+  pc.p.x = pc.p.ax = R.d[RF_X]; pc.p.y = pc.p.ay = R.d[RF_Y]; pc.p.z = pc.p.az = R.d[RF_Z];
+  pc.p.refb = R.refb; pc.p.h_list = R.d[RF_HLIST]; pc.p.bc = R.bc;
+  pc.p.tr = Traversal{R.cs, R.toff, R.tbox, R.grid, R.reach};
+  pc.p.targets = A.rows;
+  pc.p.cfirst = A.cfirst; pc.p.ccount = A.ccount; pc.p.nchunks = (const uint32_t *)(A.made + 1);
+  pc.p.list_all = k.list_all ? 1 : 0;
+  pc.p.list_adj = list_adj(k, R.hmax);
+  pc.p.list_factor = k.list_factor;
+  pc.p.del = k.bucket_edge;
+  for (int d = 0; d < 3; d++) pc.p.ext_lo[d] = k.ext_lo[d];
+  pc.p.cut = cut_test(k.cutoff);
+  pc.p.err = c->d_err;
+  pc.h = R.d[RF_H];
+  pc.cutoff2 = k.cutoff2;
+  GroupLists vl;
+  uint32_t ngr = 0;
+  PSPH_TRY(adj_lists(c, A, R, pc, vl, ngr));
   // 4. velocity filter
   if (k.lans) {
     hipLaunchKernelGGL(k_adj_vsm_pre, blocks(n), 256, 0, st, n, R.bc, R.d[RF_WNV], R.d[RF_SV2X], R.d[RF_SV2Y],
                        R.d[RF_SV2Z], l, A.aux[0], A.aux[1], A.aux[2], A.aux[3]);
     VsmAdj::Args a{R.d[RF_M], R.d[RF_RHO2], R.d[RF_H], R.d[RF_V1X], R.d[RF_V1Y], R.d[RF_V1Z], A.aux[0], A.aux[1],
                    A.aux[2], A.aux[3], R.bc, l};
-    launch_adj<VsmAdj>(c, pc, vl, R, a);
+    launch_adj<VsmAdj>(c, pc, vl, ngr, a);
   }
   // 5. density + EOS
   {
@@ -1444,7 +1342,7 @@ static int reverse_step(psph_ctx *c, Adjoint &A, StepRec &R, ThetaGrad &th) {
     DensAdj::Args a{R.d[RF_M], R.d[RF_RHO], R.d[RF_E1], R.bc, R.phase, A.aux[0], A.aux[1], A.aux[2], A.aux[3],
                     k.e_smooth_ratio, k.pghost_contrib, k.energy_smooth,
                     k.e_smooth_ratio * k.e_smooth_ratio == 16.0 ? 1 : 0, cut_test(k.cutoff), l};
-    launch_adj<DensAdj>(c, pc, vl, R, a);
+    launch_adj<DensAdj>(c, pc, vl, ngr, a);
   }
   // 6. momentum / energy
   {
@@ -1458,7 +1356,7 @@ static int reverse_step(psph_ctx *c, Adjoint &A, StepRec &R, ThetaGrad &th) {
     a.a0 = A.aux[0]; a.a1 = A.aux[1]; a.a2 = A.aux[2]; a.ae = A.aux[3];
     a.k = RhsAdjConst{k.alpha, k.beta, k.ata, k.eps_half, k.prandtl, k.lans};
     a.l = l;
-    launch_adj<RhsAdj>(c, pc, vl, R, a);
+    launch_adj<RhsAdj>(c, pc, vl, ngr, a);
   }
   hipLaunchKernelGGL(k_lam_scatter, blocks(n), 256, 0, st, n, R.pid, l, Lid);
   HIP_TRY(hipGetLastError());

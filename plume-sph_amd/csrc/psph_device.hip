@@ -330,23 +330,6 @@ struct ChunkBox {
   float lo[3], hi[3];
 };
 
-__device__ inline ChunkBox chunk_box(const Traversal &tr, const double *p) {
-  ChunkBox b;
-  const int nn[3] = {tr.g.nx, tr.g.ny, tr.g.nz};
-  for (int d = 0; d < 3; d++) {
-    const double lo = wave_min(p[d]) - tr.reach, hi = wave_max(p[d]) + tr.reach;
-    b.lo[d] = __double2float_rd(lo);
-    b.hi[d] = __double2float_ru(hi);
-    if (tr.g.inv_e > 0) {
-      b.c0[d] = cell_of(lo, tr.g.lo[d], tr.g.inv_e, nn[d]);
-      b.c1[d] = cell_of(hi, tr.g.lo[d], tr.g.inv_e, nn[d]);
-    } else {
-      b.c0[d] = b.c1[d] = 0;
-    }
-  }
-  return b;
-}
-
 __device__ inline bool tile_meets(const ChunkBox &b, const float4 *tbox, uint32_t t) {
   const float4 lo = tbox[2 * t], hi = tbox[2 * t + 1];
   return !(lo.x > b.hi[0] || hi.x < b.lo[0] || lo.y > b.hi[1] || hi.y < b.lo[1] || lo.z > b.hi[2] || hi.z < b.lo[2]);
@@ -406,14 +389,11 @@ __device__ inline ChunkBox chunk_list_box(const PairCommon &pc, const double *p,
   return b;
 }
 
-// A chunk: up to kChunk targets, consecutive in the cell's fine Morton order, so
+// A chunk: up to kChunk targets, consecutive in the order of the cell's targets, so
 // they sit within ~2 particle spacings of each other and the union of their
-// neighbourhoods is little more than one of them.  The reverse pair passes serve
-// each of a chunk's rows with kSub lanes that take every kSub-th candidate of a
-// staged tile; the partial sums are combined by a fixed shuffle tree.
-constexpr int kSub = 2;
+// neighbourhoods is little more than one of them.
 constexpr double kFar = 1.0e300;
-constexpr int kChunk = kWave / kSub;
+constexpr int kChunk = kWave / 2;
 
 // List materialisation (parity checks only): one wavefront per chunk, a target a
 // lane.  The candidates accepted are exactly the reference's list
@@ -509,24 +489,6 @@ __global__ void k_geom(uint32_t n, const double *x, const double *y, const doubl
   if (i >= n) return;
   xy[i] = make_double2(x[i], y[i]);
   zh[i] = make_double2(z[i], 0.5 * h[i]);
-}
-
-// tiles that meet each chunk's grown box (an upper bound on its visits);
-// one wavefront per chunk, chunk = blockIdx.x, zero past the last chunk; the
-// lanes take the box's cells in turn
-__device__ inline uint32_t count_meeting_tiles(const Traversal &tr, const ChunkBox &box) {
-  const GridDesc &g = tr.g;
-  const int bx = box.c1[0] - box.c0[0] + 1, by = box.c1[1] - box.c0[1] + 1, bz = box.c1[2] - box.c0[2] + 1;
-  const int nbox = bx * by * bz;
-  uint32_t cnt = 0;
-  for (int k = threadIdx.x; k < nbox; k += kWave) {
-    const int cx = box.c0[0] + k % bx, cy = box.c0[1] + (k / bx) % by, cz = box.c0[2] + k / (bx * by);
-    const uint32_t cell = ((uint32_t)cz * g.ny + cy) * g.nx + cx;
-    const uint32_t t0 = tr.toff[cell], t1 = tr.toff[cell + 1];
-    for (uint32_t t = t0; t < t1; t++) cnt += tile_meets(box, tr.tbox, t) ? 1u : 0u;
-  }
-  for (int o = 32; o > 0; o >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, o);
-  return cnt;
 }
 
 // m &= ~(1 << b) for a wave-uniform 64-bit mask in scalar registers: one
@@ -703,7 +665,9 @@ struct GroupCommon {
   Geom g;
   GroupLists gl;
   double cutx;               // cut with a relative margin of 1e-12
+  double cutj;               // of a particle's h / 2: cutx, or 2 cutx for lists of both roles
   double h_max;
+  int both;                  // lists of the adjoint: kernel boxes of the larger h of a pair
   // lists for an iteration of the adaptive h: the kernel's h over h (0: lists
   // for the three passes) and the targets that have converged
   double c_smooth;
@@ -736,12 +700,12 @@ __device__ inline double group_max(double v) {
   return v;
 }
 
-// |x_k - c_k| - b_k <= max(chh + cutx h_j / 2, ch) holds on every axis for each
+// |x_k - c_k| - b_k <= max(chh + cutj h_j / 2, ch) holds on every axis for each
 // particle j that is a pair of one of the group's targets in any of the passes
 // (b with room for the rounding of c and of the differences).
 struct GroupBox {
   double c[3], b[3];
-  double chh, ch;            // cutx h / 2 and cutx h of the group's largest h
+  double chh, ch;            // cutx h / 2 (both roles: 0) and cutx h of the group's largest h
   float lo[3], up[3];        // the grown box
 };
 
@@ -796,6 +760,12 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
       B.chh = -HUGE_VAL;
       B.ch = group_max(in ? w : 0.0);
       widest = B.ch * (1 + 1e-9);
+    } else if (gc.both) {
+      // |x_k - x_j| <= cutx max(h_i, h_j)
+      fast = false;
+      B.ch = gc.cutx * group_max(hi);
+      B.chh = 0;
+      widest = fmax(B.ch, gc.cutx * gc.h_max) * (1 + 1e-9);
     } else {
       widest = gc.cutx * fmax(0.5 * hi + 0.5 * gc.h_max, hi);
       fast = widest <= supp && (pc.list_all != 0 || (widest <= lf && widest * (1 + 1e-12) < pc.del));
@@ -878,7 +848,7 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
           const uint32_t gm = __builtin_amdgcn_readlane(meets, l);
           const uint32_t j = base + min((uint32_t)lane, cnt - 1u);
           const double2 xy = gc.g.xy[j], zh = gc.g.zh[j];
-          const double chh = gc.cutx * zh.y;
+          const double chh = gc.cutj * zh.y;
           const uint64_t valid = cnt < kWave ? (1ull << cnt) - 1 : ~0ull;
 #pragma unroll
           for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
@@ -1141,12 +1111,6 @@ __global__ __launch_bounds__(kMaxSplit * kWave, P::kWaves) void k_group_pass(Pai
     if (lane == 0 && npairs > nt) atomicAdd(a.pairs, (unsigned long long)(npairs - nt));
 }
 
-// sum of v over the kSub lanes of a target (lanes slot*kSub .. +kSub-1)
-template <int S>
-__device__ inline double sub_sum(double v) {
-  for (int o = 1; o < S; o <<= 1) v += __shfl_xor(v, o);
-  return v;
-}
 constexpr double kInvSqrtPi = 0.564189583547756;   // sph_lib.cc:207
 
 // The pair arithmetic type R is double (FP64 form) or float (FP32-pair form):
@@ -1174,30 +1138,12 @@ template <class R> __device__ inline R rabs(R x);
 template <> __device__ inline double rabs<double>(double x) { return __builtin_fabs(x); }
 template <> __device__ inline float rabs<float>(float x) { return __builtin_fabsf(x); }
 
-// exp(-e) in FP64 for 0 <= e < kETab / 8 from a table of exp(-k/8) and the
-// Taylor series of exp(-r), 0 <= r < 1/8, to r^10 (truncation < 6e-18).  The
-// table lives in each workgroup's LDS; 224 entries (1.75 KB) keep the density
-// pass at 6 waves per SIMD.
-constexpr int kETab = 224;            // covers the kernel box: e = |s|^2 <= 27
-__device__ inline void etab_fill(double *tab, int lane) {
-  for (int k = lane; k < kETab; k += kWave) tab[k] = exp(-0.125 * k);
-}
-__device__ inline double exp_neg_tab(double e, const double *tab) {
-  const double k = fmin(floor(e * 8.0), (double)(kETab - 1));
-  const double r = e - 0.125 * k;
-  double p = 1.0 / 3628800;
-  p = fma(p, -r, 1.0 / 362880); p = fma(p, -r, 1.0 / 40320); p = fma(p, -r, 1.0 / 5040);
-  p = fma(p, -r, 1.0 / 720); p = fma(p, -r, 1.0 / 120); p = fma(p, -r, 1.0 / 24);
-  p = fma(p, -r, 1.0 / 6); p = fma(p, -r, 0.5); p = fma(p, -r, 1.0); p = fma(p, -r, 1.0);
-  return tab[(int)k] * p;
-}
-
 // exp(-e) in FP64 for e >= 0 without a table (Cody and Waite's reduction: e = -k
 // ln 2 - r with k an integer, |r| <= ln 2 / 2, ln 2 in two parts; then 1 + r +
 // r^2 q(r) with q the degree-9 polynomial through the Chebyshev nodes of the
 // interval, computed for this file in 60-digit arithmetic: truncation 1.7e-17).
-// Measured over 0 <= e <= 27.5: 1.0 ulp at most, 0.30 ulp rms (the table form
-// below: 1.9 and 0.47; the C library's: 0.51 and 0.29).  16 VALU instructions
+// Measured over 0 <= e <= 27.5: 1.0 ulp at most, 0.30 ulp rms (a table of
+// exp(-k/8) and a series of degree 10: 1.9 and 0.47; the C library's: 0.51 and 0.29).  16 VALU instructions
 // and no LDS.
 __device__ inline double exp_neg(double e) {
   const double magic = 6755399441055744.0;               // 1.5 * 2^52: kd's low word is k
@@ -2867,6 +2813,13 @@ static int excl_scan(psph_ctx *c, const uint32_t *in, uint32_t *out, size_t n1) 
   return 0;
 }
 
+static void launch_order(psph_ctx *c, uint32_t n, uint32_t ncells, const uint32_t *cs, const uint32_t *tpos,
+                         const double *x, const double *y, const double *z, uint32_t *targets) {
+  // one cell holds everything: a wavefront per run, else per cell
+  const uint32_t per_cell = ncells == 1 ? (n + kRun - 1) / kRun : 1;
+  hipLaunchKernelGGL(k_order_targets, ncells * per_cell, kWave, 0, c->stream, cs, tpos, per_cell, x, y, z, targets);
+}
+
 extern "C" int psph_neighbors(psph_ctx *c) {
   if (!c) return fail(PSPH_EINVAL, "null ctx");
   PSPH_TRY(build_grid(c));
@@ -2962,12 +2915,7 @@ extern "C" int psph_neighbors(psph_ctx *c) {
   PSPH_TRY(excl_scan(c, c->cchunks, c->coff, (size_t)g.ncells + 1));
   hipLaunchKernelGGL(k_chunks, blocks(g.ncells + 1), 256, 0, s, g.ncells, c->cs, c->tpos, c->coff,
                      (uint32_t)kChunk, c->cfirst, c->ccount, c->nchunks);
-  if (n) {
-    // one cell holds everything: a wavefront per run, else per cell
-    const uint32_t per_cell = g.ncells == 1 ? (n + kRun - 1) / kRun : 1;
-    hipLaunchKernelGGL(k_order_targets, g.ncells * per_cell, kWave, 0, s, c->cs, c->tpos, per_cell, qx, qy, qz,
-                       c->targets);
-  }
+  if (n) launch_order(c, n, g.ncells, c->cs, c->tpos, qx, qy, qz, c->targets);
   HIP_TRY(hipGetLastError());
   tm.stop();
   c->grid_valid = true;
@@ -3029,27 +2977,39 @@ static void launch_list(psph_ctx *c, double reach, uint32_t *count, const uint32
   else hipLaunchKernelGGL(k_list<1>, nb, kWave, 0, c->stream, pc, count, offset, out);
 }
 
+// what the visits are made for: particles, cells, smoothing lengths and their
+// bound, the visit cursor (the number of chunks follows it), and whether a pair
+// counts for both of its particles
+struct ListOf {
+  size_t n, ncells;
+  const double *h;
+  double h_max;
+  unsigned long long *cursor;
+  bool both;
+};
+
 static GroupCommon group_common(psph_ctx *c) {
   GroupCommon gc{};
   gc.g = Geom{c->gxy, c->gzh};
   gc.gl = GroupLists{c->gvisit, c->goff, c->gnum, c->gfast, c->gcursor, c->gvisit_cap};
   gc.cutx = c->cfg.cutoff * (1.0 + 1e-12);     // a superset of the three passes' kernel boxes
+  gc.cutj = gc.cutx;
   gc.h_max = c->h_max;
   return gc;
 }
 
 // memory of the group passes: positions, record arrays, per-group offsets
-static int group_memory(psph_ctx *c) {
+static int group_memory(psph_ctx *c, size_t chunks) {
   if (!c->gxy) PSPH_TRY(dmalloc((void **)&c->gxy, c->cap * sizeof(double2)));
   if (!c->gzh) PSPH_TRY(dmalloc((void **)&c->gzh, c->cap * sizeof(double2)));
   for (auto &p : c->pk)
     if (!p) PSPH_TRY(dmalloc(&p, c->cap * 16));
-  if (c->chunk_cap > c->gchunk_cap) {
+  if (chunks > c->gchunk_cap) {
     uint32_t **arrs[] = {&c->goff, &c->gnum, &c->gfast};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
     c->gchunk_cap = 0;
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, c->chunk_cap * kGroupsPerChunk * 4));
-    c->gchunk_cap = c->chunk_cap;
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, chunks * kGroupsPerChunk * 4));
+    c->gchunk_cap = chunks;
   }
   return 0;
 }
@@ -3059,26 +3019,31 @@ static void launch_geom(psph_ctx *c, const PairCommon &pc) {
 }
 
 // the groups' visits for the boxes that c_smooth and done say (GroupCommon)
-static int build_lists(psph_ctx *c, const PairCommon &pc, double c_smooth, const uint32_t *done) {
+static int build_lists(psph_ctx *c, const PairCommon &pc, const ListOf &of, double c_smooth, const uint32_t *done,
+                       uint32_t &ngroups) {
   // a group per wave up to a quarter of a million particles: at 77k 0.15 ms against
   // 0.20 with half a chunk; a chunk per wave beyond
-  const uint32_t nsplit = c->n < (1u << 18) ? kGroupsPerChunk : 1;
-  const unsigned G = chunk_grid(c->n, c->grid.ncells, kChunk) * nsplit;
+  const uint32_t nsplit = of.n < (1u << 18) ? kGroupsPerChunk : 1;
+  const unsigned G = chunk_grid(of.n, of.ncells, kChunk) * nsplit;
   for (;;) {
     GroupCommon gc = group_common(c);
     gc.c_smooth = c_smooth;
     gc.done = done;
-    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->gcursor, 0ull, 1);
+    gc.gl.cursor = of.cursor;
+    gc.h_max = of.h_max;
+    gc.both = of.both ? 1 : 0;
+    if (of.both) gc.cutj = 2 * gc.cutx;
+    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, of.cursor, 0ull, 1);
     if (c->cfg.dim == 3)
-      hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
+      hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
     else
-      hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, c->f.h, c->cfg.cutoff2, nsplit);
+      hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
     HIP_TRY(hipGetLastError());
-    unsigned long long got[2] = {0, 0};         // visits; chunks (nchunks)
-    HIP_TRY(hipMemcpyAsync(got, c->gcursor, 16, hipMemcpyDeviceToHost, c->stream));
+    unsigned long long got[2] = {0, 0};         // visits; chunks
+    HIP_TRY(hipMemcpyAsync(got, of.cursor, 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     const unsigned long long total = got[0];
-    c->ngroups = (uint32_t)got[1] * kGroupsPerChunk;
+    ngroups = (uint32_t)got[1] * kGroupsPerChunk;
     if (total <= c->gvisit_cap) return 0;
     // the visits outgrew their memory: this call only counted
     constexpr unsigned long long kMost = 0xffffffffull;      // GroupLists::off
@@ -3092,15 +3057,19 @@ static int build_lists(psph_ctx *c, const PairCommon &pc, double c_smooth, const
   }
 }
 
+static ListOf own_lists(const psph_ctx *c) {
+  return ListOf{c->n, c->grid.ncells, c->f.h, c->h_max, c->gcursor, false};
+}
+
 // Lists and positions of the group passes (positions, h and targets fixed since
 // the last psph_neighbors / adaptation).
 static int ensure_lists(psph_ctx *c) {
   if (c->lists_valid) return 0;
   StageTimer tm(c, 1);
-  PSPH_TRY(group_memory(c));
+  PSPH_TRY(group_memory(c, c->chunk_cap));
   const PairCommon pc = make_common(c, c->reach_main);
   launch_geom(c, pc);
-  PSPH_TRY(build_lists(c, pc, 0.0, nullptr));
+  PSPH_TRY(build_lists(c, pc, own_lists(c), 0.0, nullptr, c->ngroups));
   c->lists_valid = true;
   return 0;
 }
@@ -3208,7 +3177,7 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
   double hmax = c->h_max;
   if (c->n && k.num_loop > 0) {
     HIP_TRY(hipMemsetAsync(c->usp, 0, c->n * 4, c->stream));
-    PSPH_TRY(group_memory(c));
+    PSPH_TRY(group_memory(c, c->chunk_cap));
     const PairCommon pc = make_common(c, c->reach_main);
     launch_geom(c, pc);
     // FP64 arithmetic in every form (h enters every later pass, and a
@@ -3219,7 +3188,7 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
     else launch_pack<AdaptPass<double>>(c, a, FieldCopy{});
     for (int it = 0; it < k.num_loop; it++) {
       StageTimer tm(c, 2);
-      PSPH_TRY(build_lists(c, pc, k.c_smooth, c->usp));
+      PSPH_TRY(build_lists(c, pc, own_lists(c), k.c_smooth, c->usp, c->ngroups));
       const GroupCommon gc = group_common(c);
       if (k.dim == 3) {
         if (fx) launch_group_kernel<3, AdaptPass<double, true>>(c, pc, gc, a, false);
