@@ -327,7 +327,7 @@ struct VsmAdj {
   };
   struct Rec { double mr, ih2, nrm, v[3], a[3], c; int ok; };
   struct Row { double imi, irho, mr, ih2, nrm, v[3], a[3], c; bool ok; };
-  static constexpr int kWaves = 3;             // per SIMD: at most 168 VGPRs
+  static constexpr int kWaves = 2;             // (158 VGPRs, 3 waves per SIMD; asked for 3: 453 us)
   static constexpr int NACC = 8;               // 0-2: x, 3-5: v, 6: m, 7: rho
   __device__ static void load_row(const Args &A, uint32_t i, Row &t) {
     const double mi = A.m[i], rhoi = A.rho[i], ih = 1.0 / A.h[i], nk = kInvSqrtPi * ih;
@@ -673,6 +673,30 @@ __global__ void k_adj_row_flags(uint32_t n, const int32_t *bc, const uint32_t *g
   flags[i] = (is_real(b) || b == 0 || ((b == 1 || b == 2) && gflag[i])) ? 1u : 0u;
 }
 
+// erupt ghosts of the starting state, and what their theta-gradient takes:
+// row r of out holds field f at out[f rows + r]
+__global__ void k_erupt_flags(uint32_t n, const int32_t *bc, uint32_t *flags) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n) flags[i] = (i < n && bc[i] == 0) ? 1u : 0u;
+}
+struct EruptRows { const double *f[9]; };
+__global__ void k_erupt_rows(uint32_t rows, const uint32_t *idx, EruptRows from, double *out) {
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  const uint32_t i = idx[r];
+  for (int f = 0; f < 9; f++) out[(size_t)f * rows + r] = from.f[f][i];
+}
+// three components of rows r0.. of a permutation, interleaved
+__global__ void k_rows3(uint32_t rows, uint32_t r0, const uint32_t *perm, const double *x, const double *y,
+                        const double *z, double *out) {
+  const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  const uint32_t i = perm[r0 + r];
+  out[3 * (size_t)r] = x[i];
+  out[3 * (size_t)r + 1] = y[i];
+  out[3 * (size_t)r + 2] = z[i];
+}
+
 // fixed-order block sums of one array
 __global__ void k_sum_blocks(uint32_t n, const double *v, double *part) {
   __shared__ double sh[256];
@@ -958,20 +982,24 @@ static int dev_sum(psph_ctx *c, Adjoint &A, const double *v, size_t n, double *o
   return 0;
 }
 
+static int adj_row_memory(psph_ctx *c, Adjoint &A, size_t n) {
+  if (n + 1 <= A.n_cap) return 0;
+  uint32_t **arrs[] = {&A.flags, &A.tpos, &A.rows};
+  for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
+  A.n_cap = 0;
+  const size_t cap = std::max<size_t>(c->cap, n) + 1;
+  for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, cap * 4));
+  A.n_cap = cap;
+  return 0;
+}
+
 // groups of adjoint rows of one step (chunks of kChunk consecutive rows of a cell)
 static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
   const uint32_t n = (uint32_t)R.n;
   const GridDesc &g = R.grid;
   const uint32_t ncells = g.ncells;
   hipStream_t s = c->stream;
-  if (n + 1 > A.n_cap) {
-    uint32_t **arrs[] = {&A.flags, &A.tpos, &A.rows};
-    for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
-    A.n_cap = 0;
-    const size_t cap = std::max<size_t>(c->cap, n) + 1;
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, cap * 4));
-    A.n_cap = cap;
-  }
+  PSPH_TRY(adj_row_memory(c, A, n));
   if (ncells + 1 > A.cell_cap) {
     uint32_t **arrs[] = {&A.cchunks, &A.coff};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
@@ -1461,63 +1489,73 @@ extern "C" int psph_adjoint_run(psph_ctx *c, int64_t nsteps, int64_t ckpt_every,
 
   // ---- initial state: setup ghosts and the per-particle output ----
   const Snapshot &S0 = A.ck[0];
-  std::vector<int32_t> bc0(n0);
-  std::vector<double> x0(n0), y0(n0), lam0(6 * std::max<size_t>(n0, 1));
-  std::vector<double> lm(pid_end);
+  // (id q is the q-th particle of S0.)  The setup's erupt ghosts are few: their
+  // rows are picked on the device, in order.
+  std::vector<double> er;
+  uint32_t nerupt = 0;
+  tp.mode = 0;
   if (n0) {
-    HIP_TRY(hipMemcpyAsync(bc0.data(), S0.i[0], n0 * 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(x0.data(), S0.d[0], n0 * 8, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipMemcpyAsync(y0.data(), S0.d[1], n0 * 8, hipMemcpyDeviceToHost, st));
-    const int fl[6] = {L_Z, L_VZ, L_RHO, L_E, L_T, L_CP};
-    for (int f = 0; f < 6; f++) HIP_TRY(hipMemcpyAsync(lam0.data() + f * n0, A.L[fl[f]], n0 * 8, hipMemcpyDeviceToHost, st));
+    PSPH_TRY(adj_row_memory(c, A, n0));
+    hipLaunchKernelGGL(k_erupt_flags, blocks(n0 + 1), 256, 0, st, (uint32_t)n0, S0.i[0], A.flags);
+    PSPH_TRY(excl_scan(c, A.flags, A.tpos, n0 + 1));
+    hipLaunchKernelGGL(k_targets, blocks(n0), 256, 0, st, (uint32_t)n0, A.flags, A.tpos, A.rows);
+    HIP_TRY(hipMemcpyAsync(&nerupt, A.tpos + n0, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
   }
-  if (pid_end) HIP_TRY(hipMemcpyAsync(lm.data(), A.L[L_M], (size_t)pid_end * 8, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
+  if (nerupt) {
+    double *rows = nullptr;
+    PSPH_TRY(dmalloc((void **)&rows, (size_t)nerupt * 9 * 8));
+    const EruptRows from{{A.L[L_Z], A.L[L_VZ], A.L[L_RHO], A.L[L_E], A.L[L_T], A.L[L_CP], A.L[L_M], S0.d[0], S0.d[1]}};
+    hipLaunchKernelGGL(k_erupt_rows, blocks(nerupt), 256, 0, st, nerupt, A.rows, from, rows);
+    er.resize((size_t)nerupt * 9);
+    const hipError_t got = hipMemcpyAsync(er.data(), rows, er.size() * 8, hipMemcpyDeviceToHost, st);
+    const hipError_t done = hipStreamSynchronize(st);
+    hipFree(rows);
+    HIP_TRY(got);
+    HIP_TRY(done);
+  }
+  std::vector<double> lm(pid_end - n0);
+  if (pid_end > n0) HIP_TRY(hipMemcpy(lm.data(), A.L[L_M] + n0, lm.size() * 8, hipMemcpyDeviceToHost));
   const VentDeriv vd = vent_deriv(k);
   double lm_erupt = 0;
-  for (size_t q = 0; q < n0; q++) {
-    if (bc0[q] != 0) continue;
-    double one[6];
-    for (int f = 0; f < 6; f++) one[f] = lam0[f * n0 + q];
+  for (size_t q = 0; q < nerupt; q++) {
+    double one[9];
+    for (int f = 0; f < 9; f++) one[f] = er[f * nerupt + q];
     one[0] = 0;                                   // setup ghosts: z independent of the vent velocity
     // column exit velocity (vel_prof, sph_lib.cc:1223-1243) at the ghost's column centre
-    const double rsq = x0[q] * x0[q] + y0[q] * y0[q];
+    const double rsq = one[7] * one[7] + one[8] * one[8];
     const double vel = k.vent_profile == 0 ? k.vent_v : 2 * k.vent_v * (1 - rsq / (k.vent_r * k.vent_r));
     ghost_theta(k, vd, vel, 0.0, one, th);
-    lm_erupt += lm[q];
+    lm_erupt += one[6];
   }
-  for (size_t q = n0; q < pid_end; q++) lm_erupt += lm[q];   // every ghost the inlet added
+  for (double v : lm) lm_erupt += v;                           // every ghost the inlet added
   th.T += lm_erupt * vd.dm_dT;
   th.ng0 += lm_erupt * vd.dm_dn;
 
   if (grad_v || grad_sv) {
     // psph_read order of the state at the start: live particles, THashTable order
-    std::vector<uint32_t> k0(n0), k1(n0), k2(n0);
-    if (n0) {
-      HIP_TRY(hipMemcpy(k0.data(), S0.u[0], n0 * 4, hipMemcpyDeviceToHost));
-      HIP_TRY(hipMemcpy(k1.data(), S0.u[1], n0 * 4, hipMemcpyDeviceToHost));
-      HIP_TRY(hipMemcpy(k2.data(), S0.u[2], n0 * 4, hipMemcpyDeviceToHost));
-    }
-    std::vector<uint32_t> live;
-    for (size_t q = 0; q < n0; q++) if (bc0[q] >= 0) live.push_back((uint32_t)q);
-    std::vector<uint32_t> a0(live.size()), a1(live.size()), a2(live.size());
-    for (size_t q = 0; q < live.size(); q++) { a0[q] = k0[live[q]]; a1[q] = k1[live[q]]; a2[q] = k2[live[q]]; }
-    auto perm = canonical_order(k, a0.data(), a1.data(), a2.data(), live.size());
-    if (live.size() > n_cap) { tp.mode = 0; snap_load(c, A.fin); return fail(PSPH_ECAPACITY, "adjoint: %zu particles, gradient buffers hold %zu", live.size(), n_cap); }
+    unsigned long long cnt[2];
+    PSPH_TRY(count_live(c, n0, S0.i[0], cnt));
+    const size_t live = cnt[0];
+    if (live > n_cap) { snap_load(c, A.fin); return fail(PSPH_ECAPACITY, "adjoint: %zu particles, gradient buffers hold %zu", live, n_cap); }
+    PSPH_TRY(read_order(c, (uint32_t)n0, S0.u[0], S0.u[1], S0.u[2], S0.i[0]));
+    PSPH_TRY(group_memory(c, 0));
+    // through a record array, which holds two doubles a particle
+    const size_t at_once = c->cap / 2;
     for (int which = 0; which < 2; which++) {
       double *dst = which == 0 ? grad_v : grad_sv;
       if (!dst) continue;
-      std::vector<double> g3(3 * std::max<size_t>(n0, 1));
-      for (int d = 0; d < 3; d++)
-        if (n0) HIP_TRY(hipMemcpy(g3.data() + d * n0, A.L[(which == 0 ? L_VX : L_SVX) + d], n0 * 8, hipMemcpyDeviceToHost));
-      for (size_t r = 0; r < perm.size(); r++) {
-        const uint32_t id = live[perm[r]];
-        for (int d = 0; d < 3; d++) dst[3 * r + d] = g3[d * n0 + id];
+      double *const *g = A.L + (which == 0 ? L_VX : L_SVX);
+      for (size_t r0 = 0; r0 < live; r0 += at_once) {
+        const size_t rows = std::min(at_once, live - r0);
+        hipLaunchKernelGGL(k_rows3, blocks(rows), 256, 0, st, (uint32_t)rows, (uint32_t)r0, c->idx_b, g[0], g[1], g[2],
+                           (double *)c->pk[0]);
+        HIP_TRY(hipMemcpyAsync(dst + 3 * r0, c->pk[0], rows * 24, hipMemcpyDeviceToHost, st));
       }
     }
-    out->n_particles = (int64_t)live.size();
+    HIP_TRY(hipStreamSynchronize(st));
+    out->n_particles = (int64_t)live;
   }
-  tp.mode = 0;
   PSPH_TRY(snap_load(c, A.fin));
   HIP_TRY(hipStreamSynchronize(st));
   const double t_end = now_ms();

@@ -198,10 +198,31 @@ __global__ void k_cellkey(uint32_t n, const double *x, const double *y, const do
   key[i] = ((((uint32_t)cc[2] * g.ny + cc[1]) * g.nx + cc[0]) << sh) | m;
 }
 
-template <class T>
-__global__ void k_gather(uint32_t n, const uint32_t *perm, const T *__restrict__ src, T *__restrict__ dst) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[perm[i]];
+// dst[i] = src[perm[i]] for N8 arrays of 8 bytes an element and N4 of 4: the
+// index is read once and a thread has all its loads in flight (a launch per
+// array: 75 us of a step at 240k particles, 615 us at 6.8M; so 26 and 441).
+constexpr int kMove8 = 11, kMove4 = 7;
+struct Moves {
+  const uint64_t *s8[kMove8];
+  uint64_t *d8[kMove8];
+  const uint32_t *s4[kMove4];
+  uint32_t *d4[kMove4];
+};
+template <int N8, int N4>
+__global__ void k_gather(uint32_t n, const uint32_t *perm, Moves mv) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t from = perm[i];
+  uint64_t v8[N8 ? N8 : 1];
+  uint32_t v4[N4 ? N4 : 1];
+#pragma unroll
+  for (int k = 0; k < N8; k++) v8[k] = mv.s8[k][from];
+#pragma unroll
+  for (int k = 0; k < N4; k++) v4[k] = mv.s4[k][from];
+#pragma unroll
+  for (int k = 0; k < N8; k++) mv.d8[k][i] = v8[k];
+#pragma unroll
+  for (int k = 0; k < N4; k++) mv.d4[k][i] = v4[k];
 }
 
 // cell_start[c] = first sorted index whose cell (key >> sh) >= c, c in [0, ncells]
@@ -2251,6 +2272,53 @@ __global__ __launch_bounds__(256) void k_count_real(uint32_t n, const int32_t *b
   }
 }
 
+// live particles and, of them, the real ones: grid-stride, an atomic a block each
+__global__ __launch_bounds__(256) void k_count_live(uint32_t n, const int32_t *bc, unsigned long long *out) {
+  __shared__ unsigned int part[2][256 / kWave];
+  unsigned int cnt[2] = {0, 0};
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int b = bc[i];
+    cnt[0] += b >= 0 ? 1u : 0u;
+    cnt[1] += is_real(b) ? 1u : 0u;
+  }
+  for (int q = 0; q < 2; q++) {
+    for (int o = kWave / 2; o > 0; o >>= 1) cnt[q] += (unsigned int)__shfl_xor((int)cnt[q], o);
+    if ((threadIdx.x & (kWave - 1)) == 0) part[q][threadIdx.x / kWave] = cnt[q];
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    unsigned long long sum = 0;
+    for (int w = 0; w < 256 / kWave; w++) sum += part[threadIdx.x][w];
+    if (sum) atomicAdd(out + threadIdx.x, sum);
+  }
+}
+
+// THashTable order (thashtab.cc:209-262) by three stable sorts, the last key
+// first: key2; key0 and key1; the slot, with the removed particles past every
+// slot.  The keys of the particles in the order that perm has so far:
+__global__ void k_read_key01(uint32_t n, const uint32_t *perm, const uint32_t *k0, const uint32_t *k1, uint64_t *key) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t j = perm[i];
+  key[i] = (uint64_t)k0[j] << 32 | k1[j];
+}
+// the slot as table_slot has it (psph_host.cpp): quotient, product and sum of the
+// parts each rounded as there
+__global__ void k_read_slot(uint32_t n, const uint32_t *perm, const uint32_t *k0, const uint32_t *k1, const int32_t *bc,
+                            int table_size, int dim, uint64_t *key) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t j = perm[i];
+  uint32_t slot = k0[j];                             // 1D: the hash is key0
+  if (dim != 1) {
+    const double umax = 4294967295.0;
+    const int s2 = table_size / 10, s1 = table_size - s2;
+    const int i1 = (int)((double)k0[j] / umax * s1), i2 = (int)((double)k1[j] / umax * s2);
+    slot = (uint32_t)(i1 + i2) ^ 0x80000000u;        // (the sum of the sizes is an int)
+  }
+  key[i] = (bc[j] < 0 ? (uint64_t)1 << 32 : 0) | slot;
+}
+
 __global__ void k_iota_u32(uint32_t *p, uint32_t first, uint32_t n) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = first + i;
@@ -2404,6 +2472,8 @@ struct StepRec {
 };
 struct Adjoint;
 
+constexpr int kWords = 16;       // of psph_ctx::d_u64
+
 struct psph_ctx {
   psph_config cfg{};
   hipStream_t stream = nullptr;
@@ -2421,7 +2491,7 @@ struct psph_ctx {
   size_t cs_cap = 0, tile_cap = 0, chunk_cap = 0;
   void *cub = nullptr;
   size_t cub_bytes = 0;
-  unsigned long long *d_u64 = nullptr;   // [0] dt bits [1] hmax bits [2] pairs [3] dead
+  unsigned long long *d_u64 = nullptr;   // [0] dt bits [1] hmax bits [2] pairs [3] dead [8] live [9] real
   int *d_err = nullptr;
   double *d_part = nullptr;
   // grid of the last neighbour search
@@ -2566,13 +2636,13 @@ extern "C" int psph_create(const psph_config *cfg, size_t capacity, psph_ctx **o
     if (!rc) rc = dmalloc((void **)pp, capacity * 4);
   if (!rc) rc = dmalloc((void **)&c->flags, (capacity + 1) * 4);
   if (!rc) rc = dmalloc((void **)&c->tpos, (capacity + 1) * 4);
-  if (!rc) rc = dmalloc((void **)&c->d_u64, 8 * 8);
+  if (!rc) rc = dmalloc((void **)&c->d_u64, kWords * 8);
   if (!rc) { c->gcursor = c->d_u64 + 6; c->nchunks = (uint32_t *)(c->d_u64 + 7); }   // read in one copy
   if (!rc) rc = dmalloc((void **)&c->d_err, 2 * sizeof(int));
   if (!rc) rc = dmalloc((void **)&c->d_part, kRedBlocks * 8 * 8);
   if (rc) { psph_destroy(c); return rc; }
   hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, c->d_err, 0, 2);
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64, 0ull, 8);
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64, 0ull, kWords);
   c->next_output = cfg->t_output;
   *out = c;
   return 0;
@@ -2638,14 +2708,23 @@ extern "C" int psph_load(psph_ctx *c, const psph_soa *host, size_t n, double t0,
   return 0;
 }
 
+// live and real particles of bc[0..n)
+static int count_live(psph_ctx *c, size_t n, const int32_t *bc, unsigned long long cnt[2]) {
+  unsigned long long *out = c->d_u64 + 8;
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, out, 0ull, 2);
+  if (n) hipLaunchKernelGGL(k_count_live, red_blocks(n), 256, 0, c->stream, (uint32_t)n, bc, out);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(cnt, out, 16, hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return 0;
+}
+
 extern "C" int psph_count(psph_ctx *c, size_t *n_total, size_t *n_real) {
   if (!c) return fail(PSPH_EINVAL, "null ctx");
-  std::vector<int32_t> bc(c->n);
-  if (c->n) HIP_TRY(hipMemcpy(bc.data(), c->f.bc, c->n * 4, hipMemcpyDeviceToHost));
-  size_t nt = 0, nr = 0;
-  for (auto b : bc) { if (b >= 0) nt++; if (b == 100 || b == 99) nr++; }
-  if (n_total) *n_total = nt;
-  if (n_real) *n_real = nr;
+  unsigned long long cnt[2];
+  PSPH_TRY(count_live(c, c->n, c->f.bc, cnt));
+  if (n_total) *n_total = cnt[0];
+  if (n_real) *n_real = cnt[1];
   return 0;
 }
 
@@ -2688,21 +2767,63 @@ static int download(psph_ctx *c, HostParticles &P) {
   return 0;
 }
 
+// The n particles with these keys in THashTable order, removed ones last: their
+// indices in c->idx_b.  On the host the order took 21 ms of a read of 98k
+// particles (sort, and a permutation of every field), 15 ms of the gradients of 227k.
+static int read_order(psph_ctx *c, uint32_t n, const uint32_t *k0, const uint32_t *k1, const uint32_t *k2,
+                      const int32_t *bc) {
+  if (!n) return 0;
+  hipStream_t s = c->stream;
+  uint64_t *a = (uint64_t *)c->dsp[0], *b = (uint64_t *)c->dsp[1];
+  size_t b32 = 0, b64 = 0;
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, b32, k2, c->key_b, c->idx_a, c->idx_b, (int)n, 0, 32, s));
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, b64, a, b, c->idx_a, c->idx_b, (int)n, 0, 64, s));
+  PSPH_TRY(ensure_cub(c, std::max(b32, b64)));
+  hipLaunchKernelGGL(k_iota_u32, blocks(n), 256, 0, s, c->idx_a, 0u, n);
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->cub, b32, k2, c->key_b, c->idx_a, c->idx_b, (int)n, 0, 32, s));
+  hipLaunchKernelGGL(k_read_key01, blocks(n), 256, 0, s, n, c->idx_b, k0, k1, a);
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->cub, b64, a, b, c->idx_b, c->idx_a, (int)n, 0, 64, s));
+  hipLaunchKernelGGL(k_read_slot, blocks(n), 256, 0, s, n, c->idx_a, k0, k1, bc, c->cfg.p_table_size, c->cfg.dim, a);
+  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->cub, b64, a, b, c->idx_a, c->idx_b, (int)n, 0, 33, s));
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 extern "C" int psph_read(psph_ctx *c, psph_soa *host, size_t cap, size_t *n_out) {
   if (!c || !n_out) return fail(PSPH_EINVAL, "null argument");
-  HostParticles P;
-  PSPH_TRY(download(c, P));
-  // drop removed particles, then THashTable order
-  std::vector<uint32_t> keep;
-  keep.reserve(P.size());
-  for (size_t i = 0; i < P.size(); i++) if (P.bc[i] >= 0) keep.push_back((uint32_t)i);
-  if (keep.size() != P.size()) { P.permute(keep); }
-  auto perm = canonical_order(c->cfg, P.k0.data(), P.k1.data(), P.k2.data(), P.size());
-  P.permute(perm);
-  *n_out = P.size();
+  unsigned long long cnt[2];
+  PSPH_TRY(count_live(c, c->n, c->f.bc, cnt));
+  const size_t n = cnt[0];                    // removed particles are dropped
+  *n_out = n;
   if (!host) return 0;
-  if (P.size() > cap) return fail(PSPH_ECAPACITY, "read: %zu particles, buffer holds %zu", P.size(), cap);
-  P.to_soa(host);
+  if (n > cap) return fail(PSPH_ECAPACITY, "read: %zu particles, buffer holds %zu", n, cap);
+  if (!n) return 0;
+  PSPH_TRY(read_order(c, (uint32_t)c->n, c->f.k0, c->f.k1, c->f.k2, c->f.bc));
+  // through the spare arrays, ten (nine) fields of 8 bytes and three of 4 at a time
+  const double *src8[] = {
+#define S_(a) c->f.a,
+    PSPH_DFIELDS(S_)
+#undef S_
+  };
+  double *dst8[] = {host->x, host->y, host->z, host->vx, host->vy, host->vz, host->svx, host->svy, host->svz, host->rho,
+                    host->e, host->m, host->h, host->p, host->c, host->T, host->gam, host->cp, host->xi};
+  const void *src4[] = {c->f.k0, c->f.k1, c->f.k2, c->f.bc, c->f.phase, c->f.inv};
+  void *dst4[] = {host->key0, host->key1, host->key2, host->bc, host->phase, host->involved};
+  void *spare4[] = {c->usp, c->isp, c->idx_a};
+  for (int part = 0; part < 2; part++) {
+    const int f0 = part * 10, nf = part ? 9 : 10;
+    Moves mv{};
+    for (int k = 0; k < nf; k++) { mv.s8[k] = (const uint64_t *)src8[f0 + k]; mv.d8[k] = (uint64_t *)c->dsp[k]; }
+    for (int k = 0; k < 3; k++) { mv.s4[k] = (const uint32_t *)src4[part * 3 + k]; mv.d4[k] = (uint32_t *)spare4[k]; }
+    if (part == 0) hipLaunchKernelGGL((k_gather<10, 3>), blocks(n), 256, 0, c->stream, (uint32_t)n, c->idx_b, mv);
+    else hipLaunchKernelGGL((k_gather<9, 3>), blocks(n), 256, 0, c->stream, (uint32_t)n, c->idx_b, mv);
+    HIP_TRY(hipGetLastError());
+    for (int k = 0; k < nf; k++)
+      if (dst8[f0 + k]) HIP_TRY(hipMemcpyAsync(dst8[f0 + k], c->dsp[k], n * 8, hipMemcpyDeviceToHost, c->stream));
+    for (int k = 0; k < 3; k++)
+      if (dst4[part * 3 + k]) HIP_TRY(hipMemcpyAsync(dst4[part * 3 + k], spare4[k], n * 4, hipMemcpyDeviceToHost, c->stream));
+  }
+  HIP_TRY(hipStreamSynchronize(c->stream));
   return 0;
 }
 
@@ -2848,25 +2969,39 @@ extern "C" int psph_neighbors(psph_ctx *c) {
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, c->key_a, c->key_b, c->idx_a, c->idx_b, (int)n, 0, end_bit, s));
     PSPH_TRY(ensure_cub(c, bytes));
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->cub, bytes, c->key_a, c->key_b, c->idx_a, c->idx_b, (int)n, 0, end_bit, s));
-    // gather every field into cell order
-#define G_(a) { hipLaunchKernelGGL(k_gather<double>, blocks(n), 256, 0, s, n, c->idx_b, c->f.a, c->dsp[0]); std::swap(c->f.a, c->dsp[0]); }
-    PSPH_DFIELDS(G_)
-#undef G_
-#define G_(a) { hipLaunchKernelGGL(k_gather<uint32_t>, blocks(n), 256, 0, s, n, c->idx_b, c->f.a, c->usp); std::swap(c->f.a, c->usp); }
-    PSPH_UFIELDS(G_)
-#undef G_
-#define G_(a) { hipLaunchKernelGGL(k_gather<int32_t>, blocks(n), 256, 0, s, n, c->idx_b, c->f.a, c->isp); std::swap(c->f.a, c->isp); }
-    PSPH_IFIELDS(G_)
-#undef G_
-    hipLaunchKernelGGL(k_gather<uint32_t>, blocks(n), 256, 0, s, n, c->idx_b, c->pid, c->pid_sp);
-    std::swap(c->pid, c->pid_sp);
-    if (frozen) {
-      double **pp[3] = {&c->px, &c->py, &c->pz};
-      for (auto q : pp) {
-        hipLaunchKernelGGL(k_gather<double>, blocks(n), 256, 0, s, n, c->idx_b, *q, c->dsp[0]);
-        std::swap(*q, c->dsp[0]);
-      }
+    // gather every field into cell order; the places it goes to are the spare
+    // arrays and those that this search fills only later
+    double **f8[] = {
+#define F_(a) &c->f.a,
+      PSPH_DFIELDS(F_)
+#undef F_
+      &c->px, &c->py, &c->pz};
+    double **to8[kMove8] = {&c->h_list};
+    for (int k = 0; k < 10; k++) to8[k + 1] = &c->dsp[k];
+    const int n8 = frozen ? 22 : 19;
+    static_assert(sizeof f8 / sizeof f8[0] == 2 * kMove8, "two launches move every array");
+    Moves mv;
+    for (int k = 0; k < kMove8; k++) { mv.s8[k] = (const uint64_t *)*f8[k]; mv.d8[k] = (uint64_t *)*to8[k]; }
+    uint32_t **to4[kMove4 - 1] = {&c->usp, &c->pid_sp, &c->idx_a, &c->refb, &c->targets, &c->key_a};
+    int q4 = 0;
+    auto move4 = [&](auto *&field, auto *&to) {
+      mv.s4[q4] = (const uint32_t *)field;
+      mv.d4[q4++] = (uint32_t *)to;
+      auto *was = field;
+      field = (decltype(was))to;
+      to = (std::remove_reference_t<decltype(to)>)was;
+    };
+    move4(c->f.k0, *to4[0]); move4(c->f.k1, *to4[1]); move4(c->f.k2, *to4[2]);
+    move4(c->pid, *to4[3]); move4(c->f.bc, *to4[4]); move4(c->f.phase, *to4[5]); move4(c->f.inv, c->isp);
+    hipLaunchKernelGGL((k_gather<kMove8, kMove4>), blocks(n), 256, 0, s, n, c->idx_b, mv);
+    for (int k = 0; k < kMove8; k++) std::swap(*f8[k], *to8[k]);
+    for (int k = kMove8; k < n8; k++) {
+      mv.s8[k - kMove8] = (const uint64_t *)*f8[k];
+      mv.d8[k - kMove8] = (uint64_t *)*to8[k - kMove8];
     }
+    if (frozen) hipLaunchKernelGGL((k_gather<kMove8, 0>), blocks(n), 256, 0, s, n, c->idx_b, mv);
+    else hipLaunchKernelGGL((k_gather<19 - kMove8, 0>), blocks(n), 256, 0, s, n, c->idx_b, mv);
+    for (int k = kMove8; k < n8; k++) std::swap(*f8[k], *to8[k - kMove8]);
     std::swap(c->key_a, c->key_b);   // key_a: sorted keys
   }
   // drop removed particles (their key == ncells sorts them to the tail)
