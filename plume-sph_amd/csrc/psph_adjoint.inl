@@ -820,7 +820,7 @@ static int snap_save(psph_ctx *c, Snapshot &s) {
     for (int k = 0; k < PSPH_NIF; k++) HIP_TRY(hipMemcpyAsync(s.i[k], iv[k], n * 4, hipMemcpyDeviceToDevice, st));
     HIP_TRY(hipMemcpyAsync(s.pid, c->pid, n * 4, hipMemcpyDeviceToDevice, st));
   }
-  HIP_TRY(hipMemcpyAsync(&s.dead, c->d_u64 + 3, 8, hipMemcpyDeviceToHost, st));
+  HIP_TRY(hipMemcpyAsync(&s.dead, c->words + W_DEAD, 8, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   s.n = n;
   s.time = c->time; s.next_output = c->next_output; s.step = c->step; s.ioutput = c->ioutput;
@@ -839,7 +839,7 @@ static int snap_load(psph_ctx *c, const Snapshot &s) {
     for (int k = 0; k < PSPH_NIF; k++) HIP_TRY(hipMemcpyAsync(iv[k], s.i[k], n * 4, hipMemcpyDeviceToDevice, st));
     HIP_TRY(hipMemcpyAsync(c->pid, s.pid, n * 4, hipMemcpyDeviceToDevice, st));
   }
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, st, c->d_u64 + 3, (unsigned long long)s.dead, 1);
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, st, c->words + W_DEAD, (unsigned long long)s.dead, 1);
   HIP_TRY(hipStreamSynchronize(st));
   c->n = n;
   c->time = s.time; c->next_output = s.next_output; c->step = s.step; c->ioutput = s.ioutput;
@@ -1036,9 +1036,10 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
 static int adj_lists(psph_ctx *c, Adjoint &A, const StepRec &R, const AdjCommon &pc, GroupLists &gl, uint32_t &ngroups) {
   c->lists_valid = false;
   PSPH_TRY(group_memory(c, R.n / kChunk + (size_t)R.grid.ncells + 1));
-  hipLaunchKernelGGL(k_geom, blocks(R.n), 256, 0, c->stream, (uint32_t)R.n, pc.p.x, pc.p.y, pc.p.z, pc.h, c->gxy, c->gzh);
+  hipLaunchKernelGGL(k_geom, blocks(R.n), 256, 0, c->stream, (uint32_t)R.n, pc.p.x, pc.p.y, pc.p.z, pc.h, c->gxy, c->gzh,
+                     A.made);
   const ListOf of{R.n, R.grid.ncells, pc.h, R.hmax, A.made, true};
-  PSPH_TRY(build_lists(c, pc.p, of, 0.0, nullptr, ngroups));
+  PSPH_TRY(build_lists(c, pc.p, of, 0.0, nullptr, true, ngroups));
   gl = group_common(c).gl;
   return 0;
 }
@@ -1346,7 +1347,8 @@ static int reverse_step(psph_ctx *c, Adjoint &A, StepRec &R, ThetaGrad &th) {
   pc.p.del = k.bucket_edge;
   for (int d = 0; d < 3; d++) pc.p.ext_lo[d] = k.ext_lo[d];
   pc.p.cut = cut_test(k.cutoff);
-  pc.p.err = c->d_err;
+  pc.p.err = (int *)(c->words + W_ERR);
+  pc.p.halt = pc.p.err;
   pc.h = R.d[RF_H];
   pc.cutoff2 = k.cutoff2;
   GroupLists vl;

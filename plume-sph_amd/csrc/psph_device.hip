@@ -63,6 +63,28 @@ __device__ inline void raise_err(int *err, int code, uint32_t idx) {
   if (atomicCAS(err, 0, code) == 0) err[1] = (int)idx;
 }
 
+// The words of a context that kernels leave for the host, read in one copy: a
+// step reads them where it needs them and not after every stage.
+enum Word {
+  W_DT, W_HMAX,               // bits of the least h / c and the largest h
+  W_PAIRS, W_DEAD, W_REAL,    // pairs of the RHS; particles removed; real particles left
+  W_BCOND,                    // groups of wall ghosts to refresh
+  W_CURSOR, W_CHUNKS,         // visits handed out, chunks of targets
+  W_LIVE, W_LIVE_REAL,
+  W_ERR,                      // error words, [0] code and [1] particle: of the stages without one of
+  W_ERR_RHS, W_ERR_DENS, W_ERR_VSM,   // their own, and of the passes whose errors a step reads at its end
+  W_VMAX,                     // bits of the largest speed
+  W_OVER, W_ITERS,            // lists that found no room since the last check; iterations of the adaptive h done
+  W_COUNT
+};
+// an earlier stage of this step failed (n error words from err): the stages
+// after it do nothing, as if the step had ended there
+__device__ inline bool halted(const int *err, int n) {
+  int bad = 0;
+  for (int q = 0; q < n; q++) bad |= err[2 * q];
+  return bad != 0;
+}
+
 __device__ inline bool need_neigh(int bc) { return bc == 100 || bc == 99; }
 __device__ inline bool is_real(int bc) { return bc == 100 || bc == 99; }
 __device__ inline bool contr_dens(int pg, int bc) {
@@ -134,19 +156,31 @@ __device__ inline double block_ext(double v) {
   return v;
 }
 
-// dt candidate min h/c over need_neigh particles (timestep.cc:94-135);
-// grid-stride, 256 threads per block.
+// dt candidate min h/c over need_neigh particles (timestep.cc:94-135) and max h
+// over the live ones; grid-stride, 256 threads per block.
 __global__ __launch_bounds__(256) void k_dt_min(uint32_t n, const int32_t *bc, const double *h, const double *c,
-                                                unsigned long long *out, int *err) {
-  double v = 1.0e300;
+                                                unsigned long long *words) {
+  double v = 1.0e300, hm = 0;
   for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    if (!need_neigh(bc[i])) continue;
+    const int b = bc[i];
+    if (b < 0) continue;
+    const double hi = h[i];
+    hm = fmax(hm, hi);
+    if (!need_neigh(b)) continue;
     const double ci = c[i];
-    if (!(ci > 0)) raise_err(err, PSPH_EINVARIANT, i);
-    else v = fmin(v, h[i] / ci);
+    if (!(ci > 0)) raise_err((int *)(words + W_ERR), PSPH_EINVARIANT, i);
+    else v = fmin(v, hi / ci);
   }
   v = block_ext<false>(v);
-  if (threadIdx.x == 0 && v < 1.0e300) atomicMin(out, (unsigned long long)__double_as_longlong(v));
+  hm = block_ext<true>(hm);
+  if (threadIdx.x != 0) return;
+  if (v < 1.0e300) atomicMin(words + W_DT, (unsigned long long)__double_as_longlong(v));
+  if (hm > 0) atomicMax(words + W_HMAX, (unsigned long long)__double_as_longlong(hm));
+}
+__global__ void k_step_words(unsigned long long *w) {
+  if (threadIdx.x) return;
+  w[W_DT] = 0x7FF0000000000000ull;                 // +inf
+  w[W_HMAX] = w[W_PAIRS] = w[W_REAL] = w[W_VMAX] = 0;
 }
 
 // max h over live particles (the cell edge must cover every pair support)
@@ -374,6 +408,8 @@ struct PairCommon {
   double ext_lo[3];           // origin of the reference buckets
   CutTest cut;
   int *err;
+  const int *halt;            // error words of the stages before this pass
+  int nhalt;
 };
 
 // The region a chunk's neighbour lists can reach (neighs.cc:37-211): per
@@ -499,14 +535,15 @@ constexpr int kStreams = kWave / kGroup;       // particles evaluated at a time
 constexpr int kGroupsPerChunk = kChunk / kGroup;
 constexpr int kMaxSplit = 8;                   // waves that share a group
 
-// Positions (x, y) and (z, h / 2) of every particle.
+// Positions (x, y) and (z, h / 2) of every particle; the lists made next start at visit 0.
 struct Geom {
   const double2 *xy, *zh;
 };
 
 __global__ void k_geom(uint32_t n, const double *x, const double *y, const double *z, const double *h, double2 *xy,
-                       double2 *zh) {
+                       double2 *zh, unsigned long long *cursor) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *cursor = 0;
   if (i >= n) return;
   xy[i] = make_double2(x[i], y[i]);
   zh[i] = make_double2(z[i], 0.5 * h[i]);
@@ -693,6 +730,9 @@ struct GroupCommon {
   // for the three passes) and the targets that have converged
   double c_smooth;
   const uint32_t *done;
+  // optional: set where the visits found no room, by lists whose cursor the host
+  // does not read before the pass; the pass then does nothing, else counts itself
+  unsigned long long *over;
 };
 
 // The group of this workgroup, its target for this lane (lane % kGroup; past
@@ -898,7 +938,10 @@ __global__ __launch_bounds__(kWave) void k_group_lists(PairCommon pc, GroupCommo
       for (uint32_t q = 0; q < kGroupsPerChunk; q++) room += num[q];
       if (lane == 0) first = atomicAdd(gc.gl.cursor, (unsigned long long)room);
       uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)first);
-      if (__builtin_amdgcn_readfirstlane((uint32_t)(first >> 32)) || (unsigned long long)at + room > gc.gl.cap) return;
+      if (__builtin_amdgcn_readfirstlane((uint32_t)(first >> 32)) || (unsigned long long)at + room > gc.gl.cap) {
+        if (gc.over && lane == 0) atomicOr(gc.over, 1ull);
+        return;
+      }
       for (uint32_t q = 0; q < kGroupsPerChunk; q++) {
         off[q] = at;
         at += num[q];
@@ -980,7 +1023,11 @@ __global__ __launch_bounds__(kMaxSplit * kWave, P::kWaves) void k_group_pass(Pai
   extern __shared__ char lds[];                    // a GroupLds<P> per wave
   uint32_t gid, i;
   const uint32_t nt = my_group(pc, gid, i);
-  if (!nt) return;
+  if (!nt || halted(pc.halt, pc.nhalt)) return;
+  if (gc.over) {
+    if (gc.over[0]) return;
+    if (gid == 0 && threadIdx.x == 0) atomicAdd(gc.over + (W_ITERS - W_OVER), 1ull);
+  }
   const int lane = threadIdx.x % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), split = blockDim.x / kWave;
   GroupLds<P> &own_lds = ((GroupLds<P> *)lds)[wave];
@@ -2182,25 +2229,6 @@ __global__ __launch_bounds__(kBcondWaves * kWave, 2) void k_bcond(uint32_t n, Bc
   }
 }
 
-// largest per-axis speed of the particles update_pos moves (reals with the
-// filtered velocity under LANS, erupt ghosts with v)
-__global__ __launch_bounds__(256) void k_speed_max(uint32_t n, const int32_t *bc, int lans, const double *vx,
-                                                   const double *vy, const double *vz, const double *svx,
-                                                   const double *svy, const double *svz, unsigned long long *out) {
-  double v = 0;
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const int b = bc[i];
-    if (b == 100 || b == 99) {
-      const bool s = lans != 0;
-      v = fmax(v, fmax(fabs(s ? svx[i] : vx[i]), fmax(fabs(s ? svy[i] : vy[i]), fabs(s ? svz[i] : vz[i]))));
-    } else if (b == 0) {
-      v = fmax(v, fmax(fabs(vx[i]), fmax(fabs(vy[i]), fabs(vz[i]))));
-    }
-  }
-  v = block_ext<true>(v);
-  if (threadIdx.x == 0 && v > 0) atomicMax(out, (unsigned long long)__double_as_longlong(v));
-}
-
 // ---------------------------------------------------------------------------
 // Position update + escape (update_pos.cc:34-168, bucket.cc:435-452)
 // ---------------------------------------------------------------------------
@@ -2214,61 +2242,63 @@ struct PosTape {
   int32_t *tr_step, *esc_step;
 };
 
-__global__ void k_update_pos(uint32_t n, int dim, int lans, int erupting, double dt, double *x,
-                             double *y, double *z, const double *vx, const double *vy,
-                             const double *vz, const double *svx, const double *svy,
-                             const double *svz, int32_t *bc, double *h, int32_t *inv,
-                             double ground, double h_new, double lo0, double lo1, double lo2,
-                             double hi0, double hi1, double hi2, unsigned long long *dead, PosTape tp) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int b = bc[i];
-  if (b == 100 || b == 99) {
-    if (dim == 3) {
-      double ux = lans ? svx[i] : vx[i], uy = lans ? svy[i] : vy[i], uz = lans ? svz[i] : vz[i];
-      x[i] = x[i] + dt * ux; y[i] = y[i] + dt * uy; z[i] = z[i] + dt * uz;
-    } else {
-      x[i] = x[i] + dt * (lans ? svx[i] : vx[i]);
-    }
-  } else if (b == 0 && erupting) {
-    x[i] = x[i] + dt * vx[i];
-    if (dim == 3) {
-      y[i] = y[i] + dt * vy[i];
-      z[i] = z[i] + dt * vz[i];
-      const bool turn = tp.mode == 2 ? tp.tr_step[tp.pid[i]] == tp.k : z[i] >= ground;
-      if (turn) {
-        b = 100; bc[i] = 100; h[i] = h_new; inv[i] = 2;
-        if (tp.mode == 1) tp.tr_step[tp.pid[i]] = tp.k;
+// Then, of what is left: the real particles (bc 100/99), and the largest per-axis
+// speed of the particles that move (reals with the filtered velocity under LANS,
+// erupt ghosts with v).  Grid-stride, an atomic a block each.
+__global__ __launch_bounds__(256) void k_update_pos(
+    uint32_t n, int dim, int lans, int erupting, double dt, double *x, double *y, double *z, const double *vx,
+    const double *vy, const double *vz, const double *svx, const double *svy, const double *svz, int32_t *bc, double *h,
+    int32_t *inv, double ground, double h_new, double lo0, double lo1, double lo2, double hi0, double hi1, double hi2,
+    unsigned long long *words, PosTape tp) {
+  __shared__ unsigned int part[256 / kWave];
+  if (halted((const int *)(words + W_ERR), 4)) return;
+  unsigned int reals = 0;
+  double vmax = 0;
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    int b = bc[i];
+    const bool was_real = is_real(b);
+    if (!was_real && b != 0) continue;
+    const double v[3] = {vx[i], vy[i], vz[i]};
+    double u[3] = {v[0], v[1], v[2]};              // of a real particle
+    if (lans && (was_real || erupting)) { u[0] = svx[i]; u[1] = svy[i]; u[2] = svz[i]; }
+    if (was_real) {
+      x[i] = x[i] + dt * u[0];
+      if (dim == 3) { y[i] = y[i] + dt * u[1]; z[i] = z[i] + dt * u[2]; }
+    } else if (erupting) {
+      x[i] = x[i] + dt * v[0];
+      if (dim == 3) {
+        y[i] = y[i] + dt * v[1];
+        z[i] = z[i] + dt * v[2];
+        const bool turn = tp.mode == 2 ? tp.tr_step[tp.pid[i]] == tp.k : z[i] >= ground;
+        if (turn) {
+          b = 100; bc[i] = 100; h[i] = h_new; inv[i] = 2;
+          if (tp.mode == 1) tp.tr_step[tp.pid[i]] = tp.k;
+        }
       }
     }
-  }
-  if (dim == 3 && (b == 100 || b == 99)) {
-    const double TINY = 1.0E-08;
-    bool esc = (x[i] - lo0) < -TINY || (y[i] - lo1) < -TINY || (z[i] - lo2) < -TINY ||
-               (x[i] - hi0) > TINY || (y[i] - hi1) > TINY || (z[i] - hi2) > TINY;
-    if (tp.mode == 2) esc = tp.esc_step[tp.pid[i]] == tp.k;
-    if (esc) {
-      bc[i] = -1; atomicAdd(dead, 1ull);
-      if (tp.mode == 1) tp.esc_step[tp.pid[i]] = tp.k;
+    if (dim == 3 && is_real(b)) {
+      const double TINY = 1.0E-08;
+      bool esc = (x[i] - lo0) < -TINY || (y[i] - lo1) < -TINY || (z[i] - lo2) < -TINY ||
+                 (x[i] - hi0) > TINY || (y[i] - hi1) > TINY || (z[i] - hi2) > TINY;
+      if (tp.mode == 2) esc = tp.esc_step[tp.pid[i]] == tp.k;
+      if (esc) {
+        b = -1; bc[i] = -1; atomicAdd(words + W_DEAD, 1ull);
+        if (tp.mode == 1) tp.esc_step[tp.pid[i]] = tp.k;
+      }
     }
+    reals += is_real(b) ? 1u : 0u;
+    if (is_real(b)) vmax = fmax(vmax, fmax(fabs(u[0]), fmax(fabs(u[1]), fabs(u[2]))));
+    else if (b == 0) vmax = fmax(vmax, fmax(fabs(v[0]), fmax(fabs(v[1]), fabs(v[2]))));
   }
-}
-
-// real particles (bc 100/99): grid-stride count, one atomic per block
-__global__ __launch_bounds__(256) void k_count_real(uint32_t n, const int32_t *bc, unsigned long long *out) {
-  __shared__ unsigned int part[256 / kWave];
-  unsigned int cnt = 0;
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    const int b = bc[i];
-    cnt += (b == 100 || b == 99) ? 1u : 0u;
-  }
-  for (int o = kWave / 2; o > 0; o >>= 1) cnt += (unsigned int)__shfl_xor((int)cnt, o);
-  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = cnt;
+  vmax = block_ext<true>(vmax);
+  for (int o = kWave / 2; o > 0; o >>= 1) reals += (unsigned int)__shfl_xor((int)reals, o);
+  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = reals;
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long sum = 0;
     for (int w = 0; w < 256 / kWave; w++) sum += part[w];
-    if (sum) atomicAdd(out, sum);
+    if (sum) atomicAdd(words + W_REAL, sum);
+    if (vmax > 0) atomicMax(words + W_VMAX, (unsigned long long)__double_as_longlong(vmax));
   }
 }
 
@@ -2386,8 +2416,10 @@ __global__ void k_conservation(uint32_t n, const int32_t *bc, const double *m, c
 }
 
 inline unsigned blocks(size_t n, unsigned b = 256) { return (unsigned)((n + b - 1) / b); }
-// grid of a grid-stride reduction: enough blocks to fill the chip, no more
-inline unsigned red_blocks(size_t n) { return std::min(blocks(n), 2048u); }
+// grid of a grid-stride reduction: enough blocks to fill the chip, no more, and
+// 8 elements a thread where they are few (the blocks' atomics on one word take
+// their turns: the least h / c of 227k particles 24 us with one element, 12 so)
+inline unsigned red_blocks(size_t n) { return std::min(blocks(n, 8 * 256), 2048u); }
 
 }  // namespace
 
@@ -2472,8 +2504,6 @@ struct StepRec {
 };
 struct Adjoint;
 
-constexpr int kWords = 16;       // of psph_ctx::d_u64
-
 struct psph_ctx {
   psph_config cfg{};
   hipStream_t stream = nullptr;
@@ -2491,8 +2521,10 @@ struct psph_ctx {
   size_t cs_cap = 0, tile_cap = 0, chunk_cap = 0;
   void *cub = nullptr;
   size_t cub_bytes = 0;
-  unsigned long long *d_u64 = nullptr;   // [0] dt bits [1] hmax bits [2] pairs [3] dead [8] live [9] real
-  int *d_err = nullptr;
+  unsigned long long *words = nullptr;   // on the device (Word)
+  unsigned long long *seen = nullptr;    // their last copy, in pinned memory; then 2 words of lists' cursors
+  char *up_h = nullptr, *up_d = nullptr; // particles on their way to the device (upload)
+  bool up_busy = false;
   double *d_part = nullptr;
   // grid of the last neighbour search
   bool grid_valid = false;
@@ -2573,17 +2605,34 @@ static int dmalloc(void **p, size_t bytes) {
   return 0;
 }
 
-static int check_err(psph_ctx *c, const char *stage) {
-  int he[2];
-  HIP_TRY(hipMemcpyAsync(he, c->d_err, sizeof he, hipMemcpyDeviceToHost, c->stream));
+// c->seen = the words, after everything queued so far
+static int read_words(psph_ctx *c) {
+  HIP_TRY(hipMemcpyAsync(c->seen, c->words, W_COUNT * 8, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
-  if (he[0]) {
-    int code = he[0];
-    hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, c->d_err, 0, 2);
-    return fail(code, "%s: invariant violated at device particle %d (density<=0, mass fraction>1, "
-                      "wnorm<=0 or sound speed<=0)", stage, he[1]);
+  c->up_busy = false;
+  return 0;
+}
+static double seen_double(const psph_ctx *c, Word w) {
+  double v;
+  std::memcpy(&v, &c->seen[w], 8);
+  return v;
+}
+// the first error word that is set in c->seen; stage: what W_ERR stands for
+static int seen_err(psph_ctx *c, const char *stage) {
+  const char *names[] = {stage, "rhs", "density", "vsmooth"};
+  for (int q = 0; q < 4; q++) {
+    int he[2];
+    std::memcpy(he, &c->seen[W_ERR + q], 8);
+    if (!he[0]) continue;
+    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_ERR, 0ull, 4);
+    return fail(he[0], "%s: invariant violated at device particle %d (density<=0, mass fraction>1, "
+                       "wnorm<=0 or sound speed<=0)", names[q], he[1]);
   }
   return 0;
+}
+static int check_err(psph_ctx *c, const char *stage) {
+  PSPH_TRY(read_words(c));
+  return seen_err(c, stage);
 }
 
 static int ensure_cub(psph_ctx *c, size_t bytes) {
@@ -2636,13 +2685,16 @@ extern "C" int psph_create(const psph_config *cfg, size_t capacity, psph_ctx **o
     if (!rc) rc = dmalloc((void **)pp, capacity * 4);
   if (!rc) rc = dmalloc((void **)&c->flags, (capacity + 1) * 4);
   if (!rc) rc = dmalloc((void **)&c->tpos, (capacity + 1) * 4);
-  if (!rc) rc = dmalloc((void **)&c->d_u64, kWords * 8);
-  if (!rc) { c->gcursor = c->d_u64 + 6; c->nchunks = (uint32_t *)(c->d_u64 + 7); }   // read in one copy
-  if (!rc) rc = dmalloc((void **)&c->d_err, 2 * sizeof(int));
+  if (!rc) rc = dmalloc((void **)&c->words, W_COUNT * 8);
+  if (!rc) { c->gcursor = c->words + W_CURSOR; c->nchunks = (uint32_t *)(c->words + W_CHUNKS); }
+  if (!rc && hipHostMalloc((void **)&c->seen, (W_COUNT + 2) * 8, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    c->seen = nullptr;
+    rc = fail(PSPH_ENOMEM, "hipHostMalloc");
+  }
   if (!rc) rc = dmalloc((void **)&c->d_part, kRedBlocks * 8 * 8);
   if (rc) { psph_destroy(c); return rc; }
-  hipLaunchKernelGGL(k_fill_i32, 1, 64, 0, c->stream, c->d_err, 0, 2);
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64, 0ull, kWords);
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words, 0ull, W_COUNT);
   c->next_output = cfg->t_output;
   *out = c;
   return 0;
@@ -2664,11 +2716,13 @@ extern "C" int psph_destroy(psph_ctx *c) {
   for (auto p : c->dsp) if (p) hipFree(p);
   void *ptrs[] = {c->usp, c->isp, c->h_list, c->pid, c->pid_sp, c->refb, c->key_a, c->key_b, c->idx_a, c->idx_b,
                   c->flags, c->tpos, c->targets, c->cfirst, c->ccount, c->cs, c->tcnt, c->toff,
-                  c->cchunks, c->coff, c->tbox, c->cub, c->d_u64, c->d_err, c->d_part,
+                  c->cchunks, c->coff, c->tbox, c->cub, c->words, c->up_d, c->d_part,
                   c->gvisit, c->goff, c->gnum, c->gfast, c->gxy, c->gzh, c->px, c->py, c->pz,
                   c->d_occ, c->d_conv, c->d_sides};
   for (auto p : ptrs) if (p) hipFree(p);
   for (auto p : c->pk) if (p) hipFree(p);
+  if (c->seen) hipHostFree(c->seen);
+  if (c->up_h) hipHostFree(c->up_h);
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
   if (c->stream) hipStreamDestroy(c->stream);
@@ -2676,9 +2730,53 @@ extern "C" int psph_destroy(psph_ctx *c) {
   return 0;
 }
 
+// Up to kUpload particles go through pinned memory in one copy and a kernel that
+// takes the fields apart, and nobody waits: the 25 copies of an inlet's few
+// particles, each waited for, took NNN us of a step.
+constexpr size_t kUpload = 4096;
+constexpr size_t kUploadBytes = 19 * 8 + 6 * 4;      // of a particle
+__global__ void k_append(uint32_t n, uint32_t at, const char *from, DevFields f) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double *d = (const double *)from + i;
+  const uint32_t *u = (const uint32_t *)(from + (size_t)n * 19 * 8) + i;
+#define A_(a) f.a[at + i] = *d; d += n;
+  PSPH_DFIELDS(A_)
+#undef A_
+#define A_(a) f.a[at + i] = *u; u += n;
+  PSPH_UFIELDS(A_)
+#undef A_
+#define A_(a) f.a[at + i] = (int32_t)*u; u += n;
+  PSPH_IFIELDS(A_)
+#undef A_
+}
+
+static int upload_few(psph_ctx *c, const HostParticles &P, size_t at) {
+  const size_t n = P.size();
+  if (!c->up_h) {
+    if (!c->up_d) PSPH_TRY(dmalloc((void **)&c->up_d, kUpload * kUploadBytes));
+    if (hipHostMalloc((void **)&c->up_h, kUpload * kUploadBytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->up_h = nullptr;
+      return fail(PSPH_ENOMEM, "hipHostMalloc");
+    }
+  }
+  if (c->up_busy) HIP_TRY(hipStreamSynchronize(c->stream));   // the copy before has left the pinned memory
+  char *to = c->up_h;
+#define A_(a) std::memcpy(to, P.a.data(), n * sizeof(P.a[0])); to += n * sizeof(P.a[0]);
+  PSPH_DFIELDS(A_) PSPH_UFIELDS(A_) PSPH_IFIELDS(A_)
+#undef A_
+  HIP_TRY(hipMemcpyAsync(c->up_d, c->up_h, n * kUploadBytes, hipMemcpyHostToDevice, c->stream));
+  c->up_busy = true;
+  hipLaunchKernelGGL(k_append, blocks(n), 256, 0, c->stream, (uint32_t)n, (uint32_t)at, c->up_d, c->f);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
 static int upload(psph_ctx *c, const HostParticles &P, size_t at) {
   size_t n = P.size();
   if (!n) return 0;
+  if (n <= kUpload) return upload_few(c, P, at);
 #define U_(a) HIP_TRY(hipMemcpyAsync(c->f.a + at, P.a.data(), n * sizeof(P.a[0]), hipMemcpyHostToDevice, c->stream));
   PSPH_DFIELDS(U_) PSPH_UFIELDS(U_)
   U_(bc) U_(phase)
@@ -2698,7 +2796,7 @@ extern "C" int psph_load(psph_ctx *c, const psph_soa *host, size_t n, double t0,
   c->n = n;
   if (n) hipLaunchKernelGGL(k_iota_u32, blocks(n), 256, 0, c->stream, c->pid, 0u, (uint32_t)n);
   c->next_pid = (uint32_t)n;
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 3, 0ull, 1);
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_DEAD, 0ull, 1);
   c->time = t0;
   c->step = step0;
   c->ioutput = 0;
@@ -2710,12 +2808,13 @@ extern "C" int psph_load(psph_ctx *c, const psph_soa *host, size_t n, double t0,
 
 // live and real particles of bc[0..n)
 static int count_live(psph_ctx *c, size_t n, const int32_t *bc, unsigned long long cnt[2]) {
-  unsigned long long *out = c->d_u64 + 8;
+  unsigned long long *out = c->words + W_LIVE;
   hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, out, 0ull, 2);
   if (n) hipLaunchKernelGGL(k_count_live, red_blocks(n), 256, 0, c->stream, (uint32_t)n, bc, out);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(cnt, out, 16, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
+  PSPH_TRY(read_words(c));
+  cnt[0] = c->seen[W_LIVE];
+  cnt[1] = c->seen[W_LIVE_REAL];
   return 0;
 }
 
@@ -2832,16 +2931,12 @@ extern "C" int psph_read(psph_ctx *c, psph_soa *host, size_t cap, size_t *n_out)
 // ---------------------------------------------------------------------------
 extern "C" int psph_timestep(psph_ctx *c, double *dt_out) {
   if (!c || !dt_out) return fail(PSPH_EINVAL, "null argument");
-  unsigned long long init = (unsigned long long)0x7FF0000000000000ull;   // +inf bits
   StageTimer tm(c, 0);
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64, init, 1);
-  if (c->n) hipLaunchKernelGGL(k_dt_min, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, c->f.h, c->f.c, c->d_u64, c->d_err);
+  hipLaunchKernelGGL(k_step_words, 1, 64, 0, c->stream, c->words);
+  if (c->n) hipLaunchKernelGGL(k_dt_min, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, c->f.h, c->f.c, c->words);
   tm.stop();
-  unsigned long long bits;
-  HIP_TRY(hipMemcpyAsync(&bits, c->d_u64, 8, hipMemcpyDeviceToHost, c->stream));
   PSPH_TRY(check_err(c, "timestep"));
-  double mn;
-  std::memcpy(&mn, &bits, 8);
+  const double mn = seen_double(c, W_DT);
   double dt = 1.0E+10;                    // timestep.cc:99
   if (mn < dt) dt = mn;
   *dt_out = c->cfg.cfl * dt;
@@ -2857,16 +2952,16 @@ extern "C" int psph_advance_time(psph_ctx *c, double *dt) {   // TimeProps::incr
   return 0;
 }
 
-static int build_grid(psph_ctx *c) {
+// max h over the live particles (and the other words) in c->seen
+static int reduce_hmax(psph_ctx *c) {
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_HMAX, 0ull, 1);
+  if (c->n) hipLaunchKernelGGL(k_h_max, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, c->f.h, c->words + W_HMAX);
+  return read_words(c);
+}
+
+// hmax: the largest h of the live particles
+static int build_grid(psph_ctx *c, double hmax) {
   const psph_config &k = c->cfg;
-  // h_max over live particles
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 1, 0ull, 1);
-  if (c->n) hipLaunchKernelGGL(k_h_max, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, c->f.h, c->d_u64 + 1);
-  unsigned long long bits;
-  HIP_TRY(hipMemcpyAsync(&bits, c->d_u64 + 1, 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  double hmax;
-  std::memcpy(&hmax, &bits, 8);
   if (!(hmax > 0) || !std::isfinite(hmax)) hmax = k.h_air;
   c->h_max = hmax;
   c->reach_main = k.cutoff * hmax * (1 + 1e-9);
@@ -2941,9 +3036,11 @@ static void launch_order(psph_ctx *c, uint32_t n, uint32_t ncells, const uint32_
   hipLaunchKernelGGL(k_order_targets, ncells * per_cell, kWave, 0, c->stream, cs, tpos, per_cell, x, y, z, targets);
 }
 
-extern "C" int psph_neighbors(psph_ctx *c) {
-  if (!c) return fail(PSPH_EINVAL, "null ctx");
-  PSPH_TRY(build_grid(c));
+// seen: c->seen holds the largest h and the removed particles of this state
+static int neighbors(psph_ctx *c, bool seen) {
+  if (!seen) PSPH_TRY(reduce_hmax(c));
+  const unsigned long long dead = c->seen[W_DEAD];
+  PSPH_TRY(build_grid(c, seen_double(c, W_HMAX)));
   StageTimer tm(c, 1);
   const GridDesc &g = c->grid;
   uint32_t n = (uint32_t)c->n;
@@ -2958,7 +3055,7 @@ extern "C" int psph_neighbors(psph_ctx *c) {
       PSPH_TRY(dmalloc((void **)&c->pz, c->cap * 8));
     }
     if (n) hipLaunchKernelGGL(k_pos_from_rec, blocks(n), 256, 0, s, n, c->pid, c->f.bc, tp.xrec[tp.k], tp.xrec_n[tp.k],
-                              c->f.x, c->f.y, c->f.z, c->px, c->py, c->pz, c->d_err);
+                              c->f.x, c->f.y, c->f.z, c->px, c->py, c->pz, (int *)(c->words + W_ERR));
   }
   if (n) {
     hipLaunchKernelGGL(k_cellkey, blocks(n), 256, 0, s, n, frozen ? c->px : c->f.x, frozen ? c->py : c->f.y,
@@ -3005,14 +3102,11 @@ extern "C" int psph_neighbors(psph_ctx *c) {
     std::swap(c->key_a, c->key_b);   // key_a: sorted keys
   }
   // drop removed particles (their key == ncells sorts them to the tail)
-  unsigned long long dead = 0;
-  HIP_TRY(hipMemcpyAsync(&dead, c->d_u64 + 3, 8, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   if (dead) {
     if (dead > n) return fail(PSPH_EINVARIANT, "removed-particle count %llu exceeds %u", dead, n);
     n -= (uint32_t)dead;
     c->n = n;
-    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, c->d_u64 + 3, 0ull, 1);
+    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, c->words + W_DEAD, 0ull, 1);
   }
   hipLaunchKernelGGL(k_cell_start, blocks(n + 1), 256, 0, s, n, c->key_a, 3 * g.fbits, g.ncells, c->cs);
   // tiles of each cell and their boxes
@@ -3058,6 +3152,11 @@ extern "C" int psph_neighbors(psph_ctx *c) {
   return 0;
 }
 
+extern "C" int psph_neighbors(psph_ctx *c) {
+  if (!c) return fail(PSPH_EINVAL, "null ctx");
+  return neighbors(c, false);
+}
+
 // half an ulp of the cut-off; the test above assumes its mantissa is even
 static CutTest cut_test(double cut) {
   int e;
@@ -3093,7 +3192,9 @@ static PairCommon make_common(psph_ctx *c, double reach) {
   // h_max bounds h at list time (it only grows with an adaptation)
   pc.list_adj = list_adj(c->cfg, c->h_max);
   pc.cut = cut_test(c->cfg.cutoff);
-  pc.err = c->d_err;
+  pc.err = (int *)(c->words + W_ERR);
+  pc.halt = pc.err;
+  pc.nhalt = 0;
   return pc;
 }
 
@@ -3150,33 +3251,44 @@ static int group_memory(psph_ctx *c, size_t chunks) {
 }
 
 static void launch_geom(psph_ctx *c, const PairCommon &pc) {
-  hipLaunchKernelGGL(k_geom, blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, pc.x, pc.y, pc.z, c->f.h, c->gxy, c->gzh);
+  hipLaunchKernelGGL(k_geom, blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, pc.x, pc.y, pc.z, c->f.h, c->gxy, c->gzh,
+                     c->gcursor);
 }
 
-// the groups' visits for the boxes that c_smooth and done say (GroupCommon)
-static int build_lists(psph_ctx *c, const PairCommon &pc, const ListOf &of, double c_smooth, const uint32_t *done,
-                       uint32_t &ngroups) {
+// the groups' visits for the boxes that c_smooth and done say (GroupCommon): the
+// kernel alone, its cursor at 0
+static int launch_lists(psph_ctx *c, const PairCommon &pc, const ListOf &of, double c_smooth, const uint32_t *done,
+                        unsigned long long *over) {
   // a group per wave up to a quarter of a million particles: at 77k 0.15 ms against
   // 0.20 with half a chunk; a chunk per wave beyond
   const uint32_t nsplit = of.n < (1u << 18) ? kGroupsPerChunk : 1;
   const unsigned G = chunk_grid(of.n, of.ncells, kChunk) * nsplit;
-  for (;;) {
-    GroupCommon gc = group_common(c);
-    gc.c_smooth = c_smooth;
-    gc.done = done;
-    gc.gl.cursor = of.cursor;
-    gc.h_max = of.h_max;
-    gc.both = of.both ? 1 : 0;
-    if (of.both) gc.cutj = 2 * gc.cutx;
-    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, of.cursor, 0ull, 1);
-    if (c->cfg.dim == 3)
-      hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
-    else
-      hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
-    HIP_TRY(hipGetLastError());
-    unsigned long long got[2] = {0, 0};         // visits; chunks
+  GroupCommon gc = group_common(c);
+  gc.c_smooth = c_smooth;
+  gc.done = done;
+  gc.gl.cursor = of.cursor;
+  gc.h_max = of.h_max;
+  gc.both = of.both ? 1 : 0;
+  if (of.both) gc.cutj = 2 * gc.cutx;
+  gc.over = over;
+  if (c->cfg.dim == 3)
+    hipLaunchKernelGGL(k_group_lists<3>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
+  else
+    hipLaunchKernelGGL(k_group_lists<1>, G, kWave, 0, c->stream, pc, gc, of.h, c->cfg.cutoff2, nsplit);
+  HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+// the visits, in memory that holds them; cleared: the cursor is at 0
+static int build_lists(psph_ctx *c, const PairCommon &pc, const ListOf &of, double c_smooth, const uint32_t *done,
+                       bool cleared, uint32_t &ngroups) {
+  for (;; cleared = false) {
+    if (!cleared) hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, of.cursor, 0ull, 1);
+    PSPH_TRY(launch_lists(c, pc, of, c_smooth, done, nullptr));
+    unsigned long long *got = c->seen + W_COUNT;             // visits; chunks
     HIP_TRY(hipMemcpyAsync(got, of.cursor, 16, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    c->up_busy = false;
     const unsigned long long total = got[0];
     ngroups = (uint32_t)got[1] * kGroupsPerChunk;
     if (total <= c->gvisit_cap) return 0;
@@ -3204,7 +3316,7 @@ static int ensure_lists(psph_ctx *c) {
   PSPH_TRY(group_memory(c, c->chunk_cap));
   const PairCommon pc = make_common(c, c->reach_main);
   launch_geom(c, pc);
-  PSPH_TRY(build_lists(c, pc, own_lists(c), 0.0, nullptr, c->ngroups));
+  PSPH_TRY(build_lists(c, pc, own_lists(c), 0.0, nullptr, true, c->ngroups));
   c->lists_valid = true;
   return 0;
 }
@@ -3261,9 +3373,13 @@ static void launch_group_pass(psph_ctx *c, const PairCommon &pc, const GroupComm
 }
 // the RHS, density and filter passes; PM, PX, PP, PD: the pass in the FP32-pair,
 // FP32-exp, FP32-pure and FP64 forms
+// err: the pass's error word; the passes after the RHS do nothing if an earlier
+// word is set
 template <class PM, class PX, class PP, class PD>
-static int launch_groups(psph_ctx *c, const typename PD::Args &a, const FieldCopy &fc) {
-  const PairCommon pc = make_common(c, c->reach_main);
+static int launch_groups(psph_ctx *c, Word err, const typename PD::Args &a, const FieldCopy &fc) {
+  PairCommon pc = make_common(c, c->reach_main);
+  pc.err = (int *)(c->words + err);
+  pc.nhalt = err == W_ERR_RHS ? 0 : err - W_ERR;
   const GroupCommon gc = group_common(c);
   const int form = c->cfg.precision;
   if (c->cfg.dim == 3) {
@@ -3282,16 +3398,6 @@ static int launch_groups(psph_ctx *c, const typename PD::Args &a, const FieldCop
 
 static EosConst eos_const(const psph_config &k) {
   return EosConst{k.ng0, k.cvs, k.cvg, k.cva, k.rg, k.ra, k.lans};
-}
-
-static int reduce_hmax(psph_ctx *c, double *out) {
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 1, 0ull, 1);
-  if (c->n) hipLaunchKernelGGL(k_h_max, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, c->f.h, c->d_u64 + 1);
-  unsigned long long bits;
-  HIP_TRY(hipMemcpyAsync(&bits, c->d_u64 + 1, 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  std::memcpy(out, &bits, 8);
-  return 0;
 }
 
 // the later passes of a step use the new h: widen the reach
@@ -3321,10 +3427,10 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
     const bool fx = k.precision == PSPH_FP32_EXP;
     if (fx) launch_pack<AdaptPass<double, true>>(c, a, FieldCopy{});
     else launch_pack<AdaptPass<double>>(c, a, FieldCopy{});
-    for (int it = 0; it < k.num_loop; it++) {
-      StageTimer tm(c, 2);
-      PSPH_TRY(build_lists(c, pc, own_lists(c), k.c_smooth, c->usp, c->ngroups));
-      const GroupCommon gc = group_common(c);
+    const ListOf of = own_lists(c);
+    auto pass = [&](unsigned long long *over) {
+      GroupCommon gc = group_common(c);
+      gc.over = over;
       if (k.dim == 3) {
         if (fx) launch_group_kernel<3, AdaptPass<double, true>>(c, pc, gc, a, false);
         else launch_group_kernel<3, AdaptPass<double>>(c, pc, gc, a, false);
@@ -3332,11 +3438,35 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
         if (fx) launch_group_kernel<1, AdaptPass<double, true>>(c, pc, gc, a, false);
         else launch_group_kernel<1, AdaptPass<double>>(c, pc, gc, a, false);
       }
+    };
+    // The first iteration's lists say how many groups there are and find their
+    // memory.  The others are queued behind it and nobody waits: their boxes are
+    // seldom larger, and where the memory does not hold them after all, that
+    // iteration and those after it do nothing (GroupCommon::over) and are made
+    // again from there.
+    unsigned long long *over = c->words + W_OVER;
+    for (int64_t it = 0; it < k.num_loop;) {
+      {
+        StageTimer tm(c, 2);
+        PSPH_TRY(build_lists(c, pc, of, k.c_smooth, c->usp, it == 0, c->ngroups));
+        pass(nullptr);
+      }
+      it++;
+      if (it < k.num_loop) hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, over, 0ull, 2);
+      for (int64_t q = it; q < k.num_loop; q++) {
+        StageTimer tm(c, 2);
+        hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, of.cursor, 0ull, 1);
+        PSPH_TRY(launch_lists(c, pc, of, k.c_smooth, c->usp, over));
+        pass(over);
+      }
+      HIP_TRY(hipGetLastError());
+      PSPH_TRY(reduce_hmax(c));
+      if (it >= k.num_loop || !c->ngroups || !c->seen[W_OVER]) break;
+      it += (int64_t)c->seen[W_ITERS];
     }
-    HIP_TRY(hipGetLastError());
-    PSPH_TRY(reduce_hmax(c, &hmax));
+    hmax = seen_double(c, W_HMAX);
+    PSPH_TRY(seen_err(c, "adapt_h"));
   }
-  PSPH_TRY(check_err(c, "adapt_h"));
   set_reach(c, hmax);
   return 0;
 }
@@ -3346,14 +3476,13 @@ static int h_by_id(psph_ctx *c, double *tab, int replay) {
   if (c->n) hipLaunchKernelGGL(k_h_by_id, blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->pid, c->f.h, tab, replay);
   HIP_TRY(hipGetLastError());
   if (!replay) return 0;
-  double hmax;
-  PSPH_TRY(reduce_hmax(c, &hmax));
-  set_reach(c, hmax);
+  PSPH_TRY(reduce_hmax(c));
+  set_reach(c, seen_double(c, W_HMAX));
   return 0;
 }
 
-extern "C" int psph_rhs(psph_ctx *c, double dt) {
-  if (!c) return fail(PSPH_EINVAL, "null ctx");
+// The passes of a step; psph_step reads their errors at its end (seen_err).
+static int rhs_pass(psph_ctx *c, double dt) {
   if (!c->grid_valid) return fail(PSPH_EINVAL, "rhs: call psph_neighbors first");
   const psph_config &k = c->cfg;
   uint32_t n = (uint32_t)c->n;
@@ -3372,23 +3501,29 @@ extern "C" int psph_rhs(psph_ctx *c, double dt) {
   a.dt = dt; a.g = k.g; a.cutoff = k.cutoff; a.cutoff2 = k.cutoff2; a.alpha = k.alpha; a.beta = k.beta;
   a.ata = k.ata; a.eps_half = k.eps_half; a.prandtl = k.prandtl; a.heat_scale = k.heat_scale;
   a.beta2 = 2.0 * k.beta; a.kheat = 20.0 * k.eps_half / k.prandtl;
-  a.lans = k.lans; a.dim = k.dim; a.eos = eos_const(k); a.pairs = c->d_u64 + 2;
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 2, 0ull, 1);
+  a.lans = k.lans; a.dim = k.dim; a.eos = eos_const(k); a.pairs = c->words + W_PAIRS;
   if (n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 3);
-    if (n) PSPH_TRY((launch_groups<RhsPass<float>, RhsPass<float, true, true>, RhsPass<float, false>, RhsPass<double>>(c, a, fc)));
+    if (n) PSPH_TRY((launch_groups<RhsPass<float>, RhsPass<float, true, true>, RhsPass<float, false>, RhsPass<double>>(c, W_ERR_RHS, a, fc)));
   }
   HIP_TRY(hipGetLastError());
   std::swap(c->f.vx, c->dsp[1]); std::swap(c->f.vy, c->dsp[2]); std::swap(c->f.vz, c->dsp[3]);
   std::swap(c->f.e, c->dsp[4]); std::swap(c->f.p, c->dsp[5]); std::swap(c->f.c, c->dsp[6]);
   std::swap(c->f.T, c->dsp[7]); std::swap(c->f.gam, c->dsp[8]); std::swap(c->f.cp, c->dsp[9]);
-  HIP_TRY(hipMemcpyAsync(&c->last_pairs, c->d_u64 + 2, 8, hipMemcpyDeviceToHost, c->stream));
-  return check_err(c, "rhs");
+  return 0;
 }
 
-extern "C" int psph_density(psph_ctx *c) {
+extern "C" int psph_rhs(psph_ctx *c, double dt) {
   if (!c) return fail(PSPH_EINVAL, "null ctx");
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_PAIRS, 0ull, 1);
+  PSPH_TRY(rhs_pass(c, dt));
+  PSPH_TRY(read_words(c));
+  c->last_pairs = c->seen[W_PAIRS];
+  return seen_err(c, "rhs");
+}
+
+static int density_pass(psph_ctx *c) {
   if (!c->grid_valid) return fail(PSPH_EINVAL, "density: call psph_neighbors first");
   const psph_config &k = c->cfg;
   uint32_t n = (uint32_t)c->n;
@@ -3412,16 +3547,21 @@ extern "C" int psph_density(psph_ctx *c) {
   if (n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 4);
-    if (n) PSPH_TRY((launch_groups<DensPass<float>, DensPass<float, true, true>, DensPass<float, false>, DensPass<double>>(c, a, fc)));
+    if (n) PSPH_TRY((launch_groups<DensPass<float>, DensPass<float, true, true>, DensPass<float, false>, DensPass<double>>(c, W_ERR_DENS, a, fc)));
   }
   HIP_TRY(hipGetLastError());
   std::swap(c->f.rho, c->dsp[1]);
   std::swap(c->f.e, c->dsp[2]);
+  return 0;
+}
+
+extern "C" int psph_density(psph_ctx *c) {
+  if (!c) return fail(PSPH_EINVAL, "null ctx");
+  PSPH_TRY(density_pass(c));
   return check_err(c, "density");
 }
 
-extern "C" int psph_vsmooth(psph_ctx *c) {
-  if (!c) return fail(PSPH_EINVAL, "null ctx");
+static int vsmooth_pass(psph_ctx *c) {
   if (!c->grid_valid) return fail(PSPH_EINVAL, "vsmooth: call psph_neighbors first");
   const psph_config &k = c->cfg;
   VsmArgs a{};
@@ -3433,9 +3573,15 @@ extern "C" int psph_vsmooth(psph_ctx *c) {
   if (c->n) PSPH_TRY(ensure_lists(c));
   {
     StageTimer tm(c, 5);
-    if (c->n) PSPH_TRY((launch_groups<VsmPass<float>, VsmPass<float, true>, VsmPass<float>, VsmPass<double>>(c, a, FieldCopy{})));
+    if (c->n) PSPH_TRY((launch_groups<VsmPass<float>, VsmPass<float, true>, VsmPass<float>, VsmPass<double>>(c, W_ERR_VSM, a, FieldCopy{})));
   }
   HIP_TRY(hipGetLastError());
+  return 0;
+}
+
+extern "C" int psph_vsmooth(psph_ctx *c) {
+  if (!c) return fail(PSPH_EINVAL, "null ctx");
+  PSPH_TRY(vsmooth_pass(c));
   return check_err(c, "vsmooth");
 }
 
@@ -3445,30 +3591,42 @@ static int iferupt(const psph_ctx *c) {     // TimeProps::iferupt (properties.h:
   return 1;
 }
 
-extern "C" int psph_update_pos(psph_ctx *c, double dt) {
-  if (!c) return fail(PSPH_EINVAL, "null ctx");
+// undo: the density pass was queued behind an RHS that may have failed
+static int update_pos(psph_ctx *c, double dt, bool undo) {
   const psph_config &k = c->cfg;
   uint32_t n = (uint32_t)c->n;
   PosTape tp{c->tape.mode, (int32_t)c->tape.k, c->pid, c->tape.tr_step, c->tape.esc_step};
   if (tp.mode && (!tp.tr_step || c->next_pid > c->tape.id_cap)) return fail(PSPH_EINVAL, "update_pos: tape has no id table");
   StageTimer tm(c, 6);
-  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 4, 0ull, 1);
   if (n)
-    hipLaunchKernelGGL(k_update_pos, blocks(n), 256, 0, c->stream, n, k.dim, k.lans, iferupt(c), dt,
+    hipLaunchKernelGGL(k_update_pos, red_blocks(n), 256, 0, c->stream, n, k.dim, k.lans, iferupt(c), dt,
                        c->f.x, c->f.y, c->f.z, c->f.vx, c->f.vy, c->f.vz, c->f.svx, c->f.svy, c->f.svz,
                        c->f.bc, c->f.h, c->f.inv, k.dom_lo[2], k.ratio_sml_dx * k.h_air,
                        k.dom_lo[0], k.dom_lo[1], k.dom_lo[2], k.dom_hi[0], k.dom_hi[1], k.dom_hi[2],
-                       c->d_u64 + 3, tp);
-  if (n) hipLaunchKernelGGL(k_count_real, red_blocks(n), 256, 0, c->stream, n, c->f.bc, c->d_u64 + 4);
+                       c->words, tp);
   tm.stop();
   HIP_TRY(hipGetLastError());
-  unsigned long long cnt[2] = {0, 0};      // escaped, real after the update
-  HIP_TRY(hipMemcpyAsync(cnt, c->d_u64 + 3, 16, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  c->last_removed = (int64_t)cnt[0];
-  c->last_real = (int64_t)cnt[1];
+  PSPH_TRY(read_words(c));
+  if (undo) {
+    c->last_pairs = c->seen[W_PAIRS];
+    if ((uint32_t)c->seen[W_ERR] || (uint32_t)c->seen[W_ERR_RHS]) {
+      // the density pass did nothing: its fields are where they were
+      std::swap(c->f.rho, c->dsp[1]);
+      std::swap(c->f.e, c->dsp[2]);
+    }
+    PSPH_TRY(seen_err(c, "rhs"));
+  }
+  c->last_removed = (int64_t)c->seen[W_DEAD];
+  c->last_real = (int64_t)c->seen[W_REAL];
   c->grid_valid = false;
   return 0;
+}
+
+extern "C" int psph_update_pos(psph_ctx *c, double dt) {
+  if (!c) return fail(PSPH_EINVAL, "null ctx");
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_REAL, 0ull, 1);
+  hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->words + W_VMAX, 0ull, 1);
+  return update_pos(c, dt, false);
 }
 
 // id-indexed event tables of the tape, grown to hold `need` ids (new: -1)
@@ -3590,7 +3748,7 @@ static int apply_bcond_grid(psph_ctx *c, double disp, double *wrec = nullptr, si
   const double hm = std::max(c->h_max, k.ratio_sml_dx * k.h_air);
   a.reach = k.cutoff * hm * (1 + 1e-9) + disp * (1 + 1e-9);
   const uint32_t n = (uint32_t)c->n;
-  unsigned long long *count = c->d_u64 + 5;
+  unsigned long long *count = c->words + W_BCOND;
   hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, count, 0ull, 1);
   hipLaunchKernelGGL(k_bcond_list, blocks(n), 256, 0, c->stream, n, a, c->usp, count);
   const unsigned grid = std::min(kBcondGrid, (n / kBcondGroup / kXcds + 1) * kXcds);
@@ -3617,6 +3775,7 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
   const psph_config &k = c->cfg;
   Tape &tp = c->tape;
   double dt;
+  bool seen = false;                       // c->seen is of the state that the search will find
   if (k.adapt_domain && k.dim == 3 && !c->dom_ready)
     return fail(PSPH_EINVAL, "adapt_domain: call psph_domain_init after psph_load");
   if (tp.mode == 2) {
@@ -3624,8 +3783,10 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
     dt = tp.dt[tp.k];
     c->time += dt;
     c->step++;
+    hipLaunchKernelGGL(k_step_words, 1, 64, 0, c->stream, c->words);
   } else {
     PSPH_TRY(psph_timestep(c, &dt));
+    seen = true;
     PSPH_TRY(psph_advance_time(c, &dt));
     if (tp.mode == 1) tp.dt.push_back(dt);
   }
@@ -3634,13 +3795,14 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
     // the region of real particles grows before this step's search
     // (main.cc:256-304); the wall ghosts are refreshed after it
     c->dom_pending = 0;
+    seen = false;
     PSPH_TRY(domain_adapt(c));
     if (k.wall_bc && c->n) {
       PSPH_TRY(psph_neighbors(c));
       PSPH_TRY(apply_bcond_grid(c, 0.0));
     }
   }
-  PSPH_TRY(psph_neighbors(c));
+  PSPH_TRY(neighbors(c, seen));
   if (tp.mode == 2) {
     const int slot = tp.hslot[tp.k];
     if (slot >= 0) PSPH_TRY(h_by_id(c, tp.htab[slot], 1));
@@ -3657,13 +3819,13 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
     tp.hslot.push_back(-1);
   }
   if (c->rec) PSPH_TRY(rec_capture(c, 0, dt));
-  PSPH_TRY(psph_rhs(c, dt));
+  PSPH_TRY(rhs_pass(c, dt));
   if (c->rec) PSPH_TRY(rec_capture(c, 1, dt));
-  PSPH_TRY(psph_density(c));
+  PSPH_TRY(density_pass(c));
   if (c->rec) PSPH_TRY(rec_capture(c, 2, dt));
-  if (k.lans) PSPH_TRY(psph_vsmooth(c));
+  if (k.lans) PSPH_TRY(vsmooth_pass(c));
   if (c->rec) PSPH_TRY(rec_capture(c, 3, dt));
-  PSPH_TRY(psph_update_pos(c, dt));
+  PSPH_TRY(update_pos(c, dt, true));
   int64_t added = 0;
   const uint32_t id0 = c->next_pid;
   PSPH_TRY(psph_inject(c, dt, &added));
@@ -3676,14 +3838,9 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
   if (k.wall_bc && k.dim == 3 && c->n) {
     // apply_bcond at the end of the step (main.cc:468): the grid is the one of
     // this step's neighbour search; particles have moved by at most dt vmax
-    hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, c->d_u64 + 1, 0ull, 1);
-    hipLaunchKernelGGL(k_speed_max, red_blocks(c->n), 256, 0, c->stream, (uint32_t)c->n, c->f.bc, k.lans, c->f.vx,
-                       c->f.vy, c->f.vz, c->f.svx, c->f.svy, c->f.svz, c->d_u64 + 1);
-    unsigned long long bits = 0;
-    HIP_TRY(hipMemcpyAsync(&bits, c->d_u64 + 1, 8, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    double vmax;
-    std::memcpy(&vmax, &bits, 8);
+    double vmax = seen_double(c, W_VMAX);
+    for (size_t q = 0; q < (size_t)added; q++)
+      vmax = std::max(vmax, std::max(std::fabs(c->inj.vx[q]), std::max(std::fabs(c->inj.vy[q]), std::fabs(c->inj.vz[q]))));
     double disp = std::fabs(dt) * vmax;
     const uint32_t nb = (uint32_t)c->n;
     if (tp.mode == 1 && (int64_t)tp.xrecb.size() == tp.k) {
@@ -3703,7 +3860,7 @@ extern "C" int psph_step(psph_ctx *c, psph_step_out *out) {
       if (tp.k >= (int64_t)tp.xrecb.size() || !c->px)
         return fail(PSPH_EINVAL, "replay: no recorded refresh positions for step %lld", (long long)tp.k);
       hipLaunchKernelGGL(k_pos_from_rec, blocks(nb), 256, 0, c->stream, nb, c->pid, c->f.bc, tp.xrecb[tp.k],
-                         tp.xrecb_n[tp.k], c->f.x, c->f.y, c->f.z, c->px, c->py, c->pz, c->d_err);
+                         tp.xrecb_n[tp.k], c->f.x, c->f.y, c->f.z, c->px, c->py, c->pz, (int *)(c->words + W_ERR));
       disp *= 1.01;
     }
     if (c->rec) PSPH_TRY(rec_capture(c, 4, dt));
