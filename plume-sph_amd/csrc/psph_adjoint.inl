@@ -162,7 +162,7 @@ __global__ void k_adj_rhs_pre(uint32_t n, const int32_t *bc, double dt, double g
 // ---------------------------------------------------------------------------
 // Adjoint pair passes.  Rows: the particles whose state can depend on the
 // inputs (real particles, erupt ghosts, boundary ghosts next to targets), in
-// groups as the targets of the forward passes (k_group_lists, k_order_targets).
+// groups as the targets of the forward passes (k_cell_fill, k_group_lists).
 // ---------------------------------------------------------------------------
 struct AdjCommon {
   PairCommon p;              // targets: the rows
@@ -666,12 +666,14 @@ struct RhsAdj {
 // Adjoint rows: real particles, erupt ghosts, and the boundary ghosts (bc 1,
 // 2: constant in time, but their velocity and state enter their neighbours'
 // sums) that some target's sum met in the recorded step (gflag).
-__global__ void k_adj_row_flags(uint32_t n, const int32_t *bc, const uint32_t *gflag, uint32_t *flags) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > n) return;
-  const int b = i < n ? bc[i] : -1;
-  flags[i] = (is_real(b) || b == 0 || ((b == 1 || b == 2) && gflag[i])) ? 1u : 0u;
-}
+struct IsRow {
+  const int32_t *bc;
+  const uint32_t *gflag;
+  __device__ bool operator()(uint32_t i) const {
+    const int b = bc[i];
+    return is_real(b) || b == 0 || ((b == 1 || b == 2) && gflag[i]);
+  }
+};
 
 // erupt ghosts of the starting state, and what their theta-gradient takes:
 // row r of out holds field f at out[f rows + r]
@@ -743,7 +745,8 @@ struct Adjoint {
   double *aux[8] = {};        // per-particle seeds of one pass
   double *part = nullptr;     // reduction partials
   // chunks of adjoint rows
-  uint32_t *flags = nullptr, *tpos = nullptr, *rows = nullptr, *cchunks = nullptr, *coff = nullptr;
+  uint32_t *flags = nullptr, *tpos = nullptr, *rows = nullptr;
+  CellSum *cell_has = nullptr, *cell_at = nullptr;
   uint32_t *cfirst = nullptr, *ccount = nullptr;
   unsigned long long *made = nullptr;   // visits handed out, chunks
   size_t n_cap = 0, chunk_cap = 0, cell_cap = 0;
@@ -793,7 +796,7 @@ static void adjoint_free(psph_ctx *c) {
   for (auto p : A->L) if (p) hipFree(p);
   for (auto p : A->l) if (p) hipFree(p);
   for (auto p : A->aux) if (p) hipFree(p);
-  void *ptrs[] = {A->part, A->flags, A->tpos, A->rows, A->cchunks, A->coff, A->cfirst, A->ccount,
+  void *ptrs[] = {A->part, A->flags, A->tpos, A->rows, A->cell_has, A->cell_at, A->cfirst, A->ccount,
                   A->made};
   for (auto p : ptrs) if (p) hipFree(p);
   delete A;
@@ -1001,10 +1004,10 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
   hipStream_t s = c->stream;
   PSPH_TRY(adj_row_memory(c, A, n));
   if (ncells + 1 > A.cell_cap) {
-    uint32_t **arrs[] = {&A.cchunks, &A.coff};
+    CellSum **arrs[] = {&A.cell_has, &A.cell_at};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
     A.cell_cap = 0;
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)ncells + 1) * 4));
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)ncells + 1) * sizeof(CellSum)));
     A.cell_cap = (size_t)ncells + 1;
   }
   const size_t chunks_ub = n / kChunk + (size_t)ncells + 1;
@@ -1019,14 +1022,8 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
     PSPH_TRY(dmalloc((void **)&A.made, 2 * 8));
     hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, A.made, 0ull, 2);
   }
-  hipLaunchKernelGGL(k_adj_row_flags, blocks(n + 1), 256, 0, s, n, R.bc, R.gflag, A.flags);
-  PSPH_TRY(excl_scan(c, A.flags, A.tpos, (size_t)n + 1));
-  if (n) hipLaunchKernelGGL(k_targets, blocks(n), 256, 0, s, n, A.flags, A.tpos, A.rows);
-  hipLaunchKernelGGL(k_cell_chunks, blocks(ncells + 1), 256, 0, s, ncells, R.cs, A.tpos, (uint32_t)kChunk, A.cchunks);
-  PSPH_TRY(excl_scan(c, A.cchunks, A.coff, (size_t)ncells + 1));
-  hipLaunchKernelGGL(k_chunks, blocks(ncells + 1), 256, 0, s, ncells, R.cs, A.tpos, A.coff,
-                     (uint32_t)kChunk, A.cfirst, A.ccount, (uint32_t *)(A.made + 1));
-  if (n) launch_order(c, n, ncells, R.cs, A.tpos, R.d[RF_X], R.d[RF_Y], R.d[RF_Z], A.rows);
+  PSPH_TRY(fill_cells(c, ncells, R.cs, IsRow{R.bc, R.gflag}, A.cell_has, A.cell_at, nullptr, nullptr, R.d[RF_X], R.d[RF_Y],
+                      R.d[RF_Z], A.rows, A.cfirst, A.ccount, (uint32_t *)(A.made + 1)));
   HIP_TRY(hipGetLastError());
   return 0;
 }

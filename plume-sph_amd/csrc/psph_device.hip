@@ -259,48 +259,6 @@ __global__ void k_gather(uint32_t n, const uint32_t *perm, Moves mv) {
   for (int k = 0; k < N4; k++) mv.d4[k][i] = v4[k];
 }
 
-// cell_start[c] = first sorted index whose cell (key >> sh) >= c, c in [0, ncells]
-__global__ void k_cell_start(uint32_t n, const uint32_t *key, int sh, uint32_t ncells, uint32_t *cs) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i > n) return;
-  uint32_t prev = (i == 0) ? 0u : min(key[i - 1] >> sh, ncells) + 1u;
-  uint32_t cur = (i == n) ? ncells + 1u : min(key[i] >> sh, ncells) + 1u;
-  for (uint32_t c = prev; c < cur; c++) cs[c] = i;
-}
-
-// tiles per cell (64 consecutive particles each); tcnt[ncells] = 0
-__global__ void k_tile_counts(uint32_t ncells, const uint32_t *cs, uint32_t *tcnt) {
-  uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c > ncells) return;
-  tcnt[c] = c == ncells ? 0u : (cs[c + 1] - cs[c] + kWave - 1) / kWave;
-}
-
-// Bounding box of every tile, rounded outwards to float: [lo, hi] per tile, and
-// in the w components the bits of its first particle and its particle count.
-// One wavefront per tile; the tile's cell is found by bisection of toff.
-__global__ __launch_bounds__(kWave) void k_tile_boxes(uint32_t ncells, const uint32_t *cs, const uint32_t *toff,
-                                                      const double *x, const double *y, const double *z,
-                                                      float4 *tbox) {
-  const uint32_t t = blockIdx.x;
-  if (t >= toff[ncells]) return;
-  uint32_t lo = 0, hi = ncells;              // toff[lo] <= t < toff[hi]
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) / 2;
-    if (toff[mid] <= t) lo = mid; else hi = mid;
-  }
-  const uint32_t base = cs[lo] + kWave * (t - toff[lo]);
-  const uint32_t end = min(cs[lo + 1], base + kWave);
-  const uint32_t j = base + threadIdx.x < end ? base + threadIdx.x : base;
-  const double px = x[j], py = y[j], pz = z[j];
-  const double ax = wave_min(px), ay = wave_min(py), az = wave_min(pz);
-  const double bx = wave_max(px), by = wave_max(py), bz = wave_max(pz);
-  if (threadIdx.x == 0) {
-    tbox[2 * t] = make_float4(__double2float_rd(ax), __double2float_rd(ay), __double2float_rd(az), __uint_as_float(base));
-    tbox[2 * t + 1] = make_float4(__double2float_ru(bx), __double2float_ru(by), __double2float_ru(bz),
-                                  __uint_as_float(end - base));
-  }
-}
-
 // Reference bucket (preprocessor cells of edge 8 h_air, preprocess.cc:88-133)
 // as packed coordinates: x in bits 0-9, y in bits 11-20, z in bits 22-31 (at
 // most 1023 buckets per axis; kDead outside the grid).  A list holds the own
@@ -315,54 +273,45 @@ __device__ inline bool refb_adjacent(uint32_t a, uint32_t b) {
   return (a != kDead) & (b != kDead) & ((d & 0x7ffu) - 1024u <= 2u) & (((d >> 11) & 0x7ffu) - 1024u <= 2u) & ((d >> 22) <= 2u);
 }
 
-// the smoothing length at list time, and the reference bucket
-__global__ void k_refb(uint32_t n, const double *x, const double *y, const double *z, const double *h,
-                       double lx, double ly, double lz, double del, int bx, int by, int bz,
-                       uint32_t *refb, double *h_list) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// After the sort: cs[c] = first index whose cell (key >> sh) >= c, c in [0,
+// ncells]; the smoothing length at list time; the reference bucket.  Empty cells
+// that follow each other are filled by the whole wave (one lane alone took 11 us
+// at 65k particles of 1.7k targets).
+struct RefBuckets { double lo[3], del; int nb[3]; };
+__global__ void k_sorted(uint32_t n, const uint32_t *key, int sh, uint32_t ncells, uint32_t *cs, const double *x,
+                         const double *y, const double *z, const double *h, RefBuckets b, uint32_t *refb, double *h_list) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool here = i <= n;
+  uint32_t prev = 0, cur = 0;
+  if (here) {
+    prev = (i == 0) ? 0u : min(key[i - 1] >> sh, ncells) + 1u;
+    cur = (i == n) ? ncells + 1u : min(key[i] >> sh, ncells) + 1u;
+  }
+  const bool many = cur > prev + 4;
+  if (!many)
+    for (uint32_t c = prev; c < cur; c++) cs[c] = i;
+  uint64_t left = __ballot(many);
+  while (left) {
+    const int l = __builtin_ctzll(left);
+    left &= left - 1;
+    const uint32_t a = __builtin_amdgcn_readlane(prev, l), e = __builtin_amdgcn_readlane(cur, l);
+    const uint32_t at = __builtin_amdgcn_readlane(i, l);
+    for (uint32_t c = a + threadIdx.x % kWave; c < e; c += kWave) cs[c] = at;
+  }
   if (i >= n) return;
-  double fx = floor((x[i] - lx) / del), fy = floor((y[i] - ly) / del), fz = floor((z[i] - lz) / del);
+  const double fx = floor((x[i] - b.lo[0]) / b.del), fy = floor((y[i] - b.lo[1]) / b.del),
+               fz = floor((z[i] - b.lo[2]) / b.del);
   uint32_t r = kDead;
-  if (fx >= 0 && fx < bx && fy >= 0 && fy < by && fz >= 0 && fz < bz)
+  if (fx >= 0 && fx < b.nb[0] && fy >= 0 && fy < b.nb[1] && fz >= 0 && fz < b.nb[2])
     r = refb_pack((uint32_t)fx, (uint32_t)fy, (uint32_t)fz);
   refb[i] = r;
   h_list[i] = h[i];
 }
 
-__global__ void k_target_flags(uint32_t n, const int32_t *bc, uint32_t *flags) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= n) flags[i] = (i < n && need_neigh(bc[i])) ? 1u : 0u;
-}
-
+// indices whose flag is set, in order (tpos: the flags' sums)
 __global__ void k_targets(uint32_t n, const uint32_t *flags, const uint32_t *tpos, uint32_t *targets) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n && flags[i]) targets[tpos[i]] = i;
-}
-
-// chunks: up to csz consecutive targets of one cell
-__global__ void k_cell_chunks(uint32_t ncells, const uint32_t *cs, const uint32_t *tpos, uint32_t csz,
-                              uint32_t *cell_chunks) {
-  uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r > ncells) return;
-  if (r == ncells) { cell_chunks[r] = 0; return; }
-  uint32_t a = tpos[cs[r]], b = tpos[cs[r + 1]];
-  cell_chunks[r] = (b - a + csz - 1) / csz;
-}
-
-__global__ void k_chunks(uint32_t ncells, const uint32_t *cs, const uint32_t *tpos, const uint32_t *chunk_off,
-                         uint32_t csz, uint32_t *cfirst, uint32_t *ccount, uint32_t *nchunks) {
-  uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= ncells) {
-    if (r == ncells) *nchunks = chunk_off[ncells];
-    return;
-  }
-  uint32_t a = tpos[cs[r]], b = tpos[cs[r + 1]];
-  uint32_t o = chunk_off[r];
-  for (uint32_t t = a; t < b; t += csz) {
-    cfirst[o] = t;
-    ccount[o] = min(csz, b - t);
-    o++;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -598,7 +547,7 @@ __device__ inline double swap_add(double a, double b) {
 // One wavefront per run, two targets a lane; a target's place is the number of
 // its segment's smaller keys, each key a coordinate's upper bits above the place
 // it had (no two are equal).  Bound by that count: a chain of LDS reads where
-// cells are few (12 us at 1.7k targets), 140 us at 4M.
+// cells are few (the whole of k_cell_fill 18 us at 1.7k targets), 140 us at 4M.
 // us per launch without and with it (RHS, density, filter): 1M FP64 7124, 3159,
 // 2593 / 6270, 2710, 2240; 4M FP32-exp 15203, 8077, 7212 / 13390, 7080, 6300.
 constexpr int kRun = 2 * kWave;
@@ -612,15 +561,21 @@ __device__ inline float order_value(uint32_t k) {
   return __uint_as_float(k ^ ((int32_t)k < 0 ? 0x80000000u : 0xffffffffu));
 }
 
+// what this wave wrote to LDS is there for its other lanes
+__device__ inline void wave_sync() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // the n places' segments of 2 HALF: each becomes its lower and its upper half
 template <int HALF>
-__device__ inline void halve_segments(uint32_t n, uint32_t (&key)[3][kRun], uint32_t *id) {
+__device__ inline void halve_segments(uint32_t lane, uint32_t n, uint32_t (&key)[3][kRun], uint32_t *id) {
   if (n <= HALF) return;                            // (uniform) one segment, no longer than its half
   constexpr int kAcross = 2 * HALF < kWave ? 2 * HALF : kWave;
   uint32_t own[2][3], to[2], who[2], lo[2][3], up[2][3];
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    const uint32_t p = threadIdx.x + q * kWave;
+    const uint32_t p = lane + q * kWave;
     who[q] = id[p];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
@@ -646,7 +601,7 @@ __device__ inline void halve_segments(uint32_t n, uint32_t (&key)[3][kRun], uint
   }
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    const uint32_t p = threadIdx.x + q * kWave, s0 = p & ~(2u * HALF - 1u);
+    const uint32_t p = lane + q * kWave, s0 = p & ~(2u * HALF - 1u);
     const float ex = order_value(up[q][0]) - order_value(lo[q][0]);
     const float ey = order_value(up[q][1]) - order_value(lo[q][1]);
     const float ez = order_value(up[q][2]) - order_value(lo[q][2]);
@@ -665,47 +620,141 @@ __device__ inline void halve_segments(uint32_t n, uint32_t (&key)[3][kRun], uint
     // a segment no longer than its half stays as it is
     to[q] = min(s0 + 2 * HALF, n) <= s0 + HALF ? p : s0 + below;
   }
-  __syncthreads();
+  wave_sync();
 #pragma unroll
   for (int q = 0; q < 2; q++)
-    if (threadIdx.x + q * kWave < n) {
+    if (lane + q * kWave < n) {
       id[to[q]] = who[q];
 #pragma unroll
       for (int d = 0; d < 3; d++) key[d][to[q]] = (own[q][d] & ~(uint32_t)(kRun - 1)) | to[q];
     }
-  __syncthreads();
+  wave_sync();
 }
 
-// per_cell: wavefronts a cell has (they take its runs in turn)
-__global__ __launch_bounds__(kWave) void k_order_targets(const uint32_t *cs, const uint32_t *tpos, uint32_t per_cell,
-                                                         const double *x, const double *y, const double *z,
-                                                         uint32_t *targets) {
-  __shared__ __align__(16) uint32_t key[3][kRun];
-  __shared__ uint32_t id[kRun];
+struct OrderLds {
+  uint32_t key[3][kRun], id[kRun];
+};
+// one run: t[0..n), n <= kRun
+__device__ inline void order_run(uint32_t lane, uint32_t n, const double *x, const double *y, const double *z,
+                                 uint32_t *t, OrderLds &o) {
   static_assert(kRun == 2 * kWave && kGroup == 8, "halves of 64 to 8 places");
-  const uint32_t cell = blockIdx.x / per_cell;
-  const uint32_t a = tpos[cs[cell]], b = tpos[cs[cell + 1]];
-  for (uint32_t t0 = a + blockIdx.x % per_cell * kRun; t0 < b; t0 += per_cell * kRun) {
-    const uint32_t n = min((uint32_t)kRun, b - t0);
-    if (n <= (uint32_t)kGroup) continue;
-    const uint32_t first = targets[t0];
-    const double org[3] = {x[first], y[first], z[first]};
+  const uint32_t first = t[0];
+  const double org[3] = {x[first], y[first], z[first]};
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const uint32_t p = threadIdx.x + q * kWave, i = targets[t0 + min(p, n - 1)];
-      const double at[3] = {x[i], y[i], z[i]};
-      id[p] = i;
+  for (int q = 0; q < 2; q++) {
+    const uint32_t p = lane + q * kWave, i = t[min(p, n - 1)];
+    const double at[3] = {x[i], y[i], z[i]};
+    o.id[p] = i;
 #pragma unroll
-      for (int d = 0; d < 3; d++) key[d][p] = p < n ? order_key((float)(at[d] - org[d]), p) : ~0u;
-    }
-    __syncthreads();
-    halve_segments<64>(n, key, id);
-    halve_segments<32>(n, key, id);
-    halve_segments<16>(n, key, id);
-    halve_segments<8>(n, key, id);
-    for (uint32_t p = threadIdx.x; p < n; p += kWave) targets[t0 + p] = id[p];
-    __syncthreads();
+    for (int d = 0; d < 3; d++) o.key[d][p] = p < n ? order_key((float)(at[d] - org[d]), p) : ~0u;
   }
+  wave_sync();
+  halve_segments<64>(lane, n, o.key, o.id);
+  halve_segments<32>(lane, n, o.key, o.id);
+  halve_segments<16>(lane, n, o.key, o.id);
+  halve_segments<8>(lane, n, o.key, o.id);
+  for (uint32_t p = lane; p < n; p += kWave) t[p] = o.id[p];
+  wave_sync();
+}
+
+// What a cell holds, and the sums of it over the cells before: tiles (64
+// consecutive particles each), targets, chunks of kChunk consecutive targets.
+struct CellSum { uint32_t tiles, targets, chunks; };
+struct CellAdd {
+  __host__ __device__ CellSum operator()(const CellSum &a, const CellSum &b) const {
+    return CellSum{a.tiles + b.tiles, a.targets + b.targets, a.chunks + b.chunks};
+  }
+};
+struct IsTarget {
+  const int32_t *bc;
+  __device__ bool operator()(uint32_t i) const { return need_neigh(bc[i]); }
+};
+
+// One workgroup per cell (k_cell_counts: and one more, zero): a wavefront where
+// there is a grid, kOneCell threads where one cell holds everything.
+constexpr int kOneCell = 1024;
+template <class T>
+__global__ __launch_bounds__(kOneCell) void k_cell_counts(uint32_t ncells, const uint32_t *cs, T is, CellSum *out) {
+  __shared__ uint32_t part[kOneCell / kWave];
+  const uint32_t cell = blockIdx.x;
+  const uint32_t lo = cs[cell], hi = cell < ncells ? cs[cell + 1] : lo;
+  uint32_t cnt = 0;
+  for (uint32_t i = lo + threadIdx.x; i < hi; i += blockDim.x) cnt += is(i) ? 1u : 0u;
+  for (int o = kWave / 2; o > 0; o >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, o);
+  if (blockDim.x > kWave) {
+    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = cnt;
+    __syncthreads();
+    cnt = 0;
+    for (uint32_t w = 0; w < blockDim.x / kWave; w++) cnt += part[w];
+  }
+  if (threadIdx.x == 0) out[cell] = CellSum{(hi - lo + kWave - 1) / kWave, cnt, (cnt + kChunk - 1) / kChunk};
+}
+
+// The cell's tiles with their boxes, rounded outwards to float: [lo, hi] per tile,
+// and in the w components the bits of its first particle and its particle count
+// (toff null: not these); its targets, in the order of the passes; its chunks.
+// (Counts, scans and lists in kernels of their own over particles, tiles and cells:
+// 15 launches of a search; so 5.)
+template <class T>
+__global__ __launch_bounds__(kOneCell) void k_cell_fill(uint32_t ncells, const uint32_t *cs, T is, const CellSum *sums,
+                                                        uint32_t *toff, float4 *tbox, const double *x, const double *y,
+                                                        const double *z, uint32_t *targets, uint32_t *cfirst,
+                                                        uint32_t *ccount, uint32_t *nchunks) {
+  extern __shared__ __align__(16) char lds[];      // an OrderLds per wave
+  __shared__ uint32_t part[kOneCell / kWave];
+  const uint32_t cell = blockIdx.x, lane = threadIdx.x % kWave;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), nw = blockDim.x / kWave;
+  const uint32_t lo = cs[cell], hi = cs[cell + 1];
+  const CellSum at = sums[cell], to = sums[cell + 1];
+  if (threadIdx.x == 0) {
+    if (toff) toff[cell] = at.tiles;
+    if (cell == ncells - 1) {
+      if (toff) toff[ncells] = to.tiles;
+      *nchunks = to.chunks;
+    }
+  }
+  for (uint32_t t = at.tiles + wave; toff && t < to.tiles; t += nw) {
+    const uint32_t base = lo + kWave * (t - at.tiles), end = min(hi, base + kWave);
+    const uint32_t j = base + lane < end ? base + lane : base;
+    const double px = x[j], py = y[j], pz = z[j];
+    const double ax = wave_min(px), ay = wave_min(py), az = wave_min(pz);
+    const double bx = wave_max(px), by = wave_max(py), bz = wave_max(pz);
+    if (lane == 0) {
+      tbox[2 * t] = make_float4(__double2float_rd(ax), __double2float_rd(ay), __double2float_rd(az), __uint_as_float(base));
+      tbox[2 * t + 1] = make_float4(__double2float_ru(bx), __double2float_ru(by), __double2float_ru(bz),
+                                    __uint_as_float(end - base));
+    }
+  }
+  const uint32_t nt = to.targets - at.targets;
+  if (!nt) return;
+  for (uint32_t q = threadIdx.x; q < to.chunks - at.chunks; q += blockDim.x) {
+    cfirst[at.chunks + q] = at.targets + q * kChunk;
+    ccount[at.chunks + q] = min((uint32_t)kChunk, nt - q * kChunk);
+  }
+  uint32_t next = at.targets;
+  for (uint32_t i0 = lo; i0 < hi; i0 += blockDim.x) {
+    const uint32_t i = i0 + threadIdx.x;
+    const bool mine = i < hi && is(i);
+    const uint64_t m = __ballot(mine);
+    uint32_t before = 0, all = (uint32_t)__popcll(m);
+    if (nw > 1) {
+      if (lane == 0) part[wave] = all;
+      __syncthreads();
+      all = 0;
+      for (uint32_t w = 0; w < nw; w++) {
+        if (w < wave) before += part[w];
+        all += part[w];
+      }
+      __syncthreads();
+    }
+    if (mine) targets[next + before + lanes_below(m)] = i;
+    next += all;
+  }
+  __threadfence_block();
+  __syncthreads();                                 // the cell's targets are there
+  OrderLds &o = ((OrderLds *)lds)[wave];
+  for (uint32_t t0 = wave * kRun; t0 < nt; t0 += nw * kRun)
+    if (nt - t0 > (uint32_t)kGroup) order_run(lane, min((uint32_t)kRun, nt - t0), x, y, z, targets + at.targets + t0, o);
 }
 
 // The tiles a group visits, with a 64-bit mask of the particles that can be a
@@ -2514,9 +2563,10 @@ struct psph_ctx {
   int32_t *isp = nullptr;      // spare i32 array
   double *h_list = nullptr;
   uint32_t *refb = nullptr, *key_a = nullptr, *key_b = nullptr, *idx_a = nullptr, *idx_b = nullptr;
-  uint32_t *flags = nullptr, *tpos = nullptr, *targets = nullptr;
+  uint32_t *targets = nullptr;
   uint32_t *cfirst = nullptr, *ccount = nullptr;
-  uint32_t *cs = nullptr, *tcnt = nullptr, *toff = nullptr, *cchunks = nullptr, *coff = nullptr, *nchunks = nullptr;
+  uint32_t *cs = nullptr, *toff = nullptr, *nchunks = nullptr;
+  CellSum *cell_has = nullptr, *cell_at = nullptr;   // per cell: its contents, and of the cells before
   float4 *tbox = nullptr;
   size_t cs_cap = 0, tile_cap = 0, chunk_cap = 0;
   void *cub = nullptr;
@@ -2683,8 +2733,6 @@ extern "C" int psph_create(const psph_config *cfg, size_t capacity, psph_ctx **o
   uint32_t **u32s[] = {&c->refb, &c->key_a, &c->key_b, &c->idx_a, &c->idx_b, &c->targets};
   for (auto pp : u32s)
     if (!rc) rc = dmalloc((void **)pp, capacity * 4);
-  if (!rc) rc = dmalloc((void **)&c->flags, (capacity + 1) * 4);
-  if (!rc) rc = dmalloc((void **)&c->tpos, (capacity + 1) * 4);
   if (!rc) rc = dmalloc((void **)&c->words, W_COUNT * 8);
   if (!rc) { c->gcursor = c->words + W_CURSOR; c->nchunks = (uint32_t *)(c->words + W_CHUNKS); }
   if (!rc && hipHostMalloc((void **)&c->seen, (W_COUNT + 2) * 8, hipHostMallocDefault) != hipSuccess) {
@@ -2715,8 +2763,7 @@ extern "C" int psph_destroy(psph_ctx *c) {
 #undef F_
   for (auto p : c->dsp) if (p) hipFree(p);
   void *ptrs[] = {c->usp, c->isp, c->h_list, c->pid, c->pid_sp, c->refb, c->key_a, c->key_b, c->idx_a, c->idx_b,
-                  c->flags, c->tpos, c->targets, c->cfirst, c->ccount, c->cs, c->tcnt, c->toff,
-                  c->cchunks, c->coff, c->tbox, c->cub, c->words, c->up_d, c->d_part,
+                  c->targets, c->cfirst, c->ccount, c->cs, c->toff, c->cell_has, c->cell_at, c->tbox, c->cub, c->words, c->up_d, c->d_part,
                   c->gvisit, c->goff, c->gnum, c->gfast, c->gxy, c->gzh, c->px, c->py, c->pz,
                   c->d_occ, c->d_conv, c->d_sides};
   for (auto p : ptrs) if (p) hipFree(p);
@@ -2732,7 +2779,7 @@ extern "C" int psph_destroy(psph_ctx *c) {
 
 // Up to kUpload particles go through pinned memory in one copy and a kernel that
 // takes the fields apart, and nobody waits: the 25 copies of an inlet's few
-// particles, each waited for, took NNN us of a step.
+// particles, each waited for, took about 0.2 ms of a step.
 constexpr size_t kUpload = 4096;
 constexpr size_t kUploadBytes = 19 * 8 + 6 * 4;      // of a particle
 __global__ void k_append(uint32_t n, uint32_t at, const char *from, DevFields f) {
@@ -2996,9 +3043,13 @@ static int build_grid(psph_ctx *c, double hmax) {
   c->grid = g;
   size_t need = (size_t)g.ncells + 1;
   if (need > c->cs_cap) {
-    uint32_t **arrs[] = {&c->cs, &c->tcnt, &c->toff, &c->cchunks, &c->coff};
+    uint32_t **arrs[] = {&c->cs, &c->toff};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
+    CellSum **sums[] = {&c->cell_has, &c->cell_at};
+    for (auto pp : sums) { if (*pp) hipFree(*pp); *pp = nullptr; }
+    c->cs_cap = 0;
     for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, need * 4));
+    for (auto pp : sums) PSPH_TRY(dmalloc((void **)pp, need * sizeof(CellSum)));
     c->cs_cap = need;
   }
   const size_t ub = c->n / kWave + (size_t)g.ncells + 1;
@@ -3029,11 +3080,22 @@ static int excl_scan(psph_ctx *c, const uint32_t *in, uint32_t *out, size_t n1) 
   return 0;
 }
 
-static void launch_order(psph_ctx *c, uint32_t n, uint32_t ncells, const uint32_t *cs, const uint32_t *tpos,
-                         const double *x, const double *y, const double *z, uint32_t *targets) {
-  // one cell holds everything: a wavefront per run, else per cell
-  const uint32_t per_cell = ncells == 1 ? (n + kRun - 1) / kRun : 1;
-  hipLaunchKernelGGL(k_order_targets, ncells * per_cell, kWave, 0, c->stream, cs, tpos, per_cell, x, y, z, targets);
+// The contents of the cells that cs bounds: tiles (toff not null), targets (is)
+// and their chunks.  has, at: ncells + 1 sums each.
+template <class T>
+static int fill_cells(psph_ctx *c, uint32_t ncells, const uint32_t *cs, T is, CellSum *has, CellSum *at, uint32_t *toff,
+                      float4 *tbox, const double *x, const double *y, const double *z, uint32_t *targets,
+                      uint32_t *cfirst, uint32_t *ccount, uint32_t *nchunks) {
+  const unsigned threads = ncells == 1 ? kOneCell : kWave;
+  hipLaunchKernelGGL((k_cell_counts<T>), ncells + 1, threads, 0, c->stream, ncells, cs, is, has);
+  size_t bytes = 0;
+  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)ncells + 1, c->stream));
+  PSPH_TRY(ensure_cub(c, bytes));
+  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(c->cub, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)ncells + 1, c->stream));
+  hipLaunchKernelGGL((k_cell_fill<T>), ncells, threads, threads / kWave * sizeof(OrderLds), c->stream, ncells, cs, is, at,
+                     toff, tbox, x, y, z, targets, cfirst, ccount, nchunks);
+  HIP_TRY(hipGetLastError());
+  return 0;
 }
 
 // seen: c->seen holds the largest h and the removed particles of this state
@@ -3108,10 +3170,6 @@ static int neighbors(psph_ctx *c, bool seen) {
     c->n = n;
     hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, c->words + W_DEAD, 0ull, 1);
   }
-  hipLaunchKernelGGL(k_cell_start, blocks(n + 1), 256, 0, s, n, c->key_a, 3 * g.fbits, g.ncells, c->cs);
-  // tiles of each cell and their boxes
-  hipLaunchKernelGGL(k_tile_counts, blocks(g.ncells + 1), 256, 0, s, g.ncells, c->cs, c->tcnt);
-  PSPH_TRY(excl_scan(c, c->tcnt, c->toff, (size_t)g.ncells + 1));
   // the positions every predicate of this step reads
   const double *qx = frozen ? c->px : c->f.x, *qy = frozen ? c->py : c->f.y, *qz = frozen ? c->pz : c->f.z;
   if (tp.mode == 1 && (int64_t)tp.xrec.size() == tp.k) {
@@ -3122,8 +3180,6 @@ static int neighbors(psph_ctx *c, bool seen) {
     tp.xrec_n.push_back(nrec);
     if (n) hipLaunchKernelGGL(k_pos_to_rec, blocks(n), 256, 0, s, n, c->pid, c->f.x, c->f.y, c->f.z, rec, nrec);
   }
-  hipLaunchKernelGGL(k_tile_boxes, (unsigned)(n / kWave + g.ncells + 1), kWave, 0, s, g.ncells, c->cs, c->toff,
-                     qx, qy, qz, c->tbox);
   // reference buckets (list membership) and h at list time
   int nb[3] = {1, 1, 1};
   double del = c->cfg.bucket_edge > 0 ? c->cfg.bucket_edge : 1.0;
@@ -3132,19 +3188,12 @@ static int neighbors(psph_ctx *c, bool seen) {
   for (int d = 0; d < 3; d++)
     if (nb[d] > kRefbMaxPerAxis)
       return fail(PSPH_ECAPACITY, "%d reference buckets on axis %d (at most %d)", nb[d], d, kRefbMaxPerAxis);
-  if (n) hipLaunchKernelGGL(k_refb, blocks(n), 256, 0, s, n, qx, qy, qz, c->f.h,
-                            c->cfg.ext_lo[0], c->cfg.ext_lo[1], c->cfg.ext_lo[2], del, nb[0], nb[1], nb[2],
-                            c->refb, c->h_list);
-  // targets and their chunks (<= kChunk consecutive targets of one cell)
-  hipLaunchKernelGGL(k_target_flags, blocks(n + 1), 256, 0, s, n, c->f.bc, c->flags);
-  PSPH_TRY(excl_scan(c, c->flags, c->tpos, (size_t)n + 1));
-  if (n) hipLaunchKernelGGL(k_targets, blocks(n), 256, 0, s, n, c->flags, c->tpos, c->targets);
-  hipLaunchKernelGGL(k_cell_chunks, blocks(g.ncells + 1), 256, 0, s, g.ncells, c->cs, c->tpos, (uint32_t)kChunk,
-                     c->cchunks);
-  PSPH_TRY(excl_scan(c, c->cchunks, c->coff, (size_t)g.ncells + 1));
-  hipLaunchKernelGGL(k_chunks, blocks(g.ncells + 1), 256, 0, s, g.ncells, c->cs, c->tpos, c->coff,
-                     (uint32_t)kChunk, c->cfirst, c->ccount, c->nchunks);
-  if (n) launch_order(c, n, g.ncells, c->cs, c->tpos, qx, qy, qz, c->targets);
+  const RefBuckets rb{{c->cfg.ext_lo[0], c->cfg.ext_lo[1], c->cfg.ext_lo[2]}, del, {nb[0], nb[1], nb[2]}};
+  hipLaunchKernelGGL(k_sorted, blocks((size_t)n + 1), 256, 0, s, n, c->key_a, 3 * g.fbits, g.ncells, c->cs, qx, qy, qz,
+                     c->f.h, rb, c->refb, c->h_list);
+  // tiles, targets and their chunks (<= kChunk consecutive targets of one cell)
+  PSPH_TRY(fill_cells(c, g.ncells, c->cs, IsTarget{c->f.bc}, c->cell_has, c->cell_at, c->toff, c->tbox, qx, qy, qz,
+                      c->targets, c->cfirst, c->ccount, c->nchunks));
   HIP_TRY(hipGetLastError());
   tm.stop();
   c->grid_valid = true;
