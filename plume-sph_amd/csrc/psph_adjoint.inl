@@ -817,12 +817,12 @@ static int snap_save(psph_ctx *c, Snapshot &s) {
   double *d[PSPH_NDF]; uint32_t *u[PSPH_NUF]; int32_t *iv[PSPH_NIF];
   dev_fields(c, d, u, iv);
   hipStream_t st = c->stream;
-  if (n) {
-    for (int k = 0; k < PSPH_NDF; k++) HIP_TRY(hipMemcpyAsync(s.d[k], d[k], n * 8, hipMemcpyDeviceToDevice, st));
-    for (int k = 0; k < PSPH_NUF; k++) HIP_TRY(hipMemcpyAsync(s.u[k], u[k], n * 4, hipMemcpyDeviceToDevice, st));
-    for (int k = 0; k < PSPH_NIF; k++) HIP_TRY(hipMemcpyAsync(s.i[k], iv[k], n * 4, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(s.pid, c->pid, n * 4, hipMemcpyDeviceToDevice, st));
-  }
+  Copies to{c, n};
+  for (int k = 0; k < PSPH_NDF; k++) PSPH_TRY(to.add(s.d[k], d[k]));
+  for (int k = 0; k < PSPH_NUF; k++) PSPH_TRY(to.add(s.u[k], u[k]));
+  for (int k = 0; k < PSPH_NIF; k++) PSPH_TRY(to.add(s.i[k], iv[k]));
+  PSPH_TRY(to.add(s.pid, c->pid));
+  PSPH_TRY(to.flush());
   HIP_TRY(hipMemcpyAsync(&s.dead, c->words + W_DEAD, 8, hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   s.n = n;
@@ -836,12 +836,12 @@ static int snap_load(psph_ctx *c, const Snapshot &s) {
   dev_fields(c, d, u, iv);
   hipStream_t st = c->stream;
   const size_t n = s.n;
-  if (n) {
-    for (int k = 0; k < PSPH_NDF; k++) HIP_TRY(hipMemcpyAsync(d[k], s.d[k], n * 8, hipMemcpyDeviceToDevice, st));
-    for (int k = 0; k < PSPH_NUF; k++) HIP_TRY(hipMemcpyAsync(u[k], s.u[k], n * 4, hipMemcpyDeviceToDevice, st));
-    for (int k = 0; k < PSPH_NIF; k++) HIP_TRY(hipMemcpyAsync(iv[k], s.i[k], n * 4, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(c->pid, s.pid, n * 4, hipMemcpyDeviceToDevice, st));
-  }
+  Copies from{c, n};
+  for (int k = 0; k < PSPH_NDF; k++) PSPH_TRY(from.add(d[k], s.d[k]));
+  for (int k = 0; k < PSPH_NUF; k++) PSPH_TRY(from.add(u[k], s.u[k]));
+  for (int k = 0; k < PSPH_NIF; k++) PSPH_TRY(from.add(iv[k], s.i[k]));
+  PSPH_TRY(from.add(c->pid, s.pid));
+  PSPH_TRY(from.flush());
   hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, st, c->words + W_DEAD, (unsigned long long)s.dead, 1);
   HIP_TRY(hipStreamSynchronize(st));
   c->n = n;
@@ -857,10 +857,8 @@ static int rec_capture(psph_ctx *c, int stage, double dt) {
   StepRec &r = *c->rec;
   hipStream_t st = c->stream;
   const size_t n = c->n;
-  auto cp = [&](int f, const double *src) -> int {
-    if (n) HIP_TRY(hipMemcpyAsync(r.d[f], src, n * 8, hipMemcpyDeviceToDevice, st));
-    return 0;
-  };
+  Copies to{c, stage < 4 ? n : r.n};       // (4, 5: the inlet's particles come after the first r.n)
+  auto cp = [&](int f, const double *src) -> int { return to.add(r.d[f], src); };
   if (stage == 0) {
     if (n > r.cap) {
       const size_t cap = std::max(c->cap, n);
@@ -904,17 +902,14 @@ static int rec_capture(psph_ctx *c, int stage, double dt) {
     const double *src[] = {c->f.x, c->f.y, c->f.z, c->f.h, c->f.m, c->f.rho, c->f.p, c->f.c, c->f.T, c->f.cp,
                            c->f.svx, c->f.svy, c->f.svz, c->f.vx, c->f.vy, c->f.vz, c->f.e, c->h_list};
     for (int f = RF_X; f <= RF_HLIST; f++) PSPH_TRY(cp(f, src[f]));
-    if (n) {
-      HIP_TRY(hipMemcpyAsync(r.pid, c->pid, n * 4, hipMemcpyDeviceToDevice, st));
-      HIP_TRY(hipMemcpyAsync(r.refb, c->refb, n * 4, hipMemcpyDeviceToDevice, st));
-      HIP_TRY(hipMemcpyAsync(r.ckey, c->key_a, n * 4, hipMemcpyDeviceToDevice, st));
-      HIP_TRY(hipMemcpyAsync(r.bc, c->f.bc, n * 4, hipMemcpyDeviceToDevice, st));
-      HIP_TRY(hipMemcpyAsync(r.phase, c->f.phase, n * 4, hipMemcpyDeviceToDevice, st));
-      hipLaunchKernelGGL(k_fill_i32, blocks(n), 256, 0, st, (int *)r.gflag, 0, (int)n);
-    }
-    HIP_TRY(hipMemcpyAsync(r.cs, c->cs, ncs * 4, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(r.toff, c->toff, ncs * 4, hipMemcpyDeviceToDevice, st));
-    HIP_TRY(hipMemcpyAsync(r.tbox, c->tbox, ntb * 2 * sizeof(float4), hipMemcpyDeviceToDevice, st));
+    PSPH_TRY(to.add(r.pid, c->pid)); PSPH_TRY(to.add(r.refb, c->refb)); PSPH_TRY(to.add(r.ckey, c->key_a));
+    PSPH_TRY(to.add(r.bc, c->f.bc)); PSPH_TRY(to.add(r.phase, c->f.phase));
+    if (n) hipLaunchKernelGGL(k_fill_i32, blocks(n), 256, 0, st, (int *)r.gflag, 0, (int)n);
+    Copies cells{c, ncs}, tiles{c, ntb * 4};
+    PSPH_TRY(cells.add(r.cs, c->cs)); PSPH_TRY(cells.add(r.toff, c->toff));
+    PSPH_TRY(tiles.add((uint64_t *)r.tbox, (const uint64_t *)c->tbox));
+    PSPH_TRY(cells.flush());
+    PSPH_TRY(tiles.flush());
   } else if (stage == 1) {
     PSPH_TRY(cp(RF_V1X, c->f.vx)); PSPH_TRY(cp(RF_V1Y, c->f.vy)); PSPH_TRY(cp(RF_V1Z, c->f.vz));
     PSPH_TRY(cp(RF_E1, c->f.e));
@@ -928,21 +923,16 @@ static int rec_capture(psph_ctx *c, int stage, double dt) {
     // particles come after the first r.n); 5: after it
     if (!r.d[RF_BW] || !r.bcn) return fail(PSPH_EINVARIANT, "record: no wall-ghost fields");
     const size_t m = r.n;
-    auto cpm = [&](int f, const double *src) -> int {
-      if (m) HIP_TRY(hipMemcpyAsync(r.d[f], src, m * 8, hipMemcpyDeviceToDevice, st));
-      return 0;
-    };
     if (stage == 4) {
-      PSPH_TRY(cpm(RF_XN, c->f.x)); PSPH_TRY(cpm(RF_YN, c->f.y)); PSPH_TRY(cpm(RF_ZN, c->f.z));
-      if (m) {
-        HIP_TRY(hipMemcpyAsync(r.bcn, c->f.bc, m * 4, hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(k_fill_f64, blocks(m), 256, 0, st, r.d[RF_BW], -1.0, m);
-      }
+      PSPH_TRY(cp(RF_XN, c->f.x)); PSPH_TRY(cp(RF_YN, c->f.y)); PSPH_TRY(cp(RF_ZN, c->f.z));
+      PSPH_TRY(to.add(r.bcn, c->f.bc));
+      if (m) hipLaunchKernelGGL(k_fill_f64, blocks(m), 256, 0, st, r.d[RF_BW], -1.0, m);
     } else {
-      PSPH_TRY(cpm(RF_BRHO, c->f.rho)); PSPH_TRY(cpm(RF_BE, c->f.e)); PSPH_TRY(cpm(RF_BXI, c->f.xi));
-      PSPH_TRY(cpm(RF_BVX, c->f.vx)); PSPH_TRY(cpm(RF_BVY, c->f.vy)); PSPH_TRY(cpm(RF_BVZ, c->f.vz));
+      PSPH_TRY(cp(RF_BRHO, c->f.rho)); PSPH_TRY(cp(RF_BE, c->f.e)); PSPH_TRY(cp(RF_BXI, c->f.xi));
+      PSPH_TRY(cp(RF_BVX, c->f.vx)); PSPH_TRY(cp(RF_BVY, c->f.vy)); PSPH_TRY(cp(RF_BVZ, c->f.vz));
     }
   }
+  PSPH_TRY(to.flush());
   HIP_TRY(hipGetLastError());
   return 0;
 }

@@ -273,6 +273,18 @@ __device__ inline bool refb_adjacent(uint32_t a, uint32_t b) {
   return (a != kDead) & (b != kDead) & ((d & 0x7ffu) - 1024u <= 2u) & (((d >> 11) & 0x7ffu) - 1024u <= 2u) & ((d >> 22) <= 2u);
 }
 
+// copies of n8 arrays of 8 bytes an element and n4 of 4, n elements each
+__global__ void k_copy(uint32_t n, int n8, int n4, Moves mv) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+#pragma unroll
+  for (int k = 0; k < kMove8; k++)
+    if (k < n8) mv.d8[k][i] = mv.s8[k][i];
+#pragma unroll
+  for (int k = 0; k < kMove4; k++)
+    if (k < n4) mv.d4[k][i] = mv.s4[k][i];
+}
+
 // After the sort: cs[c] = first index whose cell (key >> sh) >= c, c in [0,
 // ncells]; the smoothing length at list time; the reference bucket.  Empty cells
 // that follow each other are filled by the whole wave (one lane alone took 11 us
@@ -2575,6 +2587,7 @@ struct psph_ctx {
   unsigned long long *seen = nullptr;    // their last copy, in pinned memory; then 2 words of lists' cursors
   char *up_h = nullptr, *up_d = nullptr; // particles on their way to the device (upload)
   bool up_busy = false;
+  bool loaded_removed = false;           // removed particles (bc < 0) among those loaded
   double *d_part = nullptr;
   // grid of the last neighbour search
   bool grid_valid = false;
@@ -2839,6 +2852,7 @@ extern "C" int psph_load(psph_ctx *c, const psph_soa *host, size_t n, double t0,
   if (!host->x || !host->rho || !host->m || !host->h || !host->bc) return fail(PSPH_EINVAL, "load: x, rho, m, h and bc are required");
   HostParticles P;
   P.from_soa(host, n);
+  c->loaded_removed = std::any_of(P.bc.begin(), P.bc.end(), [](int32_t b) { return b < 0; });
   PSPH_TRY(upload(c, P, 0));
   c->n = n;
   if (n) hipLaunchKernelGGL(k_iota_u32, blocks(n), 256, 0, c->stream, c->pid, 0u, (uint32_t)n);
@@ -2852,6 +2866,35 @@ extern "C" int psph_load(psph_ctx *c, const psph_soa *host, size_t n, double t0,
   c->grid_valid = false;
   return 0;
 }
+
+// Copies between device arrays of n elements, up to 18 in a launch (one each took
+// 650 launches, and 2.4 ms of GPU time, of the gradients of 6 steps).
+struct Copies {
+  psph_ctx *c;
+  size_t n;
+  Moves mv{};
+  int n8 = 0, n4 = 0;
+  template <class T>
+  int add(T *to, const T *from) {
+    static_assert(sizeof(T) == 8 || sizeof(T) == 4, "elements of 8 or 4 bytes");
+    if (sizeof(T) == 8) {
+      if (n8 == kMove8) PSPH_TRY(flush());
+      mv.s8[n8] = (const uint64_t *)from;
+      mv.d8[n8++] = (uint64_t *)to;
+    } else {
+      if (n4 == kMove4) PSPH_TRY(flush());
+      mv.s4[n4] = (const uint32_t *)from;
+      mv.d4[n4++] = (uint32_t *)to;
+    }
+    return 0;
+  }
+  int flush() {
+    if (n && (n8 || n4)) hipLaunchKernelGGL(k_copy, blocks(n), 256, 0, c->stream, (uint32_t)n, n8, n4, mv);
+    n8 = n4 = 0;
+    HIP_TRY(hipGetLastError());
+    return 0;
+  }
+};
 
 // live and real particles of bc[0..n)
 static int count_live(psph_ctx *c, size_t n, const int32_t *bc, unsigned long long cnt[2]) {
@@ -3122,6 +3165,11 @@ static int neighbors(psph_ctx *c, bool seen) {
   if (n) {
     hipLaunchKernelGGL(k_cellkey, blocks(n), 256, 0, s, n, frozen ? c->px : c->f.x, frozen ? c->py : c->f.y,
                        frozen ? c->pz : c->f.z, c->f.bc, g, c->key_a, c->idx_a);
+  }
+  // One cell, and nothing to drop: every key is equal, and a stable sort and the
+  // gather would leave all where it is (1D: 8 launches of 30 less).
+  const bool in_order = g.ncells == 1 && g.fbits == 0 && !dead && !c->loaded_removed;
+  if (n && !in_order) {
     int end_bit = 1;
     while (end_bit < 32 && ((uint64_t)1 << end_bit) <= ((uint64_t)g.ncells << (3 * g.fbits))) end_bit++;
     size_t bytes = 0;
