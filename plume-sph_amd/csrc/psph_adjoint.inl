@@ -993,14 +993,15 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
   const uint32_t ncells = g.ncells;
   hipStream_t s = c->stream;
   PSPH_TRY(adj_row_memory(c, A, n));
-  if (ncells + 1 > A.cell_cap) {
+  const size_t parts = cell_parts(n, ncells);
+  if (parts + 1 > A.cell_cap) {
     CellSum **arrs[] = {&A.cell_has, &A.cell_at};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
     A.cell_cap = 0;
-    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, ((size_t)ncells + 1) * sizeof(CellSum)));
-    A.cell_cap = (size_t)ncells + 1;
+    for (auto pp : arrs) PSPH_TRY(dmalloc((void **)pp, (parts + 1) * sizeof(CellSum)));
+    A.cell_cap = parts + 1;
   }
-  const size_t chunks_ub = n / kChunk + (size_t)ncells + 1;
+  const size_t chunks_ub = most_chunks(n, ncells);
   if (chunks_ub > A.chunk_cap) {
     uint32_t **arrs[] = {&A.cfirst, &A.ccount};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
@@ -1012,7 +1013,7 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
     PSPH_TRY(dmalloc((void **)&A.made, 2 * 8));
     hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, s, A.made, 0ull, 2);
   }
-  PSPH_TRY(fill_cells(c, ncells, R.cs, IsRow{R.bc, R.gflag}, A.cell_has, A.cell_at, nullptr, nullptr, R.d[RF_X], R.d[RF_Y],
+  PSPH_TRY(fill_cells(c, n, ncells, R.cs, IsRow{R.bc, R.gflag}, A.cell_has, A.cell_at, nullptr, nullptr, R.d[RF_X], R.d[RF_Y],
                       R.d[RF_Z], A.rows, A.cfirst, A.ccount, (uint32_t *)(A.made + 1)));
   HIP_TRY(hipGetLastError());
   return 0;
@@ -1022,7 +1023,7 @@ static int adj_rows(psph_ctx *c, Adjoint &A, const StepRec &R) {
 // the next search makes again)
 static int adj_lists(psph_ctx *c, Adjoint &A, const StepRec &R, const AdjCommon &pc, GroupLists &gl, uint32_t &ngroups) {
   c->lists_valid = false;
-  PSPH_TRY(group_memory(c, R.n / kChunk + (size_t)R.grid.ncells + 1));
+  PSPH_TRY(group_memory(c, most_chunks(R.n, R.grid.ncells)));
   hipLaunchKernelGGL(k_geom, blocks(R.n), 256, 0, c->stream, (uint32_t)R.n, pc.p.x, pc.p.y, pc.p.z, pc.h, c->gxy, c->gzh,
                      A.made);
   const ListOf of{R.n, R.grid.ncells, pc.h, R.hmax, A.made, true};

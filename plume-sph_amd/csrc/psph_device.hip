@@ -75,6 +75,8 @@ enum Word {
   W_ERR_RHS, W_ERR_DENS, W_ERR_VSM,   // their own, and of the passes whose errors a step reads at its end
   W_VMAX,                     // bits of the largest speed
   W_OVER, W_ITERS,            // lists that found no room since the last check; iterations of the adaptive h done
+  W_ITER_CURSOR,              // and the cursors of their lists
+  W_ITER_LAST = W_ITER_CURSOR + 7,
   W_COUNT
 };
 // an earlier stage of this step failed (n error words from err): the stages
@@ -682,50 +684,55 @@ struct IsTarget {
   __device__ bool operator()(uint32_t i) const { return need_neigh(bc[i]); }
 };
 
-// One workgroup per cell (k_cell_counts: and one more, zero): a wavefront where
-// there is a grid, kOneCell threads where one cell holds everything.
-constexpr int kOneCell = 1024;
-template <class T>
-__global__ __launch_bounds__(kOneCell) void k_cell_counts(uint32_t ncells, const uint32_t *cs, T is, CellSum *out) {
-  __shared__ uint32_t part[kOneCell / kWave];
-  const uint32_t cell = blockIdx.x;
-  const uint32_t lo = cs[cell], hi = cell < ncells ? cs[cell + 1] : lo;
-  uint32_t cnt = 0;
-  for (uint32_t i = lo + threadIdx.x; i < hi; i += blockDim.x) cnt += is(i) ? 1u : 0u;
-  for (int o = kWave / 2; o > 0; o >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, o);
-  if (blockDim.x > kWave) {
-    if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = cnt;
-    __syncthreads();
-    cnt = 0;
-    for (uint32_t w = 0; w < blockDim.x / kWave; w++) cnt += part[w];
+// The particles of part p, one wavefront's: the cell p, or, where one cell holds
+// everything, its kRun particles from p kRun on (a workgroup of 1024 for the whole
+// cell took 80 us at 6.9k particles, 15 us so).  Tiles, chunks and runs start anew
+// in each part, which is on their bounds where it is kRun particles.
+__device__ inline void part_range(uint32_t p, uint32_t parts, bool one_cell, const uint32_t *cs, uint32_t &lo, uint32_t &hi) {
+  if (one_cell) {
+    lo = min(p * (uint32_t)kRun, cs[1]);
+    hi = min(lo + (uint32_t)kRun, cs[1]);
+  } else {
+    lo = cs[p];
+    hi = p < parts ? cs[p + 1] : lo;
   }
-  if (threadIdx.x == 0) out[cell] = CellSum{(hi - lo + kWave - 1) / kWave, cnt, (cnt + kChunk - 1) / kChunk};
 }
 
-// The cell's tiles with their boxes, rounded outwards to float: [lo, hi] per tile,
+// (One part more, empty, for the scan.)
+template <class T>
+__global__ __launch_bounds__(kWave) void k_cell_counts(uint32_t parts, bool one_cell, const uint32_t *cs, T is, CellSum *out) {
+  uint32_t lo, hi;
+  part_range(blockIdx.x, parts, one_cell, cs, lo, hi);
+  if (blockIdx.x == parts) hi = lo;
+  uint32_t cnt = 0;
+  for (uint32_t i = lo + threadIdx.x; i < hi; i += kWave) cnt += is(i) ? 1u : 0u;
+  for (int o = kWave / 2; o > 0; o >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, o);
+  if (threadIdx.x == 0) out[blockIdx.x] = CellSum{(hi - lo + kWave - 1) / kWave, cnt, (cnt + kChunk - 1) / kChunk};
+}
+
+// The part's tiles with their boxes, rounded outwards to float: [lo, hi] per tile,
 // and in the w components the bits of its first particle and its particle count
 // (toff null: not these); its targets, in the order of the passes; its chunks.
 // (Counts, scans and lists in kernels of their own over particles, tiles and cells:
 // 15 launches of a search; so 5.)
 template <class T>
-__global__ __launch_bounds__(kOneCell) void k_cell_fill(uint32_t ncells, const uint32_t *cs, T is, const CellSum *sums,
-                                                        uint32_t *toff, float4 *tbox, const double *x, const double *y,
-                                                        const double *z, uint32_t *targets, uint32_t *cfirst,
-                                                        uint32_t *ccount, uint32_t *nchunks) {
-  extern __shared__ __align__(16) char lds[];      // an OrderLds per wave
-  __shared__ uint32_t part[kOneCell / kWave];
-  const uint32_t cell = blockIdx.x, lane = threadIdx.x % kWave;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), nw = blockDim.x / kWave;
-  const uint32_t lo = cs[cell], hi = cs[cell + 1];
-  const CellSum at = sums[cell], to = sums[cell + 1];
-  if (threadIdx.x == 0) {
-    if (toff) toff[cell] = at.tiles;
-    if (cell == ncells - 1) {
-      if (toff) toff[ncells] = to.tiles;
+__global__ __launch_bounds__(kWave) void k_cell_fill(uint32_t parts, bool one_cell, const uint32_t *cs, T is,
+                                                     const CellSum *sums, uint32_t *toff, float4 *tbox, const double *x,
+                                                     const double *y, const double *z, uint32_t *targets,
+                                                     uint32_t *cfirst, uint32_t *ccount, uint32_t *nchunks) {
+  __shared__ __align__(16) OrderLds order;
+  const uint32_t part = blockIdx.x, lane = threadIdx.x;
+  uint32_t lo, hi;
+  part_range(part, parts, one_cell, cs, lo, hi);
+  const CellSum at = sums[part], to = sums[part + 1];
+  if (lane == 0) {
+    if (toff && (!one_cell || part == 0)) toff[part] = at.tiles;
+    if (part == parts - 1) {
+      if (toff) toff[one_cell ? 1u : parts] = to.tiles;
       *nchunks = to.chunks;
     }
   }
-  for (uint32_t t = at.tiles + wave; toff && t < to.tiles; t += nw) {
+  for (uint32_t t = at.tiles; toff && t < to.tiles; t++) {
     const uint32_t base = lo + kWave * (t - at.tiles), end = min(hi, base + kWave);
     const uint32_t j = base + lane < end ? base + lane : base;
     const double px = x[j], py = y[j], pz = z[j];
@@ -739,34 +746,21 @@ __global__ __launch_bounds__(kOneCell) void k_cell_fill(uint32_t ncells, const u
   }
   const uint32_t nt = to.targets - at.targets;
   if (!nt) return;
-  for (uint32_t q = threadIdx.x; q < to.chunks - at.chunks; q += blockDim.x) {
+  for (uint32_t q = lane; q < to.chunks - at.chunks; q += kWave) {
     cfirst[at.chunks + q] = at.targets + q * kChunk;
     ccount[at.chunks + q] = min((uint32_t)kChunk, nt - q * kChunk);
   }
   uint32_t next = at.targets;
-  for (uint32_t i0 = lo; i0 < hi; i0 += blockDim.x) {
-    const uint32_t i = i0 + threadIdx.x;
-    const bool mine = i < hi && is(i);
+  for (uint32_t i0 = lo; i0 < hi; i0 += kWave) {
+    const bool mine = i0 + lane < hi && is(i0 + lane);
     const uint64_t m = __ballot(mine);
-    uint32_t before = 0, all = (uint32_t)__popcll(m);
-    if (nw > 1) {
-      if (lane == 0) part[wave] = all;
-      __syncthreads();
-      all = 0;
-      for (uint32_t w = 0; w < nw; w++) {
-        if (w < wave) before += part[w];
-        all += part[w];
-      }
-      __syncthreads();
-    }
-    if (mine) targets[next + before + lanes_below(m)] = i;
-    next += all;
+    if (mine) targets[next + lanes_below(m)] = i0 + lane;
+    next += (uint32_t)__popcll(m);
   }
   __threadfence_block();
-  __syncthreads();                                 // the cell's targets are there
-  OrderLds &o = ((OrderLds *)lds)[wave];
-  for (uint32_t t0 = wave * kRun; t0 < nt; t0 += nw * kRun)
-    if (nt - t0 > (uint32_t)kGroup) order_run(lane, min((uint32_t)kRun, nt - t0), x, y, z, targets + at.targets + t0, o);
+  __syncthreads();                                 // the part's targets are there
+  for (uint32_t t0 = 0; t0 < nt; t0 += kRun)
+    if (nt - t0 > (uint32_t)kGroup) order_run(lane, min((uint32_t)kRun, nt - t0), x, y, z, targets + at.targets + t0, order);
 }
 
 // The tiles a group visits, with a 64-bit mask of the particles that can be a
@@ -3049,6 +3043,10 @@ static int reduce_hmax(psph_ctx *c) {
   return read_words(c);
 }
 
+// parts that the cells of n particles are filled in, and their chunks at most
+static size_t cell_parts(size_t n, size_t ncells) { return ncells == 1 ? n / kRun + 1 : ncells; }
+static size_t most_chunks(size_t n, size_t ncells) { return n / kChunk + cell_parts(n, ncells) + 1; }
+
 // hmax: the largest h of the live particles
 static int build_grid(psph_ctx *c, double hmax) {
   const psph_config &k = c->cfg;
@@ -3084,7 +3082,7 @@ static int build_grid(psph_ctx *c, double hmax) {
   while (cbits < 32 && ((uint64_t)1 << cbits) <= (uint64_t)g.ncells) cbits++;
   g.fbits = g.inv_e > 0 ? std::min(4, (32 - cbits) / 3) : 0;
   c->grid = g;
-  size_t need = (size_t)g.ncells + 1;
+  size_t need = std::max((size_t)g.ncells, cell_parts(c->n, g.ncells)) + 1;
   if (need > c->cs_cap) {
     uint32_t **arrs[] = {&c->cs, &c->toff};
     for (auto pp : arrs) { if (*pp) hipFree(*pp); *pp = nullptr; }
@@ -3096,7 +3094,7 @@ static int build_grid(psph_ctx *c, double hmax) {
     c->cs_cap = need;
   }
   const size_t ub = c->n / kWave + (size_t)g.ncells + 1;
-  const size_t cub_ = c->n / kChunk + (size_t)g.ncells + 1;
+  const size_t cub_ = most_chunks(c->n, g.ncells);
   if (ub > c->tile_cap) {
     if (c->tbox) hipFree(c->tbox);
     c->tbox = nullptr;
@@ -3124,19 +3122,20 @@ static int excl_scan(psph_ctx *c, const uint32_t *in, uint32_t *out, size_t n1) 
 }
 
 // The contents of the cells that cs bounds: tiles (toff not null), targets (is)
-// and their chunks.  has, at: ncells + 1 sums each.
+// and their chunks.  has, at: cell_parts + 1 sums each.
 template <class T>
-static int fill_cells(psph_ctx *c, uint32_t ncells, const uint32_t *cs, T is, CellSum *has, CellSum *at, uint32_t *toff,
-                      float4 *tbox, const double *x, const double *y, const double *z, uint32_t *targets,
+static int fill_cells(psph_ctx *c, size_t n, uint32_t ncells, const uint32_t *cs, T is, CellSum *has, CellSum *at,
+                      uint32_t *toff, float4 *tbox, const double *x, const double *y, const double *z, uint32_t *targets,
                       uint32_t *cfirst, uint32_t *ccount, uint32_t *nchunks) {
-  const unsigned threads = ncells == 1 ? kOneCell : kWave;
-  hipLaunchKernelGGL((k_cell_counts<T>), ncells + 1, threads, 0, c->stream, ncells, cs, is, has);
+  const bool one = ncells == 1;
+  const uint32_t parts = (uint32_t)cell_parts(n, ncells);
+  hipLaunchKernelGGL((k_cell_counts<T>), parts + 1, kWave, 0, c->stream, parts, one, cs, is, has);
   size_t bytes = 0;
-  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)ncells + 1, c->stream));
+  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(nullptr, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)parts + 1, c->stream));
   PSPH_TRY(ensure_cub(c, bytes));
-  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(c->cub, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)ncells + 1, c->stream));
-  hipLaunchKernelGGL((k_cell_fill<T>), ncells, threads, threads / kWave * sizeof(OrderLds), c->stream, ncells, cs, is, at,
-                     toff, tbox, x, y, z, targets, cfirst, ccount, nchunks);
+  HIP_TRY(hipcub::DeviceScan::ExclusiveScan(c->cub, bytes, has, at, CellAdd(), CellSum{0, 0, 0}, (int)parts + 1, c->stream));
+  hipLaunchKernelGGL((k_cell_fill<T>), parts, kWave, 0, c->stream, parts, one, cs, is, at, toff, tbox, x, y, z, targets,
+                     cfirst, ccount, nchunks);
   HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -3240,7 +3239,7 @@ static int neighbors(psph_ctx *c, bool seen) {
   hipLaunchKernelGGL(k_sorted, blocks((size_t)n + 1), 256, 0, s, n, c->key_a, 3 * g.fbits, g.ncells, c->cs, qx, qy, qz,
                      c->f.h, rb, c->refb, c->h_list);
   // tiles, targets and their chunks (<= kChunk consecutive targets of one cell)
-  PSPH_TRY(fill_cells(c, g.ncells, c->cs, IsTarget{c->f.bc}, c->cell_has, c->cell_at, c->toff, c->tbox, qx, qy, qz,
+  PSPH_TRY(fill_cells(c, n, g.ncells, c->cs, IsTarget{c->f.bc}, c->cell_has, c->cell_at, c->toff, c->tbox, qx, qy, qz,
                       c->targets, c->cfirst, c->ccount, c->nchunks));
   HIP_TRY(hipGetLastError());
   tm.stop();
@@ -3295,17 +3294,17 @@ static PairCommon make_common(psph_ctx *c, double reach) {
   return pc;
 }
 
-// workgroups for a pair pass: an upper bound on the chunks of csz targets
-// (each cell may add a partial chunk), padded so that kXcds * ceil(nchunks /
+// workgroups for a pair pass: an upper bound on the chunks (each part of the
+// cells may add a partial chunk), padded so that kXcds * ceil(nchunks /
 // kXcds) exist
-static unsigned chunk_grid(size_t n, size_t ncells, size_t csz) {
-  size_t ub = n / csz + ncells + 1 + kXcds;
+static unsigned chunk_grid(size_t n, size_t ncells) {
+  size_t ub = most_chunks(n, ncells) + kXcds;
   return (unsigned)((ub + kXcds - 1) / kXcds * kXcds);
 }
 
 static void launch_list(psph_ctx *c, double reach, uint32_t *count, const uint32_t *offset, uint32_t *out) {
   const PairCommon pc = make_common(c, reach);
-  const unsigned nb = chunk_grid(c->n, c->grid.ncells, kChunk);
+  const unsigned nb = chunk_grid(c->n, c->grid.ncells);
   if (c->cfg.dim == 3) hipLaunchKernelGGL(k_list<3>, nb, kWave, 0, c->stream, pc, count, offset, out);
   else hipLaunchKernelGGL(k_list<1>, nb, kWave, 0, c->stream, pc, count, offset, out);
 }
@@ -3359,7 +3358,7 @@ static int launch_lists(psph_ctx *c, const PairCommon &pc, const ListOf &of, dou
   // a group per wave up to a quarter of a million particles: at 77k 0.15 ms against
   // 0.20 with half a chunk; a chunk per wave beyond
   const uint32_t nsplit = of.n < (1u << 18) ? kGroupsPerChunk : 1;
-  const unsigned G = chunk_grid(of.n, of.ncells, kChunk) * nsplit;
+  const unsigned G = chunk_grid(of.n, of.ncells) * nsplit;
   GroupCommon gc = group_common(c);
   gc.c_smooth = c_smooth;
   gc.done = done;
@@ -3549,11 +3548,14 @@ extern "C" int psph_adapt_h(psph_ctx *c) {
         pass(nullptr);
       }
       it++;
-      if (it < k.num_loop) hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, over, 0ull, 2);
+      if (it < k.num_loop) hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, over, 0ull, W_ITER_LAST + 1 - W_OVER);
       for (int64_t q = it; q < k.num_loop; q++) {
         StageTimer tm(c, 2);
-        hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, of.cursor, 0ull, 1);
-        PSPH_TRY(launch_lists(c, pc, of, k.c_smooth, c->usp, over));
+        ListOf next = of;
+        next.cursor = c->words + std::min<int64_t>(W_ITER_CURSOR + (q - it), W_ITER_LAST);
+        if (W_ITER_CURSOR + (q - it) > W_ITER_LAST)
+          hipLaunchKernelGGL(k_fill_u64, 1, 64, 0, c->stream, next.cursor, 0ull, 1);
+        PSPH_TRY(launch_lists(c, pc, next, k.c_smooth, c->usp, over));
         pass(over);
       }
       HIP_TRY(hipGetLastError());
