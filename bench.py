@@ -108,8 +108,7 @@ def strong_leg(args):
     # adjoint's own arrays, visit lists and checkpoints take much of the rest
     per_step = 264.0 * S.capacity
     # the segment of step records takes at most 30 % of the free HBM: the
-    # reverse sweep's two-role visit masks (512 B per visit, ~100 GB at 16M)
-    # and the checkpoints need the rest
+    # checkpoints and the reverse sweep's own arrays and lists need the rest
     K = int(max(1, min(args.strong_adjoint, 0.30 * free / per_step)))
     if args.strong_ckpt > 0:
         K = min(K, args.strong_ckpt)

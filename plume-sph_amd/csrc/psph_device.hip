@@ -1344,7 +1344,7 @@ struct RhsArgs {
 // The FP32-pair form keeps the pressure term m_j (p_j/rho_j^2 + p_i/rho_i^2)
 // grad W in FP64: in air near hydrostatic balance its pair terms cancel to
 // about 1 % of their size, and FP32 rounding there is what the velocities
-// feel.  The kernel value comes from the exp table (FP64 at FP32-like cost);
+// feel.  The kernel value is FP64 (exp_neg, or the FP32 instruction in FX);
 // viscosity, heat conduction and the energy work terms stay FP32.
 // -2 pi^(-D/2): grad W = G dx with G = -2 W / h^2 = kGradNorm h^-(D+2) exp(-r^2/h^2)
 template <int D> constexpr double kGradNorm = -2.0 * kInvSqrtPi * kInvSqrtPi * kInvSqrtPi;
@@ -1607,7 +1607,7 @@ template <> constexpr double kNorm<1> = kInvSqrtPi;
 // does not contribute (contr_dens false or another phase) stages zero masses
 // and mr = 0, so its terms are exact zeros and no pair tests for it.
 // The FP32-pair form evaluates the density and energy-smoothing weights in
-// FP64 with the exp table: the pressure gradient of the next step amplifies
+// FP64: the pressure gradient of the next step amplifies
 // relative errors of rho and e by its cancellation.
 template <class R, bool MIXED = std::is_same<R, float>::value, bool FX = false>
 struct DensPass {
@@ -1759,7 +1759,7 @@ struct VsmArgs {
   Packs pk;
 };
 
-// The FP32-pair form evaluates the filter weights in FP64 from the exp table
+// The FP32-pair form evaluates the filter weights in FP64
 // (kernel argument, exponential, m_j / rho_j): sv moves the particles, and
 // FP32 weights (relative error ~3e-7, dominated by the rounding of s^2 and of
 // h) made the velocity filter the largest source of FP32-vs-FP64 difference,
