@@ -340,9 +340,11 @@ int psph_conservation_noalloc(const psph_soa *dev, size_t n, int32_t dim, double
  * ghosts present at the start (bc 0) are taken to hold the vent state of the
  * config, as psph_gen_plume makes them.
  * The forward run stores a checkpoint every ckpt_every steps; the reverse
- * sweep recomputes one segment at a time from its checkpoint.  grad_v and
- * grad_sv (either may be NULL) receive dH/dv and dH/dsv of the starting
- * state, 3 per particle, in psph_read order of that state (n_cap particles
+ * sweep recomputes one segment at a time from its checkpoint.  As many of the
+ * last segments as 30 % of the free device memory holds keep their records from
+ * the forward run and are not recomputed (the context holds them until
+ * psph_destroy).  grad_v and grad_sv (either may be NULL) receive dH/dv and
+ * dH/dsv of the starting state, 3 per particle, in psph_read order of that state (n_cap particles
  * at most).  On return the context holds the state after nsteps steps, and
  * the recorded schedule stays available to psph_replay_run. */
 typedef struct psph_adjoint_out {

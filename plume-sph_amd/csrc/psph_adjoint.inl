@@ -1414,18 +1414,30 @@ extern "C" int psph_adjoint_run(psph_ctx *c, int64_t nsteps, int64_t ckpt_every,
   const int64_t K = std::min(ckpt_every, nsteps);
   const int64_t nseg = (nsteps + K - 1) / K;
   if ((int64_t)A.ck.size() < nseg) A.ck.resize(nseg);
-  if ((int64_t)A.recs.size() < K) A.recs.resize(K);
   // Segments of K steps, the shorter one (if any) first: the last segment is
   // reversed straight from the recorded run, the others are recomputed from
   // their checkpoints, so a full last segment recomputes the fewest steps.
   const int64_t first_len = nsteps - (nseg - 1) * K;
   auto seg_begin = [&](int64_t seg) { return seg == 0 ? (int64_t)0 : first_len + (seg - 1) * K; };
-  const int64_t last0 = seg_begin(nseg - 1);
+  // As many of the last segments as 30 % of the free HBM holds (at least one, as
+  // asked for) are recorded in the forward run and not recomputed: a recorded step
+  // tests every pair's membership and costs half as much again as a plain one.
+  int64_t kept = nseg - 1;
+  {
+    size_t free_b = 0, total_b = 0, held = 0;
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    for (const StepRec &r : A.recs) held += r.cap ? 1 : 0;
+    const double per = (double)c->cap * ((k.wall_bc ? RF_N : RF_NBASE) * 8.0 + 7 * 4.0);
+    const int64_t fit = (int64_t)std::min(0.30 * ((double)free_b / per + (double)held), 1e9);
+    while (kept > 0 && nsteps - seg_begin(kept - 1) <= fit) kept--;
+  }
+  const int64_t rec0 = seg_begin(kept);
+  if ((int64_t)A.recs.size() < std::max(K, nsteps - rec0)) A.recs.resize(std::max(K, nsteps - rec0));
   int rc = 0;
   for (int64_t s = 0, seg = 0; s < nsteps && !rc; s++) {
     if (seg < nseg && s == seg_begin(seg)) rc = snap_save(c, A.ck[seg++]);
     if (rc) break;
-    c->rec = s >= last0 ? &A.recs[s - last0] : nullptr;
+    c->rec = s >= rec0 ? &A.recs[s - rec0] : nullptr;
     rc = psph_step(c, nullptr);
   }
   c->rec = nullptr;
@@ -1463,7 +1475,7 @@ extern "C" int psph_adjoint_run(psph_ctx *c, int64_t nsteps, int64_t ckpt_every,
   tp.mode = 2;
   for (int64_t seg = nseg - 1; seg >= 0 && !rc; seg--) {
     const int64_t s0 = seg_begin(seg), s1 = seg + 1 < nseg ? seg_begin(seg + 1) : nsteps;
-    if (seg != nseg - 1) {
+    if (seg < kept) {
       rc = snap_load(c, A.ck[seg]);
       for (int64_t s = s0; s < s1 && !rc; s++) {
         c->rec = &A.recs[s - s0];
@@ -1471,7 +1483,7 @@ extern "C" int psph_adjoint_run(psph_ctx *c, int64_t nsteps, int64_t ckpt_every,
       }
       c->rec = nullptr;
     }
-    for (int64_t s = s1 - 1; s >= s0 && !rc; s--) rc = reverse_step(c, A, A.recs[s - s0], th);
+    for (int64_t s = s1 - 1; s >= s0 && !rc; s--) rc = reverse_step(c, A, A.recs[s - (seg < kept ? s0 : rec0)], th);
   }
   c->rec = nullptr;
   if (!rc) rc = check_err(c, "adjoint");
