@@ -32,8 +32,10 @@ struct BucketGeom {
 constexpr uint32_t kOccReal = 16;   // beyond the host's OCC_* bits: a real particle
 
 // OR of the occupancy bits of every live particle into its bucket.  The
-// particles are in cell order, so a wave's lanes usually share a bucket:
-// they combine their bits first and one lane does the atomic.
+// particles are in cell order, so a wave's lanes share a few buckets: each
+// bucket's bits are combined first, and one lane does the atomic if it sets a bit
+// that is not there yet.  (An atomic a lane where a wave has more than one bucket:
+// 99 us at 51k-98k particles, the atomics on a bucket taking their turns; so 12.)
 __global__ void k_bucket_occ(uint32_t n, const double *x, const double *y, const double *z, const int32_t *bc,
                              const int32_t *inv, BucketGeom g, uint32_t *occ) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -47,12 +49,17 @@ __global__ void k_bucket_occ(uint32_t n, const double *x, const double *y, const
           ((b == 100 || b == 99) ? kOccReal : 0u);
     }
   }
-  const int64_t q0 = __shfl(q, 0);
-  if (__all(q == q0)) {
-    for (int o = 32; o > 0; o >>= 1) f |= (uint32_t)__shfl_xor((int)f, o);
-    if ((threadIdx.x & (kWave - 1)) == 0 && q0 >= 0 && f) atomicOr(occ + q0, f);
-  } else if (q >= 0) {
-    atomicOr(occ + q, f);
+  uint64_t left = __ballot(q >= 0);
+  while (left) {
+    const int l = __builtin_ctzll(left);
+    const int64_t ql = __shfl(q, l);
+    const bool same = q == ql;
+    uint32_t bits = 0;
+    for (int b = 0; b < 5; b++) bits |= __ballot(same && ((f >> b) & 1u)) ? 1u << b : 0u;
+    if ((int)(threadIdx.x & (kWave - 1)) == l &&
+        (__hip_atomic_load(occ + ql, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bits) != bits)
+      atomicOr(occ + ql, bits);
+    left &= ~__ballot(same);
   }
 }
 
